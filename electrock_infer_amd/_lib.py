@@ -46,6 +46,7 @@ EXPORTED_SYMBOLS = (
 # every function include/electrock_decoder.h declares
 DECODER_SYMBOLS = (
     "ed_version", "ed_embed", "ed_residual_norm", "ed_relu_squared", "ed_silu_gate", "ed_gated_norm", "ed_token_gate", "ed_skinny_gemm_splits", "ed_skinny_gemm",
+    "ed_decode_gemm_splits", "ed_decode_gemm_plain_pays", "ed_decode_gemm",
     "ed_token_side_supported", "ed_token_side", "ed_gla_prefill", "ed_gla_step",
     "ed_recur_record", "ed_recur_prefill", "ed_recur_step",
     "ed_attn_row_elems", "ed_attn_prepare", "ed_attn_paged", "ed_attn_prompt_supported", "ed_attn_prompt",
@@ -196,6 +197,9 @@ def load_decoder() -> ctypes.CDLL:
         "ed_embed": [vp, vp, dbl, vp, vp, i64, i64, i32, i32, vp],
         "ed_skinny_gemm_splits": [i64, i32, i32],
         "ed_skinny_gemm": [vp, vp, vp, i32, i32, i64, i32, i32, i32, vp],
+        "ed_decode_gemm_splits": [i64, i32, i32],
+        "ed_decode_gemm_plain_pays": [i64, i32, i32],
+        "ed_decode_gemm": [vp, vp, vp, i32, i32, i64, i32, i32, i32, vp],
         "ed_residual_norm": [i32, vp, vp, i32, i32, vp, vp, vp, i64, i64, i32, dbl, i32, vp],
         "ed_relu_squared": [vp, i64, i32, vp],
         "ed_silu_gate": [vp, vp, i64, i32, i32, vp],

@@ -187,9 +187,19 @@ int ed_skinny_gemm_splits(int64_t T, int N, int K) { return skinny_supported(T, 
 
 int ed_skinny_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
                    void* stream) {
+    if (dtype_ok(out_dtype) && T != 0 && !skinny_supported(T, N, K)) return EM_ERR_UNSUPPORTED;
+    return ed_decode_gemm(x, w, out, out_dtype, splits, T, N, K, act, stream);
+}
+
+int ed_decode_gemm_splits(int64_t T, int N, int K) { return decode_gemm_supported(T, N, K) ? skinny_splits(static_cast<int>(T), N, K) : 0; }
+
+int ed_decode_gemm_plain_pays(int64_t T, int N, int K) { return decode_gemm_supported(T, N, K) && decode_gemm_plain_pays(T, N, K) ? 1 : 0; }
+
+int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
+                   void* stream) {
     if (!dtype_ok(out_dtype)) return EM_ERR_BAD_DTYPE;
     if (T == 0) return 0;
-    if (!skinny_supported(T, N, K)) return EM_ERR_UNSUPPORTED;
+    if (!decode_gemm_supported(T, N, K)) return EM_ERR_UNSUPPORTED;
     if (splits < 1 || splits > 64 || splits > K / 64 || act < 0 || act > 2 ||
         (splits > 1 && (act != 0 || out_dtype != EM_DTYPE_F32)) || (act == 2 && out_dtype != EM_DTYPE_BF16))
         return EM_ERR_BAD_SHAPE;

@@ -1,154 +1,216 @@
 // out[T, N] = act(x[T, K] w[N, K]^T) for a decode batch (T <= 64), bf16: a stream over the weights.
 //
-// A workgroup owns 16 * NT columns of one of `splits` ranges of K; its eight waves share that range out, add their
-// results up in LDS, and one pass applies the activation and stores.  A wave reads the weights straight into MFMA operands: per
-// 64 elements of k a lane takes 32 consecutive bytes of one row (lane / 16 picks them, so that four lanes cover a
-// 128-byte line), for which the k order inside the step is permuted -- the token rows are read in the same order, and a
-// sum does not care.  The loads of four such steps are in flight at once.  With splits > 1 the results are float32
-// partial sums [splits, T, N] that the next kernel adds up.  GLU: w is [2 N, K], a workgroup makes 16 columns of both
-// halves and stores silu(first) * second.
+// A workgroup owns 16 * NT columns of one of `splits` ranges of K; its waves share that range out, add their results up
+// in LDS, and one pass applies the activation and stores.  Bound: the weights' bytes, and for the small matrices of a
+// layer the way from a launch to the first bytes.
+//
+// Per 64 elements of k a wave loads eight rows of 128 bytes with one instruction, eight lanes side by side on a row,
+// of the weights and of the token rows alike, and turns both into MFMA operands through a stretch of LDS of its own (pitch
+// 144 bytes: no conflicts).  Loads straight in operand layout touch sixteen half-used lines each, and the address unit, not
+// the memory, sets the pace: with 64 token rows 2048 x 4096 took 23 us that way and takes 7.5 (library: 14), with one
+// 6.5 and now 5.1.  The weights, read once, are loaded past the caches' order of use (non-temporal).  Two steps
+// are in flight per wave; requesting the next two while these are multiplied was 5-15 % slower (half the waves fit).
+// With splits > 1 the results are float32 partial sums [splits, T, N] that the next kernel adds up.  GLU: w is [2 N, K],
+// a workgroup makes the same columns of both halves and stores silu(first) * second.
 #include "decoder.h"
 #include "mma.h"
 
 namespace em {
 namespace {
 
-constexpr int kWaves = 8;
 constexpr int kStepK = 64;
-constexpr int kAhead = 4;
+constexpr int kPitch = kStepK + 8;       // elements of a row in LDS
+constexpr int kSplitGroups = 256;        // a workgroup of eight waves takes a CU
 
-template <int MT, int NT, bool F32OUT, bool GLU = false>
-__global__ __launch_bounds__(kWaves * kWave, 2) void skinny_gemm_kernel(const uint16_t* __restrict__ x,
-                                                                        const uint16_t* __restrict__ w, void* __restrict__ out,
-                                                                        int T, int N, int K, int act) {
+__device__ __forceinline__ u32x4_t load_once(const uint16_t* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+}
+__device__ __forceinline__ bf16x8_t as_frag(u32x4_t w) {
+    bf16x8_t f;
+    __builtin_memcpy(&f, &w, 16);
+    return f;
+}
+
+template <int MT, int NT, int WAVES>
+constexpr int skinny_lds() {
+    constexpr int stage = WAVES * (MT + NT) * 16 * kPitch * 2, sums = WAVES * 16 * MT * (16 * NT + 4) * 4;
+    return stage > sums ? stage : sums;
+}
+
+// MT: tiles of 16 tokens; NT: tiles of 16 weight rows; AHEAD: steps of k in flight
+template <int MT, int NT, int WAVES, int AHEAD, bool F32OUT, bool GLU>
+__global__ __launch_bounds__(WAVES * kWave) void skinny_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                                    void* __restrict__ out, int T, int N, int K, int act) {
     typedef Mma<BF16Elem> M;
-    constexpr int kCols = 16 * NT, kTile = 16 * MT * kCols, kOutCols = GLU ? 16 : kCols;
-    __shared__ float red[kWaves][kTile];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+    static_assert(!GLU || NT % 2 == 0, "tiles of both halves");
+    constexpr int kCols = 16 * NT, kOutCols = GLU ? kCols / 2 : kCols, kSumPitch = kCols + 4;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4, l8 = lane >> 3, c8 = (lane & 7) * 8;
+    uint16_t* xs = reinterpret_cast<uint16_t*>(lds) + wave * (MT + NT) * 16 * kPitch;
+    uint16_t* ws = xs + MT * 16 * kPitch;
     const int n0 = blockIdx.x * kOutCols;
     const int steps = K / kStepK, splits = gridDim.y, split = blockIdx.y;
     const int g0 = static_cast<int>(static_cast<int64_t>(steps) * split / splits);
     const int g1 = static_cast<int>(static_cast<int64_t>(steps) * (split + 1) / splits);
-    const int s0 = g0 + (g1 - g0) * wave / kWaves, s1 = g0 + (g1 - g0) * (wave + 1) / kWaves;
-
-    const uint16_t* wr[NT];
+    const int s0 = g0 + (g1 - g0) * wave / WAVES, s1 = g0 + (g1 - g0) * (wave + 1) / WAVES, last = max(s1 - 1, 0);
+    const uint16_t* wr[NT][2];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-        const int c = n0 + (GLU ? 0 : n * 16) + l16;
-        wr[n] = w + (static_cast<int64_t>(c < N ? c : N - 1) + (GLU ? n * static_cast<int64_t>(N) : 0)) * K + lq * 16;   // (columns beyond N are not stored)
-    }
-    const uint16_t* xr[MT];
+    for (int n = 0; n < NT; ++n)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int t = m * 16 + l16;
-        xr[m] = x + static_cast<int64_t>(t < T ? t : T - 1) * K + lq * 16;
-    }
+        for (int h = 0; h < 2; ++h) {
+            const int c = n0 + (GLU ? n / 2 : n) * 16 + h * 8 + l8;      // (columns beyond N are not stored)
+            wr[n][h] = w + (static_cast<int64_t>(c < N ? c : N - 1) + (GLU ? (n & 1) * static_cast<int64_t>(N) : 0)) * K + c8;
+        }
+    const uint16_t* xr[MT][2];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) xr[m][h] = x + static_cast<int64_t>(min(m * 16 + h * 8 + l8, T - 1)) * K + c8;
     f32x4_t acc[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s = s0; s < s1; s += kAhead) {
-        typename M::frag fw[kAhead][NT][2];
+    for (int s = s0; s < s1; s += AHEAD) {
+        // (a step behind the last is the last one again, so that the waits count loads in a straight line)
+        u32x4_t fw[AHEAD][NT][2], fx[AHEAD][MT][2];
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u)
-            if (s + u < s1) {
+        for (int u = 0; u < AHEAD; ++u)
 #pragma unroll
-                for (int n = 0; n < NT; ++n) {
-                    fw[u][n][0] = M::load(wr[n] + (s + u) * kStepK);
-                    fw[u][n][1] = M::load(wr[n] + (s + u) * kStepK + 8);
-                }
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) fw[u][n][h] = load_once(wr[n][h] + min(s + u, last) * kStepK);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) fx[u][m][h] = *reinterpret_cast<const u32x4_t*>(xr[m][h] + min(s + u, last) * kStepK);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            if (s + u >= s1) continue;
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4_t*>(ws + (n * 16 + h * 8 + l8) * kPitch + c8) = fw[u][n][h];
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4_t*>(xs + (m * 16 + h * 8 + l8) * kPitch + c8) = fx[u][m][h];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (the stretch is this wave's own)
+            typename M::frag ax[MT][2], aw[NT][2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) ax[m][h] = as_frag(*reinterpret_cast<const u32x4_t*>(xs + (m * 16 + l16) * kPitch + h * 32 + lq * 8));
+#pragma unroll
+                for (int n = 0; n < NT; ++n) aw[n][h] = as_frag(*reinterpret_cast<const u32x4_t*>(ws + (n * 16 + l16) * kPitch + h * 32 + lq * 8));
             }
-        typename M::frag fx[kAhead][MT][2];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u)
-            if (s + u < s1) {
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    fx[u][m][0] = M::load(xr[m] + (s + u) * kStepK);
-                    fx[u][m][1] = M::load(xr[m] + (s + u) * kStepK + 8);
-                }
-            }
+                for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u)
-            if (s + u < s1) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int m = 0; m < MT; ++m)
-#pragma unroll
-                        for (int n = 0; n < NT; ++n) acc[m][n] = M::mac(fx[u][m][h], fw[u][n][h], acc[m][n]);
-            }
+                    for (int n = 0; n < NT; ++n) acc[m][n] = M::mac(ax[m][h], aw[n][h], acc[m][n]);
+        }
     }
+    __syncthreads();
+    float* sums = reinterpret_cast<float*>(lds);                         // [WAVES][16 * MT][kSumPitch]
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) red[wave][(m * 16 + lq * 4 + r) * kCols + n * 16 + l16] = acc[m][n][r];
+            for (int r = 0; r < 4; ++r) sums[(wave * 16 * MT + m * 16 + lq * 4 + r) * kSumPitch + n * 16 + l16] = acc[m][n][r];
     __syncthreads();
-    if (GLU) {
-        for (int i = tid; i < 16 * MT * 16; i += kWaves * kWave) {
-            const int t = i / 16, c = i % 16;
-            if (t >= T || n0 + c >= N) continue;
+    for (int i = tid; i < 16 * MT * kOutCols; i += WAVES * kWave) {
+        const int t = i / kOutCols, c = i % kOutCols;
+        if (t >= T || n0 + c >= N) continue;
+        if (GLU) {
+            const float* at = sums + t * kSumPitch + c / 16 * 32 + c % 16;
             float g = 0.0f, u = 0.0f;
 #pragma unroll
-            for (int k = 0; k < kWaves; ++k) {
-                g += red[k][t * kCols + c];
-                u += red[k][t * kCols + 16 + c];
+            for (int k = 0; k < WAVES; ++k) {
+                g += at[k * 16 * MT * kSumPitch];
+                u += at[k * 16 * MT * kSumPitch + 16];
             }
             static_cast<uint16_t*>(out)[static_cast<int64_t>(t) * N + n0 + c] = f32_to_bf16_bits(silu(g) * u);
+            continue;
         }
-        return;
-    }
-    for (int i = tid; i < kTile; i += kWaves * kWave) {
-        const int t = i / kCols, c = n0 + i % kCols;
-        if (t >= T || c >= N) continue;
         float v = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) v += red[k][i];
+        for (int k = 0; k < WAVES; ++k) v += sums[(k * 16 * MT + t) * kSumPitch + c];
         if (act == 1) {
             v = fmaxf(v, 0.0f);
             v *= v;
         }
-        const int64_t at = (static_cast<int64_t>(split) * T + t) * N + c;
+        const int64_t at = (static_cast<int64_t>(split) * T + t) * N + n0 + c;
         if (F32OUT) static_cast<float*>(out)[at] = v;
         else static_cast<uint16_t*>(out)[at] = f32_to_bf16_bits(v);
     }
 }
 
+template <int MT, int NT, int WAVES, int AHEAD, bool F32OUT, bool GLU>
+int launch_one(const uint16_t* x, const uint16_t* w, void* out, int splits, int T, int N, int K, int act, hipStream_t s) {
+    const int rc = allow_lds(reinterpret_cast<const void*>(skinny_gemm_kernel<MT, NT, WAVES, AHEAD, F32OUT, GLU>), skinny_lds<MT, NT, WAVES>());
+    if (rc != 0) return rc;
+    launch((skinny_gemm_kernel<MT, NT, WAVES, AHEAD, F32OUT, GLU>),
+           dim3(static_cast<unsigned>(ceil_div(N, (GLU ? 8 : 16) * NT)), static_cast<unsigned>(splits)), dim3(WAVES * kWave),
+           (skinny_lds<MT, NT, WAVES>()), s, x, w, out, T, N, K, act);
+    return launch_status();
+}
+
+template <int MT, int NT, int WAVES, int AHEAD>
+int launch_form(const uint16_t* x, const uint16_t* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s) {
+    if constexpr (NT > 1)
+        if (act == 2) return launch_one<MT, NT, WAVES, AHEAD, false, true>(x, w, out, splits, T, N, K, 0, s);
+    return f32 ? launch_one<MT, NT, WAVES, AHEAD, true, false>(x, w, out, splits, T, N, K, act, s)
+               : launch_one<MT, NT, WAVES, AHEAD, false, false>(x, w, out, splits, T, N, K, act, s);
+}
+
+// Tiles of weight rows per workgroup: as few as leave one workgroup of eight waves to a CU (us, with 64 tokens: 3072 rows of
+// 2048 in ones 8.8, in twos 10.7; 6176 in twos 11.9, ones 17.4, fours 15.3; 8512 in fours 16.9, twos 19.5; with up to 32
+// tokens two such workgroups share a CU, and the few beyond the first 256 cost less than half of the chip without work: 8512,
+// T = 1, twos 10.0, fours 11.8).  Beyond 64 rows to a CU workgroups of four waves, of which two share a CU (32000 x 2048, T = 32: 25.0 / 29.3 with eight).  With three or four
+// tiles of tokens those carry one step of k instead of two (T = 64: 31.5 / 38.4), and partial sums take 64 rows as soon as
+// four ranges of K fill the chip that way, since the token rows are read by half as many workgroups (4096 x 12288, T = 64:
+// 26.8 / 30.5; T = 32: 22.6 / 22.6).
 template <int MT>
-int launch_glu(const uint16_t* x, const uint16_t* w, void* out, int T, int N, int K, hipStream_t s) {
-    launch((skinny_gemm_kernel<MT, 2, false, true>), dim3(static_cast<unsigned>(ceil_div(N, 16))), dim3(kWaves * kWave), 0, s, x, w, out, T, N, K, 0);
-    return launch_status();
+int launch_tokens(const uint16_t* x, const uint16_t* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s) {
+    const int rows = act == 2 ? 2 * N : N;
+    if (splits > 1) {
+        if (MT > 2 && N >= 4096) return launch_form<MT, 4, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
+        return launch_form<MT, 2, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
+    }
+    if (rows <= 16 * kSplitGroups && act != 2) return launch_form<MT, 1, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
+    if (rows <= (MT > 2 ? 32 : 36) * kSplitGroups) return launch_form<MT, 2, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
+    if (MT > 2 && rows <= 64 * kSplitGroups) return launch_form<MT, 4, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
+    return launch_form<MT, 4, 4, (MT > 2 ? 1 : 2)>(x, w, out, f32, splits, T, N, K, act, s);
 }
-
-template <int MT, int NT>
-int launch_skinny(const uint16_t* x, const uint16_t* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(ceil_div(N, 16 * NT)), static_cast<unsigned>(splits)), block(kWaves * kWave);
-    if (f32) launch((skinny_gemm_kernel<MT, NT, true>), grid, block, 0, s, x, w, out, T, N, K, act);
-    else launch((skinny_gemm_kernel<MT, NT, false>), grid, block, 0, s, x, w, out, T, N, K, act);
-    return launch_status();
-}
-
-int cols_per_group(int T, int N) { return T <= 16 && N <= 8192 ? 16 : 32; }
 
 }  // namespace
 
-// The range where this beats the library's product, which is slower to get going: up to 16 tokens unless the weights are
-// large, up to 64 tokens for small ones (us, this / library; 6144 x 2048: T = 1 8.6 / 12.4, T = 16 11.1 / 12.3, T = 32
-// 11.0 / 12.5, T = 64 15.3 / 13.0; 2048 x 2048, T = 64: 6.3 / 8.8; 12288 x 4096: T = 1 24.9 / 26.6, T = 16 29.7 / 25.7).
+// The range of ed_skinny_gemm.
 bool skinny_supported(int64_t T, int N, int K) {
-    if (T <= 0 || N <= 0 || K <= 0 || K % kStepK != 0) return false;
+    if (!decode_gemm_supported(T, N, K)) return false;
     const int64_t weights = static_cast<int64_t>(N) * K;
     return T <= 4 || (T <= 16 && weights <= (int64_t{1} << 25)) || (T <= 32 && weights <= (int64_t{1} << 24)) ||
            (T <= 64 && weights <= (int64_t{1} << 22));
 }
 
+bool decode_gemm_supported(int64_t T, int N, int K) { return T > 0 && T <= 64 && N > 0 && K > 0 && K % kStepK == 0; }
+
+// Against the library's product (us, this / library): 4096 x 4096 T = 1 8 / 16, T = 64 12.6 / 15.6; 2048 x 4096 T = 1 5.2 / 15,
+// T = 24 6.5 / 12.4, T = 64 8.2 / 14.1; 12288 x 4096 T = 12 21 / 29, T = 32 24 / 25.6, T = 48 24.7 / 26.8, T = 64 28.5 / 27.0;
+// 6720 x 4096 T = 48 19.1 / 19.0, T = 64 21.1 / 19.4; 8512 x 2048 T = 64 16.9 / 16.5.  The library is ahead with more than
+// 48 tokens and large weights, unless an activation, or a sum kept in float32, comes with the product.
+bool decode_gemm_plain_pays(int64_t T, int N, int K) { return T <= 48 || static_cast<int64_t>(N) * K <= (int64_t{1} << 24); }
+
 // Ranges of K for results that may stay partial sums: enough workgroups for the chip, a step of k for every wave.
 int skinny_splits(int T, int N, int K) {
-    const int groups = static_cast<int>(ceil_div(N, cols_per_group(T, N)));
-    const int want = static_cast<int>(ceil_div(384, groups)), most = K / (kStepK * kWaves);
+    const int groups = static_cast<int>(ceil_div(N, T > 32 && N >= 4096 ? 64 : 32));
+    const int want = static_cast<int>(kSplitGroups / groups), most = K / (kStepK * 8);
     const int s = want < most ? want : most;
     return s < 1 ? 1 : s > 8 ? 8 : s;
 }
@@ -156,11 +218,10 @@ int skinny_splits(int T, int N, int K) {
 int launch_skinny_gemm(const void* x, const void* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s) {
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     const uint16_t* wp = static_cast<const uint16_t*>(w);
-    if (act == 2) return T <= 16 ? launch_glu<1>(xp, wp, out, T, N, K, s) : T <= 32 ? launch_glu<2>(xp, wp, out, T, N, K, s) : launch_glu<4>(xp, wp, out, T, N, K, s);
-    if (cols_per_group(T, N) == 16) return launch_skinny<1, 1>(xp, wp, out, f32, splits, T, N, K, act, s);
-    if (T <= 16) return launch_skinny<1, 2>(xp, wp, out, f32, splits, T, N, K, act, s);
-    if (T <= 32) return launch_skinny<2, 2>(xp, wp, out, f32, splits, T, N, K, act, s);
-    return launch_skinny<4, 2>(xp, wp, out, f32, splits, T, N, K, act, s);
+    if (T <= 16) return launch_tokens<1>(xp, wp, out, f32, splits, T, N, K, act, s);
+    if (T <= 32) return launch_tokens<2>(xp, wp, out, f32, splits, T, N, K, act, s);
+    if (T <= 48) return launch_tokens<3>(xp, wp, out, f32, splits, T, N, K, act, s);
+    return launch_tokens<4>(xp, wp, out, f32, splits, T, N, K, act, s);
 }
 
 }  // namespace em

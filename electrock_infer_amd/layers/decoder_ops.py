@@ -15,23 +15,28 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def _skinny(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, act: int) -> torch.Tensor:
     (T, K), N = x.shape, weight.shape[0]
-    code = _lib.load_decoder().ed_skinny_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), splits,
+    code = _lib.load_decoder().ed_decode_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), splits,
                                               T, N, K, act, _lib.current_stream(x.device))
-    _lib.check_decoder(code, "skinny_gemm")
+    _lib.check_decoder(code, "decode_gemm")
     return out
 
 
 def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
-    """For a decode batch that the weight-streaming kernel takes: how many ranges of K fill the chip; else 0."""
-    if x.dtype != torch.bfloat16 or x.shape[0] > 64 or not x.is_contiguous():
+    """For a decode batch that the weight-streaming kernel takes (at most 64 rows, any size of the weights): how many ranges of
+    K fill the chip; else 0."""
+    T, (N, K) = x.shape[0], weight.shape
+    if x.dtype != torch.bfloat16 or T > 64 or not x.is_contiguous():
         return 0
-    return _lib.load_decoder().ed_skinny_gemm_splits(x.shape[0], weight.shape[0], x.shape[1])
+    lib = _lib.load_decoder()
+    if (x.data_ptr() | weight.data_ptr()) % 16 or not weight.is_contiguous():      # the library takes these
+        return lib.ed_skinny_gemm_splits(T, N, K)
+    return lib.ed_decode_gemm_splits(T, N, K)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
     """act(x @ weight^T) in x's type: a weight-streaming kernel for a decode batch, a library product otherwise;
     ``act``: None or 'relu_squared'."""
-    if _skinny_splits(x, weight):
+    if _skinny_splits(x, weight) and (act is not None or _lib.load_decoder().ed_decode_gemm_plain_pays(x.shape[0], *weight.shape)):
         return _skinny(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device), 1, int(act is not None))
     out = F.linear(x, weight)
     return relu_squared_(out) if act is not None else out
@@ -42,9 +47,9 @@ def linear_silu_gate(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     (T, _), ff = x.shape, weight.shape[0] // 2
     out = torch.empty(T, ff, dtype=x.dtype, device=x.device)
     if _skinny_splits(x, weight):
-        code = _lib.load_decoder().ed_skinny_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), 1, T, ff,
+        code = _lib.load_decoder().ed_decode_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), 1, T, ff,
                                                   x.shape[1], 2, _lib.current_stream(x.device))
-        _lib.check_decoder(code, "skinny_gemm")
+        _lib.check_decoder(code, "decode_gemm")
         return out
     u = F.linear(x, weight)
     _lib.check_decoder(_lib.load_decoder().ed_silu_gate(u.data_ptr(), out.data_ptr(), T, ff, _lib.dtype_code(x.dtype),

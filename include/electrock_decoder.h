@@ -52,6 +52,12 @@ int ed_gated_norm(void* y, const void* z, int64_t z_stride, const float* w, int6
 int ed_skinny_gemm_splits(int64_t T, int N, int K);
 int ed_skinny_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
                    void* stream);
+/* The same for every T <= 64, whatever the weights' size; ed_decode_gemm_plain_pays: 1 if that is the faster way also for a
+ * product without activation that is stored in bf16. */
+int ed_decode_gemm_splits(int64_t T, int N, int K);
+int ed_decode_gemm_plain_pays(int64_t T, int N, int K);
+int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
+                   void* stream);
 
 /* g [T, dim] = gelu_tanh(x gate^T) * table[tokens[t]][column0 + c]; x [T, W], gate [dim, W]. */
 int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const void* table, int64_t table_stride,
