@@ -1,8 +1,10 @@
 """What the kernels of libelectrock_decoder.so need to know about the batch of one forward pass: a ragged list of
 portions, one per sequence, each the next tokens of its sequence.  A decode step is the case of one token each."""
+import struct
 from dataclasses import dataclass
 from typing import List, Optional
 
+import numpy as np
 import torch
 
 from .sequence import Sequence
@@ -43,28 +45,81 @@ class DecodePadding:
     scratch_slot: int
 
 
+# From so many tokens on a portion's rows are made as arrays and copied into the batch's buffer; shorter ones are part of the
+# list of numbers that everything else is packed from.
+ARRAY_TOKENS = 64
+
+
+def _portion_pieces(s: Sequence, block_size: int):
+    """Tokens, positions and cache rows of the planned portion: arrays of a long one, else lists."""
+    start, n, table = s.num_computed_tokens, s.num_scheduled_tokens, s.block_table
+    if n < ARRAY_TOKENS:
+        return (s[start:start + n], list(range(start, start + n)),
+                [table[p // block_size] * block_size + p % block_size for p in range(start, start + n)])
+    at = np.arange(start, start + n, dtype=np.int64)
+    return (np.array(s[start:start + n], dtype=np.int32), at,
+            np.array(table, dtype=np.int64)[at // block_size] * block_size + at % block_size)
+
+
+def _add(pieces: list, piece) -> None:
+    if pieces and isinstance(piece, list) and isinstance(pieces[-1], list):
+        pieces[-1] += piece
+    else:
+        pieces.append(piece)
+
+
+def _pack(parts: dict, pinned: bool):
+    """The parts' pieces behind each other in one int32 tensor, every part at a multiple of four; name -> (place, length)."""
+    runs, flat, begin, at = [], [], 0, {}
+    for name, pieces in parts.items():
+        flat += [0] * (-(begin + len(flat)) % 4)
+        first = begin + len(flat)
+        for p in pieces:
+            if isinstance(p, np.ndarray):
+                runs += [(begin, flat), (begin + len(flat), p)]
+                begin, flat = begin + len(flat) + len(p), []
+            else:
+                flat += p
+        at[name] = (first, begin + len(flat) - first)
+    runs.append((begin, flat))
+    host = torch.empty(begin + len(flat), dtype=torch.int32, pin_memory=pinned)
+    values = host.numpy()
+    for to, run in runs:
+        if isinstance(run, np.ndarray):
+            values[to:to + len(run)] = run
+        else:
+            struct.pack_into(f"{len(run)}i", values, 4 * to, *run)
+    return host, at
+
+
 def make_ragged(seqs: List[Sequence], block_size: int, chunk_tokens: int, device, rows: Optional[List[int]] = None,
                 padding: Optional[DecodePadding] = None, into: Optional[RaggedBatch] = None) -> RaggedBatch:
     """Describe the planned portions of ``seqs``; ``rows``: batch rows whose logits are wanted (default: the last row of
     every portion).  ``into``: an earlier batch of the same ``padding``, whose buffer is overwritten."""
-    tokens, positions, cache_rows, q_begin, chunks, seq_chunks, last = [], [], [], [0], [], [0], []
-    for i, s in enumerate(seqs):
-        start, n = s.num_computed_tokens, s.num_scheduled_tokens
-        if n <= 0 or start + n > len(s) or len(s.block_table) * block_size < start + n:
-            raise ValueError("a portion needs tokens, and blocks that hold them")
-        row = q_begin[-1]
-        tokens.extend(s[start:start + n])
-        positions.extend(range(start, start + n))
-        cache_rows.extend(s.block_table[p // block_size] * block_size + p % block_size for p in range(start, start + n))
-        for at in range(0, n, chunk_tokens):
-            chunks += [i, row + at, min(chunk_tokens, n - at), 0]
-        q_begin.append(row + n)
-        seq_chunks.append(len(chunks) // 4)
-        last.append(row + n - 1)
-    starts = [s.num_computed_tokens for s in seqs]
     counts = [s.num_scheduled_tokens for s in seqs]
+    starts = [s.num_computed_tokens for s in seqs]
     slots = [s.state_slot for s in seqs]
     contexts = [a + n for a, n in zip(starts, counts)]
+    for s, n, c in zip(seqs, counts, contexts):
+        if n <= 0 or c > len(s.token_ids) or len(s.block_table) * block_size < c:
+            raise ValueError("a portion needs tokens, and blocks that hold them")
+    if all(n == 1 for n in counts):
+        tokens = [[s.token_ids[a] for s, a in zip(seqs, starts)]]
+        positions = [list(starts)]
+        cache_rows = [[s.block_table[a // block_size] * block_size + a % block_size for s, a in zip(seqs, starts)]]
+        q_begin, seq_chunks, last = list(range(len(seqs) + 1)), list(range(len(seqs) + 1)), list(range(len(seqs)))
+        chunks = [v for i in last for v in (i, i, 1, 0)]
+    else:
+        tokens, positions, cache_rows, q_begin, chunks, seq_chunks, last = [], [], [], [0], [], [0], []
+        for i, (s, n) in enumerate(zip(seqs, counts)):
+            row = q_begin[-1]
+            for pieces, piece in zip((tokens, positions, cache_rows), _portion_pieces(s, block_size)):
+                _add(pieces, piece)
+            for at in range(0, n, chunk_tokens):
+                chunks += [i, row + at, min(chunk_tokens, n - at), 0]
+            q_begin.append(row + n)
+            seq_chunks.append(len(chunks) // 4)
+            last.append(row + n - 1)
     extra = 0
     if padding is not None:
         extra = padding.batch - len(seqs)
@@ -72,8 +127,9 @@ def make_ragged(seqs: List[Sequence], block_size: int, chunk_tokens: int, device
             raise ValueError("padding is for decode steps of at most its batch")
         for i in range(len(seqs), padding.batch):
             chunks += [i, i, 1, 0]
-        tokens, positions = tokens + [0] * extra, positions + [0] * extra
-        cache_rows = cache_rows + [padding.scratch_block * block_size] * extra
+        _add(tokens, [0] * extra)
+        _add(positions, [0] * extra)
+        _add(cache_rows, [padding.scratch_block * block_size] * extra)
         q_begin, seq_chunks, last = list(range(padding.batch + 1)), list(range(padding.batch + 1)), list(range(padding.batch))
         starts, slots, contexts = starts + [0] * extra, slots + [padding.scratch_slot] * extra, contexts + [1] * extra
     k_begin = [0]
@@ -86,20 +142,16 @@ def make_ragged(seqs: List[Sequence], block_size: int, chunk_tokens: int, device
         width = padding.table_width
     tables = []
     for s, c in zip(seqs, contexts):
-        used = s.block_table[:-(-c // block_size)]
-        tables += used + [0] * (width - len(used))
+        n = -(-c // block_size)
+        tables += s.block_table[:n]
+        tables += [0] * (width - n)
     for _ in range(extra):
         tables += [padding.scratch_block] + [0] * (width - 1)
     wanted = last if rows is None else rows
-    parts = {"tokens": tokens, "positions": positions, "cache_rows": cache_rows, "q_begin": q_begin, "starts": starts,
-             "state_slots": slots, "tables": tables, "chunks": chunks, "seq_chunks": seq_chunks,
-             "k_lens": contexts, "k_begin": k_begin, "logit_rows": wanted}
-    flat, at = [], {}
-    for name, values in parts.items():
-        flat += [0] * (-len(flat) % 4)                  # 16-byte aligned views
-        at[name] = (len(flat), len(values))
-        flat += values
-    host = torch.tensor(flat, dtype=torch.int32, pin_memory=torch.device(device).type == "cuda")
+    parts = {"tokens": tokens, "positions": positions, "cache_rows": cache_rows, "q_begin": [q_begin], "starts": [starts],
+             "state_slots": [slots], "tables": [tables], "chunks": [chunks], "seq_chunks": [seq_chunks],
+             "k_lens": [contexts], "k_begin": [k_begin], "logit_rows": [list(wanted)]}
+    host, at = _pack(parts, pinned=torch.device(device).type == "cuda")
     if into is not None:
         into.buffer.copy_(host, non_blocking=True)
         return into
