@@ -6,6 +6,7 @@ namespace em {
 namespace {
 
 constexpr int kRowMaxPerThread = 32;  // floats of a row that one thread keeps in registers
+constexpr int64_t kFewRows = 256;     // up to so many rows a CU has one at most
 
 // Sum over the workgroup, the same value and the same order in every thread.  `scratch`: one float per wave.
 template <int THREADS>
@@ -55,95 +56,92 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t* __restrict__ 
     }
 }
 
-// One workgroup per row.
+// One workgroup per row, N vectors of the row per thread.
 // y may be given as float32 partial sums [y_parts, T, W].
 //   UPDATE 0: x stays          UPDATE 1: x += y / rms(y) * post_w          UPDATE 2: x = y + post_w
 //   then, when out != null: out = next_w ? x / rms(x) * next_w : x, rounded to the compute type
-template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS>
+// Bound: bytes for prompts, the way from the first load to the last store for a few rows.  Everything that a row needs is
+// requested before the first sum over it: loads behind the barriers, and partial sums one by one, cost a way to memory
+// each (four partial sums of 64 rows of 2048: 5.5 us that way, 4.9 now; two of 24 rows of 4096: 6.8, 4.9; 8192 rows of 2048:
+// 35.3, 34.5).
+template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS, int N>
 __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
     float* __restrict__ x, const typename YElem::storage* __restrict__ y, int y_parts, const float* __restrict__ post_w,
     const float* __restrict__ next_w, typename Elem::storage* __restrict__ out, int64_t out_stride, int W, float eps) {
     __shared__ float scratch[THREADS / kWave];
-    constexpr int N = kRowMaxPerThread / VEC;
+    constexpr bool kEarly = N * VEC <= 16;          // (longer rows do not fit in the registers twice)
+    constexpr int kParts = kEarly ? 4 : 1, M = kEarly ? N : 1;      // partial sums requested at once; rows of early loads
     const int64_t row = blockIdx.x;
     float* xr = x + row * W;
-    float v[N][VEC];
-    if (UPDATE != 0) {
-        const typename YElem::storage* yr = y + row * W;
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const int c = (threadIdx.x + i * THREADS) * VEC;
-            if (c < W) {
-                RowIo<YElem, VEC>::load(yr + c, v[i]);
-                for (int p = 1; p < y_parts; ++p) {
-                    float more[VEC];
-                    RowIo<YElem, VEC>::load(yr + static_cast<int64_t>(p) * gridDim.x * W + c, more);
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) v[i][j] += more[j];
-                }
-#pragma unroll
-                for (int j = 0; j < VEC; ++j) sum = fmaf(v[i][j], v[i][j], sum);
-            }
-        }
-        float rstd = 0.0f;
-        if (UPDATE == 1) rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(W) + eps);
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const int c = (threadIdx.x + i * THREADS) * VEC;
-            if (c < W) {
-                float pw[VEC];
-                if (UPDATE == 1) {
-                    float xv[VEC];
-                    RowIo<F32Elem, VEC>::load(post_w + c, pw);
-                    RowIo<F32Elem, VEC>::load(xr + c, xv);
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) v[i][j] = xv[j] + v[i][j] * rstd * pw[j];
-                } else if (post_w != nullptr) {
-                    RowIo<F32Elem, VEC>::load(post_w + c, pw);
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) v[i][j] += pw[j];
-                }
-                RowIo<F32Elem, VEC>::store(xr + c, v[i]);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const int c = (threadIdx.x + i * THREADS) * VEC;
-            if (c < W) RowIo<F32Elem, VEC>::load(xr + c, v[i]);
-        }
-    }
-    if (out == nullptr) return;
-    float rstd = 1.0f;
-    if (next_w != nullptr) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const int c = (threadIdx.x + i * THREADS) * VEC;
-            if (c < W) {
-#pragma unroll
-                for (int j = 0; j < VEC; ++j) sum = fmaf(v[i][j], v[i][j], sum);
-            }
-        }
-        rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(W) + eps);
-    }
+    float v[N][VEC], xv[M][VEC], pw[M][VEC], nw[M][VEC], sum = 0.0f;
+    const bool add_w = UPDATE == 1 || (UPDATE == 2 && post_w != nullptr), norm = out != nullptr && next_w != nullptr;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const int c = (threadIdx.x + i * THREADS) * VEC;
-        if (c < W) {
-            float o[VEC];
-            if (next_w != nullptr) {
-                float nw[VEC];
-                RowIo<F32Elem, VEC>::load(next_w + c, nw);
+        if (c >= W) continue;
+        if (UPDATE != 0) RowIo<YElem, VEC>::load(y + row * W + c, v[i]);
+        if (!kEarly) continue;
+        if (UPDATE != 2) RowIo<F32Elem, VEC>::load(xr + c, xv[i % M]);
+        if (add_w) RowIo<F32Elem, VEC>::load(post_w + c, pw[i % M]);
+        if (norm) RowIo<F32Elem, VEC>::load(next_w + c, nw[i % M]);
+    }
+    if (UPDATE != 0 && y_parts > 1) {
+        for (int p0 = 1; p0 < y_parts; p0 += kParts) {
+            float more[kParts][N][VEC];
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) o[j] = v[i][j] * rstd * nw[j];
-            } else {
+            for (int p = 0; p < kParts; ++p)
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) o[j] = v[i][j];
-            }
-            RowIo<Elem, VEC>::store(out + row * out_stride + c, o);
+                for (int i = 0; i < N; ++i) {
+                    const int c = (threadIdx.x + i * THREADS) * VEC;
+                    if (c < W) RowIo<YElem, VEC>::load(y + (static_cast<int64_t>(min(p0 + p, y_parts - 1)) * gridDim.x + row) * W + c, more[p][i]);
+                }
+#pragma unroll
+            for (int p = 0; p < kParts; ++p)
+#pragma unroll
+                for (int i = 0; i < N; ++i)
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) v[i][j] += p0 + p < y_parts ? more[p][i][j] : 0.0f;
         }
+    }
+    if (UPDATE == 1) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if ((threadIdx.x + i * THREADS) * VEC < W) {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) sum = fmaf(v[i][j], v[i][j], sum);
+            }
+    }
+    float rstd = 0.0f;
+    if (UPDATE == 1) rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(W) + eps);
+    sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int c = (threadIdx.x + i * THREADS) * VEC;
+        if (c >= W) continue;
+        if (!kEarly && UPDATE != 2) RowIo<F32Elem, VEC>::load(xr + c, xv[i % M]);
+        if (!kEarly && add_w) RowIo<F32Elem, VEC>::load(post_w + c, pw[i % M]);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            if (UPDATE == 0) v[i][j] = xv[i % M][j];
+            if (UPDATE == 1) v[i][j] = xv[i % M][j] + v[i][j] * rstd * pw[i % M][j];
+            if (UPDATE == 2 && add_w) v[i][j] += pw[i % M][j];
+            sum = fmaf(v[i][j], v[i][j], sum);
+        }
+        if (UPDATE != 0) RowIo<F32Elem, VEC>::store(xr + c, v[i]);
+    }
+    if (out == nullptr) return;
+    rstd = 1.0f;
+    if (norm) rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(W) + eps);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int c = (threadIdx.x + i * THREADS) * VEC;
+        if (c >= W) continue;
+        if (norm) {
+            if (!kEarly) RowIo<F32Elem, VEC>::load(next_w + c, nw[i % M]);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) v[i][j] = v[i][j] * rstd * nw[i % M][j];
+        }
+        RowIo<Elem, VEC>::store(out + row * out_stride + c, v[i]);
     }
 }
 
@@ -178,28 +176,35 @@ __global__ __launch_bounds__(256) void silu_gate_kernel(const typename Elem::sto
 }
 
 // y = y silu(z), normed in equal parts of `size` elements, times w, in place: one workgroup per (row, part)
-template <typename Elem, int VEC, int THREADS>
+template <typename Elem, int VEC, int THREADS, int N>
 __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::storage* __restrict__ y, const typename Elem::storage* __restrict__ z,
                                                              int64_t z_stride, const float* __restrict__ w, int size, float eps) {
     __shared__ float scratch[THREADS / kWave];
-    constexpr int N = kRowMaxPerThread / VEC;
     const int64_t row = blockIdx.x;
     const int c0 = blockIdx.y * size;
     typename Elem::storage* yr = y + (row * gridDim.y + blockIdx.y) * size;
     const typename Elem::storage* zr = z + row * z_stride + c0;
-    float v[N][VEC], sum = 0.0f;
+    constexpr bool kEarly = N * VEC <= 16;
+    constexpr int M = kEarly ? N : 1;
+    float v[N][VEC], g[M][VEC], wv[M][VEC], sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const int c = (threadIdx.x + i * THREADS) * VEC;
-        if (c < size) {
-            float g[VEC];
-            RowIo<Elem, VEC>::load(yr + c, v[i]);
-            RowIo<Elem, VEC>::load(zr + c, g);
+        if (c >= size) continue;
+        RowIo<Elem, VEC>::load(yr + c, v[i]);
+        if (!kEarly) continue;
+        RowIo<Elem, VEC>::load(zr + c, g[i % M]);
+        RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
+    }
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                v[i][j] *= silu(g[j]);
-                sum = fmaf(v[i][j], v[i][j], sum);
-            }
+    for (int i = 0; i < N; ++i) {
+        const int c = (threadIdx.x + i * THREADS) * VEC;
+        if (c >= size) continue;
+        if (!kEarly) RowIo<Elem, VEC>::load(zr + c, g[i % M]);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            v[i][j] *= silu(g[i % M][j]);
+            sum = fmaf(v[i][j], v[i][j], sum);
         }
     }
     const float rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(size) + eps);
@@ -207,10 +212,9 @@ __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::stor
     for (int i = 0; i < N; ++i) {
         const int c = (threadIdx.x + i * THREADS) * VEC;
         if (c < size) {
-            float wv[VEC];
-            RowIo<F32Elem, VEC>::load(w + c0 + c, wv);
+            if (!kEarly) RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) v[i][j] *= rstd * wv[j];
+            for (int j = 0; j < VEC; ++j) v[i][j] *= rstd * wv[i % M][j];
             RowIo<Elem, VEC>::store(yr + c, v[i]);
         }
     }
@@ -220,28 +224,39 @@ template <typename Elem, int VEC>
 int launch_gated(void* y, const void* z, int64_t z_stride, const float* w, int64_t T, int parts, int size, float eps, hipStream_t s) {
     typedef typename Elem::storage S;
     const dim3 grid(static_cast<unsigned>(T), static_cast<unsigned>(parts));
-    if (size <= 64 * kRowMaxPerThread / 4)
-        launch((gated_norm_kernel<Elem, VEC, 64>), grid, dim3(64), 0, s, static_cast<S*>(y), static_cast<const S*>(z), z_stride, w, size, eps);
-    else if (size <= 256 * kRowMaxPerThread)
-        launch((gated_norm_kernel<Elem, VEC, 256>), grid, dim3(256), 0, s, static_cast<S*>(y), static_cast<const S*>(z), z_stride, w, size, eps);
-    else
-        launch((gated_norm_kernel<Elem, VEC, 1024>), grid, dim3(1024), 0, s, static_cast<S*>(y), static_cast<const S*>(z), z_stride, w, size, eps);
+#define EM_GATED(THREADS, N) \
+    launch((gated_norm_kernel<Elem, VEC, THREADS, N>), grid, dim3(THREADS), 0, s, static_cast<S*>(y), static_cast<const S*>(z), z_stride, w, size, eps)
+    if (size <= 512) EM_GATED(64, 8 / VEC);
+    else if (VEC == 4 && T * parts <= kFewRows && size > 1024 && size <= 4096) EM_GATED(1024, 4 / VEC);
+    else if (VEC == 4 && size <= 4096) EM_GATED(256, 16 / VEC);
+    else if (size <= 256 * kRowMaxPerThread) EM_GATED(256, kRowMaxPerThread / VEC);
+    else EM_GATED(1024, kRowMaxPerThread / VEC);
+#undef EM_GATED
     return launch_status();
 }
 
+template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS, int N>
+int launch_rows(float* x, const void* y, int y_parts, const float* post_w, const float* next_w, void* out, int64_t out_stride,
+                int64_t T, int W, float eps, hipStream_t s) {
+    launch((residual_norm_kernel<Elem, YElem, UPDATE, VEC, THREADS, N>), dim3(static_cast<unsigned>(T)), dim3(THREADS), 0, s, x,
+           static_cast<const typename YElem::storage*>(y), y_parts, post_w, next_w, static_cast<typename Elem::storage*>(out), out_stride, W, eps);
+    return launch_status();
+}
+
+// One vector per thread where the rows do not fill the chip (kFewRows), so that a row is over sooner; 256 threads where they do.
 template <typename Elem, typename YElem, int UPDATE, int VEC>
 int launch_residual(float* x, const void* y, int y_parts, const float* post_w, const float* next_w, void* out, int64_t out_stride,
                     int64_t T, int W, float eps, hipStream_t s) {
-    typedef typename Elem::storage S;
-    typedef typename YElem::storage YS;
-    const dim3 grid(static_cast<unsigned>(T));
-    if (W <= 256 * kRowMaxPerThread)
-        launch((residual_norm_kernel<Elem, YElem, UPDATE, VEC, 256>), grid, dim3(256), 0, s, x,
-               static_cast<const YS*>(y), y_parts, post_w, next_w, static_cast<S*>(out), out_stride, W, eps);
-    else
-        launch((residual_norm_kernel<Elem, YElem, UPDATE, VEC, 1024>), grid, dim3(1024), 0, s, x,
-               static_cast<const YS*>(y), y_parts, post_w, next_w, static_cast<S*>(out), out_stride, W, eps);
-    return launch_status();
+#define EM_ROWS(THREADS, N) return launch_rows<Elem, YElem, UPDATE, VEC, THREADS, N>(x, y, y_parts, post_w, next_w, out, out_stride, T, W, eps, s)
+    if constexpr (VEC == 4) {
+        if (T <= kFewRows && W > 1024 && W <= 2048) EM_ROWS(512, 1);
+        if (T <= kFewRows && W > 1024 && W <= 4096) EM_ROWS(1024, 1);
+        if (W <= 2048) EM_ROWS(256, 2);
+        if (W <= 4096) EM_ROWS(256, 4);
+    }
+    if (W <= 256 * kRowMaxPerThread) EM_ROWS(256, kRowMaxPerThread / VEC);
+    EM_ROWS(1024, kRowMaxPerThread / VEC);
+#undef EM_ROWS
 }
 
 template <typename Elem, typename YElem, int VEC>
