@@ -147,10 +147,24 @@ template <> struct Precise<BF16Elem> {    // the hardware's exponential and reci
 
 // ---- any portion ----
 constexpr int kKeys = 32;
+// Cached rows are read once per step: past the caches' order of use.
+template <typename Elem>
+__device__ __forceinline__ typename Mma<Elem>::frag load_nt(const typename Elem::storage* p) {
+    constexpr int kWords = sizeof(typename Elem::storage) * 8 / 16;
+    u32x4_t w[kWords];
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p) + i);
+    typename Mma<Elem>::frag f;
+    __builtin_memcpy(&f, w, sizeof(w));
+    return f;
+}
 template <typename Elem> __host__ __device__ constexpr int value_pitch(int dvt) { return dvt * 16 + 16 / static_cast<int>(sizeof(typename Elem::storage)); }
-template <typename Elem> __host__ __device__ constexpr int paged_lds(int dvt) {   // values of a wave's tile; later the waves' results
-    return 4 * kKeys * value_pitch<Elem>(dvt) * static_cast<int>(sizeof(typename Elem::storage)) > 4 * 16 * (dvt * 16 + 4) * 4
-               ? 4 * kKeys * value_pitch<Elem>(dvt) * static_cast<int>(sizeof(typename Elem::storage)) : 4 * 16 * (dvt * 16 + 4) * 4;
+template <typename Elem> __host__ __device__ constexpr int tile_pitch(int dkt, int dvt) {     // of keys and values in one stretch
+    return sizeof(typename Elem::storage) == 2 && dkt <= 4 && dkt * 2 > dvt ? value_pitch<Elem>(dkt * 2) : value_pitch<Elem>(dvt);
+}
+template <typename Elem> __host__ __device__ constexpr int paged_lds(int dkt, int dvt) {   // keys, then values of a wave's tile; later the waves' results
+    const int tiles = 4 * kKeys * tile_pitch<Elem>(dkt, dvt) * static_cast<int>(sizeof(typename Elem::storage)), results = 4 * 16 * (dvt * 16 + 4) * 4;
+    return tiles > results ? tiles : results;
 }
 
 // DKT: 32-element steps of dim; DVT: 16-element tiles of vdim
@@ -160,7 +174,7 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
                                                                                                     float* __restrict__ part_ml) {
     typedef typename Elem::storage S;
     typedef Mma<Elem> M;
-    constexpr int LPV = value_pitch<Elem>(DVT), kPieces = kKeys * DVT * 2 / kWave, LPO = DVT * 16 + 4;
+    constexpr int LPT = tile_pitch<Elem>(DKT, DVT), kPieces = kKeys * DVT * 2 / kWave, kRowsAtOnce = kKeys / kPieces, LPO = DVT * 16 + 4;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ float wave_m[4][16], wave_l[4][16];
     const int share = p.heads / p.kv_heads;
@@ -189,43 +203,70 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
 #pragma unroll
     for (int d = 0; d < DVT; ++d) o[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     float m = -INFINITY, l = 0.0f;       // l: this lane's share
-    S* Vs = reinterpret_cast<S*>(lds_raw) + wave * kKeys * LPV;
+    S* Vs = reinterpret_cast<S*>(lds_raw) + wave * kKeys * LPT;
     const int32_t* table = p.tables + static_cast<int64_t>(seq) * p.table_width;
     const S* keys = static_cast<const S*>(p.cache) + g * dp;
-    const S* values = static_cast<const S*>(p.cache) + p.kv_heads * dp + g * vp;
-    const int pieces = vp / 8;
+    const int v_key = lane / (DVT * 2), v_col = lane % (DVT * 2) * 8;          // (columns beyond the values are never stored)
+    const S* values = static_cast<const S*>(p.cache) + p.kv_heads * dp + g * vp + min(v_col, vp - 8);
     auto row_of = [&](int tile) {
         const int key = tile * kKeys + (lane & 31);
         return key <= last_pos && tile < tile1 ? table[key / p.block_size] * p.block_size + key % p.block_size : -1;
     };
-    int next_row = row_of(tile0 + wave);
-    for (int tile = tile0 + wave; tile < tile1; tile += 4) {
-        const int row = next_row;
-        next_row = row_of(tile + 4);
-        typename M::frag fv[kPieces];
+    // Bound: a wave's way to memory, times its tiles, where sequences are few or short; bytes beyond (us for 101 MB, 64 x 768
+    // keys of 4 x (128 + 128): 35.9, of it 5 for the combination of three partial results; now 26.9 in one pass; 256 x 768: 103,
+    // now 76).  The next tile's keys and values are on their way in registers, whole rows side by side (a load in operand
+    // layout touches 16 half-used lines), and pass through the wave's LDS one after the other.  Two workgroups to a CU: with
+    // the registers of three the tiles in flight spill (35.7 against 29.7).
+    constexpr bool kAhead = sizeof(S) == 2 && DKT <= 4;
+    constexpr int kKeyPieces = kAhead ? kKeys * DKT * 4 / kWave : 1, kKeysAtOnce = kKeys / kKeyPieces;
+    typename M::frag fk[kKeyPieces], fv[kPieces];
+    const int k_key = lane / (DKT * 4), k_col = lane % (DKT * 4) * 8;
+    auto key_row = [&](int row, int key) { return keys + static_cast<int64_t>(max(__shfl(row, key), 0)) * row_elems; };
+    auto load_keys = [&](int row) {
+#pragma unroll
+        for (int i = 0; i < kKeyPieces; ++i) fk[i] = load_nt<Elem>(key_row(row, k_key + i * kKeysAtOnce) + min(k_col, dp - 8));
+    };
+    auto load_values = [&](int row) {
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
-            const int e = lane + i * kWave, key = e / pieces, c = (e - key * pieces) * 8;
-            const int r = __shfl(row, key & 31);
-            fv[i] = key < kKeys && r >= 0 ? M::load(values + static_cast<int64_t>(r) * row_elems + c) : M::zero();
+            fv[i] = load_nt<Elem>(values + static_cast<int64_t>(max(__shfl(row, v_key + i * kRowsAtOnce), 0)) * row_elems);
+        }
+    };
+    int row = row_of(tile0 + wave), next_row = row_of(tile0 + wave + 4);
+    if (kAhead && tile0 + wave < tile1) {
+        load_keys(row);
+        load_values(row);
+    }
+    for (int tile = tile0 + wave; tile < tile1; tile += 4) {
+        if (!kAhead) load_values(row);
+        if (kAhead) {
+#pragma unroll
+            for (int i = 0; i < kKeyPieces; ++i) store_frag<Elem>(Vs + (k_key + i * kKeysAtOnce) * LPT + k_col, fk[i]);
+            load_keys(next_row);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (the stretch of LDS is this wave's own)
         }
         f32x4_t s[2];
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
             s[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            const int r = __shfl(row, n * 16 + l16);
-            const S* kr = keys + static_cast<int64_t>(max(r, 0)) * row_elems;
+            const S* kr = kAhead ? Vs + (n * 16 + l16) * LPT : key_row(row, n * 16 + l16);
 #pragma unroll
             for (int k = 0; k < DKT; ++k) {
-                const int c = k * 32 + lq * 8;
-                s[n] = M::mac(c < dp && r >= 0 ? M::load(kr + c) : M::zero(), fq[k], s[n]);
+                typename M::frag f = M::load(kr + (kAhead ? k * 32 + lq * 8 : min(k * 32 + lq * 8, dp - 8)));
+                // (a key that does not exist is masked below; elements beyond dim are zero in the query)
+                if (k * 32 + 32 > dp && k * 32 + lq * 8 >= dp) f = M::zero();
+                s[n] = M::mac(f, fq[k], s[n]);
             }
         }
+        if (kAhead) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
-            const int e = lane + i * kWave, key = e / pieces, c = (e - key * pieces) * 8;
-            if (key < kKeys) store_frag<Elem>(Vs + key * LPV + c, fv[i]);
+            if (__shfl(row, v_key + i * kRowsAtOnce) < 0) fv[i] = M::zero();
+            store_frag<Elem>(Vs + (v_key + i * kRowsAtOnce) * LPT + v_col, fv[i]);
         }
+        if (kAhead) load_values(next_row);
+        row = next_row;
+        next_row = row_of(tile + 8);
         float mx = -INFINITY;
 #pragma unroll
         for (int n = 0; n < 2; ++n)
@@ -258,7 +299,7 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
         for (int d = 0; d < DVT; ++d) {
             if (d * 16 < vp) {
                 o[d] *= alpha;
-                o[d] = M::mac(load_columns<Elem>(Vs, LPV, lq * 4, 16 + lq * 4, d * 16, l16), fp, o[d]);
+                o[d] = M::mac(load_columns<Elem>(Vs, LPT, lq * 4, 16 + lq * 4, d * 16, l16), fp, o[d]);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -530,7 +571,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(AttnProblem p) {
 
 template <typename Elem, int DKT, int DVT>
 int launch_paged(const AttnProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml, int64_t T, hipStream_t s) {
-    const size_t lds = paged_lds<Elem>(DVT);
+    const size_t lds = paged_lds<Elem>(DKT, DVT);
     int rc = allow_lds(reinterpret_cast<const void*>(attn_paged_kernel<Elem, DKT, DVT>), lds);
     if (rc != 0) return rc;
     const dim3 grid(static_cast<unsigned>(ceil_div(static_cast<int64_t>(max_q) * (p.heads / p.kv_heads), 16)),
