@@ -362,6 +362,192 @@ __global__ __launch_bounds__(256) void latent_paged_kernel(LatentProblem p, int 
     }
 }
 
+// The same for bf16, a wave on its own: 16 rows against every fourth tile of 16 keys, the tile in a stretch of LDS of its
+// own and the next one on its way in registers, no barrier before the waves' results are added up.  S^T = K Q^T leaves a lane
+// keys (lane / 16) * 4 + 0..3 for one row, which is the second operand of O^T = V^T P^T as it is.  Bound: the way to
+// memory, once per tile; a workgroup has a CU to itself (its waves' accumulators, queries and tiles take over half of the
+// registers for rank 512 + 64 rotated; tiles of 32 keys do not fit).  Workgroups that read the same
+// keys for other heads run on the same XCD at the same time, so that its L2 serves all but the first.  23 sequences of
+// 1500 keys, 32 heads on 512 + 64: 44.8 us in five ranges with four barriers per tile (36.1 in ten), 31.3 now, in five; 64 of
+// 1000 keys, 16 heads: 35.4 (eight), 33.5 (four).
+// DKT: 32-element steps of a cached row; NT: 16-element tiles of the latent.
+constexpr int kWaveKeys = 16;
+template <int DKT, int NT>
+struct LatentWave {
+    static constexpr int kPitch = DKT * 32 + 8, kSums = NT * 16 + 4;
+    static constexpr int kTileBytes = kWaveKeys * kPitch * 2, kSumBytes = 16 * kSums * 4;
+    static constexpr int kLds = 4 * (kTileBytes > kSumBytes ? kTileBytes : kSumBytes);
+};
+
+// Columns col0 + l16 of rows row0 .. + 3 of an LDS matrix.
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ s16x4_t load_four_rows(const uint16_t* m, int pitch, int row0, int col0, int l16) {
+    typedef __attribute__((address_space(3))) s16x4_t* lds_ptr;
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(m + (row0 + (l16 >> 2)) * pitch + col0 + (l16 & 3) * 4));
+}
+
+template <int DKT, int NT>
+__global__ __launch_bounds__(256, 1) void latent_wave_kernel(LatentProblem p, int n_seqs, int groups, int splits, float* __restrict__ part_o,
+                                                             float* __restrict__ part_ml) {
+    typedef Mma<BF16Elem> M;
+    typedef LatentWave<DKT, NT> L;
+    constexpr int LP = L::kPitch, kXcds = 8;
+    constexpr float kSlack = 8.0f;
+    static_assert(DKT % 2 == 0 && NT * 16 <= DKT * 32, "rows of whole 128-byte pieces that hold every tile of the latent");
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
+    __shared__ float wave_m[4][16], wave_l[4][16];
+    const int slot = blockIdx.x / kXcds, group = slot % groups, pair = slot / groups * kXcds + blockIdx.x % kXcds;
+    const int seq = pair / splits, split = pair - seq * splits;
+    if (seq >= n_seqs) return;
+    const int q0 = p.q_begin[seq], rows = (p.q_begin[seq + 1] - q0) * p.heads, r0 = group * 16;
+    if (r0 >= rows) return;
+    const int start = p.starts[seq];
+    const int n_keys = start + min(r0 + 15, rows - 1) / p.heads + 1;
+    const int n_tiles = (n_keys + kWaveKeys - 1) / kWaveKeys, per_split = (n_tiles + splits - 1) / splits;
+    const int tile0 = split * per_split, tile1 = min(tile0 + per_split, n_tiles);
+    const int pitch_c = latent_pitch(p.rank), row_elems = latent_row_elems(p.rank, p.rot);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+
+    const int mine = min(r0 + l16, rows - 1), my_t = mine / p.heads, my_h = mine - my_t * p.heads, pos = start + my_t;
+    bf16x8_t fq[DKT];
+    {
+        const int64_t row = q0 + my_t;
+        const uint16_t* latent = static_cast<const uint16_t*>(p.q_latent) + (row * p.heads + my_h) * pitch_c;
+        const uint16_t* rotated = static_cast<const uint16_t*>(p.q) + row * p.q_stride + my_h * (p.dim + p.rot) + p.dim;
+        const bool vec = p.rot % 8 == 0 && p.dim % 8 == 0 && p.q_stride % 8 == 0 && reinterpret_cast<uintptr_t>(p.q) % 16 == 0;
+#pragma unroll
+        for (int k = 0; k < DKT; ++k) {
+            const int c = k * 32 + lq * 8;
+            fq[k] = M::zero();
+            if (c < pitch_c) fq[k] = load_frag<BF16Elem>(latent + c, p.rank - c, true);
+            else if (c < row_elems) fq[k] = load_frag<BF16Elem>(rotated + (c - pitch_c), p.rot - (c - pitch_c), vec);
+        }
+    }
+    uint16_t* Ks = reinterpret_cast<uint16_t*>(lds_raw + wave * (L::kLds / 4));
+    for (int i = lane; i < kWaveKeys * (DKT * 4 - row_elems / 8); i += kWave) {        // columns behind the rows stay zero
+        const int w = DKT * 4 - row_elems / 8, r = i / w;
+        store_frag<BF16Elem>(Ks + r * LP + row_elems + (i - r * w) * 8, M::zero());
+    }
+    const int32_t* table = p.tables + static_cast<int64_t>(seq) * p.table_width;
+    const uint16_t* cache = static_cast<const uint16_t*>(p.cache);
+    auto row_of = [&](int tile) {
+        const int key = tile * kWaveKeys + (lane & 15);
+        return key < n_keys && tile < tile1 ? table[key / p.block_size] * p.block_size + key % p.block_size : -1;
+    };
+    // eight lanes side by side on 128 bytes of a row, eight rows at once
+    constexpr int kCols = DKT / 2;
+    u32x4_t piece[2][kCols];
+    const int l8 = lane >> 3, c8 = (lane & 7) * 8;
+    auto fetch = [&](int row) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const uint16_t* from = cache + static_cast<int64_t>(max(__shfl(row, g * 8 + l8), 0)) * row_elems;
+#pragma unroll
+            for (int i = 0; i < kCols; ++i) piece[g][i] = *reinterpret_cast<const u32x4_t*>(from + min(i * 64 + c8, row_elems - 8));
+        }
+    };
+    f32x4_t o[NT];
+#pragma unroll
+    for (int d = 0; d < NT; ++d) o[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    float m = -INFINITY, l = 0.0f;           // l: this lane's share
+    int row = row_of(tile0 + wave), next_row = row_of(tile0 + wave + 4);
+    if (tile0 + wave < tile1) fetch(row);
+    for (int tile = tile0 + wave; tile < tile1; tile += 4) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const bool none = __shfl(row, g * 8 + l8) < 0;
+#pragma unroll
+            for (int i = 0; i < kCols; ++i) {
+                if (none) piece[g][i] = u32x4_t{0, 0, 0, 0};
+                if (i * 64 + c8 < row_elems) *reinterpret_cast<u32x4_t*>(Ks + (g * 8 + l8) * LP + i * 64 + c8) = piece[g][i];
+            }
+        }
+        fetch(next_row);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (the stretch of LDS is this wave's own)
+        f32x4_t part[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+        for (int k = 0; k < DKT; ++k) part[k & 1] = M::mac(M::load(Ks + l16 * LP + k * 32 + lq * 8), fq[k], part[k & 1]);
+        f32x4_t s = part[0] + part[1];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = tile * kWaveKeys + lq * 4 + r <= pos ? s[r] * p.scale : -INFINITY;
+            mx = fmaxf(mx, s[r]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        // m need not be the maximum: while no row's scores exceed it by more than kSlack the weights stay below e^kSlack and
+        // the accumulators as they are (their way through the vector unit costs more than the tile's products)
+        if (__any(mx > m + kSlack)) {
+            const float mn = fmaxf(m, mx), alpha = mn == -INFINITY ? 1.0f : expf(m - mn);
+            m = mn;
+            l *= alpha;
+            if (tile != tile0 + wave) {
+#pragma unroll
+                for (int d = 0; d < NT; ++d) o[d] *= alpha;
+            }
+        }
+        const float base = m == -INFINITY ? 0.0f : m;
+        s16x4_t fp;
+        float sum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float e = expf(s[r] - base);
+            sum += e;
+            fp[r] = static_cast<short>(f32_to_bf16_bits(e));
+        }
+        l += sum;
+        // (what lies behind the latent in a row is finite, and its sums are not stored)
+#pragma unroll
+        for (int d = 0; d < NT; ++d)
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(load_four_rows(Ks, LP, lq * 4, d * 16, l16), fp, o[d], 0, 0, 0);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        row = next_row;
+        next_row = row_of(tile + 8);
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (lq == 0) {
+        wave_m[wave][l16] = m;
+        wave_l[wave][l16] = l;
+    }
+    __syncthreads();
+    float* Os = reinterpret_cast<float*>(lds_raw);                   // [4][16][kSums]
+#pragma unroll
+    for (int d = 0; d < NT; ++d) *reinterpret_cast<f32x4_t*>(Os + (wave * 16 + l16) * L::kSums + d * 16 + lq * 4) = o[d];
+    __syncthreads();
+    for (int i = tid; i < 16 * (pitch_c / 4); i += 256) {
+        const int rr = i / (pitch_c / 4), c = (i - rr * (pitch_c / 4)) * 4;
+        if (r0 + rr >= rows) continue;
+        const int64_t at = static_cast<int64_t>(q0) * p.heads + r0 + rr;
+        const float sk = p.sink[(r0 + rr) % p.heads];
+        float top = splits == 1 ? sk : -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) top = fmaxf(top, wave_m[w][rr]);
+        const float base = top == -INFINITY ? 0.0f : top;
+        float sum = 0.0f;
+        f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float weight = expf(wave_m[w][rr] - base);
+            sum = fmaf(wave_l[w][rr], weight, sum);
+            v += *reinterpret_cast<const f32x4_t*>(Os + (w * 16 + rr) * L::kSums + c) * weight;
+        }
+        if (splits == 1) {
+            const float inv = 1.0f / (sum + expf(sk - base));
+            uint16_t* out = static_cast<uint16_t*>(p.out) + at * pitch_c + c;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) out[j] = f32_to_bf16_bits(c + j < p.rank ? v[j] * inv : 0.0f);
+        } else {
+            *reinterpret_cast<f32x4_t*>(part_o + (at * splits + split) * pitch_c + c) = v;
+            if (c == 0) {
+                part_ml[(at * splits + split) * 2] = top;
+                part_ml[(at * splits + split) * 2 + 1] = sum;
+            }
+        }
+    }
+}
+
 template <typename Elem>
 __global__ __launch_bounds__(128) void latent_combine_kernel(const float* __restrict__ part_o,
                                                              const float* __restrict__ part_ml,
@@ -429,11 +615,27 @@ int launch_paged(const LatentProblem& p, int n_seqs, int max_q, int splits, floa
     return launch_status();
 }
 
+template <int DKT, int NT>
+int launch_wave(const LatentProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml, hipStream_t s) {
+    constexpr int kLds = LatentWave<DKT, NT>::kLds;
+    const int rc = allow_lds(reinterpret_cast<const void*>(latent_wave_kernel<DKT, NT>), kLds);
+    if (rc != 0) return rc;
+    const int64_t groups = ceil_div(static_cast<int64_t>(max_q) * p.heads, 16), pairs = round_up(static_cast<int64_t>(n_seqs) * splits, 8);
+    launch((latent_wave_kernel<DKT, NT>), dim3(static_cast<unsigned>(groups * pairs)), dim3(256), kLds, s, p, n_seqs, static_cast<int>(groups),
+           splits, part_o, part_ml);
+    return launch_status();
+}
+
 template <typename Elem>
 int dispatch_paged(const LatentProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml, int64_t T,
                    hipStream_t s) {
     int rc;
-    if (p.rank <= 128) rc = launch_paged<Elem, 2>(p, n_seqs, max_q, splits, part_o, part_ml, s);
+    const int row = latent_row_elems(p.rank, p.rot);
+    if (sizeof(typename Elem::storage) == 2 && row <= 18 * 32) {       // (rows of which a wave's queries and accumulators fit in its registers)
+        if (p.rank <= 128 && row <= 192) rc = launch_wave<6, 8>(p, n_seqs, max_q, splits, part_o, part_ml, s);
+        else if (p.rank <= 256 && row <= 320) rc = launch_wave<10, 16>(p, n_seqs, max_q, splits, part_o, part_ml, s);
+        else rc = launch_wave<18, 32>(p, n_seqs, max_q, splits, part_o, part_ml, s);
+    } else if (p.rank <= 128) rc = launch_paged<Elem, 2>(p, n_seqs, max_q, splits, part_o, part_ml, s);
     else if (p.rank <= 256) rc = launch_paged<Elem, 4>(p, n_seqs, max_q, splits, part_o, part_ml, s);
     else rc = launch_paged<Elem, 8>(p, n_seqs, max_q, splits, part_o, part_ml, s);
     if (rc != 0 || splits == 1) return rc;

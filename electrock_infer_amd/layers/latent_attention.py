@@ -17,6 +17,7 @@ class LatentAttention(nn.Module):
 
     PROMPT_TOKENS = 64           # portions from this length on write their keys and values out, if the kernel takes the sizes
     TARGET_WORKGROUPS = 768      # the keys are shared out over workgroups until a launch has about this many
+    WAVE_ROW, WAVE_WORKGROUPS = 576, 256      # cached rows of the kernel whose workgroups have a CU to themselves: no more of them than CUs
 
     def __init__(self, width: int, heads: int, dim: int, rot_dim: int, vdim: int, kv_rank: int, scale: float,
                  rotary_base: float, eps: float, dtype):
@@ -55,6 +56,8 @@ class LatentAttention(nn.Module):
 
     def splits(self, batch) -> int:
         groups = -(-batch.max_q * self.heads // 16) * batch.n_seqs
+        if self.uk.dtype == torch.bfloat16 and self.row_elems() <= self.WAVE_ROW:
+            return max(1, min(self.WAVE_WORKGROUPS // groups, -(-batch.max_context // 128), 64))
         return max(1, min(-(-self.TARGET_WORKGROUPS // groups), -(-batch.max_context // 128), 64))
 
     def forward(self, h: torch.Tensor, batch, cache: torch.Tensor) -> torch.Tensor:
