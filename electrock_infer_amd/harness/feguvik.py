@@ -136,6 +136,14 @@ class FeguvikForCausalLM(DecoderModel):
         self.final_norm = nn.Parameter(torch.ones(W, dtype=torch.float32), requires_grad=False)
         self.head = matrix(cfg.vocab_size, W)
         self.runs = cfg.runs()
+        self.chunk_heads = max([l.mixer["heads"] for l in cfg.layers if l.kind == "gla"], default=1)
+
+    def chunk_tokens(self, tokens: int) -> int:
+        """As short as leaves the linear attention's chunks a few workgroups per CU: the blocks of a chunk are walked through
+        one after the other (us of all its kernels, 16 heads: 300 tokens in chunks of 32 32, 64 41, 256 103; 1024 in 64 44,
+        256 101; 2048 in 64 65, 256 115; 4096 in 128 108, 64 124, 256 127; 8192 in 256 188, 128 208)."""
+        work = tokens * self.chunk_heads
+        return 32 if work <= 8192 else 64 if work <= 49152 else 128 if work <= 98304 else 256
 
     # ---- forward ----
     def forward(self, batch: RaggedBatch) -> torch.Tensor:
