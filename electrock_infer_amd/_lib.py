@@ -45,7 +45,7 @@ EXPORTED_SYMBOLS = (
 
 # every function include/electrock_decoder.h declares
 DECODER_SYMBOLS = (
-    "ed_version", "ed_embed", "ed_residual_norm", "ed_relu_squared", "ed_silu_gate", "ed_gated_norm", "ed_token_gate", "ed_skinny_gemm_splits", "ed_skinny_gemm",
+    "ed_version", "ed_embed", "ed_residual_norm", "ed_relu_squared", "ed_silu_gate", "ed_gated_norm", "ed_argmax", "ed_token_gate", "ed_skinny_gemm_splits", "ed_skinny_gemm",
     "ed_decode_gemm_splits", "ed_decode_gemm_plain_pays", "ed_decode_gemm",
     "ed_token_side_supported", "ed_token_side", "ed_gla_prefill", "ed_gla_step",
     "ed_recur_record", "ed_recur_prefill", "ed_recur_step",
@@ -204,6 +204,7 @@ def load_decoder() -> ctypes.CDLL:
         "ed_relu_squared": [vp, i64, i32, vp],
         "ed_silu_gate": [vp, vp, i64, i32, i32, vp],
         "ed_gated_norm": [vp, vp, i64, vp, i64, i32, i32, dbl, i32, vp],
+        "ed_argmax": [vp, i64, i32, vp, vp],
         "ed_recur_record": [i32],
         "ed_recur_prefill": [ctypes.POINTER(RecurArgs), vp],
         "ed_recur_step": [ctypes.POINTER(RecurArgs), vp],

@@ -27,6 +27,7 @@ int launch_residual_norm(int update, float* x, const void* y, int y_dtype, int y
                          void* out, int64_t out_stride, int64_t T, int W, float eps, int dtype, hipStream_t s);
 int launch_relu_squared(void* u, int64_t n, int dtype, hipStream_t s);
 int launch_silu_gate(const void* u, void* out, int64_t T, int ff, int dtype, hipStream_t s);
+int launch_argmax(const float* x, int64_t T, int V, int32_t* out, hipStream_t s);
 int launch_gated_norm(void* y, const void* z, int64_t z_stride, const float* w, int64_t T, int parts, int size, float eps, int dtype,
                       hipStream_t s);
 

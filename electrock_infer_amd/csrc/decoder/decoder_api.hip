@@ -183,6 +183,13 @@ int ed_gated_norm(void* y, const void* z, int64_t z_stride, const float* w, int6
     return launch_gated_norm(y, z, z_stride, w, T, parts, size, static_cast<float>(eps), dtype, as_stream(stream));
 }
 
+int ed_argmax(const float* x, int64_t T, int V, int32_t* out, void* stream) {
+    if (T < 0 || T > kMaxRows || V <= 0 || V > (1 << 30)) return EM_ERR_BAD_SHAPE;
+    if (T == 0) return 0;
+    if (!x || !out) return EM_ERR_NULL_POINTER;
+    return launch_argmax(x, T, V, out, as_stream(stream));
+}
+
 int ed_skinny_gemm_splits(int64_t T, int N, int K) { return skinny_supported(T, N, K) ? skinny_splits(static_cast<int>(T), N, K) : 0; }
 
 int ed_skinny_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,

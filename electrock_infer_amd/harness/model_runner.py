@@ -5,6 +5,7 @@ from typing import List, Optional
 
 import torch
 
+from ..layers.decoder_ops import argmax_rows
 from ..utils.loader import load_model
 from .batch import make_ragged
 from .config import EngineConfig
@@ -134,7 +135,7 @@ class ModelRunner:
     def run(self, seqs: List[Sequence], is_prefill: bool, return_logits: bool = False):
         logits = self.logits(seqs, is_prefill)
         if all(s.temperature == 0 for s in seqs):
-            token_ids = logits.argmax(dim=-1).tolist()
+            token_ids = (argmax_rows(logits) if self.ragged else logits.argmax(dim=-1)).tolist()
         else:
             temperatures = self._to_device([s.temperature for s in seqs], torch.float32)
             token_ids = self.sampler(logits, temperatures).tolist()

@@ -110,6 +110,15 @@ def relu_squared_(u: torch.Tensor) -> torch.Tensor:
     return u
 
 
+def argmax_rows(x: torch.Tensor) -> torch.Tensor:
+    """int32 [T]: the place of the largest value of every row of ``x`` [T, V] (float32), the first of equal ones."""
+    x = x.contiguous()
+    out = torch.empty(x.shape[0], dtype=torch.int32, device=x.device)
+    _lib.check_decoder(_lib.load_decoder().ed_argmax(x.data_ptr(), x.shape[0], x.shape[1], out.data_ptr(),
+                                                     _lib.current_stream(x.device)), "argmax")
+    return out
+
+
 def gated_norm_(y: torch.Tensor, z_ptr: int, z_stride: int, weight: torch.Tensor, parts: int, eps: float) -> torch.Tensor:
     """y = y * silu(z), RMS-normed in equal parts of a row, times ``weight``; in place."""
     T, inner = y.shape

@@ -45,6 +45,9 @@ int ed_silu_gate(const void* u, void* out, int64_t T, int ff, int dtype, void* s
 int ed_gated_norm(void* y, const void* z, int64_t z_stride, const float* w, int64_t T, int parts, int size, double eps, int dtype,
                   void* stream);
 
+/* out [T]: place of the largest of x [T, V]'s values in every row, the first of equal ones; a NaN counts as the largest. */
+int ed_argmax(const float* x, int64_t T, int V, int32_t* out, void* stream);
+
 /* out = act(x w^T) for a decode batch, bf16 operands: x [T, K], w [N, K], T <= 64 (fewer for large
  * weights), K a multiple of 64; act 0: none,
  * 1: max(v, 0)^2, 2: w is [2 N, K], out = silu(x w_c) * (x w_(N + c)) in bf16.  splits > 1: out is float32 [splits, T, N], partial sums over K (no act).  ed_skinny_gemm_splits: how
