@@ -242,16 +242,25 @@ def check_decoder(code: int, what: str) -> None:
         raise RuntimeError(f"{what} failed: {ERROR_TEXT.get(code, 'HIP error')} (status {code})")
 
 
+_dtype_codes = {}
+
+
 def dtype_code(dtype) -> int:
-    import torch
+    if not _dtype_codes:
+        import torch
+        _dtype_codes.update({torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16})
     try:
-        return {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16}[dtype]
+        return _dtype_codes[dtype]
     except KeyError:
         raise RuntimeError(f"unsupported element type {dtype}") from None
 
 
 def current_stream(device) -> int:
+    """The handle of torch's current stream of a device (without the Stream object that wraps it: 0.3 us instead of 3.5,
+    on every launch)."""
     import torch
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
