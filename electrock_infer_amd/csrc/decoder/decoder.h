@@ -43,7 +43,8 @@ struct TokenSideProblem {
     float* x;                // [T, W]
     const uint16_t* y;       // [T, W]
     const float *post_w, *side_norm, *next_w;
-    const uint16_t *gate, *proj;   // [dim, W], [W, dim]
+    const uint16_t *gate, *proj;   // [dim, W], [W, dim]; packed: 16 x 32 pieces in operand order, k steps outside / inside
+    bool packed;
     const int32_t* tokens;
     const uint16_t* table;
     int64_t table_stride;
@@ -58,6 +59,7 @@ struct TokenSideProblem {
 int launch_token_gate(const void* x, const void* gate, const int32_t* tokens, const void* table, int64_t table_stride,
                       int column0, void* g, int64_t T, int W, int dim, int dtype, hipStream_t s);
 bool token_side_supported(int W, int dim);
+inline bool token_side_packable(int W, int dim) { return W % 128 == 0 && dim % 32 == 0; }
 int launch_token_side(TokenSideProblem p, hipStream_t s);
 
 // ---- gla.hip ----

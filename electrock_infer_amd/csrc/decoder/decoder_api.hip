@@ -229,11 +229,12 @@ int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const 
 
 int ed_token_side_supported(int W, int dim) { return token_side_supported(W, dim) ? 1 : 0; }
 
-int ed_token_side(float* x, const void* y, const float* post_w, const void* gate, const void* proj, const int32_t* tokens,
+namespace {
+int token_side(bool packed, float* x, const void* y, const float* post_w, const void* gate, const void* proj, const int32_t* tokens,
                   const void* table, int64_t table_stride, int column0, const float* side_norm, const float* next_w, void* out,
                   int64_t out_stride, int64_t T, int W, int dim, double eps, void* stream) {
     if (T < 0 || T > kMaxRows || column0 < 0 || column0 + static_cast<int64_t>(dim) > table_stride || out_stride < W) return EM_ERR_BAD_SHAPE;
-    if (!token_side_supported(W, dim) || out_stride % 4 != 0) return EM_ERR_UNSUPPORTED;
+    if (!token_side_supported(W, dim) || out_stride % 4 != 0 || (packed && !token_side_packable(W, dim))) return EM_ERR_UNSUPPORTED;
     if (T == 0) return 0;
     if (!x || !y || !post_w || !gate || !proj || !tokens || !table || !side_norm || !out) return EM_ERR_NULL_POINTER;
     if (!aligned16(x) || !aligned16(y) || !aligned16(post_w) || !aligned16(gate) || !aligned16(proj) || !aligned16(side_norm) ||
@@ -252,9 +253,25 @@ int ed_token_side(float* x, const void* y, const float* post_w, const void* gate
     p.out = static_cast<uint16_t*>(out);
     p.out_stride = out_stride;
     p.T = T;
+    p.packed = packed;
     p.W = W; p.dim = dim;
     p.eps = static_cast<float>(eps);
     return launch_token_side(p, as_stream(stream));
+}
+}  // namespace
+
+int ed_token_side(float* x, const void* y, const float* post_w, const void* gate, const void* proj, const int32_t* tokens,
+                  const void* table, int64_t table_stride, int column0, const float* side_norm, const float* next_w, void* out,
+                  int64_t out_stride, int64_t T, int W, int dim, double eps, void* stream) {
+    return token_side(false, x, y, post_w, gate, proj, tokens, table, table_stride, column0, side_norm, next_w, out, out_stride, T, W, dim, eps, stream);
+}
+
+int ed_token_side_packable(int W, int dim) { return token_side_supported(W, dim) && token_side_packable(W, dim) ? 1 : 0; }
+
+int ed_token_side_packed(float* x, const void* y, const float* post_w, const void* gate, const void* proj, const int32_t* tokens,
+                  const void* table, int64_t table_stride, int column0, const float* side_norm, const float* next_w, void* out,
+                  int64_t out_stride, int64_t T, int W, int dim, double eps, void* stream) {
+    return token_side(true, x, y, post_w, gate, proj, tokens, table, table_stride, column0, side_norm, next_w, out, out_stride, T, W, dim, eps, stream);
 }
 
 int ed_gla_prefill(const ed_gla_args* a, void* stream) {

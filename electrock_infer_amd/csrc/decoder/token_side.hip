@@ -8,7 +8,10 @@
 //     out = x / rms(x) * next_w, or x                    (what the next layer reads)
 // A workgroup takes up to 16 rows of the float32 stream.  A row belongs to one wave in the element-wise phases (its sums
 // are wave reductions, no barriers); in between, the rows' bf16 copy in LDS is the first operand of the gate product,
-// whose k range the eight waves share out, and p, rounded to bf16, takes that copy's place for the last phase.
+// whose k range the eight waves share out, and p, rounded to bf16, takes that copy's place for the last phase.  Bound: the
+// bytes of the rows and, in between, the address unit that serves the weights' fragments.  Packed weights lie in operand order,
+// a wave's load is 1 KB that lies whole instead of 16 half-used lines, and what this saves in registers keeps the rows, which
+// were read twice before (8192 rows: W = 1024 45.6 -> 30.9 us, 2048 87.7 -> 70.0, 4096 215 -> 160).
 #include "decoder.h"
 #include "mma.h"
 
@@ -86,8 +89,8 @@ __global__ __launch_bounds__(kThreads) void token_gate_kernel(const typename Ele
 
 // NV: four-element pieces of a row per lane (W <= 256 * NV).  FULL: W % 128 == 0 and dim % 32 == 0, no operand piece is
 // ragged and several weight fragments are fetched together.
-template <int NV, bool FULL>
-__global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(TokenSideProblem p) {
+template <int NV, bool FULL, int RPW, bool PACKED>
+__global__ __launch_bounds__(kThreads, NV <= 8 && (!PACKED || NV * RPW <= 8) ? 4 : 2) void token_side_kernel(TokenSideProblem p) {
     typedef Mma<BF16Elem> M;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
@@ -99,13 +102,14 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
     const int n = static_cast<int>(min(static_cast<int64_t>(p.rows_per_group), p.T - row0));
     const float inv_w = 1.0f / static_cast<float>(W);
 
-    // ---- x + normed y, as bf16, into LDS ----
-    float y_rstd[2];
+    // ---- x + normed y: as bf16 into LDS, and (KEEP) as it is in registers ----
+    constexpr bool KEEP = PACKED;
+    constexpr int R = KEEP ? RPW : 1;
+    float keep[KEEP ? R : 1][KEEP ? NV : 1][4], y_rstd[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int r = wave + i * kWaves;
-        y_rstd[i] = 0.0f;
-        if (r < n) {
+        if (i < RPW && r < n) {
             const uint16_t* yr = p.y + (row0 + r) * W;
             float y[NV][4], sum = 0.0f;
             f32x4_t x[NV];
@@ -131,7 +135,10 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
                     const f32x4_t w4 = *reinterpret_cast<const f32x4_t*>(p.post_w + c);
                     float v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = x[j][e] + y[j][e] * y_rstd[i] * w4[e];
+                    for (int e = 0; e < 4; ++e) {
+                        v[e] = x[j][e] + y[j][e] * y_rstd[i] * w4[e];
+                        if (KEEP) keep[i % R][j % (KEEP ? NV : 1)][e] = v[e];
+                    }
                     store4(Xs + r * LPX + c, v);
                 }
             }
@@ -156,7 +163,7 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
 #pragma unroll
         for (int t = 0; t < kGateTiles; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         if (FULL) {
-            constexpr int kAhead = 4;
+            constexpr int kAhead = KEEP ? 2 : 4;
             for (int s = wave; s < steps; s += kWaves * kAhead) {
                 typename M::frag fw[kAhead][kGateTiles];
 #pragma unroll
@@ -165,7 +172,8 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
 #pragma unroll
                         for (int t = 0; t < kGateTiles; ++t)
                             if (d0 + t * 16 < dim)
-                                fw[u][t] = M::load(p.gate + static_cast<int64_t>(d0 + t * 16 + l16) * W + (s + u * kWaves) * 32 + lq * 8);
+                                fw[u][t] = M::load(PACKED ? p.gate + (static_cast<int64_t>(s + u * kWaves) * (dim / 16) + d0 / 16 + t) * 512 + lane * 8
+                                                          : p.gate + static_cast<int64_t>(d0 + t * 16 + l16) * W + (s + u * kWaves) * 32 + lq * 8);
                     }
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u)
@@ -211,7 +219,7 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
     // ---- p = proj g: every wave a share of the columns ----
     const int col_tiles = (W + 15) / 16;
     if (FULL) {
-        constexpr int kAhead = 8;  // column tiles whose weights are fetched together
+        constexpr int kAhead = KEEP ? 4 : 8;  // column tiles whose weights are fetched together
         for (int t = wave; t < col_tiles; t += kWaves * kAhead) {
             f32x4_t acc[kAhead];
 #pragma unroll
@@ -221,7 +229,8 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u)
                     if (t + u * kWaves < col_tiles)
-                        fw[u] = M::load(p.proj + static_cast<int64_t>((t + u * kWaves) * 16 + l16) * dim + k);
+                        fw[u] = M::load(PACKED ? p.proj + (static_cast<int64_t>(t + u * kWaves) * (dim / 32) + k / 32) * 512 + lane * 8
+                                               : p.proj + static_cast<int64_t>((t + u * kWaves) * 16 + l16) * dim + k);
                 const typename M::frag fg = M::load(Gs + l16 * LPG + k);
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u)
@@ -249,19 +258,34 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
     __syncthreads();
     // ---- the stream and the next layer's input ----
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < RPW; ++i) {
         const int r = wave + i * kWaves;
         if (r >= n) continue;
         const int64_t row = row0 + r;
-        float sum = 0.0f, x[NV][4], y[NV][4];
+        float sum = 0.0f;
+        float x[NV][4];
+        if (KEEP) {
 #pragma unroll
-        for (int j = 0; j < NV; ++j) {
-            const int c = (lane + j * 64) * 4;
-            if (c < W) {
+            for (int j = 0; j < NV; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[j][e] = keep[i % R][j % (KEEP ? NV : 1)][e];
+        } else {
+            f32x4_t x4[NV];
+            float y[NV][4];
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int c = (lane + j * 64) * 4;
+                if (c >= W) continue;
                 load4(p.y + row * W + c, y[j]);
-                const f32x4_t x4 = *reinterpret_cast<const f32x4_t*>(p.x + row * W + c);
+                x4[j] = *reinterpret_cast<const f32x4_t*>(p.x + row * W + c);
+            }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[j][e] = x4[e];
+            for (int j = 0; j < NV; ++j) {
+                const int c = (lane + j * 64) * 4;
+                if (c >= W) continue;
+                const f32x4_t w4 = *reinterpret_cast<const f32x4_t*>(p.post_w + c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[j][e] = x4[j][e] + y[j][e] * y_rstd[i] * w4[e];
             }
         }
 #pragma unroll
@@ -282,11 +306,10 @@ __global__ __launch_bounds__(kThreads, NV <= 8 ? 4 : 2) void token_side_kernel(T
             if (c < W) {
                 float v[4];
                 load4(Xs + r * LPX + c, v);
-                const f32x4_t w4 = *reinterpret_cast<const f32x4_t*>(p.post_w + c);
                 const f32x4_t s4 = *reinterpret_cast<const f32x4_t*>(p.side_norm + c);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    x[j][e] += y[j][e] * y_rstd[i] * w4[e] + v[e] * rstd * s4[e];
+                    x[j][e] += v[e] * rstd * s4[e];
                     sum = fmaf(x[j][e], x[j][e], sum);
                 }
             }
@@ -330,12 +353,22 @@ size_t lds_bytes(int W, int dim, int* g_offset, int* part_offset) {
     return static_cast<size_t>(first) + g + (one_turn ? 0 : kPartBytes);
 }
 
+template <int NV, bool FULL, int RPW, bool PACKED>
+int launch_rows(TokenSideProblem p, size_t lds, hipStream_t s) {
+    p.rows_per_group = RPW * kWaves;
+    const int rc = allow_lds(reinterpret_cast<const void*>(token_side_kernel<NV, FULL, RPW, PACKED>), lds);
+    if (rc != 0) return rc;
+    launch((token_side_kernel<NV, FULL, RPW, PACKED>), dim3(static_cast<unsigned>(ceil_div(p.T, p.rows_per_group))), dim3(kThreads), lds, s, p);
+    return launch_status();
+}
+
+// One row per wave while two do not fill the chip; and where two would leave one workgroup to a CU, whose phases then wait for
+// each other (rows kept in registers; us for 8192 rows, one / two: W = 1024 37 / 31, 2048 70 / 82, 4096 200 / 160).
 template <int NV, bool FULL>
 int launch_side(const TokenSideProblem& p, size_t lds, hipStream_t s) {
-    const int rc = allow_lds(reinterpret_cast<const void*>(token_side_kernel<NV, FULL>), lds);
-    if (rc != 0) return rc;
-    launch((token_side_kernel<NV, FULL>), dim3(static_cast<unsigned>(ceil_div(p.T, p.rows_per_group))), dim3(kThreads), lds, s, p);
-    return launch_status();
+    if constexpr (FULL)
+        if (p.packed) return p.T <= 512 || NV == 8 ? launch_rows<NV, FULL, 1, true>(p, lds, s) : launch_rows<NV, FULL, 2, true>(p, lds, s);
+    return p.T <= 512 ? launch_rows<NV, FULL, 1, false>(p, lds, s) : launch_rows<NV, FULL, 2, false>(p, lds, s);
 }
 
 }  // namespace
@@ -361,8 +394,7 @@ bool token_side_supported(int W, int dim) {
 
 int launch_token_side(TokenSideProblem p, hipStream_t s) {
     const size_t lds = lds_bytes(p.W, p.dim, &p.g_offset, &p.part_offset);
-    p.rows_per_group = p.T <= 512 ? 8 : 16;  // one row per wave while the chip is not full
-    if (p.W % 128 == 0 && p.dim % 32 == 0) {
+    if (token_side_packable(p.W, p.dim)) {
         if (p.W <= 1024) return launch_side<4, true>(p, lds, s);
         if (p.W <= 2048) return launch_side<8, true>(p, lds, s);
         return launch_side<16, true>(p, lds, s);

@@ -111,8 +111,9 @@ class FeguvikLayer(nn.Module):
         self.post1 = (self.norm1b * self.ls1).contiguous()
         if self.mlp is not None:
             self.post2 = (self.norm2b * self.ls2).contiguous()
-        if hasattr(self.mix, "finish_loading"):
-            self.mix.finish_loading()
+        for part in (self.mix, self.side):
+            if hasattr(part, "finish_loading"):
+                part.finish_loading()
 
 
 class FeguvikForCausalLM(DecoderModel):

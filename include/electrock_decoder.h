@@ -76,6 +76,14 @@ int ed_token_side(float* x, const void* y, const float* post_w, const void* gate
                   const void* table, int64_t table_stride, int column0, const float* side_norm, const float* next_w, void* out,
                   int64_t out_stride, int64_t T, int W, int dim, double eps, void* stream);
 
+/* The same with the weights in operand order, for W a multiple of 128 and dim of 32 (ed_token_side_packable): gate as
+ * [W / 32][dim / 16] and proj as [W / 16][dim / 32] pieces of 16 rows x 32 columns, a piece as [4][16][8]: eight columns,
+ * row, columns of the eight. */
+int ed_token_side_packable(int W, int dim);
+int ed_token_side_packed(float* x, const void* y, const float* post_w, const void* gate, const void* proj, const int32_t* tokens,
+                         const void* table, int64_t table_stride, int column0, const float* side_norm, const float* next_w, void* out,
+                         int64_t out_stride, int64_t T, int W, int dim, double eps, void* stream);
+
 /*
  * Gated linear attention: S_t = diag(alpha_t) S_(t-1) + k_t v_t^T, o_t = S_t^T (q_scale q_t), alpha =
  * sigmoid(a2 a1_t + bias)^(1/tau); o is RMS-normed per head with norm_w, multiplied by silu(g), rounded to dtype.
