@@ -22,6 +22,8 @@ constexpr float kFixedCap = 40.0f;    // up to here exp(-2 cap) is a normal floa
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
+__device__ __forceinline__ f32x4_t fma4(f32x4_t a, f32x4_t b, f32x4_t c) { return __builtin_elementwise_fma(a, b, c); }
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
@@ -374,18 +376,31 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
 }
 
 // ---- long portions ----
+// What bounds it: the vector units (54 % busy) and the matrix units (26 %) take turns, as a wave's scores wait for one product
+// and its second product for the scores, with two waves on a SIMD.  So a score is kept cheap and a tile free of waits:
+//   * the cap's tanh takes two of the three slow instructions of a score (exponential, reciprocal).  Up to kTanhRange caps
+//     tanh(x) is x times a polynomial of degree four in x * x (least largest relative error, 7.3e-8: about half a unit in the
+//     last place); a wave whose 32 x 64 scores all lie there takes it, four scores in step, others take the exponential.  Caps
+//     are chosen far above ordinary scores.
+//   * the page of a tile's keys is asked for a tile ahead of its use and in front of the loads that use the one before, and the
+//     rows are read from LDS in front of the barrier; loads have no condition of their own (keys behind the last stand for it).
+// One prompt of 8192 tokens, 16 heads of 128, cap 30: 427 -> 386 us, window 1024: 119.5 -> 112.6; scores beyond the range
+// 422 -> 401, no cap 386 -> 368; 8 x 1000 tokens, heads of 64: 61.7 -> 59.4; heads of 256 / 64: 249 -> 228.  Two tiles in LDS
+// with one barrier a tile were no faster (394 us, 114).
+constexpr float kTanhRange = 0.6f;
 constexpr int kTileKeys = 64;
 constexpr int kRowsPerWave = 32;
 constexpr int kRows = 4 * kRowsPerWave;
 
 template <int DKT, int DVT>
-__global__ __launch_bounds__(256, 2) void attn_prompt_kernel(AttnProblem p) {
+__global__ __launch_bounds__(256, DKT == 2 && DVT == 4 ? 3 : 2) void attn_prompt_kernel(AttnProblem p) {
     typedef Mma<BF16Elem> M;
     constexpr int LPK = DKT * 32 + 8, LPV = DVT * 16 + 8;
+    constexpr bool kPoly = DKT <= 4;       // registers enough for a second form of the scores
     constexpr int kFetchK = kTileKeys * DKT * 4 / 256, kFetchV = kTileKeys * DVT * 2 / 256;
     __shared__ __attribute__((aligned(16))) uint16_t Ks[kTileKeys * LPK];
     __shared__ __attribute__((aligned(16))) uint16_t Vs[kTileKeys * LPV];
-    __shared__ int Kr[2][kTileKeys];                                 // cache row of every key of a tile, -1: no key
+    __shared__ int64_t Kr[2][kTileKeys];                             // where every key of a tile lies in the cache, -1: no key
     const int h = blockIdx.x, seq = blockIdx.z, g = h / (p.heads / p.kv_heads);
     const int row0 = p.q_begin[seq], nq = p.q_begin[seq + 1] - row0;
     const int t0 = (static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y)) * kRows;  // long rows start first
@@ -412,39 +427,53 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(AttnProblem p) {
     const int32_t* table = p.tables + static_cast<int64_t>(seq) * p.table_width;
     const uint16_t* keys = static_cast<const uint16_t*>(p.cache) + g * dp;
     const uint16_t* values = static_cast<const uint16_t*>(p.cache) + p.kv_heads * dp + g * vp;
-    auto find_rows = [&](int tile) {
-        if (tid < kTileKeys && tile < tile1) {
-            const int key = tile * kTileKeys + tid;
-            Kr[tile & 1][tid] = key <= last_pos ? table[key / p.block_size] * p.block_size + key % p.block_size : -1;
-        }
+    // the page of the key that thread tid < 64 looks up; keys behind the last one stand for it (their scores are masked)
+    auto key_of = [&](int tile) { return min(tile * kTileKeys + tid, last_pos); };
+    auto page_of = [&](int tile) { return tid < kTileKeys ? table[key_of(tile) / p.block_size] : 0; };
+    auto keep_rows = [&](int tile, int page) {
+        if (tid < kTileKeys) Kr[tile & 1][tid] = static_cast<int64_t>(page * p.block_size + key_of(tile) % p.block_size) * row_elems;
     };
     typename M::frag rk[kFetchK], rv[kFetchV];
-    auto fetch = [&](int tile) {
+    int64_t at_k[kFetchK], at_v[kFetchV];
+    auto read_rows = [&](int tile) {
 #pragma unroll
-        for (int i = 0; i < kFetchK; ++i) {
-            const int e = tid + i * 256, c = (e % (DKT * 4)) * 8, row = Kr[tile & 1][e / (DKT * 4)];
-            rk[i] = c < dp && row >= 0 ? M::load(keys + static_cast<int64_t>(row) * row_elems + c) : M::zero();
+        for (int i = 0; i < kFetchK; ++i) at_k[i] = Kr[tile & 1][(tid + i * 256) / (DKT * 4)];
+#pragma unroll
+        for (int i = 0; i < kFetchV; ++i) at_v[i] = Kr[tile & 1][(tid + i * 256) / (DVT * 2)];
+    };
+    const int cv = min((tid % (DVT * 2)) * 8, vp - 8);   // value columns behind the last are not stored
+    auto fetch = [&]() {
+        if (dp == DKT * 32) {
+#pragma unroll
+            for (int i = 0; i < kFetchK; ++i) rk[i] = M::load(keys + (tid + i * 256) % (DKT * 4) * 8 + at_k[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kFetchK; ++i) {
+                const int c = (tid + i * 256) % (DKT * 4) * 8;
+                rk[i] = c < dp ? M::load(keys + c + at_k[i]) : M::zero();
+            }
         }
 #pragma unroll
-        for (int i = 0; i < kFetchV; ++i) {
-            const int e = tid + i * 256, c = (e % (DVT * 2)) * 8, row = Kr[tile & 1][e / (DVT * 2)];
-            rv[i] = c < vp && row >= 0 ? M::load(values + static_cast<int64_t>(row) * row_elems + c) : M::zero();
-        }
+        for (int i = 0; i < kFetchV; ++i) rv[i] = M::load(values + cv + at_v[i]);
     };
     f32x4_t o[DVT][2];
 #pragma unroll
     for (int d = 0; d < DVT; ++d) o[d][0] = o[d][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const bool capped = p.softcap > 0.0f, fixed = capped && p.softcap <= kFixedCap;
     const float c2 = p.scale * kLog2e, cap2 = p.softcap * kLog2e, in_cap = capped ? 2.0f * kLog2e * p.scale / p.softcap : 0.0f;
-    // running maxima in units of log2 (the cap is one that never has to be raised); l: this lane's share
-    float m[2], l[2] = {0.0f, 0.0f};
-    m[0] = m[1] = fixed ? cap2 : -INFINITY;
+    const float to_cap = capped ? p.scale / p.softcap : 0.0f;
+    const float tanh0 = cap2 * 0.99999994f, tanh1 = cap2 * -0.33332309f, tanh2 = cap2 * 0.13310173f, tanh3 = cap2 * -0.05210148f, tanh4 = cap2 * 0.015475428f;
+    // running maxima in units of log2 (not kept where the cap stands for them); l: this lane's share
+    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
 
-    find_rows(tile0);
-    find_rows(tile0 + 1);
+    keep_rows(tile0, page_of(tile0));
+    keep_rows(tile0 + 1, page_of(tile0 + 1));
+    int page = page_of(tile0 + 2);
     __syncthreads();
-    fetch(tile0);
+    read_rows(tile0);
+    fetch();
     for (int tile = tile0; tile < tile1; ++tile) {
+        read_rows(tile + 1);
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < kFetchK; ++i) {
@@ -456,9 +485,12 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(AttnProblem p) {
             const int e = tid + i * 256;
             store_frag<BF16Elem>(Vs + (e / (DVT * 2)) * LPV + (e % (DVT * 2)) * 8, rv[i]);
         }
-        if (tile + 1 < tile1) fetch(tile + 1);
+        // A page is asked for one tile before its rows are kept, and in front of the next tile's loads: loads come back in
+        // order, and a wave that waited for its page behind them would wait for them all.
+        keep_rows(tile + 2, page);
+        page = page_of(tile + 3);
+        if (tile + 1 < tile1) fetch();
         __syncthreads();
-        find_rows(tile + 2);     // into the half that this tile's rows leave; read behind the next barriers
         const int k0 = tile * kTileKeys;
         // no key of this tile for this wave's queries
         if (k0 > first_pos + kRowsPerWave - 1 || k0 + kTileKeys - 1 < first_pos - window + 1) continue;
@@ -474,8 +506,34 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(AttnProblem p) {
                 s[n][0] = M::mac(fk, fq[0][k], s[n][0]);
                 s[n][1] = M::mac(fk, fq[1][k], s[n][1]);
             }
-        // scores in units of log2
-        if (capped) {
+        // scores in units of log2; with a fixed maximum their distance to it
+        if (kPoly && fixed) {
+            float top = 0.0f;
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) top = fmaxf(top, fabsf(s[n][j][r]));
+            if (__all(top * fabsf(to_cap) <= kTanhRange)) {
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const f32x4_t x = s[n][j] * to_cap, u = x * x;
+                        f32x4_t t = fma4(fma4(f32x4_t(tanh4), u, f32x4_t(tanh3)), u, f32x4_t(tanh2));
+                        t = fma4(fma4(t, u, f32x4_t(tanh1)), u, f32x4_t(tanh0));
+                        s[n][j] = fma4(x, t, f32x4_t(-cap2));
+                    }
+            } else {
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) s[n][j][r] = -2.0f * cap2 * __builtin_amdgcn_rcpf(exp2_fast(s[n][j][r] * in_cap) + 1.0f);
+            }
+        } else if (capped) {
 #pragma unroll
             for (int n = 0; n < 4; ++n)
 #pragma unroll
@@ -505,7 +563,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(AttnProblem p) {
         float alpha[2] = {1.0f, 1.0f};
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            float base = m[j];
+            float base = kPoly ? 0.0f : cap2;
             if (!fixed) {
                 float mx = -INFINITY;
 #pragma unroll
