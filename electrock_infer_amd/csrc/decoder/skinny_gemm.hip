@@ -172,10 +172,10 @@ int launch_form(const uint16_t* x, const uint16_t* w, void* out, bool f32, int s
 // Tiles of weight rows per workgroup: as few as leave one workgroup of eight waves to a CU (us, with 64 tokens: 3072 rows of
 // 2048 in ones 8.8, in twos 10.7; 6176 in twos 11.9, ones 17.4, fours 15.3; 8512 in fours 16.9, twos 19.5; with up to 32
 // tokens two such workgroups share a CU, and the few beyond the first 256 cost less than half of the chip without work: 8512,
-// T = 1, twos 10.0, fours 11.8).  Beyond 64 rows to a CU workgroups of four waves, of which two share a CU (32000 x 2048, T = 32: 25.0 / 29.3 with eight).  With three or four
-// tiles of tokens those carry one step of k instead of two (T = 64: 31.5 / 38.4), and partial sums take 64 rows as soon as
-// four ranges of K fill the chip that way, since the token rows are read by half as many workgroups (4096 x 12288, T = 64:
-// 26.8 / 30.5; T = 32: 22.6 / 22.6).
+// T = 1, twos 10.0, fours 11.8).  Beyond 64 rows to a CU workgroups of four waves, of which two share a CU (32000 x 2048,
+// T = 32: 25.0 / 29.3 with eight).  With three or four tiles of tokens those carry one step of k instead of two (T = 64:
+// 31.5 / 38.4), and partial sums take 64 rows as soon as four ranges of K fill the chip that way, since the token rows are
+// read by half as many workgroups (4096 x 12288, T = 64: 26.8 / 30.5; T = 32: 22.6 / 22.6).
 template <int MT>
 int launch_tokens(const uint16_t* x, const uint16_t* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s) {
     const int rows = act == 2 ? 2 * N : N;

@@ -17,7 +17,8 @@ class TokenSideInput(nn.Module):
         self.gate = nn.Parameter(torch.zeros(dim, width, dtype=dtype), requires_grad=False)
         self.proj = nn.Parameter(torch.zeros(width, dim, dtype=dtype), requires_grad=False)
         self.norm = nn.Parameter(torch.ones(width, dtype=torch.float32), requires_grad=False)
-        self.packed = None       # (gate, proj) in operand order
+        for name in ("gate_packed", "proj_packed"):      # in operand order; they move with the module and are not saved
+            self.register_buffer(name, None, persistent=False)
 
     def finish_loading(self) -> None:
         """Forms of the weights that the one-launch kernel reads: pieces of 16 rows x 32 columns, each as an MFMA takes it, so
@@ -25,7 +26,7 @@ class TokenSideInput(nn.Module):
         dim, W = self.gate.shape
         if self.gate.dtype == torch.bfloat16 and _lib.load_decoder().ed_token_side_packable(W, dim):
             pieces = lambda w: w.data.view(w.shape[0] // 16, 16, w.shape[1] // 32, 4, 8).permute(0, 2, 3, 1, 4)
-            self.packed = (pieces(self.gate).transpose(0, 1).contiguous(), pieces(self.proj).contiguous())
+            self.gate_packed, self.proj_packed = pieces(self.gate).transpose(0, 1).contiguous(), pieces(self.proj).contiguous()
 
     def forward(self, x: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
         """x [T, width] (the stream in the compute type) -> what is to be normed with ``norm`` and added."""
@@ -39,8 +40,9 @@ class TokenSideInput(nn.Module):
         T, W = x.shape
         lib, dim = _lib.load_decoder(), self.gate.shape[0]
         if T >= self.ONE_LAUNCH_ROWS * W and y.dim() == 2 and y.dtype == torch.bfloat16 and out.stride(0) % 4 == 0 and lib.ed_token_side_supported(W, dim) == 1:
-            gate, proj = self.packed or (self.gate, self.proj)
-            run = lib.ed_token_side_packed if self.packed else lib.ed_token_side
+            packed = self.gate_packed is not None
+            gate, proj = (self.gate_packed, self.proj_packed) if packed else (self.gate, self.proj)
+            run = lib.ed_token_side_packed if packed else lib.ed_token_side
             code = run(x.data_ptr(), y.data_ptr(), post_w.data_ptr(), gate.data_ptr(), proj.data_ptr(), tokens.data_ptr(),
                        table.data_ptr(), table.stride(0), self.column0, self.norm.data_ptr(), None if next_w is None else next_w.data_ptr(),
                        out.data_ptr(), out.stride(0), T, W, dim, float(eps), _lib.current_stream(x.device))

@@ -30,7 +30,7 @@ def test_packed_weights(W, T, dim, last):
     for packed in (False, True):
         if packed:
             side.finish_loading()
-            assert side.packed is not None
+            assert side.gate_packed is not None and "gate_packed" not in side.state_dict()
         stream, out = x.clone(), torch.full((T, W + 4), 7.0, dtype=torch.bfloat16, device="cuda")
         side.close_layer(stream, y, post, tokens, table, 1e-6, out[:, :W], nxt)
         assert bool((out[:, W:] == 7).all())
