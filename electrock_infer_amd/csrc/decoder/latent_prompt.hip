@@ -2,11 +2,12 @@
 // matrix products over the latents of the context (keys [K, heads * dim], values transposed [heads * vdim, K]) and a
 // tiled softmax attention runs on them.
 //
-// A workgroup takes 128 queries of one head, 32 per wave.  Per tile of 64 keys a wave computes S^T = K Q^T: a lane then
-// holds, for one query, keys (lane / 16) * 4 + 0..3 of every 16.  Since a sum over keys may run in any order as long as
-// both operands agree, these registers, rounded to bf16, are the second operand of O^T = V^T P^T as they are: the values
-// only have to lie in LDS in the matching key order.  Nothing of the probabilities goes through LDS, the running maximum
-// and sum of a query live in one register of its four lanes, and a lane's results are four neighbouring outputs.
+// A workgroup takes 128 queries of one head, 32 per wave, or half as many where that leaves CUs without work.  Per tile of 64
+// keys a wave computes S^T = K Q^T: a lane then holds, for one query, keys (lane / 16) * 4 + 0..3 of every 16.  Since a sum
+// over keys may run in any order as long as both operands agree, these registers, rounded to bf16, are the second operand of
+// O^T = V^T P^T as they are: the values only have to lie in LDS in the matching key order.  Nothing of the probabilities goes
+// through LDS, the running maximum and sum of a query live in one register of its four lanes, and a lane's results are four
+// neighbouring outputs.
 #include "decoder.h"
 #include "mma.h"
 
@@ -14,14 +15,13 @@ namespace em {
 namespace {
 
 constexpr int kTileKeys = 64;
-constexpr int kRowsPerWave = 32;
-constexpr int kRows = 4 * kRowsPerWave;
 constexpr float kLog2e = 1.4426950408889634f;
 
-// DKT: 32-element steps of dim + rot; DVT: 16-element tiles of vdim
-template <int DKT, int DVT>
+// DKT: 32-element steps of dim + rot; DVT: 16-element tiles of vdim; QT: 16-query tiles of a wave
+template <int DKT, int DVT, int QT>
 __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPromptProblem p) {
     typedef Mma<BF16Elem> M;
+    constexpr int kRowsPerWave = 16 * QT, kRows = 4 * kRowsPerWave;
     constexpr int LPK = DKT * 32 + 8, LPV = kTileKeys + 8;
     constexpr int kFetchK = kTileKeys * DKT * 4 / 256, kFetchV = DVT * 16 * (kTileKeys / 8) / 256;
     __shared__ __attribute__((aligned(16))) uint16_t Ks[kTileKeys * LPK];
@@ -37,9 +37,9 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPromptProbl
     const int n_tiles = (start + min(t0 + kRows, nq) + kTileKeys - 1) / kTileKeys;
     const int first_pos = start + t0 + wave * kRowsPerWave;      // of this wave's first query
 
-    typename M::frag fq[2][DKT];
+    typename M::frag fq[QT][DKT];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < QT; ++j) {
         const int t = t0 + wave * kRowsPerWave + j * 16 + l16;
         const uint16_t* q = p.q + (row0 + static_cast<int64_t>(min(t, nq - 1))) * p.q_stride + h * D;
 #pragma unroll
@@ -66,10 +66,17 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPromptProbl
         }
     };
 
-    f32x4_t o[DVT][2];
+    f32x4_t o[DVT][QT];
 #pragma unroll
-    for (int d = 0; d < DVT; ++d) o[d][0] = o[d][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};   // m in units of log2; l: this lane's share
+    for (int d = 0; d < DVT; ++d)
+#pragma unroll
+        for (int j = 0; j < QT; ++j) o[d][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    float m[QT], l[QT];   // m in units of log2; l: this lane's share
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+        m[j] = -INFINITY;
+        l[j] = 0.0f;
+    }
     const float c2 = p.scale * kLog2e;
 
     fetch(0);
@@ -94,30 +101,33 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPromptProbl
         if (tile + 1 < n_tiles) fetch(tile + 1);
         if (tile * kTileKeys > first_pos + kRowsPerWave - 1) continue;   // no key of this tile for this wave's queries
 
-        f32x4_t s[4][2];
+        f32x4_t s[4][QT];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) s[n][0] = s[n][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int j = 0; j < QT; ++j) s[n][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k = 0; k < DKT; ++k)
 #pragma unroll
             for (int n = 0; n < 4; ++n) {
                 const typename M::frag fk = M::load(Ks + (n * 16 + l16) * LPK + k * 32 + lq * 8);
-                s[n][0] = M::mac(fk, fq[0][k], s[n][0]);
-                s[n][1] = M::mac(fk, fq[1][k], s[n][1]);
+#pragma unroll
+                for (int j = 0; j < QT; ++j) s[n][j] = M::mac(fk, fq[j][k], s[n][j]);
             }
         if (tile * kTileKeys + kTileKeys - 1 > first_pos) {
 #pragma unroll
             for (int n = 0; n < 4; ++n)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < QT; ++j)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
                         if (tile * kTileKeys + n * 16 + lq * 4 + r > first_pos + j * 16 + l16) s[n][j][r] = -INFINITY;
         }
-        typename M::frag fp[2][2];   // [32-key step][query tile]
-        float alpha[2];
+        typename M::frag fp[2][QT];   // [32-key step][query tile]
+        float alpha[QT];
+        bool same = true;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < QT; ++j) {
             float mx = -INFINITY;
 #pragma unroll
             for (int n = 0; n < 4; ++n)
@@ -140,26 +150,26 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPromptProbl
                     fp[n >> 1][j][(n & 1) * 4 + r] = static_cast<__bf16>(e);
                 }
             l[j] = l[j] * alpha[j] + sum;
+            same = same && alpha[j] == 1.0f;
         }
-        if (!__all(alpha[0] == 1.0f && alpha[1] == 1.0f)) {
+        if (!__all(same)) {
 #pragma unroll
-            for (int d = 0; d < DVT; ++d) {
-                o[d][0] *= alpha[0];
-                o[d][1] *= alpha[1];
-            }
+            for (int d = 0; d < DVT; ++d)
+#pragma unroll
+                for (int j = 0; j < QT; ++j) o[d][j] *= alpha[j];
         }
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
             for (int d = 0; d < DVT; ++d) {
                 const typename M::frag fv = M::load(Vs + (d * 16 + l16) * LPV + k * 32 + lq * 8);
-                o[d][0] = M::mac(fv, fp[k][0], o[d][0]);
-                o[d][1] = M::mac(fv, fp[k][1], o[d][1]);
+#pragma unroll
+                for (int j = 0; j < QT; ++j) o[d][j] = M::mac(fv, fp[k][j], o[d][j]);
             }
     }
     const float sk = p.sink[h] * kLog2e;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < QT; ++j) {
         l[j] += __shfl_xor(l[j], 16);
         l[j] += __shfl_xor(l[j], 32);
         const float top = fmaxf(m[j], sk), w = __builtin_amdgcn_exp2f(m[j] - top);
@@ -178,11 +188,24 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPromptProbl
     }
 }
 
+template <int DKT, int DVT, int QT>
+int launch_tiles(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(p.heads), static_cast<unsigned>(ceil_div(max_q, 64 * QT)), static_cast<unsigned>(n_seqs));
+    launch((latent_prompt_kernel<DKT, DVT, QT>), grid, dim3(256), 0, s, p);
+    return launch_status();
+}
+
+// Below two workgroups of 128 queries to a CU, workgroups of 64: a workgroup's time is a chain of tiles, which is shorter with
+// half the products and exponentials to a tile, and CUs without work take the other half (us, 128 / 64 queries, heads of
+// 128 + 64: 48 workgroups, 300 tokens behind 1000, 53.5 / 35.2; 128, one prompt of 1024 42.8 / 29.1; 256, 2048 80 / 59 and
+// 4 x 512 25.7 / 24.0; 384, 3072 123 / 88; 512, 4 x 1024 55.8 / 57.1, 4096 163 / 152, behind 4000 328 / 385; 1024, 8192
+// 397 / 520).  A query's sums keep their order either way.
+constexpr int64_t kFewWorkgroups = 512;
+
 template <int DKT, int DVT>
 int launch_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(p.heads), static_cast<unsigned>(ceil_div(max_q, kRows)), static_cast<unsigned>(n_seqs));
-    launch((latent_prompt_kernel<DKT, DVT>), grid, dim3(256), 0, s, p);
-    return launch_status();
+    if (ceil_div(max_q, 128) * p.heads * n_seqs < kFewWorkgroups) return launch_tiles<DKT, DVT, 1>(p, n_seqs, max_q, s);
+    return launch_tiles<DKT, DVT, 2>(p, n_seqs, max_q, s);
 }
 
 template <int DVT>
