@@ -268,6 +268,14 @@ int ed_token_side(float* x, const void* y, const float* post_w, const void* gate
 
 int ed_token_side_packable(int W, int dim) { return token_side_supported(W, dim) && token_side_packable(W, dim) ? 1 : 0; }
 
+int ed_token_side_pack(const void* gate, const void* proj, void* gate_out, void* proj_out, int W, int dim, void* stream) {
+    if (!ed_token_side_packable(W, dim)) return EM_ERR_UNSUPPORTED;
+    if (!gate || !proj || !gate_out || !proj_out) return EM_ERR_NULL_POINTER;
+    if (!aligned16(gate) || !aligned16(proj) || !aligned16(gate_out) || !aligned16(proj_out)) return EM_ERR_ALIGNMENT;
+    return launch_token_side_pack(static_cast<const uint16_t*>(gate), static_cast<const uint16_t*>(proj), static_cast<uint16_t*>(gate_out),
+                                  static_cast<uint16_t*>(proj_out), W, dim, as_stream(stream));
+}
+
 int ed_token_side_packed(float* x, const void* y, const float* post_w, const void* gate, const void* proj, const int32_t* tokens,
                   const void* table, int64_t table_stride, int column0, const float* side_norm, const float* next_w, void* out,
                   int64_t out_stride, int64_t T, int W, int dim, double eps, void* stream) {

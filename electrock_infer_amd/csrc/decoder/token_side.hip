@@ -11,7 +11,7 @@
 // whose k range the eight waves share out, and p, rounded to bf16, takes that copy's place for the last phase.  Bound: the
 // bytes of the rows and, in between, the address unit that serves the weights' fragments.  Packed weights lie in operand order,
 // a wave's load is 1 KB that lies whole instead of 16 half-used lines, and what this saves in registers keeps the rows, which
-// were read twice before (8192 rows: W = 1024 45.6 -> 30.9 us, 2048 87.7 -> 70.0, 4096 215 -> 160).
+// were read twice before (8192 rows, with the packing: W = 1024 46.9 -> 32.7 us, 2048 84.2 -> 67.8, 4096 215 -> 145).
 #include "decoder.h"
 #include "mma.h"
 
@@ -85,6 +85,21 @@ __global__ __launch_bounds__(kThreads) void token_gate_kernel(const typename Ele
             g[(t0 + r) * dim + d] = Elem::store(gelu_tanh(z) * e);
         }
     }
+}
+
+// The weights in operand order: 16 rows x 32 columns, each piece as an MFMA takes it, 16 bytes per thread.  Made in front of every
+// call that reads them, so that there is no second copy to keep up with weights that are written later (0.25 MB each for
+// 2048 x 64: 2.0 us beside the 66 of 8192 rows).
+__global__ __launch_bounds__(256) void token_side_pack_kernel(const uint16_t* __restrict__ gate, const uint16_t* __restrict__ proj,
+                                                              uint16_t* __restrict__ gate_out, uint16_t* __restrict__ proj_out, int W, int dim) {
+    const int i = blockIdx.x * 256 + threadIdx.x, piece = i / 64, row = i % 16, c = i % 64 / 16 * 8;
+    if (i >= W / 8 * dim) return;
+    const int d0 = piece % (dim / 16) * 16, k = piece / (dim / 16) * 32;       // gate: steps of W outside
+    const int w0 = piece / (dim / 32) * 16, e = piece % (dim / 32) * 32;       // proj: steps of dim inside
+    const bf16x8_t g = Mma<BF16Elem>::load(gate + static_cast<int64_t>(d0 + row) * W + k + c);
+    const bf16x8_t v = Mma<BF16Elem>::load(proj + static_cast<int64_t>(w0 + row) * dim + e + c);
+    store_frag<BF16Elem>(gate_out + static_cast<int64_t>(i) * 8, g);
+    store_frag<BF16Elem>(proj_out + static_cast<int64_t>(i) * 8, v);
 }
 
 // NV: four-element pieces of a row per lane (W <= 256 * NV).  FULL: W % 128 == 0 and dim % 32 == 0, no operand piece is
@@ -390,6 +405,11 @@ int launch_token_gate(const void* x, const void* gate, const int32_t* tokens, co
 bool token_side_supported(int W, int dim) {
     int a, b;
     return W > 0 && W % 4 == 0 && W <= 4096 && dim > 0 && dim <= 1024 && lds_bytes(W, dim, &a, &b) <= kLdsPerCu;
+}
+
+int launch_token_side_pack(const uint16_t* gate, const uint16_t* proj, uint16_t* gate_out, uint16_t* proj_out, int W, int dim, hipStream_t s) {
+    launch(token_side_pack_kernel, dim3(static_cast<unsigned>(ceil_div(W / 8 * dim, 256))), dim3(256), 0, s, gate, proj, gate_out, proj_out, W, dim);
+    return launch_status();
 }
 
 int launch_token_side(TokenSideProblem p, hipStream_t s) {

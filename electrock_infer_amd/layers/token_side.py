@@ -17,16 +17,15 @@ class TokenSideInput(nn.Module):
         self.gate = nn.Parameter(torch.zeros(dim, width, dtype=dtype), requires_grad=False)
         self.proj = nn.Parameter(torch.zeros(width, dim, dtype=dtype), requires_grad=False)
         self.norm = nn.Parameter(torch.ones(width, dtype=torch.float32), requires_grad=False)
-        for name in ("gate_packed", "proj_packed"):      # in operand order; they move with the module and are not saved
+        # Room for the weights in operand order, so that a wave of the one-launch kernel loads 1 KB that lies whole.  Every call that
+        # reads it fills it first, and always from the weights of that moment: calls on several streams write the same bytes.
+        for name in ("gate_packed", "proj_packed"):
             self.register_buffer(name, None, persistent=False)
 
     def finish_loading(self) -> None:
-        """Forms of the weights that the one-launch kernel reads: pieces of 16 rows x 32 columns, each as an MFMA takes it, so
-        that a wave loads 1 KB that lies whole."""
         dim, W = self.gate.shape
         if self.gate.dtype == torch.bfloat16 and _lib.load_decoder().ed_token_side_packable(W, dim):
-            pieces = lambda w: w.data.view(w.shape[0] // 16, 16, w.shape[1] // 32, 4, 8).permute(0, 2, 3, 1, 4)
-            self.gate_packed, self.proj_packed = pieces(self.gate).transpose(0, 1).contiguous(), pieces(self.proj).contiguous()
+            self.gate_packed, self.proj_packed = torch.empty_like(self.gate.data), torch.empty_like(self.proj.data)
 
     def forward(self, x: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
         """x [T, width] (the stream in the compute type) -> what is to be normed with ``norm`` and added."""
@@ -40,12 +39,14 @@ class TokenSideInput(nn.Module):
         T, W = x.shape
         lib, dim = _lib.load_decoder(), self.gate.shape[0]
         if T >= self.ONE_LAUNCH_ROWS * W and y.dim() == 2 and y.dtype == torch.bfloat16 and out.stride(0) % 4 == 0 and lib.ed_token_side_supported(W, dim) == 1:
-            packed = self.gate_packed is not None
-            gate, proj = (self.gate_packed, self.proj_packed) if packed else (self.gate, self.proj)
-            run = lib.ed_token_side_packed if packed else lib.ed_token_side
+            gate, proj, run, stream = self.gate, self.proj, lib.ed_token_side, _lib.current_stream(x.device)
+            if self.gate_packed is not None:
+                gate, proj, run = self.gate_packed, self.proj_packed, lib.ed_token_side_packed
+                _lib.check_decoder(lib.ed_token_side_pack(self.gate.data_ptr(), self.proj.data_ptr(), gate.data_ptr(), proj.data_ptr(),
+                                                          W, dim, stream), "token_side_pack")
             code = run(x.data_ptr(), y.data_ptr(), post_w.data_ptr(), gate.data_ptr(), proj.data_ptr(), tokens.data_ptr(),
                        table.data_ptr(), table.stride(0), self.column0, self.norm.data_ptr(), None if next_w is None else next_w.data_ptr(),
-                       out.data_ptr(), out.stride(0), T, W, dim, float(eps), _lib.current_stream(x.device))
+                       out.data_ptr(), out.stride(0), T, W, dim, float(eps), stream)
             _lib.check_decoder(code, "token_side")
             return
         rows = torch.empty(T, W, dtype=out.dtype, device=x.device)
