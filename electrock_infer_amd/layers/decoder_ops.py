@@ -25,12 +25,9 @@ def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
     """For a decode batch that the weight-streaming kernel takes (at most 64 rows, any size of the weights): how many ranges of
     K fill the chip; else 0."""
     T, (N, K) = x.shape[0], weight.shape
-    if x.dtype != torch.bfloat16 or T > 64 or not x.is_contiguous():
+    if x.dtype != torch.bfloat16 or T > 64 or not x.is_contiguous() or not weight.is_contiguous() or (x.data_ptr() | weight.data_ptr()) % 16:
         return 0
-    lib = _lib.load_decoder()
-    if (x.data_ptr() | weight.data_ptr()) % 16 or not weight.is_contiguous():      # the library takes these
-        return lib.ed_skinny_gemm_splits(T, N, K)
-    return lib.ed_decode_gemm_splits(T, N, K)
+    return _lib.load_decoder().ed_decode_gemm_splits(T, N, K)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
