@@ -23,11 +23,14 @@ def _skinny(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: in
 
 def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
     """For a decode batch that the weight-streaming kernel takes (at most 64 rows, any size of the weights): how many ranges of
-    K fill the chip; else 0."""
-    T, (N, K) = x.shape[0], weight.shape
-    if x.dtype != torch.bfloat16 or T > 64 or not x.is_contiguous() or not weight.is_contiguous() or (x.data_ptr() | weight.data_ptr()) % 16:
+    K fill the chip; else 0: operands that do not fit each other, that are to be differentiated or that are not dense rows from a
+    16-byte boundary are the library's, to compute or to refuse."""
+    if not (x.dtype == weight.dtype == torch.bfloat16 and x.dim() == weight.dim() == 2 and x.shape[0] <= 64 and
+            x.shape[1] == weight.shape[1] and x.device == weight.device and x.is_contiguous() and weight.is_contiguous()):
         return 0
-    return _lib.load_decoder().ed_decode_gemm_splits(T, N, K)
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad) or (x.data_ptr() | weight.data_ptr()) % 16:
+        return 0
+    return _lib.load_decoder().ed_decode_gemm_splits(x.shape[0], *weight.shape)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:

@@ -46,3 +46,36 @@ def test_every_form_gives_the_product(T, N, K):
         assert off(ops.linear(x, w, "relu_squared"), F.relu(want) ** 2) < 3 * 2.0 ** -8, name
         gated = F.silu(want[:, :N // 2]) * want[:, N // 2:]
         assert off(ops.linear_silu_gate(x, w), gated) < 3 * 2.0 ** -8, name
+
+
+def bf16(*shape):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(sum(shape))).to(BF16)
+
+
+# (on the CPU: the product itself never runs on these)
+@pytest.mark.parametrize("x,w", [(bf16(8, 128), bf16(48, 64)), (bf16(8, 64), bf16(48, 128)), (bf16(64, 4096), bf16(6144, 2048)), (bf16(8, 64), bf16(48, 64).float()),
+                                 (bf16(8, 64).float(), bf16(48, 64)), (bf16(8, 64), bf16(48, 64).half())])
+def test_operands_that_do_not_fit_are_refused(x, w):
+    assert ops._skinny_splits(x, w) == 0
+    for product in (ops.linear, ops.linear_parts, lambda x, w: ops.linear(x, w, "relu_squared"), ops.linear_silu_gate):
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            product(x, w)
+
+
+def test_operands_on_two_devices_are_not_taken():
+    assert ops._skinny_splits(bf16(8, 64), torch.empty(48, 64, dtype=BF16, device="meta")) == 0
+
+
+@pytest.mark.parametrize("shape", [(64,), (1, 64), (2, 3, 64), (64, 64, 64), (3, 1, 1, 64)])
+def test_rows_of_any_shape_and_gradients_are_the_librarys(shape):
+    x, w = bf16(*shape), bf16(48, 64)
+    if len(shape) != 2:
+        assert ops._skinny_splits(x, w) == 0 and torch.equal(ops.linear(x, w), F.linear(x, w))
+    x.requires_grad_()
+    assert ops._skinny_splits(x, w) == 0
+    ops.linear(x, w).sum().backward()
+    # (sums of 48 standard normal values, about 20 at most, rounded to bf16)
+    assert float((x.grad - w.float().sum(0)).abs().max()) < 20 * 2.0 ** -8
+    if len(shape) == 2:
+        with torch.no_grad():
+            assert ops._skinny_splits(x, w) > 0
