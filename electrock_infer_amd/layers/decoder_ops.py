@@ -111,7 +111,10 @@ def relu_squared_(u: torch.Tensor) -> torch.Tensor:
 
 
 def argmax_rows(x: torch.Tensor) -> torch.Tensor:
-    """int32 [T]: the place of the largest value of every row of ``x`` [T, V] (float32), the first of equal ones."""
+    """int32 [T]: the place of the largest value of every row of ``x`` [T, V], the first of equal ones; what the kernel does not
+    take (other types, shapes, devices) goes to the library's, along the last dimension."""
+    if x.dtype != torch.float32 or x.dim() != 2 or x.shape[1] == 0 or not x.is_cuda:
+        return x.argmax(dim=-1).int()
     x = x.contiguous()
     out = torch.empty(x.shape[0], dtype=torch.int32, device=x.device)
     _lib.check_decoder(_lib.load_decoder().ed_argmax(x.data_ptr(), x.shape[0], x.shape[1], out.data_ptr(),
