@@ -86,6 +86,8 @@ def _pack(parts: dict, pinned: bool):
     values = host.numpy()
     for to, run in runs:
         if isinstance(run, np.ndarray):
+            if int(run.max()) > 0x7FFFFFFF or int(run.min()) < -0x80000000:     # (numpy would take the low bits)
+                raise OverflowError("a number of the batch does not fit 32 bits")
             values[to:to + len(run)] = run
         else:
             struct.pack_into(f"{len(run)}i", values, 4 * to, *run)
