@@ -162,6 +162,8 @@ __host__ __device__ constexpr int latent_pitch(int rank) { return (rank + 7) / 8
 __host__ __device__ constexpr int latent_row_elems(int rank, int rot) { return latent_pitch(rank) + (rot + 7) / 8 * 8; }
 constexpr int kLatentMaxSplits = 256;
 bool latent_supported(int heads, int dim, int rot, int rank);
+int latent_splits(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64_t max_q, int64_t keys);
+bool latent_waves(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64_t max_q, int64_t keys);
 int launch_latent_prepare(const LatentProblem& p, int64_t T, hipStream_t s);
 int launch_latent_paged(const LatentProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml,
                         int64_t T, hipStream_t s);

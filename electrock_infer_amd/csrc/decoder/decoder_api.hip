@@ -353,6 +353,21 @@ int ed_attn_prompt(const ed_attn_args* a, void* stream) {
 
 int ed_latent_row_elems(int rank, int rot) { return latent_row_elems(rank, rot); }
 
+namespace {
+bool latent_call_ok(int dtype, int heads, int rank, int rot, int n_seqs, int max_q, int max_context) {
+    return dtype_ok(dtype) && latent_supported(heads, 1, rot, rank) && n_seqs > 0 && n_seqs <= kMaxSeqs && max_q > 0 && max_q <= kMaxRows &&
+           max_context > 0;
+}
+}  // namespace
+
+int ed_latent_splits(int dtype, int heads, int rank, int rot, int n_seqs, int max_q, int max_context) {
+    return latent_call_ok(dtype, heads, rank, rot, n_seqs, max_q, max_context) ? latent_splits(dtype, rank, rot, heads, n_seqs, max_q, max_context) : 0;
+}
+
+int ed_latent_waves(int dtype, int heads, int rank, int rot, int n_seqs, int max_q, int max_context) {
+    return latent_call_ok(dtype, heads, rank, rot, n_seqs, max_q, max_context) && latent_waves(dtype, rank, rot, heads, n_seqs, max_q, max_context) ? 1 : 0;
+}
+
 int ed_latent_prepare(const ed_latent_args* a, void* stream) {
     const int rc = check_latent(a);
     if (rc != 0 || a->T == 0) return rc;

@@ -366,12 +366,13 @@ __global__ __launch_bounds__(256) void latent_paged_kernel(LatentProblem p, int 
 // own and the next one on its way in registers, no barrier before the waves' results are added up.  S^T = K Q^T leaves a lane
 // keys (lane / 16) * 4 + 0..3 for one row, which is the second operand of O^T = V^T P^T as it is.  Bound: the way to
 // memory, once per tile; a workgroup has a CU to itself (its waves' accumulators, queries and tiles take over half of the
-// registers for rank 512 + 64 rotated; tiles of 32 keys do not fit).  Workgroups that read the same
-// keys for other heads run on the same XCD at the same time, so that its L2 serves all but the first.  23 sequences of
-// 1500 keys, 32 heads on 512 + 64: 44.8 us in five ranges with four barriers per tile (36.1 in ten), 31.3 now, in five; 64 of
-// 1000 keys, 16 heads: 35.4 (eight), 33.5 (four).
+// registers for rank 512 + 64 rotated; tiles of 32 keys do not fit).  Workgroups that read the same keys for other rows run
+// on the same XCD at the same time, so that its L2 serves all but the first (64 sequences of 1000 keys, 64 heads: 54.9 us,
+// 64.2 without), unless that takes more rounds of the chip, for some XCDs would be idle (63 tokens behind 3000, 32 heads:
+// 283 us that way, 76.9 spread out).  23 sequences of 1500 keys, 32 heads on 512 + 64: 44.8 us in five ranges with four barriers
+// per tile (36.1 in ten), 31.3 now, in five; 64 of 1000 keys, 16 heads: 35.4 (eight), 33.5 (four).
 // DKT: 32-element steps of a cached row; NT: 16-element tiles of the latent.
-constexpr int kWaveKeys = 16;
+constexpr int kWaveKeys = 16, kXcds = 8, kXcdCus = 32;
 template <int DKT, int NT>
 struct LatentWave {
     static constexpr int kPitch = DKT * 32 + 8, kSums = NT * 16 + 4;
@@ -387,16 +388,17 @@ __device__ __forceinline__ s16x4_t load_four_rows(const uint16_t* m, int pitch, 
 }
 
 template <int DKT, int NT>
-__global__ __launch_bounds__(256, 1) void latent_wave_kernel(LatentProblem p, int n_seqs, int groups, int splits, float* __restrict__ part_o,
-                                                             float* __restrict__ part_ml) {
+__global__ __launch_bounds__(256, 1) void latent_wave_kernel(LatentProblem p, int n_seqs, int groups, int splits, bool one_xcd,
+                                                             float* __restrict__ part_o, float* __restrict__ part_ml) {
     typedef Mma<BF16Elem> M;
     typedef LatentWave<DKT, NT> L;
-    constexpr int LP = L::kPitch, kXcds = 8;
+    constexpr int LP = L::kPitch;
     constexpr float kSlack = 8.0f;
     static_assert(DKT % 2 == 0 && NT * 16 <= DKT * 32, "rows of whole 128-byte pieces that hold every tile of the latent");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     __shared__ float wave_m[4][16], wave_l[4][16];
-    const int slot = blockIdx.x / kXcds, group = slot % groups, pair = slot / groups * kXcds + blockIdx.x % kXcds;
+    const int slot = one_xcd ? blockIdx.x / kXcds : blockIdx.x, group = slot % groups;
+    const int pair = one_xcd ? slot / groups * kXcds + blockIdx.x % kXcds : slot / groups;
     const int seq = pair / splits, split = pair - seq * splits;
     if (seq >= n_seqs) return;
     const int q0 = p.q_begin[seq], rows = (p.q_begin[seq + 1] - q0) * p.heads, r0 = group * 16;
@@ -620,10 +622,71 @@ int launch_wave(const LatentProblem& p, int n_seqs, int max_q, int splits, float
     constexpr int kLds = LatentWave<DKT, NT>::kLds;
     const int rc = allow_lds(reinterpret_cast<const void*>(latent_wave_kernel<DKT, NT>), kLds);
     if (rc != 0) return rc;
-    const int64_t groups = ceil_div(static_cast<int64_t>(max_q) * p.heads, 16), pairs = round_up(static_cast<int64_t>(n_seqs) * splits, 8);
-    launch((latent_wave_kernel<DKT, NT>), dim3(static_cast<unsigned>(groups * pairs)), dim3(256), kLds, s, p, n_seqs, static_cast<int>(groups),
-           splits, part_o, part_ml);
+    const int64_t groups = ceil_div(static_cast<int64_t>(max_q) * p.heads, 16), pairs = static_cast<int64_t>(n_seqs) * splits;
+    const bool one_xcd = ceil_div(ceil_div(pairs, kXcds) * groups, kXcdCus) <= ceil_div(groups * pairs, kXcds * kXcdCus);
+    launch((latent_wave_kernel<DKT, NT>), dim3(static_cast<unsigned>(groups * (one_xcd ? round_up(pairs, kXcds) : pairs))), dim3(256), kLds, s, p,
+           n_seqs, static_cast<int>(groups), splits, one_xcd, part_o, part_ml);
     return launch_status();
+}
+
+// Which kernel a call takes, and the ranges that its keys are shared out over.  latent_paged (2 to 4 workgroups to a CU) with
+// 768 workgroups, unless the waves that work alone are ahead.  Their time is estimated in keys that a CU goes through: rounds
+// of 256 workgroups, each its range and the keys that its start and the sum over its waves are worth (fewer keys where they
+// cost more), at the best number of ranges; it is compared with
+//   * rows up to 192 on a latent up to 128: nothing, they are ahead throughout (us, 64 + 32: 512 sequences of 500 keys 22 / 31);
+//   * rows up to 320 on a latent up to 256: all keys spread evenly over the CUs, and a start.  A key costs both kernels the
+//     same, so the waves lose what a part-filled round leaves idle (256 + 64: 64 x 1000 keys, 16 heads 21.8 / 24.6, 300 x 700
+//     59 / 47);
+//   * longer rows on a latent up to 256, which they take in the form for 512, and rows on a latent up to 512: rounds of
+//     latent_paged (three and two workgroups to a CU), times what a workgroup of a full CU is slower (256 + 128: 8 x 1000
+//     keys 18.3 / 19.0, 64 x 3000 51.7 / 46.6; 512 + 64: 64 x 1000 33.8 / 35.3, 300 x 1000 with 32 heads 109 / 101, 400 x 1000
+//     114 / 137).  Here latent_paged runs in whole rounds too (400 x 1000 on 256 + 128: in twos 100, in threes 82).
+// The numbers are those that lose least over 455 measured calls (1 to 600 sequences, 1 to 63 tokens, 16 to 128 heads, 60 to 12000
+// keys): 14 % faster than latent_paged alone on the average, at most 10 % slower.
+constexpr int kRangeKeys = 128, kMostRanges = 64;
+
+struct LatentPlan {
+    bool waves;
+    int splits;
+};
+
+// The grid of the waves that work alone has one dimension, whose threads are counted in 32 bits.
+bool wave_grid_fits(int64_t n_seqs, int64_t rows, int64_t splits) { return round_up(n_seqs * splits, kXcds) * ceil_div(rows, 16) < (1 << 24); }
+
+struct Rounds {
+    double keys;
+    int splits;
+};
+
+Rounds fewest_keys(int64_t groups, int64_t keys, int slots, double start) {
+    const int most = static_cast<int>(ceil_div(keys, kRangeKeys) < kMostRanges ? ceil_div(keys, kRangeKeys) : kMostRanges);
+    Rounds best{static_cast<double>(ceil_div(groups, slots)) * (static_cast<double>(keys) + start), 1};
+    for (int s = 2; s <= most; ++s) {
+        const double k = static_cast<double>(ceil_div(groups * s, slots)) * (static_cast<double>(keys) / s + start);
+        if (k < 0.995 * best.keys) best = Rounds{k, s};
+    }
+    return best;
+}
+
+// groups: 16 rows of a sequence each; keys: of the longest sequence
+LatentPlan latent_plan(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64_t max_q, int64_t keys) {
+    constexpr int kCus = kXcds * kXcdCus, kPagedGroups = 768;
+    const int row = latent_row_elems(rank, rot);
+    const int64_t groups = ceil_div(max_q * heads, 16) * n_seqs;
+    const int64_t ranges = ceil_div(kPagedGroups, groups), most = ceil_div(keys, kRangeKeys);
+    LatentPlan paged{false, static_cast<int>(ranges < most ? (ranges < kMostRanges ? ranges : kMostRanges) : (most < kMostRanges ? most : kMostRanges))};
+    // (rows of which a wave's queries and accumulators fit in its registers)
+    if (dtype != EM_DTYPE_BF16 || row > 18 * 32 || !wave_grid_fits(n_seqs, max_q * heads, kMostRanges)) return paged;
+    if (rank <= 128 && row <= 192) return LatentPlan{true, fewest_keys(groups, keys, kCus, 400.0).splits};
+    const bool longer = rank > 256 || row > 320;
+    const Rounds waves = fewest_keys(groups, keys, kCus, longer ? 300.0 : 200.0);
+    double other = static_cast<double>(groups) * static_cast<double>(keys) / kCus + 350.0;
+    if (longer) {
+        const Rounds r = rank > 256 ? fewest_keys(groups, keys, 2 * kCus, 100.0) : fewest_keys(groups, keys, 3 * kCus, 300.0);
+        paged.splits = r.splits;
+        other = r.keys * (rank > 256 ? 2.6 : 1.8);
+    }
+    return waves.keys <= other ? LatentPlan{true, waves.splits} : paged;
 }
 
 template <typename Elem>
@@ -631,7 +694,8 @@ int dispatch_paged(const LatentProblem& p, int n_seqs, int max_q, int splits, fl
                    hipStream_t s) {
     int rc;
     const int row = latent_row_elems(p.rank, p.rot);
-    if (sizeof(typename Elem::storage) == 2 && row <= 18 * 32) {       // (rows of which a wave's queries and accumulators fit in its registers)
+    if (latent_plan(p.dtype, p.rank, p.rot, p.heads, n_seqs, max_q, static_cast<int64_t>(p.table_width) * p.block_size).waves &&
+        wave_grid_fits(n_seqs, static_cast<int64_t>(max_q) * p.heads, splits)) {
         if (p.rank <= 128 && row <= 192) rc = launch_wave<6, 8>(p, n_seqs, max_q, splits, part_o, part_ml, s);
         else if (p.rank <= 256 && row <= 320) rc = launch_wave<10, 16>(p, n_seqs, max_q, splits, part_o, part_ml, s);
         else rc = launch_wave<18, 32>(p, n_seqs, max_q, splits, part_o, part_ml, s);
@@ -673,6 +737,14 @@ int head_gemm(const void* a, int64_t a_row, int64_t a_head, const void* b, void*
 bool latent_supported(int heads, int dim, int rot, int rank) {
     // key rows of one tile per thread: 8-element pieces, at most NTW + 2 of them (see latent_paged_kernel)
     return heads > 0 && heads <= 1024 && dim > 0 && rot >= 0 && rot % 2 == 0 && rot <= 128 && rank > 0 && rank <= 512;
+}
+
+int latent_splits(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64_t max_q, int64_t keys) {
+    return latent_plan(dtype, rank, rot, heads, n_seqs, max_q, keys).splits;
+}
+
+bool latent_waves(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64_t max_q, int64_t keys) {
+    return latent_plan(dtype, rank, rot, heads, n_seqs, max_q, keys).waves;
 }
 
 int launch_latent_prepare(const LatentProblem& p, int64_t T, hipStream_t s) {

@@ -16,8 +16,6 @@ def rotary_frequencies(dims: int, base: float, factor: float = 1.0) -> torch.Ten
 class LatentAttention(nn.Module):
 
     PROMPT_TOKENS = 64           # portions from this length on write their keys and values out, if the kernel takes the sizes
-    TARGET_WORKGROUPS = 768      # the keys are shared out over workgroups until a launch has about this many
-    WAVE_ROW, WAVE_WORKGROUPS = 576, 256      # cached rows of the kernel whose workgroups have a CU to themselves: no more of them than CUs
 
     def __init__(self, width: int, heads: int, dim: int, rot_dim: int, vdim: int, kv_rank: int, scale: float,
                  rotary_base: float, eps: float, dtype):
@@ -55,10 +53,9 @@ class LatentAttention(nn.Module):
         return self.pitch + (self.rot + 7) // 8 * 8
 
     def splits(self, batch) -> int:
-        groups = -(-batch.max_q * self.heads // 16) * batch.n_seqs
-        if self.uk.dtype == torch.bfloat16 and self.row_elems() <= self.WAVE_ROW:
-            return max(1, min(self.WAVE_WORKGROUPS // groups, -(-batch.max_context // 128), 64))
-        return max(1, min(-(-self.TARGET_WORKGROUPS // groups), -(-batch.max_context // 128), 64))
+        """Ranges that the keys are shared out over."""
+        return _lib.load_decoder().ed_latent_splits(_lib.dtype_code(self.uk.dtype), self.heads, self.rank, self.rot, batch.n_seqs, batch.max_q,
+                                                    batch.max_context)
 
     def forward(self, h: torch.Tensor, batch, cache: torch.Tensor) -> torch.Tensor:
         """h [T, width] -> [T, width] (as ``linear_parts`` has it); ``cache`` [blocks, block_size, row_elems] receives the new tokens' rows first."""

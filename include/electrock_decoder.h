@@ -226,6 +226,11 @@ typedef struct ed_latent_args {
 } ed_latent_args;
 
 int ed_latent_row_elems(int rank, int rot);
+/* For a batch of n_seqs portions of at most max_q tokens whose longest context has max_context tokens: how many ranges fill the
+ * chip (0: sizes that are not taken); 1 if such a call goes to the kernel whose waves work alone.  Any number of ranges gives
+ * the same result up to the order of sums. */
+int ed_latent_splits(int dtype, int heads, int rank, int rot, int n_seqs, int max_q, int max_context);
+int ed_latent_waves(int dtype, int heads, int rank, int rot, int n_seqs, int max_q, int max_context);
 /* Norm of the latent, rotation of the key part (both into the cache) and of q's rotated parts (in place). */
 int ed_latent_prepare(const ed_latent_args* a, void* stream);
 /* out = sum_j p_j c_j per row and head, p = softmax of (q_latent . c_j + q_rot . k_rot_j) * scale over the keys
