@@ -149,9 +149,14 @@ template <> struct Precise<BF16Elem> {    // the hardware's exponential and reci
 
 // ---- any portion ----
 constexpr int kKeys = 32;
-// Cached rows are read once per step: past the caches' order of use.
-template <typename Elem>
-__device__ __forceinline__ typename Mma<Elem>::frag load_nt(const typename Elem::storage* p) {
+// Cached rows that one workgroup reads (16 rows of queries cover a portion): past the caches' order of use.  Where several row
+// groups read them, that order is what the others need (us, bf16, 16 heads on 4 of 128, past it / in it: one token of 64 behind
+// 2000 keys 59.3 / 61.7; 47 of 8 behind 2000 70.4 / 54.8, of 32 behind 1000 128.0 / 95.0, of one behind 4000 33.3 / 29.7; 64
+// sequences of one token on the same 2000 keys, which is not known here, 46.3 / 41.5), and float32 rows, of which a load takes
+// halves of lines, always go through it (64 x 2000 keys 167 / 155).
+template <typename Elem, bool ONCE>
+__device__ __forceinline__ typename Mma<Elem>::frag load_rows(const typename Elem::storage* p) {
+    if constexpr (!ONCE) return Mma<Elem>::load(p);
     constexpr int kWords = sizeof(typename Elem::storage) * 8 / 16;
     u32x4_t w[kWords];
 #pragma unroll
@@ -170,7 +175,7 @@ template <typename Elem> __host__ __device__ constexpr int paged_lds(int dkt, in
 }
 
 // DKT: 32-element steps of dim; DVT: 16-element tiles of vdim
-template <typename Elem, int DKT, int DVT>
+template <typename Elem, int DKT, int DVT, bool ONCE>
 __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) void attn_paged_kernel(AttnProblem p, int splits,
                                                                                                     float* __restrict__ part_o,
                                                                                                     float* __restrict__ part_ml) {
@@ -226,12 +231,12 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
     auto key_row = [&](int row, int key) { return keys + static_cast<int64_t>(max(__shfl(row, key), 0)) * row_elems; };
     auto load_keys = [&](int row) {
 #pragma unroll
-        for (int i = 0; i < kKeyPieces; ++i) fk[i] = load_nt<Elem>(key_row(row, k_key + i * kKeysAtOnce) + min(k_col, dp - 8));
+        for (int i = 0; i < kKeyPieces; ++i) fk[i] = load_rows<Elem, ONCE>(key_row(row, k_key + i * kKeysAtOnce) + min(k_col, dp - 8));
     };
     auto load_values = [&](int row) {
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
-            fv[i] = load_nt<Elem>(values + static_cast<int64_t>(max(__shfl(row, v_key + i * kRowsAtOnce), 0)) * row_elems);
+            fv[i] = load_rows<Elem, ONCE>(values + static_cast<int64_t>(max(__shfl(row, v_key + i * kRowsAtOnce), 0)) * row_elems);
         }
     };
     int row = row_of(tile0 + wave), next_row = row_of(tile0 + wave + 4);
@@ -627,15 +632,22 @@ __global__ __launch_bounds__(256, DKT == 2 && DVT == 4 ? 3 : 2) void attn_prompt
     }
 }
 
+template <typename Elem, int DKT, int DVT, bool ONCE>
+int launch_groups(const AttnProblem& p, int row_groups, int n_seqs, int splits, float* part_o, float* part_ml, hipStream_t s) {
+    const size_t lds = paged_lds<Elem>(DKT, DVT);
+    const int rc = allow_lds(reinterpret_cast<const void*>(attn_paged_kernel<Elem, DKT, DVT, ONCE>), lds);
+    if (rc != 0) return rc;
+    const dim3 grid(static_cast<unsigned>(row_groups), static_cast<unsigned>(n_seqs * p.kv_heads), static_cast<unsigned>(splits));
+    launch((attn_paged_kernel<Elem, DKT, DVT, ONCE>), grid, dim3(256), lds, s, p, splits, part_o, part_ml);
+    return launch_status();
+}
+
 template <typename Elem, int DKT, int DVT>
 int launch_paged(const AttnProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml, int64_t T, hipStream_t s) {
-    const size_t lds = paged_lds<Elem>(DKT, DVT);
-    int rc = allow_lds(reinterpret_cast<const void*>(attn_paged_kernel<Elem, DKT, DVT>), lds);
-    if (rc != 0) return rc;
-    const dim3 grid(static_cast<unsigned>(ceil_div(static_cast<int64_t>(max_q) * (p.heads / p.kv_heads), 16)),
-                    static_cast<unsigned>(n_seqs * p.kv_heads), static_cast<unsigned>(splits));
-    launch((attn_paged_kernel<Elem, DKT, DVT>), grid, dim3(256), lds, s, p, splits, part_o, part_ml);
-    rc = launch_status();
+    const int row_groups = static_cast<int>(ceil_div(static_cast<int64_t>(max_q) * (p.heads / p.kv_heads), 16));
+    constexpr bool kBf16 = sizeof(typename Elem::storage) == 2;
+    const int rc = kBf16 && row_groups == 1 ? launch_groups<Elem, DKT, DVT, kBf16>(p, row_groups, n_seqs, splits, part_o, part_ml, s)
+                                            : launch_groups<Elem, DKT, DVT, false>(p, row_groups, n_seqs, splits, part_o, part_ml, s);
     if (rc != 0 || splits == 1) return rc;
     launch((attn_combine_kernel<Elem>), dim3(static_cast<unsigned>(T * p.heads)), dim3(kWave), 0, s, part_o, part_ml, splits, p.vdim,
            static_cast<typename Elem::storage*>(p.out));
