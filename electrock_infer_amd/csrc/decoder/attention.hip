@@ -683,6 +683,32 @@ bool attn_supported(int heads, int kv_heads, int dim, int vdim, int rot) {
            rot >= 0 && rot % 2 == 0 && rot <= dim;
 }
 
+// Ranges that the keys of a call of the paged kernel are shared out over.  A range goes in steps of 128 keys, four waves' tiles
+// at once; more ranges are shorter chains of steps until the chip is full, and more partial results.  In steps:
+//     rounds of the chip * (1 + steps of a range) + a share of what the partial results take, and one for their launch
+// where a "round" is as many workgroups as are in flight at no cost to each other, by the form of the kernel, and only whole
+// steps count.  us with the combination, 16 heads on 4: 64 x 768 keys in ones 26.9, in threes 29.6; 24 x 2000 keys in threes
+// 34.9, fours 31.1, eights 28.8; 8 x 2000 in eights 16.0, sixteens 17.9; 64 x 4096 in ones 109.6, twos 103.1.  Forms without the
+// next tile in flight hide its way with other workgroups (float32, 64 + 64: 24 x 2000 keys in threes 50.0, eights 31.8; bf16,
+// 192 + 64 in threes 40.8, eights 30.3).
+int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int64_t max_q, int64_t keys) {
+    const int64_t row_groups = ceil_div(max_q * (heads / kv_heads), 16), groups = row_groups * n_seqs * kv_heads, most = ceil_div(keys, 4 * kKeys);
+    const bool bf16 = dtype == EM_DTYPE_BF16, ahead = bf16 && dim <= 128, once = bf16 && row_groups == 1;
+    const double in_flight = once ? 384.0 : ahead ? 256.0 : 768.0, results = once || ahead ? 0.6 : 1.0;
+    int best = 1;
+    double least = 0.0;
+    for (int64_t s = 1; s <= most && s <= kAttnMaxSplits; ++s) {
+        const int64_t steps = ceil_div(most, s);
+        if (s > 1 && ceil_div(most, s - 1) == steps) continue;
+        const double all = static_cast<double>(groups * s), rounds = all > in_flight ? all / in_flight : 1.0;
+        const double cost = rounds * static_cast<double>(1 + steps) + (s > 1 ? results * all / 256.0 + 1.0 : 0.0);
+        if (s > 1 && cost >= least) continue;
+        least = cost;
+        best = static_cast<int>(s);
+    }
+    return best;
+}
+
 int launch_attn_prepare(const AttnProblem& p, int64_t T, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(T), T <= 256 ? static_cast<unsigned>(ceil_div(p.heads + p.kv_heads, 4)) : 1u);
     const size_t lds = sizeof(float) * (p.rot > 0 ? p.rot : 1);

@@ -22,12 +22,6 @@ class CarriedValues:
 class SoftmaxAttention(nn.Module):
 
     PROMPT_TOKENS = 48           # portions from this length on go to the kernel for prompts, if it takes the sizes
-    # The keys are shared out over workgroups until a launch has one for every CU, or two where one would take long: more only
-    # bring more partial results (us with the combination, 16 heads on 4: 64 x 768 keys in ones 26.9, in threes 29.5; 16 x 1024
-    # in fours 15.9, eights 16.6; 8 x 1024 in eights 12.9, sixteens 14.8; 64 x 4096 in ones 107.6, twos 100.8, fours 101.6).
-    TARGET_WORKGROUPS = 256
-    SPLIT_KEYS = 128             # fewest keys of a workgroup
-    LONG_KEYS = 2048             # more keys than these in a workgroup: twice as many workgroups
 
     def __init__(self, width: int, heads: int, kv_heads: int, dim: int, vdim: int, scale: float, eps: float, dtype,
                  rot_dims: int = 0, rotary_base: float = 10000.0, rotary_factor: float = 1.0, softcap: float = 0.0, window: int = 0,
@@ -65,12 +59,10 @@ class SoftmaxAttention(nn.Module):
         return torch.zeros(num_blocks, block_size, self.row_elems(), dtype=self.o.dtype, device=device)
 
     def splits(self, batch) -> int:
-        groups = -(-batch.max_q * (self.heads // self.kv_heads) // 16) * batch.n_seqs * self.kv_heads
+        """Ranges that the keys are shared out over."""
         keys = min(batch.max_context, self.window + batch.max_q) if self.window else batch.max_context
-        want = -(-self.TARGET_WORKGROUPS // groups)
-        if keys > want * self.LONG_KEYS:
-            want = -(-2 * self.TARGET_WORKGROUPS // groups)
-        return max(1, min(want, -(-keys // self.SPLIT_KEYS), 64))
+        return _lib.load_decoder().ed_attn_splits(_lib.dtype_code(self.o.dtype), self.heads, self.kv_heads, self.dim, self.vdim, batch.n_seqs,
+                                                  batch.max_q, keys)
 
     def forward(self, h: torch.Tensor, batch, cache: torch.Tensor, carried: Optional[CarriedValues] = None) -> torch.Tensor:
         """h [T, width] -> [T, width] (as ``linear_parts`` has it); ``cache`` [blocks, block_size, row_elems] receives the
