@@ -60,30 +60,128 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t* __restrict__ 
 // y may be given as float32 partial sums [y_parts, T, W].
 //   UPDATE 0: x stays          UPDATE 1: x += y / rms(y) * post_w          UPDATE 2: x = y + post_w
 //   then, when out != null: out = next_w ? x / rms(x) * next_w : x, rounded to the compute type
-// Bound: bytes for prompts, the way from the first load to the last store for a few rows.  Everything that a row needs is
-// requested before the first sum over it: loads behind the barriers, and partial sums one by one, cost a way to memory
-// each (four partial sums of 64 rows of 2048: 5.5 us that way, 4.9 now; two of 24 rows of 4096: 6.8, 4.9; 8192 rows of 2048:
-// 35.3, 34.5).
-template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS, int N>
+// PARTS: y_parts > 1, of which one is requested at a time for the whole row (64 rows of 8192 in threes 8.4 -> 7.4 us).
+template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS, int N, bool PARTS>
 __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
     float* __restrict__ x, const typename YElem::storage* __restrict__ y, int y_parts, const float* __restrict__ post_w,
     const float* __restrict__ next_w, typename Elem::storage* __restrict__ out, int64_t out_stride, int W, float eps) {
     __shared__ float scratch[THREADS / kWave];
-    constexpr bool kEarly = N * VEC <= 16;          // (longer rows do not fit in the registers twice)
-    constexpr int kParts = kEarly ? 4 : 1, M = kEarly ? N : 1;      // partial sums requested at once; rows of early loads
     const int64_t row = blockIdx.x;
     float* xr = x + row * W;
-    float v[N][VEC], xv[M][VEC], pw[M][VEC], nw[M][VEC], sum = 0.0f;
+    float v[N][VEC];
+    if (UPDATE != 0) {
+        const typename YElem::storage* yr = y + row * W;
+        float sum = 0.0f;
+        auto square = [&](int i) {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) sum = fmaf(v[i][j], v[i][j], sum);
+        };
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int c = (threadIdx.x + i * THREADS) * VEC;
+            if (c < W) {
+                RowIo<YElem, VEC>::load(yr + c, v[i]);
+                if (UPDATE == 1 && !PARTS) square(i);
+            }
+        }
+        if (PARTS) {
+            for (int p = 1; p < y_parts; ++p) {
+                float more[N][VEC];
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const int c = (threadIdx.x + i * THREADS) * VEC;
+                    if (c < W) RowIo<YElem, VEC>::load(yr + static_cast<int64_t>(p) * gridDim.x * W + c, more[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < N; ++i)
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) v[i][j] += more[i][j];
+            }
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (UPDATE == 1 && (threadIdx.x + i * THREADS) * VEC < W) square(i);
+        }
+        float rstd = 0.0f;
+        if (UPDATE == 1) rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(W) + eps);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int c = (threadIdx.x + i * THREADS) * VEC;
+            if (c < W) {
+                float pw[VEC];
+                if (UPDATE == 1) {
+                    float xv[VEC];
+                    RowIo<F32Elem, VEC>::load(post_w + c, pw);
+                    RowIo<F32Elem, VEC>::load(xr + c, xv);
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) v[i][j] = xv[j] + v[i][j] * rstd * pw[j];
+                } else if (post_w != nullptr) {
+                    RowIo<F32Elem, VEC>::load(post_w + c, pw);
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) v[i][j] += pw[j];
+                }
+                RowIo<F32Elem, VEC>::store(xr + c, v[i]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int c = (threadIdx.x + i * THREADS) * VEC;
+            if (c < W) RowIo<F32Elem, VEC>::load(xr + c, v[i]);
+        }
+    }
+    if (out == nullptr) return;
+    float rstd = 1.0f;
+    if (next_w != nullptr) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int c = (threadIdx.x + i * THREADS) * VEC;
+            if (c < W) {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) sum = fmaf(v[i][j], v[i][j], sum);
+            }
+        }
+        rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(W) + eps);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int c = (threadIdx.x + i * THREADS) * VEC;
+        if (c < W) {
+            float o[VEC];
+            if (next_w != nullptr) {
+                float nw[VEC];
+                RowIo<F32Elem, VEC>::load(next_w + c, nw);
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) o[j] = v[i][j] * rstd * nw[j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) o[j] = v[i][j];
+            }
+            RowIo<Elem, VEC>::store(out + row * out_stride + c, o);
+        }
+    }
+}
+
+// The same for short rows that are few.  Bound: the way from the first load to the last store.  Everything that a row needs is
+// requested before the first sum over it: loads behind the barriers, and partial sums one by one, cost a way to memory each.
+template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS, int N>
+__global__ __launch_bounds__(THREADS) void residual_norm_early_kernel(
+    float* __restrict__ x, const typename YElem::storage* __restrict__ y, int y_parts, const float* __restrict__ post_w,
+    const float* __restrict__ next_w, typename Elem::storage* __restrict__ out, int64_t out_stride, int W, float eps) {
+    __shared__ float scratch[THREADS / kWave];
+    constexpr int kParts = 4;          // partial sums requested at once
+    const int64_t row = blockIdx.x;
+    float* xr = x + row * W;
+    float v[N][VEC], xv[N][VEC], pw[N][VEC], nw[N][VEC], sum = 0.0f;
     const bool add_w = UPDATE == 1 || (UPDATE == 2 && post_w != nullptr), norm = out != nullptr && next_w != nullptr;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const int c = (threadIdx.x + i * THREADS) * VEC;
         if (c >= W) continue;
         if (UPDATE != 0) RowIo<YElem, VEC>::load(y + row * W + c, v[i]);
-        if (!kEarly) continue;
-        if (UPDATE != 2) RowIo<F32Elem, VEC>::load(xr + c, xv[i % M]);
-        if (add_w) RowIo<F32Elem, VEC>::load(post_w + c, pw[i % M]);
-        if (norm) RowIo<F32Elem, VEC>::load(next_w + c, nw[i % M]);
+        if (UPDATE != 2) RowIo<F32Elem, VEC>::load(xr + c, xv[i]);
+        if (add_w) RowIo<F32Elem, VEC>::load(post_w + c, pw[i]);
+        if (norm) RowIo<F32Elem, VEC>::load(next_w + c, nw[i]);
     }
     if (UPDATE != 0 && y_parts > 1) {
         for (int p0 = 1; p0 < y_parts; p0 += kParts) {
@@ -118,13 +216,11 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
     for (int i = 0; i < N; ++i) {
         const int c = (threadIdx.x + i * THREADS) * VEC;
         if (c >= W) continue;
-        if (!kEarly && UPDATE != 2) RowIo<F32Elem, VEC>::load(xr + c, xv[i % M]);
-        if (!kEarly && add_w) RowIo<F32Elem, VEC>::load(post_w + c, pw[i % M]);
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
-            if (UPDATE == 0) v[i][j] = xv[i % M][j];
-            if (UPDATE == 1) v[i][j] = xv[i % M][j] + v[i][j] * rstd * pw[i % M][j];
-            if (UPDATE == 2 && add_w) v[i][j] += pw[i % M][j];
+            if (UPDATE == 0) v[i][j] = xv[i][j];
+            if (UPDATE == 1) v[i][j] = xv[i][j] + v[i][j] * rstd * pw[i][j];
+            if (UPDATE == 2 && add_w) v[i][j] += pw[i][j];
             sum = fmaf(v[i][j], v[i][j], sum);
         }
         if (UPDATE != 0) RowIo<F32Elem, VEC>::store(xr + c, v[i]);
@@ -137,9 +233,8 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
         const int c = (threadIdx.x + i * THREADS) * VEC;
         if (c >= W) continue;
         if (norm) {
-            if (!kEarly) RowIo<F32Elem, VEC>::load(next_w + c, nw[i % M]);
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) v[i][j] = v[i][j] * rstd * nw[i % M][j];
+            for (int j = 0; j < VEC; ++j) v[i][j] = v[i][j] * rstd * nw[i][j];
         }
         RowIo<Elem, VEC>::store(out + row * out_stride + c, v[i]);
     }
@@ -175,7 +270,9 @@ __global__ __launch_bounds__(256) void silu_gate_kernel(const typename Elem::sto
     RowIo<Elem, VEC>::store(out + i, v);
 }
 
-// y = y silu(z), normed in equal parts of `size` elements, times w, in place: one workgroup per (row, part)
+// y = y silu(z), normed in equal parts of `size` elements, times w, in place: one workgroup per (row, part).  Rows of up to 4096
+// elements request everything before the sum; longer ones take the product as it comes, or the registers hold both operands
+// (float32, 300 rows of 9001: 35.8 us that way, spilled, 13.2 now; bf16, 3505 of 8192: 36.2, 31.2).
 template <typename Elem, int VEC, int THREADS, int N>
 __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::storage* __restrict__ y, const typename Elem::storage* __restrict__ z,
                                                              int64_t z_stride, const float* __restrict__ w, int size, float eps) {
@@ -187,25 +284,26 @@ __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::stor
     constexpr bool kEarly = N * VEC <= 16;
     constexpr int M = kEarly ? N : 1;
     float v[N][VEC], g[M][VEC], wv[M][VEC], sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const int c = (threadIdx.x + i * THREADS) * VEC;
-        if (c >= size) continue;
-        RowIo<Elem, VEC>::load(yr + c, v[i]);
-        if (!kEarly) continue;
-        RowIo<Elem, VEC>::load(zr + c, g[i % M]);
-        RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const int c = (threadIdx.x + i * THREADS) * VEC;
-        if (c >= size) continue;
-        if (!kEarly) RowIo<Elem, VEC>::load(zr + c, g[i % M]);
+    auto times_silu = [&](int i) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
             v[i][j] *= silu(g[i % M][j]);
             sum = fmaf(v[i][j], v[i][j], sum);
         }
+    };
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int c = (threadIdx.x + i * THREADS) * VEC;
+        if (c >= size) continue;
+        RowIo<Elem, VEC>::load(yr + c, v[i]);
+        RowIo<Elem, VEC>::load(zr + c, g[i % M]);
+        if (kEarly) RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
+        else times_silu(i);
+    }
+    if (kEarly) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if ((threadIdx.x + i * THREADS) * VEC < size) times_silu(i);
     }
     const float rstd = 1.0f / sqrtf(block_sum<THREADS>(sum, scratch) / static_cast<float>(size) + eps);
 #pragma unroll
@@ -289,27 +387,41 @@ int launch_gated(void* y, const void* z, int64_t z_stride, const float* w, int64
     return launch_status();
 }
 
-template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS, int N>
-int launch_rows(float* x, const void* y, int y_parts, const float* post_w, const float* next_w, void* out, int64_t out_stride,
-                int64_t T, int W, float eps, hipStream_t s) {
-    launch((residual_norm_kernel<Elem, YElem, UPDATE, VEC, THREADS, N>), dim3(static_cast<unsigned>(T)), dim3(THREADS), 0, s, x,
-           static_cast<const typename YElem::storage*>(y), y_parts, post_w, next_w, static_cast<typename Elem::storage*>(out), out_stride, W, eps);
-    return launch_status();
-}
-
-// One vector per thread where the rows do not fill the chip (kFewRows), so that a row is over sooner; 256 threads where they do.
+// Few rows leave CUs without one, and a row is over sooner with one vector per thread and everything requested at once (us, 64 rows
+// of 2048 in fours 4.6 -> 3.9, one of 4096 in twos 5.2 -> 4.5).  Where rows fill the chip, their bytes are the bound and rows in flight
+// count for more than a row's way: the normed update, which keeps four rows of floats that way, waits with its weights and the
+// stream (rows of 4096, at once / in turn: 300 6.0 / 5.8, 1024 11.0 / 8.6, 3505 32.0 / 26.9, 16384 206 / 148; 8192 of 2048 31.8 / 30.4);
+// y + w, which keeps three, does so for long rows in large numbers only (rows of 4096: 768 6.6 / 6.9, 1500 10.9 / 9.7, 16384 133 / 113;
+// 8192 of 2048 21.4 / 21.9), x alone never (8192 of 4096 29.6 / 30.8).
 template <typename Elem, typename YElem, int UPDATE, int VEC>
 int launch_residual(float* x, const void* y, int y_parts, const float* post_w, const float* next_w, void* out, int64_t out_stride,
                     int64_t T, int W, float eps, hipStream_t s) {
-#define EM_ROWS(THREADS, N) return launch_rows<Elem, YElem, UPDATE, VEC, THREADS, N>(x, y, y_parts, post_w, next_w, out, out_stride, T, W, eps, s)
+#define EM_ROWS(THREADS, ...)                                                                                                             \
+    do {                                                                                                                                  \
+        launch((__VA_ARGS__), dim3(static_cast<unsigned>(T)), dim3(THREADS), 0, s, x, static_cast<const typename YElem::storage*>(y), y_parts, \
+               post_w, next_w, static_cast<typename Elem::storage*>(out), out_stride, W, eps);                                            \
+        return launch_status();                                                                                                           \
+    } while (0)
+#define EM_EARLY(THREADS, N) EM_ROWS(THREADS, residual_norm_early_kernel<Elem, YElem, UPDATE, VEC, THREADS, N>)
+#define EM_LATE(THREADS, N)                                                                                       \
+    do {                                                                                                          \
+        if constexpr (UPDATE != 0 && sizeof(typename YElem::storage) == 4)                                        \
+            if (y_parts > 1) EM_ROWS(THREADS, residual_norm_kernel<Elem, YElem, UPDATE, VEC, THREADS, N, true>);  \
+        EM_ROWS(THREADS, residual_norm_kernel<Elem, YElem, UPDATE, VEC, THREADS, N, false>);                      \
+    } while (0)
     if constexpr (VEC == 4) {
-        if (T <= kFewRows && W > 1024 && W <= 2048) EM_ROWS(512, 1);
-        if (T <= kFewRows && W > 1024 && W <= 4096) EM_ROWS(1024, 1);
-        if (W <= 2048) EM_ROWS(256, 2);
-        if (W <= 4096) EM_ROWS(256, 4);
+        if (T <= kFewRows && W > 1024 && W <= 2048) EM_EARLY(512, 1);
+        if (T <= kFewRows && W > 1024 && W <= 4096) EM_EARLY(1024, 1);
+        const bool early = T <= kFewRows || UPDATE == 0 || (UPDATE == 2 && (W <= 2048 || T <= 4 * kFewRows));
+        if (early && W <= 2048) EM_EARLY(256, 2);
+        if (early && W <= 4096) EM_EARLY(256, 4);
+        if (W <= 2048) EM_LATE(256, 2);
+        if (W <= 4096) EM_LATE(256, 4);
     }
-    if (W <= 256 * kRowMaxPerThread) EM_ROWS(256, kRowMaxPerThread / VEC);
-    EM_ROWS(1024, kRowMaxPerThread / VEC);
+    if (W <= 256 * kRowMaxPerThread) EM_LATE(256, kRowMaxPerThread / VEC);
+    EM_LATE(1024, kRowMaxPerThread / VEC);
+#undef EM_LATE
+#undef EM_EARLY
 #undef EM_ROWS
 }
 
