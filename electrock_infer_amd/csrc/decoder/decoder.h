@@ -34,7 +34,7 @@ int launch_gated_norm(void* y, const void* z, int64_t z_stride, const float* w, 
 // ---- skinny_gemm.hip ----
 bool skinny_supported(int64_t T, int N, int K);
 bool decode_gemm_supported(int64_t T, int N, int K);
-bool decode_gemm_plain_pays(int64_t T, int N, int K);
+bool decode_gemm_pays(int64_t T, int rows, int K, int act, bool f32);
 int skinny_splits(int T, int N, int K);
 int launch_skinny_gemm(const void* x, const void* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s);
 

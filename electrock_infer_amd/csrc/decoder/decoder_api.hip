@@ -200,7 +200,12 @@ int ed_skinny_gemm(const void* x, const void* w, void* out, int out_dtype, int s
 
 int ed_decode_gemm_splits(int64_t T, int N, int K) { return decode_gemm_supported(T, N, K) ? skinny_splits(static_cast<int>(T), N, K) : 0; }
 
-int ed_decode_gemm_plain_pays(int64_t T, int N, int K) { return decode_gemm_supported(T, N, K) && decode_gemm_plain_pays(T, N, K) ? 1 : 0; }
+int ed_decode_gemm_pays(int64_t T, int N, int K, int act, int out_dtype) {
+    if (act < 0 || act > 2 || N > (1 << 30) || !dtype_ok(out_dtype)) return 0;
+    return decode_gemm_pays(T, act == 2 ? 2 * N : N, K, act, out_dtype == EM_DTYPE_F32) ? 1 : 0;
+}
+
+int ed_decode_gemm_plain_pays(int64_t T, int N, int K) { return ed_decode_gemm_pays(T, N, K, 0, EM_DTYPE_BF16); }
 
 int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
                    void* stream) {

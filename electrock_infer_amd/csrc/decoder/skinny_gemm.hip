@@ -201,11 +201,35 @@ bool skinny_supported(int64_t T, int N, int K) {
 
 bool decode_gemm_supported(int64_t T, int N, int K) { return T > 0 && T <= 64 && N > 0 && K > 0 && K % kStepK == 0; }
 
-// Against the library's product (us, this / library): 4096 x 4096 T = 1 8 / 16, T = 64 12.6 / 15.6; 2048 x 4096 T = 1 5.2 / 15,
-// T = 24 6.5 / 12.4, T = 64 8.2 / 14.1; 12288 x 4096 T = 12 21 / 29, T = 32 24 / 25.6, T = 48 24.7 / 26.8, T = 64 28.5 / 27.0;
-// 6720 x 4096 T = 48 19.1 / 19.0, T = 64 21.1 / 19.4; 8512 x 2048 T = 64 16.9 / 16.5.  The library is ahead with more than
-// 48 tokens and large weights, unless an activation, or a sum kept in float32, comes with the product.
-bool decode_gemm_plain_pays(int64_t T, int N, int K) { return T <= 48 || static_cast<int64_t>(N) * K <= (int64_t{1} << 24); }
+// Where a product without partial sums is faster this way than by the library (and the kernel of its activation): measured at rows
+// of 1024 to 24576, k of 1024 to 16384, T of 2 to 64, weights read from memory; 0.86 / 0.86 / 0.77 / 0.80 of the library's time on the
+// average (bf16, float32, squared ReLU, gated), at most a tenth more anywhere but float32 sums of 24576 rows.  The library shares k
+// out over the chip, so it is ahead where here
+//   * rows are few and k is long: a quarter or half of the CUs walk through all of it (us, this / library, T = 64: 1024 x 8192
+//     21.0 / 14.1; gated, 2048 rows x 12288, T = 40 34.4 / 23.3), or one tile to a CU still takes 16384 steps;
+//   * rows of 64 to a workgroup leave CUs without one (9216 to 15360; 12288 x 4096, T = 24 28.5 / 26.5, T = 8 26.4 / 30.4);
+//   * there are more than 48 tokens, whose rows every workgroup reads: unless the weights are small or an activation comes along.
+bool decode_gemm_pays(int64_t T, int rows, int K, int act, bool f32) {
+    if (!decode_gemm_supported(T, rows, K)) return false;
+    if (rows <= 2048) {
+        if (T <= 16) return act != 2 || K <= 8192;
+        if (act == 1 && T <= 32) return true;
+        if (f32 && rows <= 1024 && T > 32) return K <= 2048;
+        return K <= (T > 32 || rows <= 1024 ? 4096 : 6144);
+    }
+    if (K > 12288 && rows < 8192) return false;
+    if (act == 2) return rows > 4096 || K <= (T > 48 ? 3072 : rows > 3072 || T <= 32 ? 8192 : 6144);
+    if (act == 1) return true;
+    const bool small = static_cast<int64_t>(rows) * K <= (int64_t{1} << 24);
+    if (T > 48 && rows < 16384) return (small && K <= 4096) || (rows >= 6144 && rows <= 8192 && K <= 3072);
+    if (T > 48) return f32 || small;
+    if (rows >= 9216 && rows < 15360) {
+        if (T <= 16) return K <= (f32 ? 2048 : 4096) || (rows >= 12288 && K > 4096 && K <= 6144);
+        if (T <= 32) return K <= 2048;
+        return rows < 12288 || K <= 2048 || K >= 6144;
+    }
+    return true;
+}
 
 // Ranges of K for results that may stay partial sums: enough workgroups for the chip, a step of k for every wave.
 int skinny_splits(int T, int N, int K) {

@@ -33,10 +33,15 @@ def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
     return _lib.load_decoder().ed_decode_gemm_splits(x.shape[0], *weight.shape)
 
 
+def _streams(x: torch.Tensor, weight: torch.Tensor, out_rows: int, act: int = 0, out_dtype: int = _lib.DTYPE_BF16) -> bool:
+    """Whether the weight-streaming kernel takes the product and is the faster way."""
+    return _skinny_splits(x, weight) > 0 and _lib.load_decoder().ed_decode_gemm_pays(x.shape[0], out_rows, x.shape[1], act, out_dtype) == 1
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
     """act(x @ weight^T) in x's type: a weight-streaming kernel for a decode batch, a library product otherwise;
     ``act``: None or 'relu_squared'."""
-    if _skinny_splits(x, weight) and (act is not None or _lib.load_decoder().ed_decode_gemm_plain_pays(x.shape[0], *weight.shape)):
+    if _streams(x, weight, weight.shape[0], int(act is not None)):
         return _skinny(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device), 1, int(act is not None))
     out = F.linear(x, weight)
     return relu_squared_(out) if act is not None else out
@@ -46,7 +51,7 @@ def linear_silu_gate(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T) for ``weight`` = [gate; up]: one launch for a decode batch."""
     (T, _), ff = x.shape, weight.shape[0] // 2
     out = torch.empty(T, ff, dtype=x.dtype, device=x.device)
-    if _skinny_splits(x, weight):
+    if _streams(x, weight, ff, 2):
         code = _lib.load_decoder().ed_decode_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), 1, T, ff,
                                                   x.shape[1], 2, _lib.current_stream(x.device))
         _lib.check_decoder(code, "decode_gemm")
@@ -61,7 +66,7 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x @ weight^T with the float32 accumulators as the result, for sums that stay float32."""
     if x.dtype == torch.float32:
         return F.linear(x, weight)
-    if _skinny_splits(x, weight):
+    if _streams(x, weight, weight.shape[0], 0, _lib.DTYPE_F32):
         return _skinny(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), 1, 0)
     return torch.mm(x, weight.t(), out_dtype=torch.float32)
 

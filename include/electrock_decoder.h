@@ -55,9 +55,10 @@ int ed_argmax(const float* x, int64_t T, int V, int32_t* out, void* stream);
 int ed_skinny_gemm_splits(int64_t T, int N, int K);
 int ed_skinny_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
                    void* stream);
-/* The same for every T <= 64, whatever the weights' size; ed_decode_gemm_plain_pays: 1 if that is the faster way also for a
- * product without activation that is stored in bf16. */
+/* The same for every T <= 64, whatever the weights' size; ed_decode_gemm_pays: 1 if that (with one range) is faster than the library's
+ * product and the kernel of its activation (ed_decode_gemm_plain_pays: without one, stored in bf16). */
 int ed_decode_gemm_splits(int64_t T, int N, int K);
+int ed_decode_gemm_pays(int64_t T, int N, int K, int act, int out_dtype);
 int ed_decode_gemm_plain_pays(int64_t T, int N, int K);
 int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
                    void* stream);
