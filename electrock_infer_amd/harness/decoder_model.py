@@ -28,6 +28,10 @@ class DecoderModel(nn.Module):
         """Tokens that one workgroup of the recurrent mixers' prompt kernels takes in a step of ``tokens``."""
         return 256
 
+    def chunk_for(self, portions: List[int]) -> int:
+        """The same for a step of these portions."""
+        return self.chunk_tokens(sum(portions))
+
     # ---- weights ----
     def checkpoint_target(self, name: str):
         """(parameter name, section or None) of a checkpoint tensor, or None."""

@@ -146,6 +146,12 @@ class FeguvikForCausalLM(DecoderModel):
         work = tokens * self.chunk_heads
         return 32 if work <= 8192 else 64 if work <= 49152 else 128 if work <= 98304 else 256
 
+    def chunk_for(self, portions: List[int]) -> int:
+        """Where the portions alone give half of the CUs a chunk, shorter ones only bring more states to pass on (us with the
+        projections, 32 heads: 8 x 128 tokens in chunks of 64 199, 128 178; 4 x 60 in 32 92, 64 and 128 86; 8 heads, 8 x 128 in 32 62, 128 73)."""
+        chunk = self.chunk_tokens(sum(portions))
+        return max(chunk, 128) if len(portions) * self.chunk_heads >= 128 else chunk
+
     # ---- forward ----
     def forward(self, batch: RaggedBatch) -> torch.Tensor:
         """Normed output [T, width] of every token of the batch."""

@@ -68,7 +68,7 @@ class ModelRunner:
         """The planned portions of any batch, for models that take RaggedBatch; ``rows``: batch rows whose logits are
         wanted (default: the last one of every sequence)."""
         self.check_slots(seqs)
-        chunk = self.model.chunk_tokens(sum(s.num_scheduled_tokens for s in seqs))
+        chunk = self.model.chunk_for([s.num_scheduled_tokens for s in seqs])
         return make_ragged(seqs, self.block_size, chunk, self.device, rows)
 
     def prepare_prefill(self, seqs: List[Sequence]):

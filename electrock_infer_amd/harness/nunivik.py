@@ -117,8 +117,9 @@ class NunivikForCausalLM(DecoderModel):
     def chunk_tokens(self, tokens: int) -> int:
         """Fewer, longer chunks where there are enough of them to fill the chip: the scan over them is sequential (us of both
         mixers' kernels, width 4096, five prompts of 600 tokens: chunks of 128 929, 256 894, 512 1294; width 2048: 8192 tokens
-        512 981, 256 1043; 4096 256 535, 512 576; 1024 128 214, 256 269; 300 64 145, 128 173)."""
-        work = tokens * self.cfg.width // 2048
+        512 981, 256 1043; 4096 256 535, 512 576; 1024 128 214, 256 269; 300 64 145, 128 173; width 1024 is no different, with the
+        projections: 8 prompts of 128 64 119, 128 100; 3 of 2500 128 387, 256 354)."""
+        work = tokens * max(1, self.cfg.width // 2048)
         return 512 if work >= 8192 else 256 if work >= 4096 else 128 if work >= 1024 else 64
 
     def forward(self, batch: RaggedBatch) -> torch.Tensor:
