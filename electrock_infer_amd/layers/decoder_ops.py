@@ -117,8 +117,11 @@ def relu_squared_(u: torch.Tensor) -> torch.Tensor:
 
 def argmax_rows(x: torch.Tensor) -> torch.Tensor:
     """int32 [T]: the place of the largest value of every row of ``x`` [T, V], the first of equal ones; what the kernel does not
-    take (other types, shapes, devices) goes to the library's, along the last dimension."""
-    if x.dtype != torch.float32 or x.dim() != 2 or x.shape[1] == 0 or not x.is_cuda:
+    take (other types, shapes, devices, more workgroups than a launch has threads for) goes to the library's, along the last
+    dimension, and so does one row that is long enough to be shared out over the chip (us, kernel / library: one of 128256 22.8 /
+    29.1, of 160000 27.7 / 11.8; two of 160000 27.8 / 35.6)."""
+    if (x.dtype != torch.float32 or x.dim() != 2 or x.shape[1] == 0 or not x.is_cuda or x.shape[0] >= 1 << 22 or
+            (x.shape[0] == 1 and x.shape[1] > 1 << 17)):
         return x.argmax(dim=-1).int()
     x = x.contiguous()
     out = torch.empty(x.shape[0], dtype=torch.int32, device=x.device)

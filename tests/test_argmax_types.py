@@ -29,3 +29,12 @@ def test_host_rows(dtype):
 def test_device_rows(dtype):
     announce(f"argmax of {dtype}")
     check(dtype, "cuda")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,V", [(1, 1 << 17), (1, (1 << 17) + 1), (2, (1 << 17) + 1), (1, 500001), ((1 << 22) - 1, 3), (1 << 22, 3)])
+def test_long_rows_and_many(T, V):
+    announce(f"argmax {T} x {V}")
+    x = torch.randn(T, V, generator=torch.Generator(device="cuda").manual_seed(V), device="cuda")
+    x[:, V // 2] = x[:, V - 1] = 9.0                           # the first of equal ones
+    assert bool((argmax_rows(x) == V // 2).all())
