@@ -199,12 +199,16 @@ int launch_tiles(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_
 // half the products and exponentials to a tile, and CUs without work take the other half (us, 128 / 64 queries, heads of
 // 128 + 64: 48 workgroups, 300 tokens behind 1000, 53.5 / 35.2; 128, one prompt of 1024 42.8 / 29.1; 256, 2048 80 / 59 and
 // 4 x 512 25.7 / 24.0; 384, 3072 123 / 88; 512, 4 x 1024 55.8 / 57.1, 4096 163 / 152, behind 4000 328 / 385; 1024, 8192
-// 397 / 520).  A query's sums keep their order either way.
-constexpr int64_t kFewWorkgroups = 512;
+// 397 / 520; a little below 512, portions that end early in their last 128 queries lose: 480, 15 x 200, heads of 128 + 32 21.5 /
+// 24.2).  Keys of up to 128 elements under values of more than 64 gain little from it, and only while the workgroups of 64 have a
+// CU each (96 + 32, values of 128: 128, 1000 behind 1000 56.6 / 51.4; 256, 2 x 1000 behind 3000 107 / 126).  A query's sums keep
+// their order either way.
+template <int DKT, int DVT>
+constexpr int64_t few_workgroups() { return DKT <= 4 && DVT > 4 ? 160 : 448; }
 
 template <int DKT, int DVT>
 int launch_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s) {
-    if (ceil_div(max_q, 128) * p.heads * n_seqs < kFewWorkgroups) return launch_tiles<DKT, DVT, 1>(p, n_seqs, max_q, s);
+    if (ceil_div(max_q, 128) * p.heads * n_seqs < few_workgroups<DKT, DVT>()) return launch_tiles<DKT, DVT, 1>(p, n_seqs, max_q, s);
     return launch_tiles<DKT, DVT, 2>(p, n_seqs, max_q, s);
 }
 
