@@ -384,14 +384,15 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
 // What bounds it: the vector units (54 % busy) and the matrix units (26 %) take turns, as a wave's scores wait for one product
 // and its second product for the scores, with two waves on a SIMD.  So a score is kept cheap and a tile free of waits:
 //   * the cap's tanh takes two of the three slow instructions of a score (exponential, reciprocal).  Up to kTanhRange caps
-//     tanh(x) is x times a polynomial of degree four in x * x (least largest relative error, 7.3e-8: about half a unit in the
-//     last place); a wave whose 32 x 64 scores all lie there takes it, four scores in step, others take the exponential.  Caps
+//     tanh(x) is x times a polynomial of degree four in x * x (its coefficients as written: 9.1e-8 of the value at the end of the
+//     range, in float32 with the cap in them 1.5e-7, one to two units in the last place); a wave whose 32 x 64 scores all lie there takes it, four scores in step, others take the exponential.  Caps
 //     are chosen far above ordinary scores.
 //   * the page of a tile's keys is asked for a tile ahead of its use and in front of the loads that use the one before, and the
 //     rows are read from LDS in front of the barrier; loads have no condition of their own (keys behind the last stand for it).
 // One prompt of 8192 tokens, 16 heads of 128, cap 30: 427 -> 386 us, window 1024: 119.5 -> 112.6; scores beyond the range
-// 422 -> 401, no cap 386 -> 368; 8 x 1000 tokens, heads of 64: 61.7 -> 59.4; heads of 256 / 64: 249 -> 228.  Two tiles in LDS
-// with one barrier a tile were no faster (394 us, 114).
+// 422 -> 401, no cap 386 -> 368; 8 x 1000 tokens, heads of 64: 63.4 -> 60.3 (three workgroups to a CU, three registers of
+// them spilled: 300 tokens 13.3 -> 13.7); heads of 256 / 64: 249 -> 228, 256 / 128 644 -> 608.  Two tiles in LDS with one barrier a
+// tile were no faster (394 us, 114).
 constexpr float kTanhRange = 0.6f;
 constexpr int kTileKeys = 64;
 constexpr int kRowsPerWave = 32;

@@ -319,8 +319,8 @@ __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::stor
 }
 
 // Place of the largest value of a row, the first one where several are equal; a NaN is larger than every number.  One
-// workgroup per row, eight vectors of it requested at once: 32000 columns take a way to memory and the sum over the workgroup
-// (4.5 us; the library's two passes 15).
+// workgroup per row, eight vectors of it requested at once: 32000 columns take a way to memory and the comparison over the workgroup
+// (one row 8.1 us, 64 rows 8.6; the library 10.7 and 11.3).
 constexpr int kArgmaxThreads = 1024;
 __device__ __forceinline__ bool argmax_before(float a, int ia, float b, int ib) {
     const bool na = a != a, nb = b != b;

@@ -52,6 +52,7 @@ int ed_argmax(const float* x, int64_t T, int V, int32_t* out, void* stream);
  * weights), K a multiple of 64; act 0: none,
  * 1: max(v, 0)^2, 2: w is [2 N, K], out = silu(x w_c) * (x w_(N + c)) in bf16.  splits > 1: out is float32 [splits, T, N], partial sums over K (no act).  ed_skinny_gemm_splits: how
  * many fill the chip, 0 if the shape is not taken. */
+/* (ed_skinny_gemm: the first form of ed_decode_gemm, for callers of it; it refuses what it refused.) */
 int ed_skinny_gemm_splits(int64_t T, int N, int K);
 int ed_skinny_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
                    void* stream);
