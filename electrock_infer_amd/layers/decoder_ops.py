@@ -21,21 +21,23 @@ def _skinny(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: in
     return out
 
 
+def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Operands of the weight-streaming kernel: at most 64 rows.  What does not fit each other, is to be differentiated or is no dense
+    row from a 16-byte boundary is the library's, to compute or to refuse."""
+    shape, rows = x.shape, weight.shape
+    return (len(shape) == 2 and shape[0] <= 64 and len(rows) == 2 and shape[1] == rows[1] and x.dtype == weight.dtype == torch.bfloat16 and
+            x.device == weight.device and x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
+            not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)))
+
+
 def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
-    """For a decode batch that the weight-streaming kernel takes (at most 64 rows, any size of the weights): how many ranges of
-    K fill the chip; else 0: operands that do not fit each other, that are to be differentiated or that are not dense rows from a
-    16-byte boundary are the library's, to compute or to refuse."""
-    if not (x.dtype == weight.dtype == torch.bfloat16 and x.dim() == weight.dim() == 2 and x.shape[0] <= 64 and
-            x.shape[1] == weight.shape[1] and x.device == weight.device and x.is_contiguous() and weight.is_contiguous()):
-        return 0
-    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad) or (x.data_ptr() | weight.data_ptr()) % 16:
-        return 0
-    return _lib.load_decoder().ed_decode_gemm_splits(x.shape[0], *weight.shape)
+    """For a decode batch that the weight-streaming kernel takes: how many ranges of K fill the chip; else 0."""
+    return _lib.load_decoder().ed_decode_gemm_splits(x.shape[0], *weight.shape) if _fits(x, weight) else 0
 
 
 def _streams(x: torch.Tensor, weight: torch.Tensor, out_rows: int, act: int = 0, out_dtype: int = _lib.DTYPE_BF16) -> bool:
     """Whether the weight-streaming kernel takes the product and is the faster way."""
-    return _skinny_splits(x, weight) > 0 and _lib.load_decoder().ed_decode_gemm_pays(x.shape[0], out_rows, x.shape[1], act, out_dtype) == 1
+    return _fits(x, weight) and _lib.load_decoder().ed_decode_gemm_pays(x.shape[0], out_rows, weight.shape[1], act, out_dtype) == 1
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
