@@ -691,11 +691,15 @@ bool attn_supported(int heads, int kv_heads, int dim, int vdim, int rot) {
 // steps count.  us with the combination, 16 heads on 4: 64 x 768 keys in ones 26.9, in threes 29.6; 24 x 2000 keys in threes
 // 34.9, fours 31.1, eights 28.8; 8 x 2000 in eights 16.0, sixteens 17.9; 64 x 4096 in ones 109.6, twos 103.1.  Forms without the
 // next tile in flight hide its way with other workgroups (float32, 64 + 64: 24 x 2000 keys in threes 50.0, eights 31.8; bf16,
-// 192 + 64 in threes 40.8, eights 30.3).
+// 192 + 64 in threes 40.8, eights 30.3).  A CU's second workgroup of the form that reads its rows once gains little, as the pages
+// come near memory's rate: where every CU has one without a split, that is worth a launch only behind long contexts (64 sequences
+// of 1024 keys in ones 33.5, twos 35.0; 2048 keys 58.9 / 58.5, 4096 108.5 / 102.8; and a recorded step plans for up to twice the
+// keys that it has: 1064 of 2048 36.3 / 38.9).
 int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int64_t max_q, int64_t keys) {
     const int64_t row_groups = ceil_div(max_q * (heads / kv_heads), 16), groups = row_groups * n_seqs * kv_heads, most = ceil_div(keys, 4 * kKeys);
     const bool bf16 = dtype == EM_DTYPE_BF16, ahead = bf16 && dim <= 128, once = bf16 && row_groups == 1;
     const double in_flight = once ? 384.0 : ahead ? 256.0 : 768.0, results = once || ahead ? 0.6 : 1.0;
+    if (once && groups >= 256 && keys <= 2048) return 1;
     int best = 1;
     double least = 0.0;
     for (int64_t s = 1; s <= most && s <= kAttnMaxSplits; ++s) {

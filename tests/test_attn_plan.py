@@ -25,6 +25,12 @@ def test_forms_that_wait_for_their_keys_have_more_workgroups_in_flight():
     assert 96 * splits(F32, 64, 64) >= 750 and 96 * splits(F32, 128, 128) >= 750 and 96 * splits(BF16, 64, 64) > 288 < 96 * splits(BF16, 192, 64)
 
 
+def test_a_full_chip_is_split_behind_long_contexts_only():
+    """64 sequences on four key heads: one row group for every CU."""
+    splits = lambda n, keys: _lib.load_decoder().ed_attn_splits(BF16, 16, 4, 128, 128, n, 1, keys)
+    assert [splits(64, k) for k in (128, 1024, 2048)] == [1, 1, 1] and splits(64, 4096) == 2 and splits(63, 2048) > 1
+
+
 def test_a_window_bounds_the_keys():
     import torch
     batch = type("B", (), {"max_q": 1, "n_seqs": 1, "max_context": 8192})()
