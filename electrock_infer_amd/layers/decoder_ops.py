@@ -4,6 +4,7 @@ import ctypes
 from typing import Optional
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
 
 from .. import _lib
@@ -22,10 +23,11 @@ def _skinny(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: in
 
 
 def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Operands of the weight-streaming kernel: at most 64 rows.  What does not fit each other, is to be differentiated or is no dense
-    row from a 16-byte boundary is the library's, to compute or to refuse."""
+    """Operands of the weight-streaming kernel: at most 64 rows.  What does not fit each other, is to be differentiated (backward or
+    forward), mapped or traced, or is no dense row from a 16-byte boundary is the library's, to compute or to refuse."""
     shape, rows = x.shape, weight.shape
-    return (len(shape) == 2 and shape[0] <= 64 and len(rows) == 2 and shape[1] == rows[1] and x.dtype == weight.dtype == torch.bfloat16 and
+    return (forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active() and torch._C._get_tracing_state() is None and
+            len(shape) == 2 and shape[0] <= 64 and len(rows) == 2 and shape[1] == rows[1] and x.dtype == weight.dtype == torch.bfloat16 and
             x.device == weight.device and x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
             not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)))
 

@@ -79,3 +79,17 @@ def test_rows_of_any_shape_and_gradients_are_the_librarys(shape):
     if len(shape) == 2:
         with torch.no_grad():
             assert ops._skinny_splits(x, w) > 0
+
+
+def test_mapped_forward_differentiated_and_traced_calls_are_the_librarys():
+    x, w, t = bf16(3, 8, 64), bf16(48, 64), bf16(8, 64)
+    assert torch.equal(torch.func.vmap(lambda a: ops.linear(a, w))(x), torch.func.vmap(lambda a: F.linear(a, w))(x))
+    product = lambda f: torch.func.jvp(lambda a: f(a, w), (x[0],), (t,))
+    assert all(torch.equal(a, b) for a, b in zip(product(ops.linear), product(F.linear)))
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x[0], t)
+        assert ops._skinny_splits(dual, w) == 0
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(ops.linear(dual, w)).tangent, F.linear(t, w))
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda a: ops.linear(a, w), x[0], check_trace=False)
+        assert torch.equal(traced(x[1]), F.linear(x[1], w)) and ops._skinny_splits(x[0], w) > 0
