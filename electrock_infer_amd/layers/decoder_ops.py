@@ -39,7 +39,7 @@ def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
 
 def _streams(x: torch.Tensor, weight: torch.Tensor, out_rows: int, act: int = 0, out_dtype: int = _lib.DTYPE_BF16) -> bool:
     """Whether the weight-streaming kernel takes the product and is the faster way."""
-    return _fits(x, weight) and _lib.load_decoder().ed_decode_gemm_pays(x.shape[0], out_rows, weight.shape[1], act, out_dtype) == 1
+    return x.is_cuda and _fits(x, weight) and _lib.load_decoder().ed_decode_gemm_pays(x.shape[0], out_rows, weight.shape[1], act, out_dtype) == 1
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
@@ -78,7 +78,7 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 def linear_parts(x: torch.Tensor, weight: torch.Tensor, exact: bool = False) -> torch.Tensor:
     """x @ weight^T as ``residual_norm`` takes it: [T, N], or float32 partial sums [parts, T, N] of a decode batch.
     ``exact``: not rounded to the compute type on the way."""
-    splits = _skinny_splits(x, weight)
+    splits = _skinny_splits(x, weight) if x.is_cuda else 0
     if splits > 1:
         return _skinny(x, weight, torch.empty(splits, x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), splits, 0)
     return linear_f32(x, weight) if exact else linear(x, weight)

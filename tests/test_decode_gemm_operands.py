@@ -93,3 +93,10 @@ def test_mapped_forward_differentiated_and_traced_calls_are_the_librarys():
     with torch.no_grad():
         traced = torch.jit.trace(lambda a: ops.linear(a, w), x[0], check_trace=False)
         assert torch.equal(traced(x[1]), F.linear(x[1], w)) and ops._skinny_splits(x[0], w) > 0
+
+
+@pytest.mark.parametrize("T,N,K", SIZES + [(20, 4608, 4096)])
+def test_host_tensors_are_the_librarys(T, N, K):
+    x, w = bf16(T, K), bf16(N, K)
+    want = F.linear(x, w)
+    assert torch.equal(ops.linear(x, w), want) and torch.equal(ops.linear_parts(x, w), want)
