@@ -7,6 +7,7 @@ namespace {
 
 constexpr int kRowMaxPerThread = 32;  // floats of a row that one thread keeps in registers
 constexpr int64_t kFewRows = 256;     // up to so many rows a CU has one at most
+constexpr int kPartPiece = 16;        // elements of a partial sum's row that a thread requests at once where it takes them one by one
 
 // Sum over the workgroup, the same value and the same order in every thread.  `scratch`: one float per wave.
 template <int THREADS>
@@ -60,7 +61,9 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t* __restrict__ 
 // y may be given as float32 partial sums [y_parts, T, W].
 //   UPDATE 0: x stays          UPDATE 1: x += y / rms(y) * post_w          UPDATE 2: x = y + post_w
 //   then, when out != null: out = next_w ? x / rms(x) * next_w : x, rounded to the compute type
-// PARTS: y_parts > 1, of which one is requested at a time for the whole row (64 rows of 8192 in threes 8.4 -> 7.4 us).
+// PARTS: y_parts > 1, of which one is requested at a time, for the whole row (64 rows of 8192 in threes 8.4 -> 7.4 us), or in pieces
+// where elements go one by one: a whole row's addresses spill, and short rows would ask 32 times for a few (float32, in eights, element
+// by element / whole rows / pieces: 64 rows of 9001 15.1 / 21.3 / 13.8, 300 of 1022 8.7 / 9.7 / 8.6, 64 of 20001 51 / 36 / 27).
 template <typename Elem, typename YElem, int UPDATE, int VEC, int THREADS, int N, bool PARTS>
 __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
     float* __restrict__ x, const typename YElem::storage* __restrict__ y, int y_parts, const float* __restrict__ post_w,
@@ -85,17 +88,22 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
             }
         }
         if (PARTS) {
-            for (int p = 1; p < y_parts; ++p) {
-                float more[N][VEC];
+            constexpr int kPiece = VEC == 1 ? kPartPiece : N;
 #pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    const int c = (threadIdx.x + i * THREADS) * VEC;
-                    if (c < W) RowIo<YElem, VEC>::load(yr + static_cast<int64_t>(p) * gridDim.x * W + c, more[i]);
+            for (int i0 = 0; i0 < N; i0 += kPiece) {
+                if (i0 * THREADS * VEC >= W) break;
+                for (int p = 1; p < y_parts; ++p) {
+                    float more[kPiece][VEC];
+#pragma unroll
+                    for (int i = 0; i < kPiece; ++i) {
+                        const int c = (threadIdx.x + (i0 + i) * THREADS) * VEC;
+                        if (c < W) RowIo<YElem, VEC>::load(yr + static_cast<int64_t>(p) * gridDim.x * W + c, more[i]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < kPiece; ++i)
+#pragma unroll
+                        for (int j = 0; j < VEC; ++j) v[i0 + i][j] += more[i][j];
                 }
-#pragma unroll
-                for (int i = 0; i < N; ++i)
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) v[i][j] += more[i][j];
             }
 #pragma unroll
             for (int i = 0; i < N; ++i)
@@ -392,7 +400,8 @@ int launch_gated(void* y, const void* z, int64_t z_stride, const float* w, int64
 // count for more than a row's way: the normed update, which keeps four rows of floats that way, waits with its weights and the
 // stream (rows of 4096, at once / in turn: 300 6.0 / 5.8, 1024 11.0 / 8.6, 3505 32.0 / 26.9, 16384 206 / 148; 8192 of 2048 31.8 / 30.4);
 // y + w, which keeps three, does so for long rows in large numbers only (rows of 4096: 768 6.6 / 6.9, 1500 10.9 / 9.7, 16384 133 / 113;
-// 8192 of 2048 21.4 / 21.9), x alone never (8192 of 4096 29.6 / 30.8).
+// 8192 of 2048 21.4 / 21.9), and not with partial sums, which it requests in fours (300 of 4096 in twos 6.0 / 5.1), x alone never (8192 of
+// 4096 29.6 / 30.8).
 template <typename Elem, typename YElem, int UPDATE, int VEC>
 int launch_residual(float* x, const void* y, int y_parts, const float* post_w, const float* next_w, void* out, int64_t out_stride,
                     int64_t T, int W, float eps, hipStream_t s) {
@@ -412,7 +421,7 @@ int launch_residual(float* x, const void* y, int y_parts, const float* post_w, c
     if constexpr (VEC == 4) {
         if (T <= kFewRows && W > 1024 && W <= 2048) EM_EARLY(512, 1);
         if (T <= kFewRows && W > 1024 && W <= 4096) EM_EARLY(1024, 1);
-        const bool early = T <= kFewRows || UPDATE == 0 || (UPDATE == 2 && (W <= 2048 || T <= 4 * kFewRows));
+        const bool early = T <= kFewRows || UPDATE == 0 || (UPDATE == 2 && y_parts == 1 && (W <= 2048 || T <= 4 * kFewRows));
         if (early && W <= 2048) EM_EARLY(256, 2);
         if (early && W <= 4096) EM_EARLY(256, 4);
         if (W <= 2048) EM_LATE(256, 2);

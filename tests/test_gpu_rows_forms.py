@@ -46,6 +46,14 @@ def test_residual_norm(T, W, y_dtype, dtype, parts):
             near(stream, (x.double() + rms(whole) * post.double() if update == ops.ADD_NORMED else whole + post.double()).cpu(), F32)
 
 
+# partial sums element by element: one piece of 16 elements a thread (256 threads up to 4096 columns), two, and the same of 1024 threads;
+# more rows than are requested at once
+@pytest.mark.parametrize("T,W", [(2, 4095), (2, 4097), (1, 8190), (2, 9001), (2, 16383), (2, 16385), (1, 32767), (300, 4096), (300, 2048)])
+@pytest.mark.parametrize("dtype,parts", [(F32, 2), (BF16, 3), (F32, 8)])
+def test_partial_sums_in_pieces(T, W, dtype, parts):
+    test_residual_norm(T, W, F32, dtype, parts)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("T,parts,size", [(3, 1, 512), (3, 1, 516), (3, 1, 1024), (2, 3, 1028), (256, 1, 4096), (257, 1, 4096), (128, 2, 2048), (129, 2, 2048),
                                           (3, 1, 4100), (3, 1, 8192), (2, 1, 8196), (300, 1, 8192), (3, 2, 1021), (3, 1, 8191), (2, 1, 9001), (1, 1, 32768)])
