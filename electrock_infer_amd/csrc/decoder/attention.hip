@@ -390,16 +390,17 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
 //   * the page of a tile's keys is asked for a tile ahead of its use and in front of the loads that use the one before, and the
 //     rows are read from LDS in front of the barrier; loads have no condition of their own (keys behind the last stand for it).
 // One prompt of 8192 tokens, 16 heads of 128, cap 30: 427 -> 386 us, window 1024: 119.5 -> 112.6; scores beyond the range
-// 422 -> 401, no cap 386 -> 368; 8 x 1000 tokens, heads of 64: 63.4 -> 60.3 (three workgroups to a CU, three registers of
-// them spilled: 300 tokens 13.3 -> 13.7); heads of 256 / 64: 249 -> 228, 256 / 128 644 -> 608.  Two tiles in LDS with one barrier a
-// tile were no faster (394 us, 114).
+// 422 -> 401, no cap 386 -> 368; 8 x 1000 tokens, heads of 64: 63.4 -> 60.3; heads of 256 / 64: 249 -> 228, 256 / 128
+// 644 -> 608.  Two tiles in LDS with one barrier a tile were no faster (394 us, 114).  Capped portions of up to 500 tokens with heads of up
+// to 64, whose few tiles do not pay for the second form of the scores, are 1 to 4 % slower (1 x 173 8.5 -> 8.7).
 constexpr float kTanhRange = 0.6f;
 constexpr int kTileKeys = 64;
 constexpr int kRowsPerWave = 32;
 constexpr int kRows = 4 * kRowsPerWave;
 
-template <int DKT, int DVT>
-__global__ __launch_bounds__(256, DKT == 2 && DVT == 4 ? 3 : 2) void attn_prompt_kernel(AttnProblem p) {
+// GROUPS: workgroups that a CU is to hold
+template <int DKT, int DVT, int GROUPS>
+__global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p) {
     typedef Mma<BF16Elem> M;
     constexpr int LPK = DKT * 32 + 8, LPV = DVT * 16 + 8;
     constexpr bool kPoly = DKT <= 4;       // registers enough for a second form of the scores
@@ -669,11 +670,24 @@ int keys_paged(const AttnProblem& p, int n_seqs, int max_q, int splits, float* p
     return values_paged<Elem, 8>(p, n_seqs, max_q, splits, part_o, part_ml, T, s);
 }
 
+// Heads of up to 64 elements: three workgroups to a CU, which costs three spilled registers, where two would leave some for a further round
+// (us, two / three: 32 heads, 8 x 291 tokens, 768 workgroups, 26.1 / 21.2; 1 x 4450, 1120, 53.5 / 46.7; 16 heads, 8 x 639 behind 4000, 640,
+// 47.5 / 38.6; 8 x 221, 512, 13.2 / 13.8; 16 x 59, 128, 5.3 / 5.7).
+constexpr int64_t kTwoPerCu = 512;
+
 template <int DKT>
 int launch_prompt(const AttnProblem& p, int n_seqs, int max_q, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(p.heads), static_cast<unsigned>(ceil_div(max_q, kRows)), static_cast<unsigned>(n_seqs));
-    if (p.vdim <= 64) launch((attn_prompt_kernel<DKT, 4>), grid, dim3(256), 0, s, p);
-    else launch((attn_prompt_kernel<DKT, 8>), grid, dim3(256), 0, s, p);
+    if (p.vdim > 64) {
+        launch((attn_prompt_kernel<DKT, 8, 2>), grid, dim3(256), 0, s, p);
+        return launch_status();
+    }
+    if constexpr (DKT == 2)
+        if (static_cast<int64_t>(grid.x) * grid.y * grid.z > kTwoPerCu) {
+            launch((attn_prompt_kernel<DKT, 4, 3>), grid, dim3(256), 0, s, p);
+            return launch_status();
+        }
+    launch((attn_prompt_kernel<DKT, 4, 2>), grid, dim3(256), 0, s, p);
     return launch_status();
 }
 

@@ -59,3 +59,33 @@ def test_scores_in_every_form_of_the_cap(dim, vdim, n, first, window, cap, stren
     bound = size * (2.0 ** -8 + 4e-4) + want.abs() * 2.0 ** -8 + 1e-6
     worst = ((out.cpu().double() - want).abs() / bound).max().item()
     assert worst <= 1, worst
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (40, 8)])
+@pytest.mark.parametrize("cap,strength", [(30.0, 1.0), (30.0, 4.5), (60.0, 4.0), (0.0, 1.0)])
+def test_both_numbers_of_workgroups_to_a_cu(dim, vdim, cap, strength):
+    """Portions that alone make 64 workgroups and together 576, which is more than two to a CU: the same sums in the same order."""
+    n, first, window, S, H, G = 200, 37, 90, 9, 32, 8
+    total, pages = first + n, -(-(first + n) // BLOCK)
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    q = (torch.randn(S * n, H, dim, generator=g, device=DEV) * strength).to(BF16)
+    cache = torch.randn(S * pages, BLOCK, G * (dim + vdim), generator=g, device=DEV).to(BF16)
+    tables = torch.randperm(S * pages, generator=g, device=DEV).int().view(S, pages)
+    spare = torch.zeros(S * n, dtype=torch.int64, device=DEV)
+
+    def attend(at, count):
+        announce(f"attn prompt groups {dim} {vdim} cap {cap} x {strength} portions {at} + {count}")
+        begin = (torch.arange(count + 1, device=DEV) * n).int()
+        starts, out = torch.full((count,), first, device=DEV).int(), torch.full((count * n, H, vdim), float("nan"), dtype=BF16, device=DEV)
+        mine, pages_of = q[at * n:(at + count) * n].contiguous(), tables[at:at + count].contiguous()
+        a = _lib.AttnArgs(q=mine.data_ptr(), k=mine.data_ptr(), v=mine.data_ptr(), stride=H * dim, positions=spare.data_ptr(), cache_rows=spare.data_ptr(),
+                          cache=cache.data_ptr(), q_rows=mine.data_ptr(), out=out.data_ptr(), q_begin=begin.data_ptr(), starts=starts.data_ptr(),
+                          tables=pages_of.data_ptr(), T=count * n, n_seqs=count, max_q=n, table_width=pages, block_size=BLOCK, splits=1, heads=H,
+                          kv_heads=G, dim=dim, vdim=vdim, rot=0, window=window, dtype=_lib.DTYPE_BF16, scale=dim ** -0.5, softcap=cap, eps=1e-6)
+        assert _lib.load_decoder().ed_attn_prompt(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return out
+
+    assert total <= pages * BLOCK
+    together = attend(0, S)
+    assert bool(torch.isfinite(together).all()) and torch.equal(together, torch.cat([attend(i, 1) for i in range(S)]))
