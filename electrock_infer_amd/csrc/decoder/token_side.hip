@@ -377,12 +377,14 @@ int launch_rows(TokenSideProblem p, size_t lds, hipStream_t s) {
     return launch_status();
 }
 
-// One row per wave while two do not fill the chip; and where two would leave one workgroup to a CU, whose phases then wait for
-// each other (rows kept in registers; us for 8192 rows, one / two: W = 1024 37 / 31, 2048 70 / 82, 4096 200 / 160).
+// One row per wave while two do not fill the chip; and with eight pieces a lane, whose two rows in registers take a CU to themselves, where
+// the LDS lets a second workgroup in: phases of one then run while the other waits (us for 8192 rows, one / two: W = 1024 37 / 31,
+// 2048 66 / 79, 4096 200 / 160).  With LDS for one workgroup only (W = 1536 from dim 96, 1280 from 256) half of a tile's rows would be
+// empty for nothing: W = 1536, dim 96 98.8 / 69.1, 3072 rows 47.2 / 34.4 (40.2 before the weights were packed), 2048 x 256 191 / 126.
 template <int NV, bool FULL>
 int launch_side(const TokenSideProblem& p, size_t lds, hipStream_t s) {
     if constexpr (FULL)
-        if (p.packed) return p.T <= 512 || NV == 8 ? launch_rows<NV, FULL, 1, true>(p, lds, s) : launch_rows<NV, FULL, 2, true>(p, lds, s);
+        if (p.packed) return p.T <= 512 || (NV == 8 && 2 * lds <= kLdsPerCu) ? launch_rows<NV, FULL, 1, true>(p, lds, s) : launch_rows<NV, FULL, 2, true>(p, lds, s);
     return p.T <= 512 ? launch_rows<NV, FULL, 1, false>(p, lds, s) : launch_rows<NV, FULL, 2, false>(p, lds, s);
 }
 

@@ -37,3 +37,10 @@ def test_packed_weights(W, T, dim, last):
         got.append((stream, out[:, :W].float()))
     # the same products in the same order: nothing but the order of the rows' registers differs
     assert float((got[0][0] - got[1][0]).abs().max()) <= 2 ** -20 * float(x.abs().max()) and torch.equal(got[0][1], got[1][1])
+
+
+# eight pieces a lane on both sides of the LDS that two workgroups share, with whole and ragged groups of rows
+@pytest.mark.parametrize("W,dim", [(1280, 192), (1280, 256), (1408, 96), (1408, 128), (1536, 96), (2048, 256)])
+@pytest.mark.parametrize("T", [512, 513, 521, 544])
+def test_rows_of_a_wave_by_lds(W, T, dim):
+    test_packed_weights(W, T, dim, False)
