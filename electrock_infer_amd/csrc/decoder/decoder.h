@@ -60,6 +60,7 @@ int launch_token_gate(const void* x, const void* gate, const int32_t* tokens, co
                       int column0, void* g, int64_t T, int W, int dim, int dtype, hipStream_t s);
 bool token_side_supported(int W, int dim);
 inline bool token_side_packable(int W, int dim) { return W % 128 == 0 && dim % 32 == 0; }
+bool token_side_pack_pays(int64_t T, int W, int dim);
 int launch_token_side_pack(const uint16_t* gate, const uint16_t* proj, uint16_t* gate_out, uint16_t* proj_out, int W, int dim, hipStream_t s);
 int launch_token_side(TokenSideProblem p, hipStream_t s);
 

@@ -273,6 +273,8 @@ int ed_token_side(float* x, const void* y, const float* post_w, const void* gate
 
 int ed_token_side_packable(int W, int dim) { return token_side_supported(W, dim) && token_side_packable(W, dim) ? 1 : 0; }
 
+int ed_token_side_pack_pays(int64_t T, int W, int dim) { return ed_token_side_packable(W, dim) && token_side_pack_pays(T, W, dim) ? 1 : 0; }
+
 int ed_token_side_pack(const void* gate, const void* proj, void* gate_out, void* proj_out, int W, int dim, void* stream) {
     if (!ed_token_side_packable(W, dim)) return EM_ERR_UNSUPPORTED;
     if (!gate || !proj || !gate_out || !proj_out) return EM_ERR_NULL_POINTER;

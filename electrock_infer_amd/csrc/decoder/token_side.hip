@@ -409,6 +409,16 @@ bool token_side_supported(int W, int dim) {
     return W > 0 && W % 4 == 0 && W <= 4096 && dim > 0 && dim <= 1024 && lds_bytes(W, dim, &a, &b) <= kLdsPerCu;
 }
 
+// Packing is a launch of its own, 0.5 to 2 us behind whose rows the loads in operand order have to come out ahead (us, as they are / packed
+// and packing): rows of up to 256 with few columns do not (128 x 64, 1024 rows 9.8 / 11.2; 256 x 96, 4096 13.3 / 14.4), 32 columns only
+// with long or many rows (512, 4096 rows 13.6 / 14.3, 8192 17.9 / 17.1; 1024, 4096 25.1 / 22.2), and rows of 1152 to 1920 with 32 lose
+// where twice as many workgroups, of one row per wave, take a round more (1536, 4000 rows 33 / 24, 6144 41.6 / 44.6, 9216 71.5 / 65.2).
+bool token_side_pack_pays(int64_t T, int W, int dim) {
+    if (dim >= 64) return W >= 384 || W * dim >= 65536 || (W * dim > 16384 && T > 4096);
+    if (W <= 1024) return W >= (T > 4096 ? 384 : 1024);
+    return W >= 2048 || T <= 4096 || T > 8192;
+}
+
 int launch_token_side_pack(const uint16_t* gate, const uint16_t* proj, uint16_t* gate_out, uint16_t* proj_out, int W, int dim, hipStream_t s) {
     launch(token_side_pack_kernel, dim3(static_cast<unsigned>(ceil_div(W / 8 * dim, 256))), dim3(256), 0, s, gate, proj, gate_out, proj_out, W, dim);
     return launch_status();

@@ -40,7 +40,7 @@ class TokenSideInput(nn.Module):
         lib, dim = _lib.load_decoder(), self.gate.shape[0]
         if T >= self.ONE_LAUNCH_ROWS * W and y.dim() == 2 and y.dtype == torch.bfloat16 and out.stride(0) % 4 == 0 and lib.ed_token_side_supported(W, dim) == 1:
             gate, proj, run, stream = self.gate, self.proj, lib.ed_token_side, _lib.current_stream(x.device)
-            if self.gate_packed is not None:
+            if self.gate_packed is not None and lib.ed_token_side_pack_pays(T, W, dim) == 1:
                 gate, proj, run = self.gate_packed, self.proj_packed, lib.ed_token_side_packed
                 _lib.check_decoder(lib.ed_token_side_pack(self.gate.data_ptr(), self.proj.data_ptr(), gate.data_ptr(), proj.data_ptr(),
                                                           W, dim, stream), "token_side_pack")

@@ -82,7 +82,8 @@ int ed_token_side(float* x, const void* y, const float* post_w, const void* gate
  * [W / 32][dim / 16] and proj as [W / 16][dim / 32] pieces of 16 rows x 32 columns, a piece as [4][16][8]: eight columns,
  * row, columns of the eight. */
 int ed_token_side_packable(int W, int dim);
-/* Both weights into that order. */
+/* Both weights into that order; ed_token_side_pack_pays: 1 if that, in front of a call of T rows, is faster than the weights as they are. */
+int ed_token_side_pack_pays(int64_t T, int W, int dim);
 int ed_token_side_pack(const void* gate, const void* proj, void* gate_out, void* proj_out, int W, int dim, void* stream);
 int ed_token_side_packed(float* x, const void* y, const float* post_w, const void* gate, const void* proj, const int32_t* tokens,
                          const void* table, int64_t table_stride, int column0, const float* side_norm, const float* next_w, void* out,
