@@ -278,10 +278,12 @@ __global__ __launch_bounds__(256) void silu_gate_kernel(const typename Elem::sto
     RowIo<Elem, VEC>::store(out + i, v);
 }
 
-// y = y silu(z), normed in equal parts of `size` elements, times w, in place: one workgroup per (row, part).  Rows of up to 4096
-// elements request everything before the sum; longer ones take the product as it comes, or the registers hold both operands
-// (float32, 300 rows of 9001: 35.8 us that way, spilled, 13.2 now; bf16, 3505 of 8192: 36.2, 31.2).
-template <typename Elem, int VEC, int THREADS, int N>
+// y = y silu(z), normed in equal parts of `size` elements, times w, in place: one workgroup per (row, part).  EARLY: everything is
+// requested before the sum; else the product is taken as it comes and the weights wait.  Rows of more than 4096 elements would not keep
+// both operands in registers (float32, 300 rows of 9001: 35.8 us that way, spilled, 13.2 now; bf16, 3505 of 8192: 36.2, 31.2); rows
+// of 1025 to 4096 elements of 16 bits that fill the chip are better off with more rows in flight (early / in turn: 3000 of 4096 17.1 /
+// 16.2, 8192 of 2048 21.7 / 20.8), in 32 bits and shorter ones not (3000 of 3000 17.8 / 18.4, 8192 of 1000 bf16 13.3 / 13.5).
+template <typename Elem, int VEC, int THREADS, int N, bool EARLY>
 __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::storage* __restrict__ y, const typename Elem::storage* __restrict__ z,
                                                              int64_t z_stride, const float* __restrict__ w, int size, float eps) {
     __shared__ float scratch[THREADS / kWave];
@@ -289,8 +291,7 @@ __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::stor
     const int c0 = blockIdx.y * size;
     typename Elem::storage* yr = y + (row * gridDim.y + blockIdx.y) * size;
     const typename Elem::storage* zr = z + row * z_stride + c0;
-    constexpr bool kEarly = N * VEC <= 16;
-    constexpr int M = kEarly ? N : 1;
+    constexpr int M = EARLY ? N : 1;
     float v[N][VEC], g[M][VEC], wv[M][VEC], sum = 0.0f;
     auto times_silu = [&](int i) {
 #pragma unroll
@@ -305,10 +306,10 @@ __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::stor
         if (c >= size) continue;
         RowIo<Elem, VEC>::load(yr + c, v[i]);
         RowIo<Elem, VEC>::load(zr + c, g[i % M]);
-        if (kEarly) RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
+        if (EARLY) RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
         else times_silu(i);
     }
-    if (kEarly) {
+    if (EARLY) {
 #pragma unroll
         for (int i = 0; i < N; ++i)
             if ((threadIdx.x + i * THREADS) * VEC < size) times_silu(i);
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::stor
     for (int i = 0; i < N; ++i) {
         const int c = (threadIdx.x + i * THREADS) * VEC;
         if (c < size) {
-            if (!kEarly) RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
+            if (!EARLY) RowIo<F32Elem, VEC>::load(w + c0 + c, wv[i % M]);
 #pragma unroll
             for (int j = 0; j < VEC; ++j) v[i][j] *= rstd * wv[i % M][j];
             RowIo<Elem, VEC>::store(yr + c, v[i]);
@@ -384,13 +385,15 @@ template <typename Elem, int VEC>
 int launch_gated(void* y, const void* z, int64_t z_stride, const float* w, int64_t T, int parts, int size, float eps, hipStream_t s) {
     typedef typename Elem::storage S;
     const dim3 grid(static_cast<unsigned>(T), static_cast<unsigned>(parts));
-#define EM_GATED(THREADS, N) \
-    launch((gated_norm_kernel<Elem, VEC, THREADS, N>), grid, dim3(THREADS), 0, s, static_cast<S*>(y), static_cast<const S*>(z), z_stride, w, size, eps)
-    if (size <= 512) EM_GATED(64, 8 / VEC);
-    else if (VEC == 4 && T * parts <= kFewRows && size > 1024 && size <= 4096) EM_GATED(1024, 4 / VEC);
-    else if (VEC == 4 && size <= 4096) EM_GATED(256, 16 / VEC);
-    else if (size <= 256 * kRowMaxPerThread) EM_GATED(256, kRowMaxPerThread / VEC);
-    else EM_GATED(1024, kRowMaxPerThread / VEC);
+#define EM_GATED(THREADS, N, EARLY) \
+    launch((gated_norm_kernel<Elem, VEC, THREADS, N, EARLY>), grid, dim3(THREADS), 0, s, static_cast<S*>(y), static_cast<const S*>(z), z_stride, w, size, eps)
+    const bool few = T * parts <= kFewRows;
+    if (size <= 512) EM_GATED(64, 8 / VEC, true);
+    else if (VEC == 4 && few && size > 1024 && size <= 4096) EM_GATED(1024, 4 / VEC, true);
+    else if (VEC == 4 && !few && size > 1024 && size <= 4096 && sizeof(S) == 2) EM_GATED(256, 16 / VEC, false);
+    else if (VEC == 4 && size <= 4096) EM_GATED(256, 16 / VEC, true);
+    else if (size <= 256 * kRowMaxPerThread) EM_GATED(256, kRowMaxPerThread / VEC, false);
+    else EM_GATED(1024, kRowMaxPerThread / VEC, false);
 #undef EM_GATED
     return launch_status();
 }

@@ -65,3 +65,10 @@ def test_gated_norm(T, parts, size, dtype):
     v = y.double() * torch.nn.functional.silu(z[:, :parts * size].double())
     want = (rms(v.view(T, parts, size)).flatten(1) * w.double()).cpu()
     near(ops.gated_norm_(y, z.data_ptr(), z.stride(0), w, parts, EPS), want, dtype)
+
+
+# many rows: loads at once up to 1024 elements, in turn beyond in bf16
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("T,parts,size", [(257, 1, 1024), (257, 1, 1028), (86, 3, 1028), (300, 1, 3000), (257, 1, 4100)])
+def test_gated_norm_of_many_rows(T, parts, size, dtype):
+    test_gated_norm(T, parts, size, dtype)
