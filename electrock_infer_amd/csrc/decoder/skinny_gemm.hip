@@ -169,18 +169,31 @@ int launch_form(const uint16_t* x, const uint16_t* w, void* out, bool f32, int s
                : launch_one<MT, NT, WAVES, AHEAD, false, false>(x, w, out, splits, T, N, K, act, s);
 }
 
+// Ranges of K that fill the chip with `groups` workgroups each, a step of k for every wave at least.
+int ranges_of(int groups, int K) {
+    const int want = kSplitGroups / groups, most = K / (kStepK * 8), s = want < most ? want : most;
+    return s < 1 ? 1 : s > 8 ? 8 : s;
+}
+
+// 64 rows of weights to a workgroup for partial sums, instead of 32: where K is long enough for as many workgroups.
+bool wide_parts(int T, int N, int K) {
+    const int narrow = static_cast<int>(ceil_div(N, 32)), wide = static_cast<int>(ceil_div(N, 64));
+    return T > 32 && N >= 4096 && wide * ranges_of(wide, K) >= narrow * ranges_of(narrow, K);
+}
+
 // Tiles of weight rows per workgroup: as few as leave one workgroup of eight waves to a CU (us, with 64 tokens: 3072 rows of
 // 2048 in ones 8.8, in twos 10.7; 6176 in twos 11.9, ones 17.4, fours 15.3; 8512 in fours 16.9, twos 19.5; with up to 32
 // tokens two such workgroups share a CU, and the few beyond the first 256 cost less than half of the chip without work: 8512,
 // T = 1, twos 10.0, fours 11.8).  Beyond 64 rows to a CU workgroups of four waves, of which two share a CU (32000 x 2048,
 // T = 32: 25.0 / 29.3 with eight).  With three or four tiles of tokens those carry one step of k instead of two (T = 64:
 // 31.5 / 38.4), and partial sums take 64 rows as soon as four ranges of K fill the chip that way, since the token rows are
-// read by half as many workgroups (4096 x 12288, T = 64: 26.8 / 30.5; T = 32: 22.6 / 22.6).
+// read by half as many workgroups (4096 x 12288, T = 64: 26.8 / 30.5; T = 32: 22.6 / 22.6); K too short for that many ranges would leave
+// CUs without work (4096 x 1024, T = 64, with the norm that adds the ranges up 13.9 / 12.0; 4096 x 1536 15.0 / 12.9).
 template <int MT>
 int launch_tokens(const uint16_t* x, const uint16_t* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s) {
     const int rows = act == 2 ? 2 * N : N;
     if (splits > 1) {
-        if (MT > 2 && N >= 4096) return launch_form<MT, 4, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
+        if (MT > 2 && wide_parts(T, N, K)) return launch_form<MT, 4, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
         return launch_form<MT, 2, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
     }
     if (rows <= 16 * kSplitGroups && act != 2) return launch_form<MT, 1, 8, 2>(x, w, out, f32, splits, T, N, K, act, s);
@@ -232,12 +245,7 @@ bool decode_gemm_pays(int64_t T, int rows, int K, int act, bool f32) {
 }
 
 // Ranges of K for results that may stay partial sums: enough workgroups for the chip, a step of k for every wave.
-int skinny_splits(int T, int N, int K) {
-    const int groups = static_cast<int>(ceil_div(N, T > 32 && N >= 4096 ? 64 : 32));
-    const int want = static_cast<int>(kSplitGroups / groups), most = K / (kStepK * 8);
-    const int s = want < most ? want : most;
-    return s < 1 ? 1 : s > 8 ? 8 : s;
-}
+int skinny_splits(int T, int N, int K) { return ranges_of(static_cast<int>(ceil_div(N, wide_parts(T, N, K) ? 64 : 32)), K); }
 
 int launch_skinny_gemm(const void* x, const void* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s) {
     const uint16_t* xp = static_cast<const uint16_t*>(x);

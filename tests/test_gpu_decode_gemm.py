@@ -64,3 +64,9 @@ def test_rows_that_lie_apart_go_to_the_library():
     assert ops._skinny_splits(x, wide) == 0 and off(ops.linear(x, wide), want) < BF16_TOL
     shifted = torch.empty(20 * 4608 + 1, dtype=BF16, device="cuda")[1:].view(20, 4608).copy_(x)
     assert ops._skinny_splits(shifted, w) == 0 and off(ops.linear(shifted, w), want) < BF16_TOL
+
+
+# rows in 64s and in 32s to a workgroup, by how many ranges K has room for
+@pytest.mark.parametrize("T,N,K", [(33, 4096, 1024), (64, 4096, 1024), (48, 4096, 1536), (64, 4096, 1984), (64, 4096, 2048), (49, 4160, 1536), (64, 6144, 1024)])
+def test_partial_sums_of_short_rows(T, N, K):
+    test_partial_sums(T, N, K)
