@@ -9,6 +9,9 @@ import torch.nn.functional as F
 
 from .. import _lib
 
+# (looked up once: these are asked in front of every product)
+_transforms_active, _tracing_state, _BF16 = torch._C._are_functorch_transforms_active, torch._C._get_tracing_state, torch.bfloat16
+
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
@@ -26,10 +29,10 @@ def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Operands of the weight-streaming kernel: at most 64 rows.  What does not fit each other, is to be differentiated (backward or
     forward), mapped or traced, or is no dense row from a 16-byte boundary is the library's, to compute or to refuse."""
     shape, rows = x.shape, weight.shape
-    return (forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active() and torch._C._get_tracing_state() is None and
-            len(shape) == 2 and shape[0] <= 64 and len(rows) == 2 and shape[1] == rows[1] and x.dtype == weight.dtype == torch.bfloat16 and
+    return (len(shape) == 2 and shape[0] <= 64 and len(rows) == 2 and shape[1] == rows[1] and x.dtype is _BF16 and weight.dtype is _BF16 and
+            forward_ad._current_level < 0 and not _transforms_active() and _tracing_state() is None and
             x.device == weight.device and x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
-            not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)))
+            not ((x.requires_grad or weight.requires_grad) and torch.is_grad_enabled()))
 
 
 def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
