@@ -1,8 +1,7 @@
 """Build recipe for libelectrock_moe.so and libelectrock_decoder.so (gfx950 only).
 
 Two libraries, so that a model compiles what it needs: csrc/*.hip is the MoE layer, csrc/decoder/*.hip the kernels of
-decoders with a float32 stream, linear attention, recurrences, latent and softmax attention (no hand-counted copies
-there: the checks below are about the first one).
+decoders with a float32 stream, linear attention, recurrences, latent and softmax attention.
 
 The MoE library is compiled in-tree with plain hipcc; there is no CPU build of the
 kernels and no fallback: importing the ops without the built library fails.
@@ -56,6 +55,10 @@ GUARDED_KERNELS = {
 }
 
 
+# The same for libelectrock_decoder.so (at least four waves per CU, of which two share a SIMD).
+GUARDED_DECODER_KERNELS = {"tile_gemm_kernel": {"max_vgprs": 256, "min_vgprs": 40, "lds": 0}}
+
+
 def hipcc_path() -> str:
     for cand in (os.environ.get("HIPCC"), shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
         if cand and os.path.exists(cand):
@@ -98,12 +101,12 @@ def parse_kernel_resources(log: str) -> dict:
     return out
 
 
-def check_kernel_resources(resources: dict) -> list:
+def check_kernel_resources(resources: dict, guarded: dict = GUARDED_KERNELS) -> list:
     """Raise if a guarded kernel uses scratch memory, spills vector registers or leaves its register / LDS bounds;
     returns the checked (name, report) pairs."""
     checked, problems = [], []
     for name, rep in sorted(resources.items()):
-        for frag, lim in GUARDED_KERNELS.items():
+        for frag, lim in guarded.items():
             # mangled names hold the length-prefixed identifier, e.g. 16gemm_tile_kernel
             if f"{len(frag)}{frag}" not in name:
                 continue
@@ -115,14 +118,32 @@ def check_kernel_resources(resources: dict) -> list:
                                 f"[{lim['min_vgprs']}, {lim['max_vgprs']}]")
             if rep.get("lds", -1) != lim["lds"]:
                 problems.append(f"{name}: {rep.get('lds')} B of static LDS, expected {lim['lds']}")
-    found = {frag for frag in GUARDED_KERNELS if any(f"{len(frag)}{frag}" in n for n, _ in checked)}
-    for frag in GUARDED_KERNELS:
+    found = {frag for frag in guarded if any(f"{len(frag)}{frag}" in n for n, _ in checked)}
+    for frag in guarded:
         if frag not in found:
             problems.append(f"no resource report for any {frag}: the build no longer emits the remarks")
     if problems:
         raise RuntimeError("kernel resource check failed (the hand-counted copy pipelines need kernels without "
                            "compiler-made memory traffic):\n  " + "\n  ".join(problems))
     return checked
+
+
+def readable(output: str) -> str:
+    """What the compiler printed, without the resource remarks (each is three lines: the remark, the source line, a caret) and
+    without the harmless line of hipcc's host pass about the packed-fp32 feature."""
+    log, skip = [], 0
+    for l in output.splitlines():
+        if "packed-fp32-ops" in l:
+            continue
+        if "[-Rpass-analysis=kernel-resource-usage]" in l:
+            skip = 2
+            continue
+        if skip and (re.match(r"^\s*\d+ \|", l) or re.match(r"^\s*\|\s*\^", l)):
+            skip -= 1
+            continue
+        skip = 0
+        log.append(l)
+    return "\n".join(log)
 
 
 def build(verbose: bool = False) -> str:
@@ -133,20 +154,7 @@ def build(verbose: bool = False) -> str:
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc, *HIPCC_FLAGS, *sources(), "-o", tmp]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    # hipcc's host pass prints one harmless line per file about the packed-fp32 feature
-    lines = [l for l in proc.stdout.splitlines() if "packed-fp32-ops" not in l]
-    # everything but the resource remarks (each is three lines: the remark, the source line, a caret)
-    log, skip = [], 0
-    for l in lines:
-        if "[-Rpass-analysis=kernel-resource-usage]" in l:
-            skip = 2
-            continue
-        if skip and (re.match(r"^\s*\d+ \|", l) or re.match(r"^\s*\|\s*\^", l)):
-            skip -= 1
-            continue
-        skip = 0
-        log.append(l)
-    log = "\n".join(log)
+    log = readable(proc.stdout)
     if proc.returncode != 0:
         raise RuntimeError("hipcc failed:\n" + log)
     checked = check_kernel_resources(parse_kernel_resources(proc.stdout))
@@ -167,7 +175,8 @@ def build_decoder() -> str:
     """Compile csrc/decoder/*.hip, side by side, into lib/libelectrock_decoder.so; returns its path."""
     os.makedirs(LIB_DIR, exist_ok=True)
     hipcc = hipcc_path()
-    flags = [f for f in HIPCC_FLAGS if f != "-shared" and not f.startswith("-Rpass")]
+    check_compiler(hipcc)
+    flags = [f for f in HIPCC_FLAGS if f != "-shared"]
     with tempfile.TemporaryDirectory(dir=LIB_DIR) as tmp:
         def compile_one(src):
             obj = os.path.join(tmp, os.path.basename(src) + ".o")
@@ -175,9 +184,9 @@ def build_decoder() -> str:
             return obj, proc
         with ThreadPoolExecutor(max_workers=8) as pool:
             done = list(pool.map(compile_one, decoder_sources()))
-        log = "\n".join(l for _, p in done for l in p.stdout.splitlines() if "packed-fp32-ops" not in l)
         if any(p.returncode != 0 for _, p in done):
-            raise RuntimeError("hipcc failed:\n" + log)
+            raise RuntimeError("hipcc failed:\n" + "\n".join(readable(p.stdout) for _, p in done))
+        check_kernel_resources({k: v for _, p in done for k, v in parse_kernel_resources(p.stdout).items()}, GUARDED_DECODER_KERNELS)
         out = os.path.join(tmp, "lib.so")
         proc = subprocess.run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", *[o for o, _ in done], "-o", out],
                               stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -190,7 +199,7 @@ def build_decoder() -> str:
 def ensure_decoder() -> str:
     """Build the decoder library if it is missing or older than its sources."""
     deps = decoder_sources() + glob.glob(os.path.join(DECODER_CSRC_DIR, "*.h")) + \
-        [os.path.join(CSRC_DIR, "common.h")] + glob.glob(os.path.join(os.path.dirname(PKG_DIR), "include", "*.h"))
+        [os.path.join(CSRC_DIR, h) for h in ("common.h", "lds_copy.h")] + glob.glob(os.path.join(os.path.dirname(PKG_DIR), "include", "*.h"))
     if not os.path.exists(DECODER_LIB_PATH) or os.path.getmtime(DECODER_LIB_PATH) < max(map(os.path.getmtime, deps)):
         build_decoder()
     return DECODER_LIB_PATH

@@ -38,6 +38,20 @@ bool decode_gemm_pays(int64_t T, int rows, int K, int act, bool f32);
 int skinny_splits(int T, int N, int K);
 int launch_skinny_gemm(const void* x, const void* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s);
 
+// ---- tile_gemm.hip ----
+struct TileGemm {
+    const uint16_t *x, *w;       // rows x_stride and w_stride elements apart
+    void* out;
+    int64_t x_stride, w_stride;
+    bool f32;
+    int splits, T, N, K, act;
+};
+constexpr int64_t kTileGemmRows = 1 << 20;
+bool tile_gemm_supported(int64_t T, int N, int K);
+bool tile_gemm_pays(int64_t T, int N, int K, int act, bool parts);
+int tile_gemm_splits(int64_t T, int N, int K);
+int launch_tile_gemm(const TileGemm& g, hipStream_t s);
+
 // ---- token_side.hip ----
 struct TokenSideProblem {
     float* x;                // [T, W]

@@ -220,6 +220,32 @@ int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int s
     return launch_skinny_gemm(x, w, out, out_dtype == EM_DTYPE_F32, splits, static_cast<int>(T), N, K, act, as_stream(stream));
 }
 
+int ed_tile_gemm_splits(int64_t T, int N, int K) {
+    return tile_gemm_pays(T, N, K, 0, true) ? tile_gemm_splits(T, N, K) : 0;
+}
+
+int ed_tile_gemm_pays(int64_t T, int N, int K, int act) { return act >= 0 && act <= 2 && tile_gemm_pays(T, N, K, act, false) ? 1 : 0; }
+
+int ed_tile_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out, int out_dtype, int splits, int64_t T, int N,
+                 int K, int act, void* stream) {
+    if (out_dtype != EM_DTYPE_BF16 && out_dtype != EM_DTYPE_F32) return EM_ERR_BAD_DTYPE;
+    if (T == 0) return 0;
+    if (!tile_gemm_supported(T, N, K)) return EM_ERR_UNSUPPORTED;
+    if (splits < 1 || splits > 64 || splits > K / 64 || act < 0 || act > 2 || (splits > 1 && (act != 0 || out_dtype != EM_DTYPE_F32)) ||
+        (act != 0 && out_dtype != EM_DTYPE_BF16) || x_stride < K || w_stride < K)
+        return EM_ERR_BAD_SHAPE;
+    if (!x || !w || !out) return EM_ERR_NULL_POINTER;
+    if (!aligned16(x) || !aligned16(w) || !aligned16(out) || x_stride % 8 != 0 || w_stride % 8 != 0) return EM_ERR_ALIGNMENT;
+    TileGemm g{};
+    g.x = static_cast<const uint16_t*>(x);
+    g.w = static_cast<const uint16_t*>(w);
+    g.out = out;
+    g.x_stride = x_stride; g.w_stride = w_stride;
+    g.f32 = out_dtype == EM_DTYPE_F32;
+    g.splits = splits; g.T = static_cast<int>(T); g.N = N; g.K = K; g.act = act;
+    return launch_tile_gemm(g, as_stream(stream));
+}
+
 int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const void* table, int64_t table_stride,
                   int column0, void* g, int64_t T, int W, int dim, int dtype, void* stream) {
     if (!dtype_ok(dtype)) return EM_ERR_BAD_DTYPE;

@@ -1,0 +1,291 @@
+// out[T, N] = act(x[T, K] w[N, K]^T) for short prompts (from 65 rows to several hundred), bf16 on the matrix units.
+//
+// A workgroup makes BM token rows x BN weight rows, a wave 16 x 16 pieces of it.  Both operands go from memory straight to LDS,
+// 128 bytes of a row per step, in a ring of STAGES stages of which all but the one that is multiplied are in flight.
+// Bound: what a CU takes in.  Rows that lie apart arrive at about 70 bytes per ns and CU whatever the tile, the waves and the
+// depth of the ring (64 x 64: 0.23 us a step, 64 x 128 0.33, 128 x 128 0.48, 128 x 256 0.78; 1 KB pieces would reach 105),
+// so a tile is as large as still leaves every CU one, and K is split where the results may stay partial sums.  us, this / the
+// library's product (and the kernel of its activation), weights from memory: 300 tokens, 6144 x 2048 squared ReLU 16.7 / 17.7 + 4.2,
+// 2048 x 6144 parts 18.1 / 26.9, 2048 x 2048 parts 8.5 / 11.5, 4096 x 12288 parts 45.9 / 66.1, 2048 x 512 5.1 / 7.0; and a call
+// costs the host 3 us instead of 20.
+// The sum of a result runs over K from a place that depends on its tile of columns (tiles side by side ask for different
+// parts of their rows at a time).
+#include "decoder.h"
+#include "mma.h"
+#include "../lds_copy.h"
+
+namespace em {
+namespace {
+
+constexpr int kStepK = 64;               // elements of a row per stage: 128 bytes
+constexpr int kXcds = 8;
+
+template <int BM, int BN, int WAVES, int STAGES>
+struct TileGeo {
+    static constexpr int kXBytes = BM * kStepK * 2, kWBytes = BN * kStepK * 2, kStageBytes = kXBytes + kWBytes;
+    static constexpr int kLdsBytes = STAGES * kStageBytes;
+    static constexpr int kXCopies = BM / 8 / WAVES, kWCopies = BN / 8 / WAVES, kCopies = kXCopies + kWCopies;   // of a wave and stage
+    static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "a copy is eight rows");
+    static_assert((STAGES - 1) * kCopies < 64, "vmcnt counts to 63");
+};
+
+// at most `stages` stages of this wave's copies still in flight
+template <int COPIES, int MOST>
+__device__ __forceinline__ void wait_stages(int stages) {
+    switch (stages < MOST ? stages : MOST) {
+        case 0: wait_dma<0>(); break;
+        case 1: wait_dma<COPIES>(); break;
+        case 2: wait_dma<(MOST > 1 ? 2 : MOST) * COPIES>(); break;
+        case 3: wait_dma<(MOST > 2 ? 3 : MOST) * COPIES>(); break;
+        case 4: wait_dma<(MOST > 3 ? 4 : MOST) * COPIES>(); break;
+        default: wait_dma<MOST * COPIES>(); break;
+    }
+}
+
+// `x_stride`, `w_stride`: elements from row to row.  ACT: 0 none, 1 squared ReLU, 2 silu(first half) * second half of w [2 N, K]
+template <int BM, int BN, int WAVES, int WM, int STAGES, int ACT, bool F32OUT>
+__global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                                  void* __restrict__ out, int64_t x_stride, int64_t w_stride, int T, int N, int K,
+                                                                  int m_tiles, int n_tiles) {
+    typedef TileGeo<BM, BN, WAVES, STAGES> G;
+    typedef Mma<BF16Elem> M;
+    constexpr int WN = WAVES / WM, MF = BM / 16 / WM, NF = BN / 16 / WN;      // fragments of a wave
+    constexpr int kOutCols = ACT == 2 ? BN / 2 : BN;
+    static_assert(ACT != 2 || NF % 2 == 0, "fragments of both halves");
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
+    const int wm = wave % WM, wn = wave / WM;
+    // an XCD takes neighbouring tiles, those of one column first: its L2 reads a weight row once
+    const int tiles = m_tiles * n_tiles, per_xcd = (tiles + kXcds - 1) / kXcds;
+    const int local = blockIdx.x / kXcds, tile = blockIdx.x % kXcds * per_xcd + local;
+    if (local >= per_xcd || tile >= tiles) return;
+    const int nt = tile / m_tiles, m0 = (tile - nt * m_tiles) * BM, n0 = nt * kOutCols;
+    const int splits = gridDim.y, split = blockIdx.y, steps = K / kStepK;
+    const int s0 = static_cast<int>(static_cast<int64_t>(steps) * split / splits);
+    const int nk = static_cast<int>(static_cast<int64_t>(steps) * (split + 1) / splits) - s0;
+
+    // Copies of a stage: 16-byte piece c of LDS holds piece q ^ (u & 7) of the two-row group u = c / 16 (q = row & 1, piece).
+    const uint16_t* src[G::kCopies];
+#pragma unroll
+    for (int i = 0; i < G::kCopies; ++i) {
+        const bool is_x = i < G::kXCopies;
+        const int c = (is_x ? i : i - G::kXCopies) * WAVES * kWave + wave * kWave + lane;
+        const int u = c >> 4, q = (c & 15) ^ (u & 7), r = u * 2 + (q >> 3), piece = (q & 7) * 8;
+        if (is_x) {
+            src[i] = x + min(m0 + r, T - 1) * x_stride;
+        } else {
+            const int f = r / 16;        // (rows beyond the last are read twice and not stored)
+            const int64_t col = ACT == 2 ? min(n0 + f / 2 * 16 + r % 16, N - 1) + (f & 1) * static_cast<int64_t>(N) : static_cast<int64_t>(min(n0 + r, N - 1));
+            src[i] = w + col * w_stride;
+        }
+        src[i] += static_cast<int64_t>(s0) * kStepK + piece;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + wave * 1024);
+    const int rot = (nt * 5) % nk;       // tiles side by side start at different places of their rows
+    auto place = [&](int step) {         // elements into the range of K
+        const int k = step + rot;
+        return (k >= nk ? k - nk : k) * kStepK;
+    };
+    auto copy = [&](int i, int at, int slot) {
+        dma16(src[i] + at, lds0 + slot * G::kStageBytes +
+                               (i < G::kXCopies ? i * WAVES * 1024 : G::kXBytes + (i - G::kXCopies) * WAVES * 1024));
+    };
+    f32x4_t acc[NF][MF];
+#pragma unroll
+    for (int n = 0; n < NF; ++n)
+#pragma unroll
+        for (int m = 0; m < MF; ++m) acc[n][m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    int x_at[2], w_at[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int piece = (h * 4 + lq) ^ ((l16 >> 1) & 7), row = (l16 >> 1) * 256 + ((l16 & 1) * 8 + piece) * 16;
+        x_at[h] = wm * MF * 2048 + row;
+        w_at[h] = G::kXBytes + wn * NF * 2048 + row;
+    }
+    M::frag fx[2][MF], fw[2][NF];
+    auto read = [&](int slot, int h) {
+        const uint8_t* s = smem + slot * G::kStageBytes;
+#pragma unroll
+        for (int n = 0; n < NF; ++n) fw[h][n] = *reinterpret_cast<const M::frag*>(s + w_at[h] + n * 2048);
+#pragma unroll
+        for (int m = 0; m < MF; ++m) fx[h][m] = *reinterpret_cast<const M::frag*>(s + x_at[h] + m * 2048);
+    };
+    auto multiply = [&](int h) {
+#pragma unroll
+        for (int n = 0; n < NF; ++n)
+#pragma unroll
+            for (int m = 0; m < MF; ++m) acc[n][m] = M::mac(fw[h][n], fx[h][m], acc[n][m]);
+    };
+    for (int s = 0; s < STAGES && s < nk; ++s)
+#pragma unroll
+        for (int i = 0; i < G::kCopies; ++i) copy(i, place(s), s);
+    wait_stages<G::kCopies, STAGES - 1>(nk - 1);
+    block_barrier();
+    read(0, 0);
+    int slot = 0;
+    auto advance = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // this wave has read its own of the stage
+        block_barrier();
+    };
+    int k = 0;
+    for (; k + STAGES < nk; ++k) {
+        read(slot, 1);
+        multiply(0);
+        wait_dma<(STAGES - 2) * G::kCopies>();                     // the next stage has landed
+        advance();
+        // the copies into the slot that is free now, one by one between products: back to back they would hold the wave up
+        const int next = slot + 1 == STAGES ? 0 : slot + 1, at = place(k + STAGES);
+        read(next, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NF * MF; ++j) {
+            acc[j / MF][j % MF] = M::mac(fw[1][j / MF], fx[1][j % MF], acc[j / MF][j % MF]);
+            constexpr int kProducts = NF * MF;
+            if ((j + 1) * G::kCopies / kProducts > j * G::kCopies / kProducts) {
+#pragma unroll
+                for (int i = j * G::kCopies / kProducts; i < (j + 1) * G::kCopies / kProducts; ++i) copy(i, at, slot);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        slot = next;
+    }
+    for (; k + 1 < nk; ++k) {
+        read(slot, 1);
+        multiply(0);
+        wait_stages<G::kCopies, STAGES - 2>(nk - 2 - k);
+        advance();
+        slot = slot + 1 == STAGES ? 0 : slot + 1;
+        read(slot, 0);
+        multiply(1);
+    }
+    read(slot, 1);
+    multiply(0);
+    multiply(1);
+
+    // element i of a fragment: token l16, column lq * 4 + i
+#pragma unroll
+    for (int m = 0; m < MF; ++m) {
+        const int t = m0 + (wm * MF + m) * 16 + l16;
+        if (t >= T) continue;
+        const int64_t row = (static_cast<int64_t>(split) * T + t) * N;
+#pragma unroll
+        for (int n = 0; n < NF; n += ACT == 2 ? 2 : 1) {
+            const int c = n0 + (wn * NF + n) / (ACT == 2 ? 2 : 1) * 16 + lq * 4;
+            f32x4_t v = acc[n][m];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (ACT == 1) v[i] = fmaxf(v[i], 0.0f) * fmaxf(v[i], 0.0f);
+                if (ACT == 2) v[i] = silu(v[i]) * acc[n + 1][m][i];
+            }
+            if (N % 4 == 0) {
+                if (c >= N) continue;
+                if (F32OUT) {
+                    *reinterpret_cast<f32x4_t*>(static_cast<float*>(out) + row + c) = v;
+                } else {
+                    *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(out) + row + c) = u32x2_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (c + i >= N) continue;
+                    if (F32OUT) static_cast<float*>(out)[row + c + i] = v[i];
+                    else static_cast<uint16_t*>(out)[row + c + i] = f32_to_bf16_bits(v[i]);
+                }
+            }
+        }
+    }
+}
+
+template <int BM, int BN, int WAVES, int STAGES, int ACT, bool F32OUT>
+int launch_one(const TileGemm& g, hipStream_t s) {
+    typedef TileGeo<BM, BN, WAVES, STAGES> G;
+    const auto kernel = tile_gemm_kernel<BM, BN, WAVES, 2, STAGES, ACT, F32OUT>;
+    const int rc = allow_lds(reinterpret_cast<const void*>(kernel), G::kLdsBytes);
+    if (rc != 0) return rc;
+    const int m_tiles = static_cast<int>(ceil_div(g.T, BM)), n_tiles = static_cast<int>(ceil_div(g.N, ACT == 2 ? BN / 2 : BN));
+    launch(kernel, dim3(static_cast<unsigned>(round_up(static_cast<int64_t>(m_tiles) * n_tiles, kXcds)), static_cast<unsigned>(g.splits)),
+           dim3(WAVES * kWave), G::kLdsBytes, s, g.x, g.w, g.out, g.x_stride, g.w_stride, g.T, g.N, g.K, m_tiles, n_tiles);
+    return launch_status();
+}
+
+template <int BM, int BN, int WAVES, int STAGES>
+int launch_form(const TileGemm& g, hipStream_t s) {
+    if (g.act == 2) return launch_one<BM, BN, WAVES, STAGES, 2, false>(g, s);
+    if (g.act == 1) return launch_one<BM, BN, WAVES, STAGES, 1, false>(g, s);
+    return g.f32 ? launch_one<BM, BN, WAVES, STAGES, 0, true>(g, s) : launch_one<BM, BN, WAVES, STAGES, 0, false>(g, s);
+}
+
+// The forms of a workgroup and what a step of theirs takes (us): where few CUs have one, where all have, and two on every CU (0:
+// the ring leaves room for one).  Fitted, with what the rest of a launch takes, to 140 shapes of 65 to 1024 rows, 2048 to 16960
+// weight rows and K of 512 to 12288: the form that the estimate picks takes 1.02 of the best one's time on the average.
+struct Form {
+    int bm, bn;
+    double few, all, two;
+};
+constexpr Form kForms[] = {{64, 64, 0.219, 0.238, 0.41}, {128, 64, 0.318, 0.352, 0.60}, {64, 128, 0.303, 0.377, 0.0}, {128, 128, 0.452, 0.516, 0.0},
+                           {128, 256, 0.738, 0.843, 0.0}};
+constexpr double kLaunch = 3.0, kStoreRate = 3.3e6, kStreamRate = 5e6, kAddRate = 5e6;      // us; bytes per us
+
+double estimate(const Form& f, int64_t T, int64_t rows, int K, int splits, int64_t out_bytes) {
+    const int64_t groups = ceil_div(T, f.bm) * ceil_div(rows, f.bn) * splits, steps = ceil_div(K / kStepK, splits);
+    const double one = f.few + (f.all - f.few) * static_cast<double>(groups < 256 ? groups : 256) / 256.0;
+    const int64_t whole = groups / (f.two > 0 ? 512 : 256), rest = groups % (f.two > 0 ? 512 : 256);
+    double us = static_cast<double>(whole * steps) * (f.two > 0 ? f.two : one);
+    if (rest > 0) us += static_cast<double>(steps) * (rest <= 256 ? one : f.two);
+    const double stream = static_cast<double>(rows) * K * 2 / kStreamRate;
+    // (the next kernel reads all partial sums instead of one result)
+    return kLaunch + (us > stream ? us + 0.1 * stream : stream + 0.1 * us) + static_cast<double>(out_bytes) / kStoreRate +
+           (splits > 1 ? static_cast<double>(out_bytes) * (1.0 - 0.5 / splits) / kAddRate : 0.0);
+}
+
+struct Plan {
+    int form, splits;
+    double us;
+};
+Plan plan(int64_t T, int N, int K, int act, bool f32, int least, int most) {
+    Plan best{0, least, 1e30};
+    for (int splits = least; splits <= most; ++splits) {
+        if (splits > 1 && K / kStepK < 2 * splits && splits > least) break;
+        for (int i = 0; i < static_cast<int>(sizeof(kForms) / sizeof(kForms[0])); ++i) {
+            const double us = estimate(kForms[i], T, act == 2 ? 2 * static_cast<int64_t>(N) : N, K, splits, T * N * (f32 || splits > 1 ? 4 * splits : 2));
+            if (us < best.us) best = Plan{i, splits, us};
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+bool tile_gemm_supported(int64_t T, int N, int K) {
+    return T > 0 && T <= kTileGemmRows && N > 0 && N <= (1 << 28) && T * N <= (int64_t{1} << 40) && K > 0 && K % kStepK == 0;
+}
+
+// Where this is the faster way (and the host's 15 us a call come on top): up to as many rows as the library needs for tiles of
+// 256 x 256 that leave no CU without one, which depends on the weights' size.  us, this / library: 2048 x 2048, 1024 rows
+// 14.2 / 16.2; 8192 x 2048 500 rows 23.0 / 25.3, 700 31.6 / 28.5; 6144 x 4096 300 rows 28.5 / 29.7, 420 33.6 / 31.8; 12288 x 4096 200 rows
+// 37.0 / 40.1, 300 51.3 / 50.3.  An activation saves the kernel behind the library's product (12288 x 4096, 512 rows 58.1 / 51.7 + 6.5); partial sums
+// fill the chip where rows and weights are few (4096 x 8192, 512 rows 42.8 / 52.6, 700 60.4 / 54.8; 2048 x 6144, 1024 rows 36.4 / 40.8).
+bool tile_gemm_pays(int64_t T, int N, int K, int act, bool parts) {
+    if (!tile_gemm_supported(T, N, K)) return false;
+    const int64_t rows = act == 2 ? 2 * static_cast<int64_t>(N) : N, few = T < rows ? T : rows, many = T < rows ? rows : T, size = many * K;
+    if (few <= 64 || many < 1024) return false;
+    if (parts) return K >= 512 && (few <= 512 || (few <= 1024 && many <= 2048 && size <= (int64_t{1} << 24)));
+    if (K > many) return false;
+    if (act != 0) return few <= (size <= (int64_t{1} << 24) ? 1024 : size <= (int64_t{1} << 26) ? 512 : 96);
+    return few <= (size <= (int64_t{1} << 21) ? 1536 : size <= (int64_t{1} << 23) ? 1024 : size <= (int64_t{1} << 24) ? 512 :
+                   size <= (int64_t{1} << 25) ? 320 : size <= (int64_t{1} << 26) ? 224 : 96);
+}
+
+int tile_gemm_splits(int64_t T, int N, int K) { return plan(T, N, K, 0, true, 1, 8).splits; }
+
+int launch_tile_gemm(const TileGemm& g, hipStream_t s) {
+    switch (plan(g.T, g.N, g.K, g.act, g.f32, g.splits, g.splits).form) {
+        case 0: return launch_form<64, 64, 4, 4>(g, s);
+        case 1: return launch_form<128, 64, 4, 3>(g, s);
+        case 2: return launch_form<64, 128, 8, 6>(g, s);
+        case 3: return launch_form<128, 128, 8, 5>(g, s);
+        default: return launch_form<128, 256, 8, 3>(g, s);
+    }
+}
+
+}  // namespace em

@@ -25,14 +25,42 @@ def _skinny(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: in
     return out
 
 
-def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Operands of the weight-streaming kernel: at most 64 rows.  What does not fit each other, is to be differentiated (backward or
-    forward), mapped or traced, or is no dense row from a 16-byte boundary is the library's, to compute or to refuse."""
+def _plain(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Operands that the product kernels read: what does not fit each other, is to be differentiated (backward or forward), mapped
+    or traced, or lies on two devices is the library's, to compute or to refuse."""
     shape, rows = x.shape, weight.shape
-    return (len(shape) == 2 and shape[0] <= 64 and len(rows) == 2 and shape[1] == rows[1] and x.dtype is _BF16 and weight.dtype is _BF16 and
-            forward_ad._current_level < 0 and not _transforms_active() and _tracing_state() is None and
-            x.device == weight.device and x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
+    return (len(shape) == 2 and len(rows) == 2 and shape[1] == rows[1] and x.dtype is _BF16 and weight.dtype is _BF16 and
+            forward_ad._current_level < 0 and not _transforms_active() and _tracing_state() is None and x.device == weight.device and
             not ((x.requires_grad or weight.requires_grad) and torch.is_grad_enabled()))
+
+
+def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Operands of the weight-streaming kernel: at most 64 rows, dense, from a 16-byte boundary."""
+    return (len(x.shape) == 2 and x.shape[0] <= 64 and _plain(x, weight) and x.is_contiguous() and weight.is_contiguous() and
+            (x.data_ptr() | weight.data_ptr()) % 16 == 0)
+
+
+def _rows_apart(t: torch.Tensor) -> bool:
+    """Whole rows from 16-byte boundaries."""
+    return t.stride(1) == 1 and t.stride(0) >= t.shape[1] and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+
+
+def _tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Operands of the tiled kernel: any rows beyond a decode batch's, from 16-byte boundaries."""
+    return x.is_cuda and len(x.shape) == 2 and x.shape[0] > 64 and _plain(x, weight) and _rows_apart(x) and _rows_apart(weight)
+
+
+def _tile(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
+    code = _lib.load_decoder().ed_tile_gemm(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(),
+                                            _lib.dtype_code(out.dtype), splits, x.shape[0], cols, x.shape[1], act,
+                                            _lib.current_stream(x.device))
+    _lib.check_decoder(code, "tile_gemm")
+    return out
+
+
+def _tiles(x: torch.Tensor, weight: torch.Tensor, cols: int, act: int = 0) -> bool:
+    """Whether the tiled kernel takes the product and is the faster way."""
+    return _tiles_fit(x, weight) and _lib.load_decoder().ed_tile_gemm_pays(x.shape[0], cols, weight.shape[1], act) == 1
 
 
 def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
@@ -46,16 +74,18 @@ def _streams(x: torch.Tensor, weight: torch.Tensor, out_rows: int, act: int = 0,
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
-    """act(x @ weight^T) in x's type: a weight-streaming kernel for a decode batch, a library product otherwise;
-    ``act``: None or 'relu_squared'."""
+    """act(x @ weight^T) in x's type: a weight-streaming kernel for a decode batch, a tiled one for a short prompt, a library product
+    otherwise; ``act``: None or 'relu_squared'."""
     if _streams(x, weight, weight.shape[0], int(act is not None)):
         return _skinny(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device), 1, int(act is not None))
+    if _tiles(x, weight, weight.shape[0], int(act is not None)):
+        return _tile(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device), 1, weight.shape[0], int(act is not None))
     out = F.linear(x, weight)
     return relu_squared_(out) if act is not None else out
 
 
 def linear_silu_gate(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """silu(x @ gate^T) * (x @ up^T) for ``weight`` = [gate; up]: one launch for a decode batch."""
+    """silu(x @ gate^T) * (x @ up^T) for ``weight`` = [gate; up]: one launch for a decode batch or a short prompt."""
     (T, _), ff = x.shape, weight.shape[0] // 2
     out = torch.empty(T, ff, dtype=x.dtype, device=x.device)
     if _streams(x, weight, ff, 2):
@@ -63,6 +93,8 @@ def linear_silu_gate(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
                                                   x.shape[1], 2, _lib.current_stream(x.device))
         _lib.check_decoder(code, "decode_gemm")
         return out
+    if _tiles(x, weight, ff, 2) and weight.shape[0] == 2 * ff:
+        return _tile(x, weight, out, 1, ff, 2)
     u = F.linear(x, weight)
     _lib.check_decoder(_lib.load_decoder().ed_silu_gate(u.data_ptr(), out.data_ptr(), T, ff, _lib.dtype_code(x.dtype),
                                                         _lib.current_stream(x.device)), "silu_gate")
@@ -75,15 +107,24 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         return F.linear(x, weight)
     if _streams(x, weight, weight.shape[0], 0, _lib.DTYPE_F32):
         return _skinny(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), 1, 0)
+    if _tiles(x, weight, weight.shape[0]):
+        return _tile(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), 1, weight.shape[0], 0)
     return torch.mm(x, weight.t(), out_dtype=torch.float32)
 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor, exact: bool = False) -> torch.Tensor:
-    """x @ weight^T as ``residual_norm`` takes it: [T, N], or float32 partial sums [parts, T, N] of a decode batch.
+    """x @ weight^T as ``residual_norm`` takes it: [T, N], or float32 partial sums [parts, T, N] of a decode batch or a short prompt.
     ``exact``: not rounded to the compute type on the way."""
     splits = _skinny_splits(x, weight) if x.is_cuda else 0
     if splits > 1:
         return _skinny(x, weight, torch.empty(splits, x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), splits, 0)
+    if _tiles_fit(x, weight):
+        (T, K), N = x.shape, weight.shape[0]
+        splits = _lib.load_decoder().ed_tile_gemm_splits(T, N, K)
+        if splits > 1:
+            return _tile(x, weight, torch.empty(splits, T, N, dtype=torch.float32, device=x.device), splits, N, 0)
+        if splits == 1:
+            return _tile(x, weight, torch.empty(T, N, dtype=torch.float32 if exact else x.dtype, device=x.device), 1, N, 0)
     return linear_f32(x, weight) if exact else linear(x, weight)
 
 

@@ -1,11 +1,10 @@
 """Latent attention (csrc/decoder/latent_attention.hip): keys and values of all heads are projections of one cached
 latent per token; a rotated key part is shared by the heads; the softmax has a learned sink per head."""
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .. import _lib
-from .decoder_ops import StackedLinear, byref, head_gemm, linear_parts, pad_k
+from .decoder_ops import StackedLinear, byref, head_gemm, linear, linear_parts, pad_k
 
 
 def rotary_frequencies(dims: int, base: float, factor: float = 1.0) -> torch.Tensor:
@@ -103,8 +102,7 @@ class LatentAttention(nn.Module):
                                                 -(-batch.max_context // 64) * 64, row, rows.data_ptr(),
                                                 _lib.dtype_code(o.dtype), stream), "latent_gather")
         latents = rows[:, :self.rank]
-        k = F.linear(latents, self.uk)
-        vt = torch.mm(self.uv, latents.t())
+        k, vt = linear(latents, self.uk), linear(self.uv, latents)
         a = _lib.LatentPromptArgs(q=self.in_proj.section_ptr(p, "q"), q_stride=p.stride(0), k=k.data_ptr(), k_stride=k.stride(0),
                                   k_rot=rows.data_ptr() + self.pitch * rows.element_size(), k_rot_stride=row, vt=vt.data_ptr(),
                                   v_stride=vt.stride(0), out=o.data_ptr(), sink=self.sink.data_ptr(),

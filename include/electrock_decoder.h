@@ -64,6 +64,14 @@ int ed_decode_gemm_plain_pays(int64_t T, int N, int K);
 int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int splits, int64_t T, int N, int K, int act,
                    void* stream);
 
+/* The same product and activations for any number of rows, x_stride and w_stride elements apart (multiples of 8; x, w, out from a
+ * 16-byte boundary); float32 results without an activation.  ed_tile_gemm_pays: 1 if that is faster than the library's product and
+ * the kernel of its activation; ed_tile_gemm_splits: ranges of K where the results may stay partial sums, 0 if the library is faster. */
+int ed_tile_gemm_splits(int64_t T, int N, int K);
+int ed_tile_gemm_pays(int64_t T, int N, int K, int act);
+int ed_tile_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out, int out_dtype, int splits, int64_t T, int N,
+                 int K, int act, void* stream);
+
 /* g [T, dim] = gelu_tanh(x gate^T) * table[tokens[t]][column0 + c]; x [T, W], gate [dim, W]. */
 int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const void* table, int64_t table_stride,
                   int column0, void* g, int64_t T, int W, int dim, int dtype, void* stream);

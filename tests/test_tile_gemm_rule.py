@@ -1,0 +1,45 @@
+"""Which products the tiled kernel of short prompts takes, and what its entry point refuses (nothing runs on a GPU here)."""
+import itertools
+
+import pytest
+import torch
+
+from electrock_infer_amd import _lib
+from electrock_infer_amd.layers import decoder_ops as ops
+
+F32, BF16 = _lib.DTYPE_F32, _lib.DTYPE_BF16
+
+
+def test_the_rule():
+    lib = _lib.load_decoder()
+    # decode batches have a kernel of their own, long prompts are the library's
+    for T, N, K in itertools.product((0, 1, 64, 8192), (2048, 4096, 12288), (1024, 2048, 4096)):
+        assert lib.ed_tile_gemm_splits(T, N, K) == 0, (T, N, K)
+        assert not any(lib.ed_tile_gemm_pays(T, N, K, act) for act in (0, 1, 2)), (T, N, K)
+    assert lib.ed_tile_gemm_pays(300, 6144, 2048, 1) == lib.ed_tile_gemm_pays(1024, 4096, 2048, 2) == lib.ed_tile_gemm_pays(1344, 2048, 512, 0) == 1
+    assert lib.ed_tile_gemm_pays(2048, 1344, 512, 0) == 1                      # (the sides' roles do not matter)
+    assert lib.ed_tile_gemm_pays(300, 6144, 2048, 3) == lib.ed_tile_gemm_pays(300, 6144, 2050, 0) == lib.ed_tile_gemm_pays(300, 512, 512, 0) == 0
+    # ranges of K never shorter than two steps, and a decode batch's widest shapes stay whole
+    for T, N, K in itertools.product((65, 200, 512), (1024, 2048, 4096, 12288), (512, 576, 2048, 12288)):
+        splits = lib.ed_tile_gemm_splits(T, N, K)
+        assert 1 <= splits <= 8 and splits * 2 <= K // 64, (T, N, K)
+
+
+@pytest.mark.parametrize("change,code", [({"T": -1}, -4), ({"K": 100}, -4), ({"N": 0}, -4), ({"splits": 0}, -2), ({"splits": 3, "K": 128}, -2),
+                                         ({"splits": 2}, -2), ({"act": 3}, -2), ({"act": 1, "dtype": F32}, -2), ({"x_stride": 64}, -2),
+                                         ({"w_stride": 64}, -2), ({"dtype": 7}, -3), ({"x": None}, -1), ({"w": 24}, -7), ({"out": 8}, -7),
+                                         ({"x_stride": 132}, -7), ({"T": 1 << 21}, -4), ({"T": 1 << 20, "N": 1 << 21}, -4)])
+def test_refused(change, code):
+    a = {"x": 16, "x_stride": 128, "w": 16, "w_stride": 128, "out": 16, "dtype": BF16, "splits": 1, "T": 100, "N": 64, "K": 128, "act": 0, **change}
+    assert _lib.load_decoder().ed_tile_gemm(a["x"], a["x_stride"], a["w"], a["w_stride"], a["out"], a["dtype"], a["splits"], a["T"], a["N"], a["K"],
+                                            a["act"], None) == code
+
+
+def test_no_rows_are_no_work():
+    assert _lib.load_decoder().ed_tile_gemm(None, 64, None, 64, None, BF16, 1, 0, 64, 64, 0, None) == 0
+
+
+def test_host_tensors_and_gradients_are_the_librarys():
+    x, w = torch.randn(100, 512).to(torch.bfloat16), torch.randn(1024, 512).to(torch.bfloat16)
+    assert not ops._tiles_fit(x, w) and torch.equal(ops.linear(x, w), torch.nn.functional.linear(x, w))
+    assert ops._plain(x, w) and not ops._plain(x.requires_grad_(), w)
