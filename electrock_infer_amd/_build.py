@@ -55,8 +55,8 @@ GUARDED_KERNELS = {
 }
 
 
-# The same for libelectrock_decoder.so (at least four waves per CU, of which two share a SIMD).
-GUARDED_DECODER_KERNELS = {"tile_gemm_kernel": {"max_vgprs": 256, "min_vgprs": 40, "lds": 0}}
+# The same for libelectrock_decoder.so (two waves share a SIMD).
+GUARDED_DECODER_KERNELS = {"tile_gemm_kernel": {"max_vgprs": 256, "min_vgprs": 24, "lds": 0}}
 
 
 def hipcc_path() -> str:

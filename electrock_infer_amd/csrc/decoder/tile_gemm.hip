@@ -1,13 +1,22 @@
-// out[T, N] = act(x[T, K] w[N, K]^T) for short prompts (from 65 rows to several hundred), bf16 on the matrix units.
+// out[T, N] = act(x[T, K] w[N, K]^T) for decode batches and short prompts (up to several hundred rows), bf16 on the matrix units.
 //
 // A workgroup makes BM token rows x BN weight rows, a wave 16 x 16 pieces of it.  Both operands go from memory straight to LDS,
 // 128 bytes of a row per step, in a ring of STAGES stages of which all but the one that is multiplied are in flight.
-// Bound: what a CU takes in.  Rows that lie apart arrive at about 70 bytes per ns and CU whatever the tile, the waves and the
-// depth of the ring (64 x 64: 0.23 us a step, 64 x 128 0.33, 128 x 128 0.48, 128 x 256 0.78; 1 KB pieces would reach 105),
+//
+// Short prompts.  Bound: what a CU takes in.  Rows that lie apart arrive at about 70 bytes per ns and CU whatever the tile, the waves
+// and the depth of the ring (64 x 64: 0.23 us a step, 64 x 128 0.33, 128 x 128 0.48, 128 x 256 0.78; 1 KB pieces would reach 105),
 // so a tile is as large as still leaves every CU one, and K is split where the results may stay partial sums.  us, this / the
 // library's product (and the kernel of its activation), weights from memory: 300 tokens, 6144 x 2048 squared ReLU 16.7 / 17.7 + 4.2,
 // 2048 x 6144 parts 18.1 / 26.9, 2048 x 2048 parts 8.5 / 11.5, 4096 x 12288 parts 45.9 / 66.1, 2048 x 512 5.1 / 7.0; and a call
 // costs the host 3 us instead of 20.
+//
+// Decode batches.  Bound: the weights' stream.  One tile of tokens, weights past the caches' order of use (non-temporal), and the
+// ring keeps 40-80 KB per workgroup in flight without a register, while the kernel of skinny_gemm.hip asks for a step's rows, waits and
+// multiplies.  us, this / that one, weights from memory: 12288 x 4096, 23 tokens 20.1 / 25.5, one 18.9 / 22.8; 4096 x 12288 parts, 64 tokens
+// 21.0 / 26.3, one 17.4 / 20.2; 2048 x 6144 parts, 64 tokens 9.4 / 12.7; gated 2 x 4096 x 2048, 64 tokens 10.9 / 14.5; 32000 x 4096
+// float32, 64 tokens 43.0 / 53.0 (6.1 TB/s).  That one shares K out over a workgroup's waves and stays ahead where the rows are few and the
+// results whole (3072 x 2048, one token 7.7 / 5.7).
+//
 // The sum of a result runs over K from a place that depends on its tile of columns (tiles side by side ask for different
 // parts of their rows at a time).
 #include "decoder.h"
@@ -24,26 +33,23 @@ template <int BM, int BN, int WAVES, int STAGES>
 struct TileGeo {
     static constexpr int kXBytes = BM * kStepK * 2, kWBytes = BN * kStepK * 2, kStageBytes = kXBytes + kWBytes;
     static constexpr int kLdsBytes = STAGES * kStageBytes;
-    static constexpr int kXCopies = BM / 8 / WAVES, kWCopies = BN / 8 / WAVES, kCopies = kXCopies + kWCopies;   // of a wave and stage
-    static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "a copy is eight rows");
+    // of a wave and stage; a copy is eight rows (where the tokens' do not go round, some are copied twice: every wave counts the same)
+    static constexpr int kXPieces = BM / 8, kXCopies = (kXPieces + WAVES - 1) / WAVES, kWCopies = BN / 8 / WAVES, kCopies = kXCopies + kWCopies;
+    static_assert(BM % 16 == 0 && BN % (8 * WAVES) == 0, "a copy is eight rows");
     static_assert((STAGES - 1) * kCopies < 64, "vmcnt counts to 63");
 };
 
-// at most `stages` stages of this wave's copies still in flight
+// at most min(stages, MOST) stages of this wave's copies still in flight
 template <int COPIES, int MOST>
 __device__ __forceinline__ void wait_stages(int stages) {
-    switch (stages < MOST ? stages : MOST) {
-        case 0: wait_dma<0>(); break;
-        case 1: wait_dma<COPIES>(); break;
-        case 2: wait_dma<(MOST > 1 ? 2 : MOST) * COPIES>(); break;
-        case 3: wait_dma<(MOST > 2 ? 3 : MOST) * COPIES>(); break;
-        case 4: wait_dma<(MOST > 3 ? 4 : MOST) * COPIES>(); break;
-        default: wait_dma<MOST * COPIES>(); break;
-    }
+    if constexpr (MOST == 0) wait_dma<0>();
+    else if (stages >= MOST) wait_dma<MOST * COPIES>();
+    else wait_stages<COPIES, MOST - 1>(stages);
 }
 
-// `x_stride`, `w_stride`: elements from row to row.  ACT: 0 none, 1 squared ReLU, 2 silu(first half) * second half of w [2 N, K]
-template <int BM, int BN, int WAVES, int WM, int STAGES, int ACT, bool F32OUT>
+// `x_stride`, `w_stride`: elements from row to row.  ACT: 0 none, 1 squared ReLU, 2 silu(first half) * second half of w
+// [2 N, K].  ONCE: one tile of tokens, so that the weights are read once.
+template <int BM, int BN, int WAVES, int WM, int STAGES, int ACT, bool F32OUT, bool ONCE>
 __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
                                                                   void* __restrict__ out, int64_t x_stride, int64_t w_stride, int T, int N, int K,
                                                                   int m_tiles, int n_tiles) {
@@ -51,7 +57,8 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
     typedef Mma<BF16Elem> M;
     constexpr int WN = WAVES / WM, MF = BM / 16 / WM, NF = BN / 16 / WN;      // fragments of a wave
     constexpr int kOutCols = ACT == 2 ? BN / 2 : BN;
-    static_assert(ACT != 2 || NF % 2 == 0, "fragments of both halves");
+    constexpr bool kMixed = ACT == 2 && NF % 2 != 0;             // a fragment holds eight columns of both halves, else two take turns
+    constexpr int kPair = ACT == 2 && !kMixed ? 2 : 1;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
     const int wm = wave % WM, wn = wave / WM;
@@ -69,26 +76,30 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
 #pragma unroll
     for (int i = 0; i < G::kCopies; ++i) {
         const bool is_x = i < G::kXCopies;
-        const int c = (is_x ? i : i - G::kXCopies) * WAVES * kWave + wave * kWave + lane;
+        const int c = (is_x ? (i * WAVES + wave) % G::kXPieces : (i - G::kXCopies) * WAVES + wave) * kWave + lane;
         const int u = c >> 4, q = (c & 15) ^ (u & 7), r = u * 2 + (q >> 3), piece = (q & 7) * 8;
         if (is_x) {
             src[i] = x + min(m0 + r, T - 1) * x_stride;
         } else {
-            const int f = r / 16;        // (rows beyond the last are read twice and not stored)
-            const int64_t col = ACT == 2 ? min(n0 + f / 2 * 16 + r % 16, N - 1) + (f & 1) * static_cast<int64_t>(N) : static_cast<int64_t>(min(n0 + r, N - 1));
+            const int f = r / 16, e = r % 16;        // (rows beyond the last are read twice and not stored)
+            const int64_t col = kMixed      ? min(n0 + f * 8 + e % 8, N - 1) + (e / 8) * static_cast<int64_t>(N)
+                                : ACT == 2 ? min(n0 + f / 2 * 16 + e, N - 1) + (f & 1) * static_cast<int64_t>(N)
+                                           : static_cast<int64_t>(min(n0 + r, N - 1));
             src[i] = w + col * w_stride;
         }
         src[i] += static_cast<int64_t>(s0) * kStepK + piece;
     }
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + wave * 1024);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
     const int rot = (nt * 5) % nk;       // tiles side by side start at different places of their rows
     auto place = [&](int step) {         // elements into the range of K
         const int k = step + rot;
         return (k >= nk ? k - nk : k) * kStepK;
     };
     auto copy = [&](int i, int at, int slot) {
-        dma16(src[i] + at, lds0 + slot * G::kStageBytes +
-                               (i < G::kXCopies ? i * WAVES * 1024 : G::kXBytes + (i - G::kXCopies) * WAVES * 1024));
+        const uint32_t to = lds0 + slot * G::kStageBytes + (i < G::kXCopies ? (i * WAVES + wave) % G::kXPieces * 1024
+                                                                             : G::kXBytes + ((i - G::kXCopies) * WAVES + wave) * 1024);
+        if (ONCE && i >= G::kXCopies) dma16_stream(src[i] + at, to);
+        else dma16(src[i] + at, to);
     };
     f32x4_t acc[NF][MF];
 #pragma unroll
@@ -166,17 +177,17 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
         const int t = m0 + (wm * MF + m) * 16 + l16;
-        if (t >= T) continue;
         const int64_t row = (static_cast<int64_t>(split) * T + t) * N;
 #pragma unroll
-        for (int n = 0; n < NF; n += ACT == 2 ? 2 : 1) {
-            const int c = n0 + (wn * NF + n) / (ACT == 2 ? 2 : 1) * 16 + lq * 4;
+        for (int n = 0; n < NF; n += kPair) {
+            const int c = kMixed ? n0 + (wn * NF + n) * 8 + (lq & 1) * 4 : n0 + (wn * NF + n) / kPair * 16 + lq * 4;
             f32x4_t v = acc[n][m];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (ACT == 1) v[i] = fmaxf(v[i], 0.0f) * fmaxf(v[i], 0.0f);
-                if (ACT == 2) v[i] = silu(v[i]) * acc[n + 1][m][i];
+                if (ACT == 2) v[i] = silu(v[i]) * (kMixed ? __shfl_xor(v[i], 32) : acc[n + kPair - 1][m][i]);
             }
+            if (t >= T || (kMixed && lq >= 2)) continue;
             if (N % 4 == 0) {
                 if (c >= N) continue;
                 if (F32OUT) {
@@ -196,10 +207,11 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
     }
 }
 
-template <int BM, int BN, int WAVES, int STAGES, int ACT, bool F32OUT>
+template <int BM, int BN, int WAVES, int WM, int STAGES, int ACT, bool F32OUT>
 int launch_one(const TileGemm& g, hipStream_t s) {
     typedef TileGeo<BM, BN, WAVES, STAGES> G;
-    const auto kernel = tile_gemm_kernel<BM, BN, WAVES, 2, STAGES, ACT, F32OUT>;
+    constexpr bool kOnce = BM < 64 || WAVES == 3 || BN == 32 || (BM == 64 && WM == 1);       // the forms of decode batches
+    const auto kernel = tile_gemm_kernel<BM, BN, WAVES, WM, STAGES, ACT, F32OUT, kOnce>;
     const int rc = allow_lds(reinterpret_cast<const void*>(kernel), G::kLdsBytes);
     if (rc != 0) return rc;
     const int m_tiles = static_cast<int>(ceil_div(g.T, BM)), n_tiles = static_cast<int>(ceil_div(g.N, ACT == 2 ? BN / 2 : BN));
@@ -208,34 +220,38 @@ int launch_one(const TileGemm& g, hipStream_t s) {
     return launch_status();
 }
 
-template <int BM, int BN, int WAVES, int STAGES>
+template <int BM, int BN, int WAVES, int WM, int STAGES>
 int launch_form(const TileGemm& g, hipStream_t s) {
-    if (g.act == 2) return launch_one<BM, BN, WAVES, STAGES, 2, false>(g, s);
-    if (g.act == 1) return launch_one<BM, BN, WAVES, STAGES, 1, false>(g, s);
-    return g.f32 ? launch_one<BM, BN, WAVES, STAGES, 0, true>(g, s) : launch_one<BM, BN, WAVES, STAGES, 0, false>(g, s);
+    if (g.act == 2) return launch_one<BM, BN, WAVES, WM, STAGES, 2, false>(g, s);
+    if (g.act == 1) return launch_one<BM, BN, WAVES, WM, STAGES, 1, false>(g, s);
+    return g.f32 ? launch_one<BM, BN, WAVES, WM, STAGES, 0, true>(g, s) : launch_one<BM, BN, WAVES, WM, STAGES, 0, false>(g, s);
 }
 
 // The forms of a workgroup and what a step of theirs takes (us): where few CUs have one, where all have, and two on every CU (0:
 // the ring leaves room for one).  Fitted, with what the rest of a launch takes, to 140 shapes of 65 to 1024 rows, 2048 to 16960
-// weight rows and K of 512 to 12288: the form that the estimate picks takes 1.02 of the best one's time on the average.
+// weight rows and K of 512 to 12288: the form that the estimate picks takes 1.02 of the best one's time on the average; and of decode
+// batches to 20 shapes of 1024 to 32000 rows with 1 to 64 tokens (1.01).
 struct Form {
     int bm, bn;
     double few, all, two;
 };
-constexpr Form kForms[] = {{64, 64, 0.219, 0.238, 0.41}, {128, 64, 0.318, 0.352, 0.60}, {64, 128, 0.303, 0.377, 0.0}, {128, 128, 0.452, 0.516, 0.0},
-                           {128, 256, 0.738, 0.843, 0.0}};
-constexpr double kLaunch = 3.0, kStoreRate = 3.3e6, kStreamRate = 5e6, kAddRate = 5e6;      // us; bytes per us
+constexpr Form kPromptForms[] = {{64, 64, 0.219, 0.238, 0.41}, {128, 64, 0.318, 0.352, 0.60}, {64, 128, 0.303, 0.377, 0.0}, {128, 128, 0.452, 0.516, 0.0},
+                                 {128, 256, 0.738, 0.843, 0.0}};
+constexpr Form kDecodeForms[3][4] = {{{16, 32, 0.143, 0.143, 0.178}, {16, 48, 0.157, 0.157, 0.290}, {16, 64, 0.183, 0.183, 0.288}, {16, 128, 0.317, 0.317, 0.567}},
+                                     {{32, 32, 0.156, 0.156, 0.253}, {32, 48, 0.184, 0.193, 0.364}, {32, 64, 0.204, 0.204, 0.363}, {32, 128, 0.340, 0.378, 0.630}},
+                                     {{64, 32, 0.208, 0.208, 0.384}, {64, 48, 0.239, 0.240, 0.466}, {64, 64, 0.271, 0.271, 0.493}, {64, 128, 0.430, 0.471, 0.0}}};
+// us; bytes per us: stores, weights from memory, further partial sums that the next kernel reads (the whole chip, or one CU a row)
+constexpr double kLaunch = 3.0, kStoreRate = 3.3e6, kPromptStream = 5e6, kDecodeStream = 6e6, kAddRate = 5e6, kAddRow = 5.7e4;
 
-double estimate(const Form& f, int64_t T, int64_t rows, int K, int splits, int64_t out_bytes) {
+double estimate(const Form& f, bool decode, int64_t T, int N, int64_t rows, int K, int splits, int out_bytes) {
     const int64_t groups = ceil_div(T, f.bm) * ceil_div(rows, f.bn) * splits, steps = ceil_div(K / kStepK, splits);
     const double one = f.few + (f.all - f.few) * static_cast<double>(groups < 256 ? groups : 256) / 256.0;
     const int64_t whole = groups / (f.two > 0 ? 512 : 256), rest = groups % (f.two > 0 ? 512 : 256);
     double us = static_cast<double>(whole * steps) * (f.two > 0 ? f.two : one);
     if (rest > 0) us += static_cast<double>(steps) * (rest <= 256 ? one : f.two);
-    const double stream = static_cast<double>(rows) * K * 2 / kStreamRate;
-    // (the next kernel reads all partial sums instead of one result)
-    return kLaunch + (us > stream ? us + 0.1 * stream : stream + 0.1 * us) + static_cast<double>(out_bytes) / kStoreRate +
-           (splits > 1 ? static_cast<double>(out_bytes) * (1.0 - 0.5 / splits) / kAddRate : 0.0);
+    const double stream = static_cast<double>(rows) * K * 2 / (decode ? kDecodeStream : kPromptStream), stored = static_cast<double>(T) * N * out_bytes * splits;
+    const double add = splits == 1 ? 0.0 : decode ? splits * (N * 4.0 / kAddRow + 0.1) : stored * (1.0 - 0.5 / splits) / kAddRate;
+    return kLaunch + (us > stream ? us : stream) + (decode ? 0.35 : 0.1) * (us > stream ? stream : us) + stored / kStoreRate + add;
 }
 
 struct Plan {
@@ -244,10 +260,12 @@ struct Plan {
 };
 Plan plan(int64_t T, int N, int K, int act, bool f32, int least, int most) {
     Plan best{0, least, 1e30};
+    const bool decode = T <= 64;
+    const Form* forms = decode ? kDecodeForms[T <= 16 ? 0 : T <= 32 ? 1 : 2] : kPromptForms;
     for (int splits = least; splits <= most; ++splits) {
-        if (splits > 1 && K / kStepK < 2 * splits && splits > least) break;
-        for (int i = 0; i < static_cast<int>(sizeof(kForms) / sizeof(kForms[0])); ++i) {
-            const double us = estimate(kForms[i], T, act == 2 ? 2 * static_cast<int64_t>(N) : N, K, splits, T * N * (f32 || splits > 1 ? 4 * splits : 2));
+        if (splits > least && K / kStepK < 2 * splits) break;
+        for (int i = 0; i < (decode ? 4 : 5); ++i) {
+            const double us = estimate(forms[i], decode, T, N, act == 2 ? 2 * static_cast<int64_t>(N) : N, K, splits, f32 ? 4 : 2);
             if (us < best.us) best = Plan{i, splits, us};
         }
     }
@@ -260,6 +278,20 @@ bool tile_gemm_supported(int64_t T, int N, int K) {
     return T > 0 && T <= kTileGemmRows && N > 0 && N <= (1 << 28) && T * N <= (int64_t{1} << 40) && K > 0 && K % kStepK == 0;
 }
 
+namespace {
+// Where a decode batch is faster this way than by the weight-streaming kernel, which shares K out over a workgroup's waves and so
+// makes twice as many, smaller pieces, and than by the library (11 sizes of 1024 to 32000 rows, K of 512 to 12288, T of 1 to 64; this /
+// the better of the two: 0.74 to 0.90 of its time beyond 8192 rows, 0.90 for partial sums with the norm behind them):
+//   * results stay partial sums, unless K leaves no steps to share out (4096 x 512, one token 7.3 / 6.7 us, 64 tokens 8.2 / 8.5);
+//   * or the rows are a CU's worth of tiles: 6144 (6144 x 4096, T = 17 13.6 / 14.6, one 12.6 / 12.9; 4096 x 4096, T = 17 11.9 / 9.8), which a
+//     short K (8192 x 1024, T = 16 9.1 / 8.6) or a gate (its fragments mix both halves: 8192 x 4096, one token 14.9 / 14.3, T = 32 15.7 / 16.4) moves up.
+bool decode_pays(int64_t T, int64_t rows, int K, int act, bool parts) {
+    if (parts) return K >= 1024;
+    if (act == 2) return (rows >= 10240 && K >= 1024) || (rows >= 8192 && T > 8 && K > 1024) || (rows >= 6144 && T > 32);
+    return rows > 8192 || (rows >= 6144 && (T > 32 || (K > 1024 && (T > 4 || rows >= 8192))));
+}
+}  // namespace
+
 // Where this is the faster way (and the host's 15 us a call come on top): up to as many rows as the library needs for tiles of
 // 256 x 256 that leave no CU without one, which depends on the weights' size.  us, this / library: 2048 x 2048, 1024 rows
 // 14.2 / 16.2; 8192 x 2048 500 rows 23.0 / 25.3, 700 31.6 / 28.5; 6144 x 4096 300 rows 28.5 / 29.7, 420 33.6 / 31.8; 12288 x 4096 200 rows
@@ -267,7 +299,9 @@ bool tile_gemm_supported(int64_t T, int N, int K) {
 // fill the chip where rows and weights are few (4096 x 8192, 512 rows 42.8 / 52.6, 700 60.4 / 54.8; 2048 x 6144, 1024 rows 36.4 / 40.8).
 bool tile_gemm_pays(int64_t T, int N, int K, int act, bool parts) {
     if (!tile_gemm_supported(T, N, K)) return false;
-    const int64_t rows = act == 2 ? 2 * static_cast<int64_t>(N) : N, few = T < rows ? T : rows, many = T < rows ? rows : T, size = many * K;
+    const int64_t rows = act == 2 ? 2 * static_cast<int64_t>(N) : N;
+    if (T <= 64) return decode_pays(T, rows, K, act, parts);
+    const int64_t few = T < rows ? T : rows, many = T < rows ? rows : T, size = many * K;
     if (few <= 64 || many < 1024) return false;
     if (parts) return K >= 512 && (few <= 512 || (few <= 1024 && many <= 2048 && size <= (int64_t{1} << 24)));
     if (K > many) return false;
@@ -279,12 +313,37 @@ bool tile_gemm_pays(int64_t T, int N, int K, int act, bool parts) {
 int tile_gemm_splits(int64_t T, int N, int K) { return plan(T, N, K, 0, true, 1, 8).splits; }
 
 int launch_tile_gemm(const TileGemm& g, hipStream_t s) {
-    switch (plan(g.T, g.N, g.K, g.act, g.f32, g.splits, g.splits).form) {
-        case 0: return launch_form<64, 64, 4, 4>(g, s);
-        case 1: return launch_form<128, 64, 4, 3>(g, s);
-        case 2: return launch_form<64, 128, 8, 6>(g, s);
-        case 3: return launch_form<128, 128, 8, 5>(g, s);
-        default: return launch_form<128, 256, 8, 3>(g, s);
+    const int form = plan(g.T, g.N, g.K, g.act, g.f32, g.splits, g.splits).form;
+    if (g.T <= 16) {
+        switch (form) {
+            case 0: return launch_form<16, 32, 2, 1, 10>(g, s);
+            case 1: return launch_form<16, 48, 3, 1, 10>(g, s);
+            case 2: return launch_form<16, 64, 4, 1, 8>(g, s);
+            default: return launch_form<16, 128, 4, 1, 4>(g, s);
+        }
+    }
+    if (g.T <= 32) {
+        switch (form) {
+            case 0: return launch_form<32, 32, 4, 2, 10>(g, s);
+            case 1: return launch_form<32, 48, 3, 1, 8>(g, s);
+            case 2: return launch_form<32, 64, 4, 1, 6>(g, s);
+            default: return launch_form<32, 128, 4, 1, 4>(g, s);
+        }
+    }
+    if (g.T <= 64) {
+        switch (form) {
+            case 0: return launch_form<64, 32, 4, 2, 6>(g, s);
+            case 1: return launch_form<64, 48, 3, 1, 5>(g, s);
+            case 2: return launch_form<64, 64, 4, 1, 5>(g, s);
+            default: return launch_form<64, 128, 4, 1, 6>(g, s);
+        }
+    }
+    switch (form) {
+        case 0: return launch_form<64, 64, 4, 2, 4>(g, s);
+        case 1: return launch_form<128, 64, 4, 2, 3>(g, s);
+        case 2: return launch_form<64, 128, 8, 2, 6>(g, s);
+        case 3: return launch_form<128, 128, 8, 2, 5>(g, s);
+        default: return launch_form<128, 256, 8, 2, 3>(g, s);
     }
 }
 

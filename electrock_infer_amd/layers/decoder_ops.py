@@ -17,14 +17,6 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-def _skinny(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, act: int) -> torch.Tensor:
-    (T, K), N = x.shape, weight.shape[0]
-    code = _lib.load_decoder().ed_decode_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), splits,
-                                              T, N, K, act, _lib.current_stream(x.device))
-    _lib.check_decoder(code, "decode_gemm")
-    return out
-
-
 def _plain(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Operands that the product kernels read: what does not fit each other, is to be differentiated (backward or forward), mapped
     or traced, or lies on two devices is the library's, to compute or to refuse."""
@@ -40,9 +32,13 @@ def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
             (x.data_ptr() | weight.data_ptr()) % 16 == 0)
 
 
+def _row_stride(t: torch.Tensor) -> int:
+    return t.stride(0) if t.shape[0] > 1 else t.shape[1]       # (a single row's may be anything)
+
+
 def _rows_apart(t: torch.Tensor) -> bool:
     """Whole rows from 16-byte boundaries."""
-    return t.stride(1) == 1 and t.stride(0) >= t.shape[1] and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+    return t.stride(1) == 1 and _row_stride(t) >= t.shape[1] and _row_stride(t) % 8 == 0 and t.data_ptr() % 16 == 0
 
 
 def _tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -50,36 +46,47 @@ def _tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return x.is_cuda and len(x.shape) == 2 and x.shape[0] > 64 and _plain(x, weight) and _rows_apart(x) and _rows_apart(weight)
 
 
-def _tile(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
-    code = _lib.load_decoder().ed_tile_gemm(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(),
+def _decode_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
+    code = _lib.load_decoder().ed_decode_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), splits,
+                                              x.shape[0], cols, x.shape[1], act, _lib.current_stream(x.device))
+    _lib.check_decoder(code, "decode_gemm")
+    return out
+
+
+def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
+    code = _lib.load_decoder().ed_tile_gemm(x.data_ptr(), _row_stride(x), weight.data_ptr(), _row_stride(weight), out.data_ptr(),
                                             _lib.dtype_code(out.dtype), splits, x.shape[0], cols, x.shape[1], act,
                                             _lib.current_stream(x.device))
     _lib.check_decoder(code, "tile_gemm")
     return out
 
 
-def _tiles(x: torch.Tensor, weight: torch.Tensor, cols: int, act: int = 0) -> bool:
-    """Whether the tiled kernel takes the product and is the faster way."""
-    return _tiles_fit(x, weight) and _lib.load_decoder().ed_tile_gemm_pays(x.shape[0], cols, weight.shape[1], act) == 1
+def _own(x: torch.Tensor, weight: torch.Tensor, cols: int, act: int = 0, dtype: torch.dtype = _BF16) -> Optional[torch.Tensor]:
+    """act(x @ weight^T) by the tiled or the weight-streaming kernel, where one of them takes it and is the faster way; else None."""
+    if not x.is_cuda or not (_fits(x, weight) or _tiles_fit(x, weight)):
+        return None
+    lib, (T, K) = _lib.load_decoder(), x.shape
+    if lib.ed_tile_gemm_pays(T, cols, K, act) == 1:
+        return _tile_gemm(x, weight, torch.empty(T, cols, dtype=dtype, device=x.device), 1, cols, act)
+    if T <= 64 and lib.ed_decode_gemm_pays(T, cols, K, act, _lib.dtype_code(dtype)) == 1:
+        return _decode_gemm(x, weight, torch.empty(T, cols, dtype=dtype, device=x.device), 1, cols, act)
+    return None
 
 
 def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
-    """For a decode batch that the weight-streaming kernel takes: how many ranges of K fill the chip; else 0."""
-    return _lib.load_decoder().ed_decode_gemm_splits(x.shape[0], *weight.shape) if _fits(x, weight) else 0
-
-
-def _streams(x: torch.Tensor, weight: torch.Tensor, out_rows: int, act: int = 0, out_dtype: int = _lib.DTYPE_BF16) -> bool:
-    """Whether the weight-streaming kernel takes the product and is the faster way."""
-    return x.is_cuda and _fits(x, weight) and _lib.load_decoder().ed_decode_gemm_pays(x.shape[0], out_rows, weight.shape[1], act, out_dtype) == 1
+    """For a decode batch that the product kernels take: how many ranges of K fill the chip; else 0."""
+    if not _fits(x, weight):
+        return 0
+    lib = _lib.load_decoder()
+    return lib.ed_tile_gemm_splits(x.shape[0], *weight.shape) or lib.ed_decode_gemm_splits(x.shape[0], *weight.shape)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
-    """act(x @ weight^T) in x's type: a weight-streaming kernel for a decode batch, a tiled one for a short prompt, a library product
-    otherwise; ``act``: None or 'relu_squared'."""
-    if _streams(x, weight, weight.shape[0], int(act is not None)):
-        return _skinny(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device), 1, int(act is not None))
-    if _tiles(x, weight, weight.shape[0], int(act is not None)):
-        return _tile(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device), 1, weight.shape[0], int(act is not None))
+    """act(x @ weight^T) in x's type: a kernel of this package for decode batches and short prompts, a library product otherwise;
+    ``act``: None or 'relu_squared'."""
+    out = _own(x, weight, weight.shape[0], int(act is not None))
+    if out is not None:
+        return out
     out = F.linear(x, weight)
     return relu_squared_(out) if act is not None else out
 
@@ -87,15 +94,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> 
 def linear_silu_gate(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T) for ``weight`` = [gate; up]: one launch for a decode batch or a short prompt."""
     (T, _), ff = x.shape, weight.shape[0] // 2
-    out = torch.empty(T, ff, dtype=x.dtype, device=x.device)
-    if _streams(x, weight, ff, 2):
-        code = _lib.load_decoder().ed_decode_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _lib.dtype_code(out.dtype), 1, T, ff,
-                                                  x.shape[1], 2, _lib.current_stream(x.device))
-        _lib.check_decoder(code, "decode_gemm")
+    out = _own(x, weight, ff, 2) if weight.shape[0] == 2 * ff else None
+    if out is not None:
         return out
-    if _tiles(x, weight, ff, 2) and weight.shape[0] == 2 * ff:
-        return _tile(x, weight, out, 1, ff, 2)
-    u = F.linear(x, weight)
+    out, u = torch.empty(T, ff, dtype=x.dtype, device=x.device), F.linear(x, weight)
     _lib.check_decoder(_lib.load_decoder().ed_silu_gate(u.data_ptr(), out.data_ptr(), T, ff, _lib.dtype_code(x.dtype),
                                                         _lib.current_stream(x.device)), "silu_gate")
     return out
@@ -105,26 +107,22 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x @ weight^T with the float32 accumulators as the result, for sums that stay float32."""
     if x.dtype == torch.float32:
         return F.linear(x, weight)
-    if _streams(x, weight, weight.shape[0], 0, _lib.DTYPE_F32):
-        return _skinny(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), 1, 0)
-    if _tiles(x, weight, weight.shape[0]):
-        return _tile(x, weight, torch.empty(x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), 1, weight.shape[0], 0)
-    return torch.mm(x, weight.t(), out_dtype=torch.float32)
+    out = _own(x, weight, weight.shape[0], 0, torch.float32)
+    return out if out is not None else torch.mm(x, weight.t(), out_dtype=torch.float32)
 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor, exact: bool = False) -> torch.Tensor:
     """x @ weight^T as ``residual_norm`` takes it: [T, N], or float32 partial sums [parts, T, N] of a decode batch or a short prompt.
     ``exact``: not rounded to the compute type on the way."""
-    splits = _skinny_splits(x, weight) if x.is_cuda else 0
-    if splits > 1:
-        return _skinny(x, weight, torch.empty(splits, x.shape[0], weight.shape[0], dtype=torch.float32, device=x.device), splits, 0)
-    if _tiles_fit(x, weight):
-        (T, K), N = x.shape, weight.shape[0]
-        splits = _lib.load_decoder().ed_tile_gemm_splits(T, N, K)
+    if x.is_cuda and (_fits(x, weight) or _tiles_fit(x, weight)):
+        (T, K), N, lib = x.shape, weight.shape[0], _lib.load_decoder()
+        splits = lib.ed_tile_gemm_splits(T, N, K)
+        run = _tile_gemm if splits > 0 else _decode_gemm
+        splits = splits or lib.ed_decode_gemm_splits(T, N, K)
         if splits > 1:
-            return _tile(x, weight, torch.empty(splits, T, N, dtype=torch.float32, device=x.device), splits, N, 0)
-        if splits == 1:
-            return _tile(x, weight, torch.empty(T, N, dtype=torch.float32 if exact else x.dtype, device=x.device), 1, N, 0)
+            return run(x, weight, torch.empty(splits, T, N, dtype=torch.float32, device=x.device), splits, N, 0)
+        if splits == 1 and T > 64:
+            return _tile_gemm(x, weight, torch.empty(T, N, dtype=torch.float32 if exact else x.dtype, device=x.device), 1, N, 0)
     return linear_f32(x, weight) if exact else linear(x, weight)
 
 

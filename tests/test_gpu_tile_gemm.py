@@ -1,4 +1,4 @@
-"""The tiled product of short prompts at the edges of its tiles, of its ring and of the rule that takes calls to it."""
+"""The tiled product of decode batches and short prompts at the edges of its tiles, of its ring and of the rule that takes calls to it."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -35,9 +35,10 @@ def product(x, w, cols, splits=1, act=0, dtype=BF16):
     return full[:-1].view(splits, T, cols)
 
 
-# rows around the tiles' edges; columns of one tile, remainders of 16 and of 4; K of one step, fewer than a ring, more than the deepest
-@pytest.mark.parametrize("T", [1, 63, 64, 65, 127, 129, 300, 1030])
-@pytest.mark.parametrize("N,K", [(64, 64), (70, 128), (1028, 320), (2056, 448), (4099, 832), (16400, 192)])
+# rows around the tiles' edges; columns of one tile, remainders of 16 and of 4; K of one step, fewer than a ring, more than the
+# deepest; enough columns for every form of a decode batch
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 63, 64, 65, 127, 129, 300, 1030])
+@pytest.mark.parametrize("N,K", [(34, 64), (70, 128), (1028, 320), (2056, 448), (4099, 832), (12290, 832), (20000, 192)])
 def test_products(T, N, K):
     announce(f"tile gemm {T} {N} {K}")
     x, w, want = operands(T, N, K)
@@ -59,14 +60,14 @@ def test_rows_that_lie_apart(T, N, K, x_stride, w_stride):
 
 
 @pytest.mark.parametrize("T,N,K", [(65, 1024, 512), (300, 2048, 2048), (300, 2048, 6144), (512, 4096, 4096), (1024, 2048, 4096), (513, 4096, 4096),
-                                   (64, 2048, 2048), (300, 1000, 512), (300, 2048, 2056), (700, 6144, 2048)])
+                                   (64, 2048, 2048), (64, 12288, 1024), (23, 6720, 1088), (16, 10240, 1024), (1, 8512, 2048), (300, 1000, 512), (300, 2048, 2056), (700, 6144, 2048)])
 def test_every_route_gives_the_product(T, N, K):
     """What the rule takes and what it leaves to the library."""
     announce(f"tile gemm routes {T} {N} {K}")
     x, w, want = operands(T, N, K)
     parts, lib = ops.linear_parts(x, w), _lib.load_decoder()
     splits = lib.ed_tile_gemm_splits(T, N, K)
-    if T > 64:
+    if splits > 0:
         assert parts.dim() == (3 if splits > 1 else 2)
     assert off(parts.sum(0) if parts.dim() == 3 else parts, want) < BF16_TOL
     exact = ops.linear_parts(x, w, exact=True)
@@ -79,5 +80,5 @@ def test_every_route_gives_the_product(T, N, K):
     # operands off the kernel's boundaries are the library's
     wide = torch.cat([x, x[:, :4]], 1)[:, :K]
     shifted = torch.empty(N * K + 1, dtype=BF16, device="cuda")[1:].view(N, K).copy_(w)
-    assert not ops._tiles_fit(wide, w) and not ops._tiles_fit(x, shifted)
+    assert not ops._tiles_fit(wide, w) and not ops._tiles_fit(x, shifted) and not ops._fits(x, shifted)
     assert off(ops.linear(wide, w), want) < BF16_TOL and off(ops.linear(x, shifted), want) < BF16_TOL

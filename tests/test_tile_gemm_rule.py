@@ -1,4 +1,4 @@
-"""Which products the tiled kernel of short prompts takes, and what its entry point refuses (nothing runs on a GPU here)."""
+"""Which products the tiled kernel takes, and what its entry point refuses (nothing runs on a GPU here)."""
 import itertools
 
 import pytest
@@ -12,10 +12,16 @@ F32, BF16 = _lib.DTYPE_F32, _lib.DTYPE_BF16
 
 def test_the_rule():
     lib = _lib.load_decoder()
-    # decode batches have a kernel of their own, long prompts are the library's
-    for T, N, K in itertools.product((0, 1, 64, 8192), (2048, 4096, 12288), (1024, 2048, 4096)):
+    # long prompts are the library's; whole results of few rows in a decode batch, and short sums of one, another kernel's
+    for T, N, K in itertools.product((0, 8192), (2048, 4096, 12288), (1024, 2048, 4096)):
         assert lib.ed_tile_gemm_splits(T, N, K) == 0, (T, N, K)
         assert not any(lib.ed_tile_gemm_pays(T, N, K, act) for act in (0, 1, 2)), (T, N, K)
+    for T, K in itertools.product((1, 16, 40, 64), (64, 512, 2048, 12288)):
+        assert not any(lib.ed_tile_gemm_pays(T, N, K, act) for N, act in ((4096, 0), (4096, 1), (2048, 2)))
+        assert (lib.ed_tile_gemm_splits(T, 4096, K) > 0) == (K >= 1024)
+        assert lib.ed_tile_gemm_pays(T, 12288, K, 0) == 1 and lib.ed_tile_gemm_pays(T, 8192, max(K, 1024), 2) == 1
+    assert [lib.ed_tile_gemm_pays(T, 8192, 1024, 0) for T in (32, 33)] == [lib.ed_tile_gemm_pays(T, 6144, 4096, 0) for T in (4, 5)] == \
+        [lib.ed_tile_gemm_pays(T, 4096, 2048, 2) for T in (8, 9)] == [0, 1]
     assert lib.ed_tile_gemm_pays(300, 6144, 2048, 1) == lib.ed_tile_gemm_pays(1024, 4096, 2048, 2) == lib.ed_tile_gemm_pays(1344, 2048, 512, 0) == 1
     assert lib.ed_tile_gemm_pays(2048, 1344, 512, 0) == 1                      # (the sides' roles do not matter)
     assert lib.ed_tile_gemm_pays(300, 6144, 2048, 3) == lib.ed_tile_gemm_pays(300, 6144, 2050, 0) == lib.ed_tile_gemm_pays(300, 512, 512, 0) == 0
