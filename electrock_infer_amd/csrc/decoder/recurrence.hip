@@ -14,8 +14,8 @@
 //     o_t = c_t S^T q_t + sum_{s <= t} (c_t / c_s) (q_t . k_s) u_s
 //     S  <- c_16 S + sum_s (c_16 / c_s) k_s u_s^T
 // block_kernel makes (I + A)^-1 diag(beta) and the 16 x 16 scores of every block, all blocks in parallel.  chunk_kernel
-// walks through the blocks of a chunk with float32 MFMAs, a wave holding 16 columns of the state in the registers in
-// which an MFMA leaves them, which are the next MFMA's second operand as they are.  With several chunks in a sequence a
+// walks through the blocks of a chunk, a wave holding 16 columns of the float32 state in the registers in which an MFMA
+// leaves them, which, split into bf16 parts, are the next MFMA's second operand as they lie.  With several chunks in a sequence a
 // first pass starts every chunk from zero, and for the delta rule, whose chunks multiply the state by a matrix, runs the
 // identity's columns along, which gives that matrix; a scan over the chunks makes the states in front of them, and the
 // output pass starts from there.  Ratios of decays are powers of differences of logarithms, never positive ones.
@@ -278,39 +278,117 @@ __global__ __launch_bounds__(256) void recur_block_kernel(RecurProblem p, int he
 }
 
 // ---- prompts: a chunk's blocks, one after the other ----
-// One workgroup per (chunk, head, group of column tiles), one wave per tile of 16 state columns; waves without a tile help
-// with the loads.  OUTPUT: from the state in front of the chunk; else from zero, with the identity's columns behind the
-// state's for the delta rule.
-template <typename Elem, int NDT, bool DELTA, bool OUTPUT, int THREADS>
-__global__ __launch_bounds__(THREADS) void recur_chunk_kernel(RecurProblem p) {
-    typedef typename Elem::storage S;
-    constexpr int D = NDT * 16, DP = D + 4, kPieces = (NDT + 3) / 4;   // four-float pieces of a block's k (q) per thread
-    constexpr int kTile = kBlock * DP;
-    const int waves = blockDim.x / kWave;
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    float* Ks = lds;                                  // [2][16][DP]
-    float* Qs = Ks + 2 * kTile;                       // [2][16][DP]
-    float* Rs = Qs + (OUTPUT ? 2 * kTile : 0);        // [2][waves][16] partial sums of squares
+// Products with the state (but the additive rule's read-out) run on the bf16 matrix units, every float32 operand as the sum of three
+// bf16 values: 8 bits each, rounded to nearest, so that the first two leave a remainder of 2^-18 and all three one of 2^-27 at most.  Of
+// the nine products the six that reach 2^-24 are added up, in float32, the smallest first.  Against float64 this is no further off than
+// float32 products (1536 tokens, decays from 1 - 6e-6 to e^-2.7 a token: 7.7e-7 / 8.0e-7 where everything is kept, 5.2e-7 / 5.3e-7 where
+// it fades); six bf16 products take 96 cycles where eight float32 ones take 256.  (An infinite operand makes NaN, not infinity.)
+//
+// What bounds the kernel now is instructions: a block is 60-80 matrix and 130-500 vector instructions per wave (splitting the state 180,
+// scaling it 32, a share of the keys 50), and the chain from the barrier through LDS, sums, u and update.  So operands are read from LDS
+// ahead of their products, row sums rotate inside the vector unit (16 shuffles through LDS before), addresses are kept from block to
+// block, and the passes that fit 128 registers run with four waves per SIMD.  us at 8192 tokens, 16 heads of 128 x 128 (delta) and 64 of
+// 128 x 64 with one key, before / now: first pass 206 / 138 and 103 / 72, output pass 193 / 135 and 222 / 170.
+struct Split2 {
+    uint32_t part[3];
+};
+__device__ __forceinline__ Split2 split2(float a, float b) {
+    Split2 s;
+    s.part[0] = pack_bf16(a, b);
+    asm("" : "+v"(s.part[0]));        // (else the compiler converts every value once more instead of shifting it back)
+    const float a1 = a - bf16_lo(s.part[0]), b1 = b - bf16_hi(s.part[0]);
+    s.part[1] = pack_bf16(a1, b1);
+    asm("" : "+v"(s.part[1]));
+    s.part[2] = pack_bf16(a1 - bf16_lo(s.part[1]), b1 - bf16_hi(s.part[1]));
+    return s;
+}
+struct Split4 {
+    u32x2_t part[3];
+};
+__device__ __forceinline__ Split4 split4(f32x4_t v) {
+    const Split2 lo = split2(v[0], v[1]), hi = split2(v[2], v[3]);
+    Split4 s;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) s.part[i] = u32x2_t{lo.part[i], hi.part[i]};
+    return s;
+}
+// the sum over the 16 lanes that share lane / 16, in all of them (rotations inside the vector unit, nothing goes through LDS)
+template <int ROTATE>
+__device__ __forceinline__ float add_rotated(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + ROTATE, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_sum(float v) { return add_rotated<1>(add_rotated<2>(add_rotated<4>(add_rotated<8>(v)))); }
+// two packed halves side by side
+__device__ __forceinline__ bf16x8_t join(u32x2_t lo, u32x2_t hi) {
+    const u32x4_t w = {lo[0], lo[1], hi[0], hi[1]};
+    bf16x8_t f;
+    __builtin_memcpy(&f, &w, 16);
+    return f;
+}
+struct Split8 {
+    bf16x8_t part[3];
+};
+__device__ __forceinline__ Split8 split8(f32x4_t lo, f32x4_t hi) {
+    const Split4 l = split4(lo), h = split4(hi);
+    Split8 s;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) s.part[i] = join(l.part[i], h.part[i]);
+    return s;
+}
+__device__ __forceinline__ f32x4_t mma(bf16x8_t a, bf16x8_t b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+// four rows of a column: ds_read_b64_tr_b16, for which the 16 lanes of a group name the four-element pieces of four rows
+__device__ __forceinline__ u32x2_t read_column(const uint16_t* piece) {
+    typedef short s16x4_t __attribute__((ext_vector_type(4)));
+    const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(piece));
+    u32x2_t w;
+    __builtin_memcpy(&w, &v, 8);
+    return w;
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+// One workgroup per (chunk, head, group of column tiles), one wave per tile of 16 state columns; waves without a tile help
+// with the loads.  Additive rule: a workgroup may take all columns of several heads that share keys (`group`), which then are split
+// once.  OUTPUT: from the state in front of the chunk; else from zero, with the identity's columns behind the state's for the
+// delta rule.
+template <typename Elem, int NDT, bool DELTA, bool OUTPUT, int THREADS>
+__global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void recur_chunk_kernel(RecurProblem p, int group) {
+    typedef typename Elem::storage S;
+    constexpr int D = NDT * 16, DP = D + 8, kPieces = (NDT + 7) / 8;   // four-float pieces of a block's k (q) per thread
+    constexpr int kPart = kBlock * DP, kTile = 3 * kPart;
+    static_assert(NDT % 2 == 0, "a step of the products is two tiles");
+    constexpr bool kRoom = THREADS <= 512 && NDT <= 8;                 // for operands ahead of their products in registers
+    const int waves = blockDim.x / kWave;
+    extern __shared__ __attribute__((aligned(16))) uint16_t operands[];
+    uint16_t* Ks = operands;                               // [2][3 parts][16][DP]
+    // Q by its parts as well, [2][3 parts][16][DP], where the delta rule splits the state for K anyway; for the additive rule as it is,
+    // [2][16][D + 4]: splitting the state costs more than the float32 products it saves
+    constexpr int kQPitch = D + 4;
+    uint16_t* Qs = Ks + 2 * kTile;
+    float* Qf = reinterpret_cast<float*>(Qs);
+    float* Rs = reinterpret_cast<float*>(Qs + 2 * kTile);              // [2][THREADS / 64][16] partial sums of squares (delta rule)
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
     const int4 ch = p.chunks[blockIdx.x];
-    const int h = blockIdx.y, dim = p.dim, vdim = p.vdim, dp = (dim + 15) / 16 * 16;
+    const int dim = p.dim, vdim = p.vdim, dp = (dim + 15) / 16 * 16, v_tiles = (vdim + 15) / 16;
+    const bool several = !DELTA && group > 1;
+    const int h = several ? blockIdx.y * group + min(wave / v_tiles, group - 1) : blockIdx.y, tile = several ? wave % v_tiles : blockIdx.z * waves + wave;
     const int g = h / (p.heads / p.kv_heads);
-    const int v_tiles = (vdim + 15) / 16, tile = blockIdx.z * waves + wave;
     const bool identity = !OUTPUT && DELTA && tile >= v_tiles;
-    const bool has_tile = tile < v_tiles || (identity && tile < v_tiles + dp / 16);
+    const bool has_tile = (several ? wave < group * v_tiles : tile < v_tiles) || (identity && tile < v_tiles + dp / 16);
     const int col = (identity ? tile - v_tiles : tile) * 16 + l16;
-    const bool v_ok = tile < v_tiles && col < vdim;
+    const bool v_ok = has_tile && tile < v_tiles && col < vdim;
     const int64_t kq_pitch = static_cast<int64_t>(p.kv_heads) * dp, v_pitch = static_cast<int64_t>(p.heads) * vdim;
     const float* kg = p.k_f + g * dp;
     const float* qg = p.q_f + g * dp;
-    const S* vg = static_cast<const S*>(p.v_f) + h * vdim + col;
-    const S* gate = OUTPUT && DELTA ? static_cast<const S*>(p.gate) + h * vdim + col : nullptr;
+    const S* vg = static_cast<const S*>(p.v_f) + h * vdim + tile * 16;
+    const S* gate = OUTPUT && DELTA ? static_cast<const S*>(p.gate) + h * vdim + tile * 16 : nullptr;
     const int n_blocks = (ch.z + kBlock - 1) / kBlock;
     const int64_t rec_pitch = static_cast<int64_t>(p.heads) * recur_record(DELTA);
     const float* rec0 = p.blocks + (static_cast<int64_t>(blockIdx.x) * (p.chunk_tokens / kBlock) * p.heads + h) * recur_record(DELTA);
 
-    f32x4_t st[NDT];                                  // rows dt * 16 + lq * 4 + r, column `col`
+    // Column `col` of the state, rows lq * D / 4 + dt * 4 + r: two tiles are eight rows of a lane that lie side by side, as a
+    // product over the state takes them, and the pieces of a key that one tile takes lie a quarter of its row apart (so that they,
+    // and 16 rows of either operand, fall on different banks).
+    f32x4_t st[NDT];
     const int64_t head_state = static_cast<int64_t>(dim) * vdim;
     float* slot = p.states + (static_cast<int64_t>(p.slots[ch.x]) * p.heads + h) * head_state;
     const bool chunked = p.chunk_states != nullptr;
@@ -320,29 +398,37 @@ __global__ __launch_bounds__(THREADS) void recur_chunk_kernel(RecurProblem p) {
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int d = dt * 16 + lq * 4 + r;
+            const int d = lq * (D / 4) + dt * 4 + r;
             st[dt][r] = identity ? (d == col ? 1.0f : 0.0f) : (!from_zero && v_ok && d < dim) ? mine[static_cast<int64_t>(d) * vdim + col] : 0.0f;
         }
     const float norm_w = OUTPUT && DELTA && v_ok ? p.norm_w[col] : 0.0f;
     const float skip = OUTPUT && p.skip != nullptr ? p.skip[h] : 0.0f;
     const float inv_vdim = 1.0f / static_cast<float>(vdim);
 
-    // a block's operands, in flight while the one before is computed
+    // A block's operands, in flight while the one before is computed: loads of rows and columns that exist, without conditions around
+    // them (what does not exist is made zero where it is used).
+    // (The additive rule's output pass and the delta rule's first one ask for a block's record when they start on it: one set of registers instead of two is what lets
+    // a CU have four waves per SIMD.)
+    constexpr bool kLate = OUTPUT != DELTA;
     f32x4_t rk[kPieces], rq[kPieces], scores, inverse, decay, rest, beta;
     float block_decay, block_log;
-    S v[4], gt[4];                                    // (as stored: a conversion here would wait for the load)
-    auto fetch = [&](int b) {
-        const int n = min(kBlock, ch.z - b * kBlock);
-        const int64_t row0 = static_cast<int64_t>(ch.y) + b * kBlock;
+    S v[4] = {}, gt[4] = {};                          // (as stored: a conversion here would wait for the load)
+    int k_at[kPieces], v_at[4];                       // a lane's elements, from a block's first row
+    int64_t gate_at[4];
+    auto place = [&](int last) {                      // ... of whose rows `last` is the last
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
             const int e = tid + i * static_cast<int>(blockDim.x), t = e / (D / 4), d = (e - t * (D / 4)) * 4;
-            rk[i] = rq[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            if (t < n && d < dp) {
-                rk[i] = *reinterpret_cast<const f32x4_t*>(kg + (row0 + t) * kq_pitch + d);
-                if (OUTPUT) rq[i] = *reinterpret_cast<const f32x4_t*>(qg + (row0 + t) * kq_pitch + d);
-            }
+            k_at[i] = min(t, last) * static_cast<int>(kq_pitch) + min(d, dp - 4);
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = min(lq * 4 + r, last), c = v_ok ? l16 : 0;
+            v_at[r] = t * static_cast<int>(v_pitch) + c;
+            if (OUTPUT && DELTA) gate_at[r] = t * p.stride + c;
+        }
+    };
+    auto records = [&](int b) {
         const float* rec = rec0 + b * rec_pitch;
         if (OUTPUT) scores = *reinterpret_cast<const f32x4_t*>(rec + kRecScores + l16 * kBlock + lq * 4);
         if (DELTA) inverse = *reinterpret_cast<const f32x4_t*>(rec + kRecInverse + l16 * kBlock + lq * 4);
@@ -351,12 +437,23 @@ __global__ __launch_bounds__(THREADS) void recur_chunk_kernel(RecurProblem p) {
         rest = *reinterpret_cast<const f32x4_t*>(rec + kRecRest + lq * 4);
         block_decay = rec[kRecDecay + kBlock - 1];
         block_log = rec[kRecLog];
+    };
+    auto fetch = [&](int b) {
+        const int64_t row0 = static_cast<int64_t>(ch.y) + b * kBlock;
+        if (b == 0 || b == n_blocks - 1) place(min(kBlock, ch.z - b * kBlock) - 1);
+        const float *k0 = kg + row0 * kq_pitch, *q0 = qg + row0 * kq_pitch;
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            rk[i] = *reinterpret_cast<const f32x4_t*>(k0 + k_at[i]);
+            if (OUTPUT) rq[i] = *reinterpret_cast<const f32x4_t*>(q0 + k_at[i]);
+        }
+        if (!kLate) records(b);
+        if (tile >= v_tiles) return;
+        const S *v0 = vg + row0 * v_pitch, *gate0 = gate + (OUTPUT && DELTA ? row0 * p.stride : 0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int t = lq * 4 + r;
-            const bool ok = v_ok && t < n;
-            v[r] = ok ? vg[(row0 + t) * v_pitch] : S(0);
-            if (OUTPUT && DELTA) gt[r] = ok ? gate[(row0 + t) * p.stride] : S(0);
+            v[r] = v0[v_at[r]];
+            if (OUTPUT && DELTA) gt[r] = gate0[gate_at[r]];
         }
     };
     // a block's results wait for the row sums of the other waves until the next barrier
@@ -366,54 +463,128 @@ __global__ __launch_bounds__(THREADS) void recur_chunk_kernel(RecurProblem p) {
         const int n = min(kBlock, ch.z - b * kBlock);
         const int64_t row0 = static_cast<int64_t>(ch.y) + b * kBlock;
         f32x4_t ss = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int w = 0; w < waves; ++w) ss += *reinterpret_cast<const f32x4_t*>(Rs + ((b & 1) * waves + w) * kBlock + lq * 4);
+#pragma unroll
+        for (int w0 = 0; w0 < THREADS / kWave; w0 += 4) {
+            f32x4_t part[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) part[w] = *reinterpret_cast<const f32x4_t*>(Rs + ((b & 1) * (THREADS / kWave) + w0 + w) * kBlock + lq * 4);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) ss += part[w];
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int t = lq * 4 + r;
-            if (v_ok && t < n) {
-                const float y = held[r] * __builtin_amdgcn_rsqf(ss[r] * inv_vdim + p.eps) * norm_w;
-                static_cast<S*>(p.out)[(row0 + t) * v_pitch + h * vdim + col] = Elem::store(y * silu_fast(held_gate[r]));
-            }
+            const float y = held[r] * __builtin_amdgcn_rsqf(ss[r] * inv_vdim + p.eps) * norm_w * silu_fast(held_gate[r]);
+            if (v_ok && t < n) static_cast<S*>(p.out)[(row0 + t) * v_pitch + h * vdim + col] = Elem::store(y);
         }
     };
+    if (OUTPUT && DELTA)              // (waves that do not exist add nothing)
+        for (int i = tid; i < 2 * THREADS / kWave * kBlock; i += static_cast<int>(blockDim.x)) Rs[i] = 0.0f;
     float log_sum = 0.0f;
     fetch(0);
     for (int b = 0; b < n_blocks; ++b) {
-        float* kb = Ks + (b & 1) * kTile;
-        float* qb = Qs + (b & 1) * kTile;
+        uint16_t* kb = Ks + (b & 1) * kTile;
+        uint16_t* qb = Qs + (b & 1) * kTile;
+        float* qf = Qf + (b & 1) * kBlock * kQPitch;
+        const int n = min(kBlock, ch.z - b * kBlock);
+        auto keep = [&](uint16_t* to, f32x4_t v, bool exists) {
+            const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            const Split4 s = split4(exists ? v : zero);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2_t*>(to + i * kPart) = s.part[i];
+        };
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
             const int e = tid + i * static_cast<int>(blockDim.x), t = e / (D / 4), d = (e - t * (D / 4)) * 4;
             if (t < kBlock) {
-                *reinterpret_cast<f32x4_t*>(kb + t * DP + d) = rk[i];
-                if (OUTPUT) *reinterpret_cast<f32x4_t*>(qb + t * DP + d) = rq[i];
+                keep(kb + t * DP + d, rk[i], t < n && d < dp);
+                if (DELTA && OUTPUT) keep(qb + t * DP + d, rq[i], t < n && d < dp);
+                if (!DELTA && OUTPUT) *reinterpret_cast<f32x4_t*>(qf + t * kQPitch + d) = d < dp ? rq[i] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
             }
         }
-        const f32x4_t scores_b = scores, inverse_b = inverse, decay_b = decay, rest_b = rest, beta_b = beta;
-        const float whole = block_decay;
+        f32x4_t scores_b, inverse_b, decay_b, rest_b, beta_b;
+        float whole;
+        auto take = [&]() {
+            scores_b = scores, inverse_b = inverse, decay_b = decay, rest_b = rest, beta_b = beta;
+            whole = block_decay;
+            log_sum += block_log;
+        };
+        if (!kLate) take();
         float v_b[4], gt_b[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            v_b[r] = Elem::load(v[r]);
-            gt_b[r] = OUTPUT && DELTA ? Elem::load(gt[r]) : 0.0f;
+            const bool ok = v_ok && lq * 4 + r < n;
+            v_b[r] = ok ? Elem::load(v[r]) : 0.0f;
+            gt_b[r] = OUTPUT && DELTA && ok ? Elem::load(gt[r]) : 0.0f;
         }
-        log_sum += block_log;
         __syncthreads();              // (the block before last, in the same half, has been used)
+        if (kLate) {
+            records(b);
+            take();
+        }
         if (b + 1 < n_blocks) fetch(b + 1);
-        if (OUTPUT && DELTA && b > 0) finish(b - 1);
         if (!has_tile) {
-            if (OUTPUT && DELTA && lane < kBlock) Rs[((b & 1) * waves + wave) * kBlock + lane] = 0.0f;
+            if (OUTPUT && DELTA && b > 0) finish(b - 1);
             continue;
         }
-        f32x4_t u;
+        // Operands from LDS a step ahead of the products, K's and Q's sums in turn: every product of a sum waits for the one before.
+        f32x4_t u, ks = {0.0f, 0.0f, 0.0f, 0.0f}, o = {0.0f, 0.0f, 0.0f, 0.0f};
         if (DELTA) {
-            f32x4_t ks = {0.0f, 0.0f, 0.0f, 0.0f};
+            constexpr int kTwo = kRoom && OUTPUT ? 1 : 0;
+            Split8 ka[1 + kTwo], qa[1 + kTwo];
+            auto rows = [&](int k) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const int at = i * kPart + l16 * DP + lq * (D / 4) + k * 8;
+                    ka[k & kTwo].part[i] = *reinterpret_cast<const bf16x8_t*>(kb + at);
+                    if (OUTPUT) qa[k & kTwo].part[i] = *reinterpret_cast<const bf16x8_t*>(qb + at);
+                }
+            };
+            Split8 s8[1 + kTwo];
+            if (kTwo) {
+                rows(0);
+                s8[0] = split8(st[0], st[1]);
+            }
+#pragma unroll
+            for (int k = 0; k < NDT / 2; ++k) {
+                if (!kTwo) rows(k);
+                else if (k + 1 < NDT / 2) rows(k + 1);
+                if (kRoom) __builtin_amdgcn_sched_barrier(0);
+                if (!kTwo) s8[0] = split8(st[2 * k], st[2 * k + 1]);
+                else if (k + 1 < NDT / 2) s8[(k + 1) & kTwo] = split8(st[2 * k + 2], st[2 * k + 3]);
+                // the smallest products first
+                constexpr int kFirst[6] = {2, 1, 0, 1, 0, 0}, kSecond[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+                for (int i = 0; i < 6; ++i) {
+                    ks = mma(ka[k & kTwo].part[kFirst[i]], s8[k & kTwo].part[kSecond[i]], ks);
+                    if (OUTPUT) o = mma(qa[k & kTwo].part[kFirst[i]], s8[k & kTwo].part[kSecond[i]], o);
+                }
+            }
+        }
+        if (!DELTA && OUTPUT) {
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) {
-                const f32x4_t k4 = *reinterpret_cast<const f32x4_t*>(kb + l16 * DP + dt * 16 + lq * 4);
+                const f32x4_t q4 = *reinterpret_cast<const f32x4_t*>(qf + l16 * kQPitch + lq * (D / 4) + dt * 4);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) ks = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[r], st[dt][r], ks, 0, 0, 0);
+                for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[r], st[dt][r], o, 0, 0, 0);
+                if (kRoom && dt % 2 != 0) __builtin_amdgcn_sched_barrier(0);      // (all of them at once do not fit the registers)
             }
+        }
+        if (OUTPUT && DELTA && b > 0) finish(b - 1);
+        // the keys by column, for the update: on their way while u is made
+        const uint16_t* kc = kb + (lq * 4 + (l16 >> 2)) * DP + (l16 & 3) * (D / 4);
+        constexpr int kRing = !kRoom ? 1 : OUTPUT || DELTA ? 2 : 4;
+        u32x2_t kt[kRing][3];
+        auto columns = [&](int dt) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) kt[dt % kRing][i] = read_column(kc + i * kPart + dt * 4);
+        };
+        if (kRoom) {
+#pragma unroll
+            for (int dt = 0; dt < kRing && dt < NDT; ++dt) columns(dt);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (DELTA) {
             f32x4_t right;
 #pragma unroll
             for (int r = 0; r < 4; ++r) right[r] = v_b[r] - decay_b[r] * ks[r];
@@ -425,44 +596,41 @@ __global__ __launch_bounds__(THREADS) void recur_chunk_kernel(RecurProblem p) {
             for (int r = 0; r < 4; ++r) u[r] = beta_b[r] * v_b[r];
         }
         if (OUTPUT) {
-            f32x4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-                const f32x4_t q4 = *reinterpret_cast<const f32x4_t*>(qb + l16 * DP + dt * 16 + lq * 4);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[r], st[dt][r], o, 0, 0, 0);
-            }
             o *= decay_b;
 #pragma unroll
             for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f32_16x16x4f32(scores_b[r], u[r], o, 0, 0, 0);
-            if (DELTA) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float ss = o[r] * o[r];
-#pragma unroll
-                    for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
-                    if (l16 == 0) Rs[((b & 1) * waves + wave) * kBlock + lq * 4 + r] = ss;
-                    held_gate[r] = gt_b[r];
-                }
-                held = o;
-            } else {
-                const int n = min(kBlock, ch.z - b * kBlock);
-                const int64_t row0 = static_cast<int64_t>(ch.y) + b * kBlock;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int t = lq * 4 + r;
-                    if (v_ok && t < n)
-                        static_cast<S*>(p.out)[(row0 + t) * v_pitch + h * vdim + col] = Elem::store(fmaf(skip, v_b[r], o[r]));
-                }
-            }
         }
         u *= rest_b;
+        // A product over 16 tokens fills half of an instruction: the halves take two of the six products of parts.
+        const Split4 us = split4(u);
+        const bf16x8_t u32 = join(us.part[2], us.part[1]), u21 = join(us.part[1], us.part[0]), u11 = join(us.part[0], us.part[0]);
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
+            if (!kRoom) columns(dt);
+            const bf16x8_t k12 = join(kt[dt % kRing][0], kt[dt % kRing][1]), k13 = join(kt[dt % kRing][0], kt[dt % kRing][2]);
+            if (kRoom && dt + kRing < NDT) columns(dt + kRing);
             st[dt] *= whole;
-            const float* kc = kb + lq * 4 * DP + dt * 16 + l16;
+            st[dt] = mma(k12, u32, st[dt]);           // k1 u3 + k2 u2
+            st[dt] = mma(k13, u21, st[dt]);           // k1 u2 + k3 u1
+            st[dt] = mma(k12, u11, st[dt]);           // k1 u1 + k2 u1
+        }
+        if (OUTPUT && DELTA) {
+            f32x4_t ss;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) st[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[r * DP], u[r], st[dt], 0, 0, 0);
+            for (int r = 0; r < 4; ++r) {
+                ss[r] = row_sum(o[r] * o[r]);
+                held_gate[r] = gt_b[r];
+            }
+            if (l16 == 0) *reinterpret_cast<f32x4_t*>(Rs + ((b & 1) * (THREADS / kWave) + wave) * kBlock + lq * 4) = ss;
+            held = o;
+        } else if (OUTPUT) {
+            const int64_t row0 = static_cast<int64_t>(ch.y) + b * kBlock;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = lq * 4 + r;
+                if (v_ok && t < n)
+                    static_cast<S*>(p.out)[(row0 + t) * v_pitch + h * vdim + col] = Elem::store(fmaf(skip, v_b[r], o[r]));
+            }
         }
     }
     if (OUTPUT && DELTA) {
@@ -477,7 +645,7 @@ __global__ __launch_bounds__(THREADS) void recur_chunk_kernel(RecurProblem p) {
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int d = dt * 16 + lq * 4 + r;
+                    const int d = lq * (D / 4) + dt * 4 + r;
                     if (d < dp) m[d * dp + col] = st[dt][r];
                 }
         }
@@ -487,7 +655,7 @@ __global__ __launch_bounds__(THREADS) void recur_chunk_kernel(RecurProblem p) {
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int d = dt * 16 + lq * 4 + r;
+            const int d = lq * (D / 4) + dt * 4 + r;
             if (v_ok && d < dim) mine[static_cast<int64_t>(d) * vdim + col] = st[dt][r];
         }
     if (!OUTPUT && !DELTA && tile == 0 && lane == 0) p.chunk_trans[static_cast<int64_t>(blockIdx.x) * p.heads + h] = log_sum;
@@ -744,13 +912,14 @@ int launch_conv(const RecurProblem& p, hipStream_t s) {
 }
 
 template <typename Elem, int NDT, bool DELTA, bool OUTPUT, int THREADS>
-int launch_chunks(const RecurProblem& p, int tiles, int waves, hipStream_t s) {
-    const size_t lds = sizeof(float) * (static_cast<size_t>(OUTPUT ? 4 : 2) * kBlock * (NDT * 16 + 4) + 2 * waves * kBlock);
+int launch_chunks(const RecurProblem& p, int tiles, int waves, int group, hipStream_t s) {
+    const size_t keys = sizeof(uint16_t) * 2 * 3 * kBlock * (NDT * 16 + 8), queries = DELTA ? keys : sizeof(float) * 2 * kBlock * (NDT * 16 + 4);
+    const size_t lds = keys + (OUTPUT ? queries : 0) + (DELTA && OUTPUT ? sizeof(float) * 2 * THREADS / kWave * kBlock : 0);
     const int rc = allow_lds(reinterpret_cast<const void*>(recur_chunk_kernel<Elem, NDT, DELTA, OUTPUT, THREADS>), lds);
     if (rc != 0) return rc;
     launch((recur_chunk_kernel<Elem, NDT, DELTA, OUTPUT, THREADS>),
-           dim3(static_cast<unsigned>(p.n_chunks), static_cast<unsigned>(p.heads), static_cast<unsigned>(ceil_div(tiles, waves))),
-           dim3(static_cast<unsigned>(waves * kWave)), lds, s, p);
+           dim3(static_cast<unsigned>(p.n_chunks), static_cast<unsigned>(p.heads / group), static_cast<unsigned>(group > 1 ? 1 : ceil_div(tiles, waves))),
+           dim3(static_cast<unsigned>(waves * kWave)), lds, s, p, group);
     return launch_status();
 }
 
@@ -758,10 +927,14 @@ template <typename Elem, int NDT, bool DELTA, bool OUTPUT>
 int size_chunks(const RecurProblem& p, hipStream_t s) {
     const int v_tiles = static_cast<int>(ceil_div(p.vdim, 16));
     const int tiles = v_tiles + (DELTA && !OUTPUT ? static_cast<int>(ceil_div(p.dim, 16)) : 0);
-    // (a head's norm needs all of its columns in one workgroup; at least four waves move the operands)
-    if (DELTA && OUTPUT && tiles > 8) return launch_chunks<Elem, NDT, DELTA, OUTPUT, DELTA && OUTPUT ? 1024 : 512>(p, tiles, tiles, s);
-    const int groups = static_cast<int>(ceil_div(tiles, 8));
-    return launch_chunks<Elem, NDT, DELTA, OUTPUT, 512>(p, tiles, std::max(4, static_cast<int>(ceil_div(tiles, groups))), s);
+    // (a head's norm needs all of its columns in one workgroup; eight waves move the operands)
+    if (DELTA && OUTPUT && tiles > 8) return launch_chunks<Elem, NDT, DELTA, OUTPUT, DELTA && OUTPUT ? 1024 : 512>(p, tiles, tiles, 1, s);
+    if (!DELTA) {
+        int group = std::max(1, 8 / v_tiles);         // heads that fill eight waves
+        while (p.heads / p.kv_heads % group != 0) --group;
+        if (group > 1) return launch_chunks<Elem, NDT, DELTA, OUTPUT, 512>(p, tiles, 8, group, s);
+    }
+    return launch_chunks<Elem, NDT, DELTA, OUTPUT, 512>(p, tiles, 8, 1, s);
 }
 
 template <typename Elem, bool DELTA, bool OUTPUT>
