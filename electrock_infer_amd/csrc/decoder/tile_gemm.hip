@@ -282,11 +282,12 @@ namespace {
 // Where a decode batch is faster this way than by the weight-streaming kernel, which shares K out over a workgroup's waves and so
 // makes twice as many, smaller pieces, and than by the library (11 sizes of 1024 to 32000 rows, K of 512 to 12288, T of 1 to 64; this /
 // the better of the two: 0.74 to 0.90 of its time beyond 8192 rows, 0.90 for partial sums with the norm behind them):
-//   * results stay partial sums, unless K leaves no steps to share out (4096 x 512, one token 7.3 / 6.7 us, 64 tokens 8.2 / 8.5);
+//   * results stay partial sums, unless K leaves no steps to share out (4096 x 512, one token 7.3 / 6.7 us, 64 tokens 8.2 / 8.5) or up
+//     to 16 tokens take a few MB (in a step of one token 2048 x 2048 and x 4096 5.6 / 5.0 on the average);
 //   * or the rows are a CU's worth of tiles: 6144 (6144 x 4096, T = 17 13.6 / 14.6, one 12.6 / 12.9; 4096 x 4096, T = 17 11.9 / 9.8), which a
 //     short K (8192 x 1024, T = 16 9.1 / 8.6) or a gate (its fragments mix both halves: 8192 x 4096, one token 14.9 / 14.3, T = 32 15.7 / 16.4) moves up.
 bool decode_pays(int64_t T, int64_t rows, int K, int act, bool parts) {
-    if (parts) return K >= 1024;
+    if (parts) return K >= 1024 && (T > 16 || rows * K > (int64_t{1} << 23));
     if (act == 2) return (rows >= 10240 && K >= 1024) || (rows >= 8192 && T > 8 && K > 1024) || (rows >= 6144 && T > 32);
     return rows > 8192 || (rows >= 6144 && (T > 32 || (K > 1024 && (T > 4 || rows >= 8192))));
 }

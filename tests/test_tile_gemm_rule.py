@@ -18,7 +18,7 @@ def test_the_rule():
         assert not any(lib.ed_tile_gemm_pays(T, N, K, act) for act in (0, 1, 2)), (T, N, K)
     for T, K in itertools.product((1, 16, 40, 64), (64, 512, 2048, 12288)):
         assert not any(lib.ed_tile_gemm_pays(T, N, K, act) for N, act in ((4096, 0), (4096, 1), (2048, 2)))
-        assert (lib.ed_tile_gemm_splits(T, 4096, K) > 0) == (K >= 1024)
+        assert (lib.ed_tile_gemm_splits(T, 4096, K) > 0) == (K > 2048 or (K == 2048 and T > 16))
         assert lib.ed_tile_gemm_pays(T, 12288, K, 0) == 1 and lib.ed_tile_gemm_pays(T, 8192, max(K, 1024), 2) == 1
     assert [lib.ed_tile_gemm_pays(T, 8192, 1024, 0) for T in (32, 33)] == [lib.ed_tile_gemm_pays(T, 6144, 4096, 0) for T in (4, 5)] == \
         [lib.ed_tile_gemm_pays(T, 4096, 2048, 2) for T in (8, 9)] == [0, 1]
