@@ -106,6 +106,91 @@ __global__ __launch_bounds__(256) void attn_prepare_kernel(AttnProblem p) {
     }
 }
 
+// The same for the rows of a prompt, bf16: a wave per token, L lanes with eight elements each to a head, everything a group of heads
+// needs requested before the first of them is normed.  Bound: the rows' bytes (8192 tokens, 16 + 4 heads of 128, 100 MB: 56 -> 35 us;
+// a workgroup per token took a head per wave, four bytes per lane and a load's way at a time).
+template <int L>
+__global__ __launch_bounds__(256) void attn_prepare_rows_kernel(AttnProblem p, int64_t T) {
+    constexpr int kHeads = kWave / L, kAhead = 4;
+    __shared__ __attribute__((aligned(16))) float turns[4][2][L * 4];          // cosines and sines of a token's pairs
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane / L, j = lane % L, c = j * 8;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+    if (t >= T) return;                                                        // (waves share nothing)
+    const int half = p.rot / 2, all = p.heads + p.kv_heads, vp = attn_pitch(p.vdim), row = attn_row_elems(p.kv_heads, L * 8, p.vdim);
+    const uint16_t *q = static_cast<const uint16_t*>(p.q) + t * p.stride + c, *k = static_cast<const uint16_t*>(p.k) + t * p.stride + c;
+    uint16_t* q_out = static_cast<uint16_t*>(p.q_out) + t * p.heads * (L * 8) + c;
+    uint16_t* cached = static_cast<uint16_t*>(p.cache) + static_cast<int64_t>(p.cache_rows[t]) * row;
+    const float pos = static_cast<float>(p.positions[t]);
+    for (int i = lane; i < half; i += kWave) sincosf(pos * p.inv_freq[i], &turns[wave][1][i], &turns[wave][0][i]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const bool turned = c < p.rot;
+    f32x4_t cosine = {1.0f, 1.0f, 1.0f, 1.0f}, sine = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (turned) {
+        cosine = *reinterpret_cast<const f32x4_t*>(&turns[wave][0][j * 4]);
+        sine = *reinterpret_cast<const f32x4_t*>(&turns[wave][1][j * 4]);
+    }
+    float wq[8], wk[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        wq[i] = p.q_norm != nullptr ? p.q_norm[c + i] : 1.0f;
+        wk[i] = p.k_norm != nullptr ? p.k_norm[c + i] : 1.0f;
+    }
+    for (int u0 = sub; u0 < all + sub; u0 += kHeads * kAhead) {
+        u32x4_t rows[kAhead];
+#pragma unroll
+        for (int n = 0; n < kAhead; ++n) {
+            const int u = min(u0 + n * kHeads, all - 1);
+            rows[n] = *reinterpret_cast<const u32x4_t*>(u < p.heads ? q + u * (L * 8) : k + (u - p.heads) * (L * 8));
+        }
+#pragma unroll
+        for (int n = 0; n < kAhead; ++n) {
+            const int u = u0 + n * kHeads;
+            const bool is_q = u < p.heads;
+            float x[8], ss = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[2 * i] = bf16_lo(rows[n][i]);
+                x[2 * i + 1] = bf16_hi(rows[n][i]);
+                ss = fmaf(x[2 * i], x[2 * i], fmaf(x[2 * i + 1], x[2 * i + 1], ss));
+            }
+            if ((is_q ? p.q_norm : p.k_norm) != nullptr) {
+#pragma unroll
+                for (int off = L / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+                const float rstd = 1.0f / sqrtf(ss / static_cast<float>(L * 8) + p.eps);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] *= rstd * (is_q ? wq[i] : wk[i]);
+            }
+            u32x4_t out;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float a = x[2 * i], b = x[2 * i + 1];
+                out[i] = turned ? pack_bf16(a * cosine[i] - b * sine[i], b * cosine[i] + a * sine[i]) : pack_bf16(a, b);
+            }
+            if (u < all) *reinterpret_cast<u32x4_t*>(is_q ? q_out + u * (L * 8) : cached + (u - p.heads) * (L * 8) + c) = out;
+        }
+    }
+    const float lambda = p.mix != nullptr ? *p.mix : 0.0f;
+    for (int i = lane * 8; i < p.kv_heads * vp; i += kWave * 8) {              // (vdim is a multiple of eight: heads side by side)
+        u32x4_t v = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(p.v) + t * p.stride + i);
+        if (p.mix != nullptr) {
+            const u32x4_t f = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(p.v_first) + t * p.v_first_stride + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = pack_bf16((1.0f - lambda) * bf16_lo(v[e]) + lambda * bf16_lo(f[e]), (1.0f - lambda) * bf16_hi(v[e]) + lambda * bf16_hi(f[e]));
+        }
+        *reinterpret_cast<u32x4_t*>(cached + p.kv_heads * (L * 8) + i) = v;
+    }
+}
+
+// Heads of 64, 128 or 256 elements from 16-byte boundaries, turned in whole lanes; from kPrepareRows tokens on.
+constexpr int64_t kPrepareRows = 256;
+bool prepare_rows(const AttnProblem& p, int64_t T) {
+    auto aligned = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };
+    return p.dtype == EM_DTYPE_BF16 && T >= kPrepareRows && (p.dim == 64 || p.dim == 128 || p.dim == 256) && p.vdim % 8 == 0 && p.rot % 8 == 0 &&
+           p.stride % 8 == 0 && aligned(p.q) && aligned(p.k) && aligned(p.v) &&
+           (p.mix == nullptr || (p.v_first_stride % 8 == 0 && aligned(p.v_first)));
+}
+
 // Columns col0 + l16 of two groups of four rows of an LDS matrix, as one operand fragment.
 template <typename Elem>
 __device__ __forceinline__ typename Mma<Elem>::frag load_columns(const typename Elem::storage* m, int pitch, int row_lo, int row_hi,
@@ -729,6 +814,13 @@ int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int
 }
 
 int launch_attn_prepare(const AttnProblem& p, int64_t T, hipStream_t s) {
+    if (prepare_rows(p, T)) {
+        const dim3 rows(static_cast<unsigned>(ceil_div(T, 4)));
+        if (p.dim == 64) launch(attn_prepare_rows_kernel<8>, rows, dim3(256), 0, s, p, T);
+        else if (p.dim == 128) launch(attn_prepare_rows_kernel<16>, rows, dim3(256), 0, s, p, T);
+        else launch(attn_prepare_rows_kernel<32>, rows, dim3(256), 0, s, p, T);
+        return launch_status();
+    }
     const dim3 grid(static_cast<unsigned>(T), T <= 256 ? static_cast<unsigned>(ceil_div(p.heads + p.kv_heads, 4)) : 1u);
     const size_t lds = sizeof(float) * (p.rot > 0 ? p.rot : 1);
     const size_t two = 2 * (p.dtype == EM_DTYPE_BF16 ? 2 : 4);

@@ -58,6 +58,60 @@ __global__ __launch_bounds__(256) void latent_prepare_kernel(LatentProblem p) {
     }
 }
 
+// The same for the rows of a prompt, bf16: a wave per token, eight elements of the latent to a lane, and of a head's rotated part the
+// pieces of both halves that belong together.  Bound: the rows' bytes (8192 tokens, rank 512 + 64, 16 heads, 52 MB: 30 -> 16 us).
+__global__ __launch_bounds__(256) void latent_prepare_rows_kernel(LatentProblem p, int64_t T) {
+    __shared__ __attribute__((aligned(16))) float turns[4][2][64];             // cosines and sines of a token's pairs
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = p.rot / 2, c = lane * 8;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+    if (t >= T) return;                                                        // (waves share nothing)
+    const uint16_t* down = static_cast<const uint16_t*>(p.down) + t * p.down_stride;
+    uint16_t* cached = static_cast<uint16_t*>(p.cache) + static_cast<int64_t>(p.cache_rows[t]) * latent_row_elems(p.rank, p.rot);
+    uint16_t* q = static_cast<uint16_t*>(p.q) + t * p.q_stride;
+    const u32x4_t zero = {0, 0, 0, 0};
+    const u32x4_t latent = c < p.rank ? *reinterpret_cast<const u32x4_t*>(down + c) : zero;
+    const float pos = static_cast<float>(p.positions[t]);
+    for (int i = lane; i < half; i += kWave) sincosf(pos * p.inv_freq[i], &turns[wave][1][i], &turns[wave][0][i]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum = fmaf(bf16_lo(latent[i]), bf16_lo(latent[i]), fmaf(bf16_hi(latent[i]), bf16_hi(latent[i]), sum));
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    const float rms = sqrtf(sum / static_cast<float>(p.rank) + p.eps);
+    if (c < p.rank) {
+        u32x4_t out;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = pack_bf16(bf16_lo(latent[i]) / rms * p.latent_w[c + 2 * i], bf16_hi(latent[i]) / rms * p.latent_w[c + 2 * i + 1]);
+        *reinterpret_cast<u32x4_t*>(cached + c) = out;
+    }
+    // the key's rotated part (unit 0), then the heads': a lane takes eight elements of either half
+    const int lanes = half / 8;
+    for (int i = lane; i < (p.heads + 1) * lanes; i += kWave) {
+        const int unit = i / lanes, at = (i - unit * lanes) * 8;
+        const uint16_t* src = unit == 0 ? down + p.rank : q + (unit - 1) * (p.dim + p.rot) + p.dim;
+        uint16_t* dst = unit == 0 ? cached + p.rank : q + (unit - 1) * (p.dim + p.rot) + p.dim;
+        const u32x4_t a = *reinterpret_cast<const u32x4_t*>(src + at), b = *reinterpret_cast<const u32x4_t*>(src + half + at);
+        u32x4_t x, y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float c0 = turns[wave][0][at + 2 * e], c1 = turns[wave][0][at + 2 * e + 1], s0 = turns[wave][1][at + 2 * e], s1 = turns[wave][1][at + 2 * e + 1];
+            x[e] = pack_bf16(bf16_lo(a[e]) * c0 - bf16_lo(b[e]) * s0, bf16_hi(a[e]) * c1 - bf16_hi(b[e]) * s1);
+            y[e] = pack_bf16(bf16_lo(b[e]) * c0 + bf16_lo(a[e]) * s0, bf16_hi(b[e]) * c1 + bf16_hi(a[e]) * s1);
+        }
+        *reinterpret_cast<u32x4_t*>(dst + at) = x;
+        *reinterpret_cast<u32x4_t*>(dst + half + at) = y;
+    }
+}
+
+// Whole lanes from 16-byte boundaries; from kPrepareRows tokens on.
+constexpr int64_t kPrepareRows = 256;
+bool prepare_rows(const LatentProblem& p, int64_t T) {
+    auto aligned = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };
+    return p.dtype == EM_DTYPE_BF16 && T >= kPrepareRows && p.rank % 8 == 0 && p.rank <= 512 && p.rot % 16 == 0 && p.rot <= 128 && p.dim % 8 == 0 &&
+           p.q_stride % 8 == 0 && p.down_stride % 8 == 0 && aligned(p.q) && aligned(p.down) && aligned(p.cache);
+}
+
 // ---- per-head product  out[t, h, n] = sum_k a[t, h, k] b[h][n][k],  b's rows padded with zeros to 32 elements ----
 // A wave makes MT * 16 rows by 64 columns.  KSPLIT: the workgroup's four waves make the same tile, each from a quarter of
 // the k steps, and add up in LDS (few tiles of long rows); else they stand side by side along the columns.
@@ -748,6 +802,10 @@ bool latent_waves(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64
 }
 
 int launch_latent_prepare(const LatentProblem& p, int64_t T, hipStream_t s) {
+    if (prepare_rows(p, T)) {
+        launch(latent_prepare_rows_kernel, dim3(static_cast<unsigned>(ceil_div(T, 4))), dim3(256), 0, s, p, T);
+        return launch_status();
+    }
     const dim3 grid(static_cast<unsigned>(T));
     const size_t lds = sizeof(float) * (p.rot > 0 ? p.rot : 1);
     if (p.dtype == EM_DTYPE_BF16) launch((latent_prepare_kernel<BF16Elem>), grid, dim3(256), lds, s, p);
