@@ -36,8 +36,9 @@ constexpr int64_t kStreamW2MaxT = 8;
 //     128-row kernel stays: it cuts the rest of a round into narrower tiles, a round of half the length (8x7B w13
 //     T=128 / 256: 291 / 293 us against 308 / 309), up to the batch sizes where most experts still fit one of its
 //     tiles: 352 tokens for the w13 GEMM (with even routing it would stay ahead up to 470 tokens, 318 against 334 us
-//     at 448; with the Zipf bias the 256-row tiles win from 200 tokens, 313 against 359 us at 224: the earlier switch
-//     is kept), 448 for the w2 GEMM (8x22B T=352: 270 against 299 us).
+//     at 448; with the Zipf bias the 256-row tiles won from 200 tokens, 313 against 359 us at 224, before uneven
+//     experts' tiles were dealt to all XCDs, which took 20 us off here and 55 at 333: the earlier switch is kept),
+//     448 for the w2 GEMM (8x22B T=352: 270 against 299 us).
 // 64-row tiles are as fast as 128-row tiles with even routing from 65 to 192 tokens and a fifth slower with the Zipf
 // bias (8x7B layer, T=128: 0.451 / 0.451 ms even, 0.597 / 0.491 ms uneven): the large-batch path does not use them.
 constexpr int kCus = 256;  // of the GPU this library is tuned for

@@ -48,7 +48,8 @@ template <int MI, int NT> struct Geo {
     static constexpr int kRF = 2 * MI;                           // 16-row fragments per wave
     static constexpr int kCF = NT / 64;                          // 16-column fragments per wave
 };
-constexpr int kGroupM = 4;
+constexpr int kGroupM = 4;      // row tiles of a group; with uneven experts at most kMostGroupM, in equal groups
+constexpr int kMostGroupM = 5;
 constexpr int kXcds = 8;
 constexpr int kRowUnit = 16;  // rows of an MFMA fragment: sorted blocks are multiples of it
 
@@ -79,32 +80,55 @@ __device__ __forceinline__ void tile_body(const MoeProblem& p, const int32_t* __
                   kCopiesA = G::kCopiesA, kStages = G::kStages, kRF = G::kRF, kCF = G::kCF;
     static_assert(kStages >= 3, "ring depth");
 
-    int mtiles = 0;
-    for (int e = 0; e < p.E; ++e) mtiles += (seg_begin[e + 1] - seg_begin[e] + kTM - 1) / kTM;
-    const int total = mtiles * ntiles_n;
-    const int per_xcd = (total + kXcds - 1) / kXcds;
+    // one expert per lane: its rows, its row tiles and those up to its last (no chain of loads, one expert after the other)
+    const int ex = threadIdx.x & 63, seg = ex < p.E ? seg_begin[ex] : 0, rows = ex < p.E ? seg_begin[ex + 1] - seg : 0;
+    const int tiles = (rows + kTM - 1) / kTM;
+    int upto = tiles, most = rows;
+    for (int off = 1; off < p.E; off *= 2) {
+        const int before = __shfl_up(upto, off), other = __shfl_xor(most, off);
+        upto += ex >= off ? before : 0;
+        most = max(most, other);
+    }
+    const int mtiles = __builtin_amdgcn_readlane(upto, p.E - 1), all = seg_begin[p.E];
     const int xcd = block % kXcds;
     const int local = block / kXcds;
-    const int logical = xcd * per_xcd + local;
+    // Each XCD has a range of the tiles, in groups of four row tiles whose token rows its L2 holds.  With the largest expert half
+    // as large again as the average, such a range may be a few experts' row tiles, with little to stream, and another more than
+    // its share of the weights: then column tiles that divide evenly are dealt to the XCDs, each with all row tiles.
+    const bool even = ntiles_n % kXcds == 0 && __builtin_amdgcn_readfirstlane(most) * 2 * p.E > all * 3;
+    const int groups = (mtiles + kMostGroupM - 1) / kMostGroupM, group_m = even ? (mtiles + groups - 1) / groups : kGroupM;
+    if (even && mtiles > __popcll(__ballot(tiles > 0)) + 1) {
+        // Several experts' second tiles: the experts go to the groups in turn, the largest first, so that each group streams as
+        // many experts' weights.  (Even experts, and one with a second tile, are faster in their order.  8x7B layer, Zipf bias, us
+        // as a range per XCD / dealt / and by size: T = 128 485 / 474 / 483, 160 493 / 478 / 493, 256 556 / 530 / 543;
+        // 288 570 / 557 / 553, 333 652 / 613 / 597, 352 666 / 624 / 603.  Even routing, T = 333: 465, dealt 475.)
+        int rank = 0;
+        for (int e = 0; e < p.E; ++e) {
+            const int other = __builtin_amdgcn_readlane(rows, e);
+            rank += other > rows || (other == rows && e < ex);
+        }
+        const int place = ex < p.E ? rank % groups * p.E + rank / groups : p.E * p.E;
+        upto = 0;
+        for (int e = 0; e < p.E; ++e) upto += __builtin_amdgcn_readlane(place, e) <= place ? __builtin_amdgcn_readlane(tiles, e) : 0;
+    }
+    const int ntn = even ? ntiles_n / kXcds : ntiles_n;
+    const int total = mtiles * ntn;
+    const int per_xcd = even ? total : (total + kXcds - 1) / kXcds;
+    const int logical = even ? local : xcd * per_xcd + local;
     if (local >= per_xcd || logical >= total) return;
-    const int group_sz = kGroupM * ntiles_n;
+    const int group_sz = group_m * ntn;
     const int group = logical / group_sz;
     const int in_group = logical - group * group_sz;
-    const int rows_in_group = (mtiles - group * kGroupM < kGroupM) ? mtiles - group * kGroupM : kGroupM;
-    const int nt = in_group / rows_in_group;
-    int mt = group * kGroupM + in_group % rows_in_group;
-    int expert = 0;
-    for (; expert < p.E - 1; ++expert) {
-        const int t = (seg_begin[expert + 1] - seg_begin[expert] + kTM - 1) / kTM;
-        if (mt < t) break;
-        mt -= t;
-    }
+    const int rows_in_group = (mtiles - group * group_m < group_m) ? mtiles - group * group_m : group_m;
+    const int nt = (even ? xcd * ntn : 0) + in_group / rows_in_group;
+    int mt = group * group_m + in_group % rows_in_group;
+    const int expert = __builtin_ctzll(__ballot(upto > mt && upto - tiles <= mt));
     // the expert's 16-row fragments are dealt evenly to its tiles
-    const int e_rows = seg_begin[expert + 1] - seg_begin[expert];
-    const int e_tiles = (e_rows + kTM - 1) / kTM;
-    const int e_frags = e_rows / kRowUnit;
+    const int e_tiles = __builtin_amdgcn_readlane(tiles, expert), e_begin = __builtin_amdgcn_readlane(seg, expert);
+    mt -= __builtin_amdgcn_readlane(upto, expert) - e_tiles;
+    const int e_frags = __builtin_amdgcn_readlane(rows, expert) / kRowUnit;
     const int frag_base = e_frags / e_tiles, frag_rem = e_frags % e_tiles;
-    const int64_t m0 = seg_begin[expert] + static_cast<int64_t>(mt * frag_base + (mt < frag_rem ? mt : frag_rem)) * kRowUnit;
+    const int64_t m0 = e_begin + static_cast<int64_t>(mt * frag_base + (mt < frag_rem ? mt : frag_rem)) * kRowUnit;
     const int valid = (frag_base + (mt < frag_rem ? 1 : 0)) * kRowUnit;  // multiple of 16, at most kTM
 
     const int tid = threadIdx.x;
