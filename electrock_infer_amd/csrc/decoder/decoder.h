@@ -11,6 +11,13 @@ __device__ __forceinline__ float gelu_tanh(float z) {
     return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
 
+// the sum over the 16 lanes that share lane / 16, in all of them (rotations inside the vector unit, nothing goes through LDS)
+template <int ROTATE>
+__device__ __forceinline__ float add_rotated(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + ROTATE, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_sum(float v) { return add_rotated<1>(add_rotated<2>(add_rotated<4>(add_rotated<8>(v)))); }
+
 // Lets a kernel take `bytes` of dynamic LDS (one CU has 160 KB); 0, or the runtime's error.
 constexpr size_t kLdsPerCu = 160 * 1024;
 inline int allow_lds(const void* kernel, size_t bytes) {

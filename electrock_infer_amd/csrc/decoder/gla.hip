@@ -8,7 +8,10 @@
 //     S    <- exp(tot) S + sum_s (k_s exp(tot - bl_s)) v_s^T
 // which are float32 MFMAs: a wave keeps the state's 16 columns of one v tile in registers, in the layout in which an
 // MFMA leaves its result; the same registers, as they are, are the second operand of the float32 16x16x4 MFMA.  One
-// workgroup is one (chunk, head), one wave a v tile.  Everything that reaches the state is float32: the operands are
+// workgroup is one (chunk, head), one wave a v tile.  Bound: instructions and the chain through a block (its matrix units are a third
+// busy), so a block loaded ahead has two barriers: its operands lie in one of two places, and the norm of its outputs, which needs all waves' sums
+// of squares, is finished in the next one (us for 8 x 1024 tokens, 16 heads of 64 x 128, before and now: first pass 43 and 37, output
+// pass 102 and 90; loads without branches are half of it).  Everything that reaches the state is float32: the operands are
 // products of the bf16 projections with float32 decays, and no exponent is positive except in the block's own 16 x 16
 // scores, where exp(-bl_s) is used as a factor only while the whole block decays by less than 2^-kFactorLimit.  (The
 // logarithms are kept to base 2.)
@@ -110,22 +113,30 @@ struct BlockRegs {
     uint16_t v[4], g[4];
 };
 
-// PAIRS > 0 (bf16, even dim, at most PAIRS * 2 * threads channel values per block, at most 512 threads): the next
-// block's operands are in flight while this one is computed.  PAIRS == 0: any size, element by element.
+// LDS of the chunk kernels: waves that the row sums have room for, blocks whose operands lie side by side, parts of the scores (with
+// PAIRS == 0 as few as there are: there the LDS decides how many workgroups a CU takes).
+constexpr int chunk_most_waves(int pairs) { return pairs > 0 ? 8 : 16; }
+constexpr int chunk_halves(int pairs) { return pairs > 0 ? 2 : 1; }
+__host__ __device__ constexpr int chunk_score_parts(int pairs, int ndt, int waves) { return pairs > 0 && ndt > waves ? ndt : waves; }
+
+// PAIRS > 0 (bf16, even dim, at most PAIRS * 2 * threads channel values per block, at most 512 threads, rows near enough for 32-bit
+// offsets inside a block): the next block's operands are in flight while this one is computed.  PAIRS == 0: any size, element by element.
 template <typename Elem, int NDT, bool OUTPUT, int PAIRS>
 __global__ __launch_bounds__(PAIRS > 0 ? 512 : 1024, PAIRS > 0 && NDT > 4 ? 2 : 4) void gla_chunk_kernel(GlaArgs p) {
     typedef typename Elem::storage S;
     constexpr int D = NDT * 16;
     constexpr int DP = D + 4;
-    const int waves = blockDim.x / kWave;
+    constexpr int kMostWaves = chunk_most_waves(PAIRS), kOperands = 2 * kBlock * DP + D * kPitchA + D;
+    const int waves = blockDim.x / kWave, slots = chunk_score_parts(PAIRS, NDT, waves);
+    // (PAIRS > 0) the operands of two blocks: one is made while slower waves read the other
     extern __shared__ float lds[];
-    float* Qp = lds;                                  // [16][DP]  q exp(bl)
-    float* Kn = Qp + kBlock * DP;                     // [16][DP]  k exp(-bl)
-    float* Kt = Kn + kBlock * DP;                     // [D][20]   k exp(tot - bl), transposed
-    float* Et = Kt + D * kPitchA;                     // [D]       exp(tot)
-    float* Ap = Et + D;                               // [waves][16][20] partial scores
-    float* Rs = Ap + waves * kBlock * kPitchA;        // [waves][16] partial row sums
-    float* Bl = Rs + waves * kBlock;                  // [16][DP]  bl, for blocks with a large decay
+    float* Qp0 = lds;                                 // [16][DP]  q exp(bl)
+    float* Kn0 = Qp0 + kBlock * DP;                   // [16][DP]  k exp(-bl)
+    float* Kt0 = Kn0 + kBlock * DP;                   // [D][20]   k exp(tot - bl), transposed
+    float* Et0 = Kt0 + D * kPitchA;                   // [D]       exp(tot)
+    float* Ap = lds + chunk_halves(PAIRS) * kOperands;  // [slots][16][20] partial scores
+    float* Rs = Ap + slots * kBlock * kPitchA;        // [kMostWaves][16] partial row sums
+    float* Bl = Rs + kMostWaves * kBlock;             // [16][DP]  bl, for blocks with a large decay
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, lq = lane >> 4;
@@ -159,37 +170,64 @@ __global__ __launch_bounds__(PAIRS > 0 ? 512 : 1024, PAIRS > 0 && NDT > 4 ? 2 : 
         for (int d = tid; d < dim; d += blockDim.x) Bl[d] = 0.0f;  // here: the chunk's decay so far
 
     BlockRegs<PAIRS ? PAIRS : 1> regs;
+    // (every lane loads, from the last row and channel where there is none, and a select at the use puts the zero: no branches, and
+    // addresses that are a uniform base and a lane's 32-bit offset)
+    const int stride = static_cast<int>(p.stride);
     auto fetch = [&](int first) {
         const int n = min(kBlock, ch.z - first);
         const int64_t row0 = static_cast<int64_t>(ch.y) + first;
+        const S *q0 = qg + row0 * p.stride, *k0 = kg + row0 * p.stride, *v0 = vg + row0 * p.stride, *g0 = gg + row0 * p.stride;
+        const float* b0 = p.bl + row0 * C + h * dim;
 #pragma unroll
         for (int i = 0; i < PAIRS; ++i) {
             const int e = (tid + i * static_cast<int>(blockDim.x)) * 2, t = e / D, d = e - t * D;
-            regs.q[i] = regs.k[i] = 0;
-            regs.b[i] = regs.tot[i] = f32x2_t{0.0f, 0.0f};
-            if (t < kBlock && d < dim) {
-                regs.tot[i] = *reinterpret_cast<const f32x2_t*>(p.bl + (row0 + n - 1) * C + h * dim + d);
-                regs.b[i] = regs.tot[i];
-                if (t < n) {
-                    regs.b[i] = *reinterpret_cast<const f32x2_t*>(p.bl + (row0 + t) * C + h * dim + d);
-                    regs.k[i] = *reinterpret_cast<const uint32_t*>(kg + (row0 + t) * p.stride + d);
-                    if (OUTPUT) regs.q[i] = *reinterpret_cast<const uint32_t*>(qg + (row0 + t) * p.stride + d);
-                }
-            }
+            const int tc = min(t, n - 1), dc = min(d, dim - 2);
+            regs.tot[i] = *reinterpret_cast<const f32x2_t*>(b0 + ((n - 1) * C + dc));
+            regs.b[i] = *reinterpret_cast<const f32x2_t*>(b0 + (tc * C + dc));
+            regs.k[i] = *reinterpret_cast<const uint32_t*>(k0 + (tc * stride + dc));
+            if (OUTPUT) regs.q[i] = *reinterpret_cast<const uint32_t*>(q0 + (tc * stride + dc));
+        }
+        const int vcc = min(vc, vdim - 1);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = lq * 4 + r, at = min(t, n - 1) * stride + vcc;
+            regs.v[r] = static_cast<uint16_t>(v0[at]);
+            if (OUTPUT) regs.g[r] = static_cast<uint16_t>(g0[at]);
+        }
+    };
+    // a block's results wait for the row sums of the other waves until the next block's first barrier
+    f32x4_t held = {0.0f, 0.0f, 0.0f, 0.0f};
+    float held_gate[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int out_stride = p.heads * vdim;
+    auto finish = [&](int first) {
+        const int n = min(kBlock, ch.z - first);
+        S* out0 = static_cast<S*>(p.out) + (static_cast<int64_t>(ch.y) + first) * out_stride + h * vdim;
+        f32x4_t ss = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w0 = 0; w0 < kMostWaves; w0 += 4) {
+            f32x4_t part[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) part[w] = *reinterpret_cast<const f32x4_t*>(Rs + (w0 + w) * kBlock + lq * 4);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) ss += part[w];
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int t = lq * 4 + r;
-            const bool ok = v_ok && t < n;
-            regs.v[r] = ok ? static_cast<uint16_t>(vg[(row0 + t) * p.stride + vc]) : 0;
-            if (OUTPUT) regs.g[r] = ok ? static_cast<uint16_t>(gg[(row0 + t) * p.stride + vc]) : 0;
+            const float y = held[r] * __builtin_amdgcn_rsqf(ss[r] * inv_vdim + p.eps) * nw;
+            if (v_ok && t < n) out0[t * out_stride + vc] = Elem::store(y * silu_fast(held_gate[r]));
         }
     };
-    if (PAIRS > 0) fetch(0);
+    if (OUTPUT) {                                     // (waves and channel tiles that do not exist add nothing)
+        for (int i = tid; i < slots * kBlock * kPitchA; i += blockDim.x) Ap[i] = 0.0f;
+        for (int i = tid; i < kMostWaves * kBlock; i += blockDim.x) Rs[i] = 0.0f;
+    }
+    if (PAIRS > 0 && ch.z > 0) fetch(0);
 
     for (int first = 0; first < ch.z; first += kBlock) {
-        const int n = min(kBlock, ch.z - first);
+        const int n = min(kBlock, ch.z - first), half = PAIRS > 0 ? (first / kBlock & 1) * kOperands : 0;
         const int64_t row0 = static_cast<int64_t>(ch.y) + first;
+        float *Qp = Qp0 + half, *Kn = Kn0 + half, *Kt = Kt0 + half, *Et = Et0 + half;
         // ---- operands of the block ----
         bool factor_ok = true;
         auto place = [&](int t, int d, float q, float k, float b, float tot) {
@@ -207,13 +245,16 @@ __global__ __launch_bounds__(PAIRS > 0 ? 512 : 1024, PAIRS > 0 && NDT > 4 ? 2 : 
             for (int i = 0; i < PAIRS; ++i) {
                 const int e = (tid + i * static_cast<int>(blockDim.x)) * 2, t = e / D, d = e - t * D;
                 if (t < kBlock) {
-                    place(t, d, bf16_lo(regs.q[i]) * p.q_scale, bf16_lo(regs.k[i]), regs.b[i][0], regs.tot[i][0]);
-                    place(t, d + 1, bf16_hi(regs.q[i]) * p.q_scale, bf16_hi(regs.k[i]), regs.b[i][1], regs.tot[i][1]);
+                    const bool in = d < dim;
+                    const uint32_t q = in && t < n ? regs.q[i] : 0, k = in && t < n ? regs.k[i] : 0;
+                    const float b_lo = in ? regs.b[i][0] : 0.0f, b_hi = in ? regs.b[i][1] : 0.0f, tot_lo = in ? regs.tot[i][0] : 0.0f, tot_hi = in ? regs.tot[i][1] : 0.0f;
+                    place(t, d, bf16_lo(q) * p.q_scale, bf16_lo(k), b_lo, tot_lo);
+                    place(t, d + 1, bf16_hi(q) * p.q_scale, bf16_hi(k), b_hi, tot_hi);
                 }
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                v[r] = bf16_bits_to_f32(regs.v[r]);
+                v[r] = v_ok && lq * 4 + r < n ? bf16_bits_to_f32(regs.v[r]) : 0.0f;
                 gate[r] = OUTPUT ? bf16_bits_to_f32(regs.g[r]) : 0.0f;
             }
             if (first + kBlock < ch.z) fetch(first + kBlock);
@@ -242,6 +283,7 @@ __global__ __launch_bounds__(PAIRS > 0 ? 512 : 1024, PAIRS > 0 && NDT > 4 ? 2 : 
         }
         if (OUTPUT) {
             factor_ok = __syncthreads_and(factor_ok);
+            if (first > 0) finish(first - kBlock);
             // ---- scores of the block, shared out over the waves by channel tile ----
             f32x4_t a = {0.0f, 0.0f, 0.0f, 0.0f};
             if (factor_ok) {
@@ -291,9 +333,20 @@ __global__ __launch_bounds__(PAIRS > 0 ? 512 : 1024, PAIRS > 0 && NDT > 4 ? 2 : 
                 for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[r], st[dt][r], o, 0, 0, 0);
             }
             f32x4_t a4 = {0.0f, 0.0f, 0.0f, 0.0f};
-            const int parts = factor_ok ? min(waves, NDT) : waves;
-            for (int w = 0; w < parts; ++w)
-                a4 += *reinterpret_cast<const f32x4_t*>(Ap + (w * kBlock + l16) * kPitchA + lq * 4);
+            if (PAIRS > 0 && factor_ok) {
+                constexpr int kGroup = NDT < 4 ? NDT : 4;
+#pragma unroll
+                for (int w0 = 0; w0 < NDT; w0 += kGroup) {
+                    f32x4_t part[kGroup];
+#pragma unroll
+                    for (int w = 0; w < kGroup; ++w) part[w] = *reinterpret_cast<const f32x4_t*>(Ap + ((w0 + w) * kBlock + l16) * kPitchA + lq * 4);
+#pragma unroll
+                    for (int w = 0; w < kGroup; ++w) a4 += part[w];
+                }
+            } else {
+                const int parts = factor_ok ? min(waves, NDT) : waves;
+                for (int w = 0; w < parts; ++w) a4 += *reinterpret_cast<const f32x4_t*>(Ap + (w * kBlock + l16) * kPitchA + lq * 4);
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[r], v[r], o, 0, 0, 0);
         } else {
@@ -310,27 +363,20 @@ __global__ __launch_bounds__(PAIRS > 0 ? 512 : 1024, PAIRS > 0 && NDT > 4 ? 2 : 
         }
         if (OUTPUT) {
             // ---- norm over the head's vdim outputs, gate ----
+            f32x4_t ss;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float ss = o[r] * o[r];
-#pragma unroll
-                for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
-                if (l16 == 0) Rs[wave * kBlock + lq * 4 + r] = ss;
+                ss[r] = row_sum(o[r] * o[r]);
+                held_gate[r] = gate[r];
             }
+            if (l16 == 0) *reinterpret_cast<f32x4_t*>(Rs + wave * kBlock + lq * 4) = ss;
+            held = o;
         }
-        __syncthreads();  // the block's LDS operands are no longer needed
-        if (OUTPUT) {
-            f32x4_t ss = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int w = 0; w < waves; ++w) ss += *reinterpret_cast<const f32x4_t*>(Rs + w * kBlock + lq * 4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = lq * 4 + r;
-                if (v_ok && t < n) {
-                    const float y = o[r] * __builtin_amdgcn_rsqf(ss[r] * inv_vdim + p.eps) * nw;
-                    static_cast<S*>(p.out)[(row0 + t) * p.heads * vdim + h * vdim + vc] = Elem::store(y * silu_fast(gate[r]));
-                }
-            }
-        }
+        if (PAIRS == 0) __syncthreads();  // the block's LDS operands are no longer needed
+    }
+    if (OUTPUT) {
+        __syncthreads();
+        finish((ch.z - 1) / kBlock * kBlock);
     }
     if (!OUTPUT || p.chunk_states == nullptr) {
 #pragma unroll
@@ -461,16 +507,17 @@ __global__ __launch_bounds__(256) void gla_step_kernel(GlaArgs p, const typename
     }
 }
 
-size_t chunk_lds_bytes(int ndt, int waves) {
+size_t chunk_lds_bytes(int ndt, int waves, int pairs) {
     const int D = ndt * 16, DP = D + 4;
-    return sizeof(float) * (3 * kBlock * DP + D * kPitchA + D + waves * kBlock * kPitchA + waves * kBlock);
+    return sizeof(float) * (chunk_halves(pairs) * (2 * kBlock * DP + D * kPitchA + D) + chunk_score_parts(pairs, ndt, waves) * kBlock * kPitchA +
+                            chunk_most_waves(pairs) * kBlock + kBlock * DP);
 }
 
 template <typename Elem, int NDT, bool OUTPUT, int PAIRS>
 int launch_chunk_kernel(const GlaArgs& p, int n_chunks, hipStream_t s) {
     const int waves = static_cast<int>(ceil_div(p.vdim, 16));
     const dim3 grid(static_cast<unsigned>(n_chunks), static_cast<unsigned>(p.heads)), block(static_cast<unsigned>(waves * kWave));
-    const size_t lds = chunk_lds_bytes(NDT, waves);
+    const size_t lds = chunk_lds_bytes(NDT, waves, PAIRS);
     const int rc = allow_lds(reinterpret_cast<const void*>(gla_chunk_kernel<Elem, NDT, OUTPUT, PAIRS>), lds);
     if (rc != 0) return rc;
     launch((gla_chunk_kernel<Elem, NDT, OUTPUT, PAIRS>), grid, block, lds, s, p);
@@ -481,7 +528,7 @@ template <typename Elem, int NDT>
 int launch_chunks(const GlaArgs& p, int n_chunks, bool output, hipStream_t s) {
     const int threads = static_cast<int>(ceil_div(p.vdim, 16)) * kWave;
     const int pairs = static_cast<int>(ceil_div(kBlock * NDT * 16 / 2, threads));
-    if (std::is_same<Elem, BF16Elem>::value && p.dim % 2 == 0 && pairs <= 2 && threads <= 512) {
+    if (std::is_same<Elem, BF16Elem>::value && p.dim % 2 == 0 && pairs <= 2 && threads <= 512 && p.stride < (1 << 26)) {
         if (pairs == 1)
             return output ? launch_chunk_kernel<BF16Elem, NDT, true, 1>(p, n_chunks, s)
                           : launch_chunk_kernel<BF16Elem, NDT, false, 1>(p, n_chunks, s);

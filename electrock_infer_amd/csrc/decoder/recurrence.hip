@@ -312,12 +312,6 @@ __device__ __forceinline__ Split4 split4(f32x4_t v) {
     for (int i = 0; i < 3; ++i) s.part[i] = u32x2_t{lo.part[i], hi.part[i]};
     return s;
 }
-// the sum over the 16 lanes that share lane / 16, in all of them (rotations inside the vector unit, nothing goes through LDS)
-template <int ROTATE>
-__device__ __forceinline__ float add_rotated(float v) {
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + ROTATE, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float row_sum(float v) { return add_rotated<1>(add_rotated<2>(add_rotated<4>(add_rotated<8>(v)))); }
 // two packed halves side by side
 __device__ __forceinline__ bf16x8_t join(u32x2_t lo, u32x2_t hi) {
     const u32x4_t w = {lo[0], lo[1], hi[0], hi[1]};
