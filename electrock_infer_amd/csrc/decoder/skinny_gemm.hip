@@ -1,4 +1,5 @@
-// out[T, N] = act(x[T, K] w[N, K]^T) for a decode batch (T <= 64), bf16: a stream over the weights.
+// out[T, N] = act(x[T, K] w[N, K]^T) for a decode batch (T <= 64), bf16: a stream over the weights, for products whose rows or
+// ranges of K do not fill the chip with the tiled kernel's workgroups (decode_pays in tile_gemm.hip has the measured line).
 //
 // A workgroup owns 16 * NT columns of one of `splits` ranges of K; its waves share that range out, add their results up
 // in LDS, and one pass applies the activation and stores.  Bound: the weights' bytes, and for the small matrices of a
