@@ -6,23 +6,42 @@ from typing import Optional
 import torch
 import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from .. import _lib
 
 # (looked up once: these are asked in front of every product)
 _transforms_active, _tracing_state, _BF16 = torch._C._are_functorch_transforms_active, torch._C._get_tracing_state, torch.bfloat16
+_dispatch_modes, _function_modes, _autocast, _is_compiling = (torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack,
+                                                              torch._C._is_any_autocast_enabled, torch.compiler.is_compiling)
+_PLAIN_TYPES, _STRIDED = (torch.Tensor, torch.nn.Parameter), torch.strided
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+def _names_a_device() -> bool:
+    """Whether the function modes only name the default device, which changes no product."""
+    return all(type(m) is DeviceContext for m in _get_current_function_mode_stack())
+
+
+def _stays_bf16(device: torch.device) -> bool:
+    return not torch.is_autocast_enabled(device.type) or torch.get_autocast_dtype(device.type) is _BF16
+
+
 def _plain(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Operands that the product kernels read: what does not fit each other, is to be differentiated (backward or forward), mapped
-    or traced, or lies on two devices is the library's, to compute or to refuse."""
+    """Operands that the product kernels read: what does not fit each other, is to be differentiated (backward or forward), mapped,
+    compiled, traced, seen by a mode or cast, is of a type of its own, or lies on two devices is the library's, to compute or to refuse.
+    (Asked before any address: a tensor that only stands for one has none.)"""
+    if _is_compiling() or type(x) not in _PLAIN_TYPES or type(weight) not in _PLAIN_TYPES:
+        return False
     shape, rows = x.shape, weight.shape
     return (len(shape) == 2 and len(rows) == 2 and shape[1] == rows[1] and x.dtype is _BF16 and weight.dtype is _BF16 and
-            forward_ad._current_level < 0 and not _transforms_active() and _tracing_state() is None and x.device == weight.device and
+            x.layout is _STRIDED and weight.layout is _STRIDED and
+            forward_ad._current_level < 0 and not _transforms_active() and _tracing_state() is None and _dispatch_modes() == 0 and
+            (_function_modes() == 0 or _names_a_device()) and (not _autocast() or _stays_bf16(x.device)) and x.device == weight.device and
             not ((x.requires_grad or weight.requires_grad) and torch.is_grad_enabled()))
 
 
