@@ -15,7 +15,7 @@ from .. import _lib
 _transforms_active, _tracing_state, _BF16 = torch._C._are_functorch_transforms_active, torch._C._get_tracing_state, torch.bfloat16
 _dispatch_modes, _function_modes, _autocast, _is_compiling = (torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack,
                                                               torch._C._is_any_autocast_enabled, torch.compiler.is_compiling)
-_PLAIN_TYPES, _STRIDED = (torch.Tensor, torch.nn.Parameter), torch.strided
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -39,16 +39,13 @@ def _plain(x: torch.Tensor, weight: torch.Tensor) -> bool:
         return False
     shape, rows = x.shape, weight.shape
     return (len(shape) == 2 and len(rows) == 2 and shape[1] == rows[1] and x.dtype is _BF16 and weight.dtype is _BF16 and
-            x.layout is _STRIDED and weight.layout is _STRIDED and
             forward_ad._current_level < 0 and not _transforms_active() and _tracing_state() is None and _dispatch_modes() == 0 and
             (_function_modes() == 0 or _names_a_device()) and (not _autocast() or _stays_bf16(x.device)) and x.device == weight.device and
             not ((x.requires_grad or weight.requires_grad) and torch.is_grad_enabled()))
 
 
-def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Operands of the weight-streaming kernel: at most 64 rows, dense, from a 16-byte boundary."""
-    return (len(x.shape) == 2 and x.shape[0] <= 64 and _plain(x, weight) and x.is_contiguous() and weight.is_contiguous() and
-            (x.data_ptr() | weight.data_ptr()) % 16 == 0)
+def _dense(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0
 
 
 def _row_stride(t: torch.Tensor) -> int:
@@ -60,9 +57,19 @@ def _rows_apart(t: torch.Tensor) -> bool:
     return t.stride(1) == 1 and _row_stride(t) >= t.shape[1] and _row_stride(t) % 8 == 0 and t.data_ptr() % 16 == 0
 
 
+def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Operands of a decode batch, whichever kernel takes it: at most 64 rows, dense, from a 16-byte boundary."""
+    return _plain(x, weight) and x.shape[0] <= 64 and _dense(x, weight)
+
+
 def _tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Operands of the tiled kernel: any rows beyond a decode batch's, from 16-byte boundaries."""
-    return x.is_cuda and len(x.shape) == 2 and x.shape[0] > 64 and _plain(x, weight) and _rows_apart(x) and _rows_apart(weight)
+    """Operands of the tiled kernel beyond a decode batch: any rows from 16-byte boundaries."""
+    return x.is_cuda and _plain(x, weight) and x.shape[0] > 64 and _rows_apart(x) and _rows_apart(weight)
+
+
+def _taken(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Either of the two, asked once."""
+    return x.is_cuda and _plain(x, weight) and (_dense(x, weight) if x.shape[0] <= 64 else _rows_apart(x) and _rows_apart(weight))
 
 
 def _decode_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
@@ -82,7 +89,7 @@ def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits:
 
 def _own(x: torch.Tensor, weight: torch.Tensor, cols: int, act: int = 0, dtype: torch.dtype = _BF16) -> Optional[torch.Tensor]:
     """act(x @ weight^T) by the tiled or the weight-streaming kernel, where one of them takes it and is the faster way; else None."""
-    if not x.is_cuda or not (_fits(x, weight) or _tiles_fit(x, weight)):
+    if not _taken(x, weight):
         return None
     lib, (T, K) = _lib.load_decoder(), x.shape
     if lib.ed_tile_gemm_pays(T, cols, K, act) == 1:
@@ -133,7 +140,7 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 def linear_parts(x: torch.Tensor, weight: torch.Tensor, exact: bool = False) -> torch.Tensor:
     """x @ weight^T as ``residual_norm`` takes it: [T, N], or float32 partial sums [parts, T, N] of a decode batch or a short prompt.
     ``exact``: not rounded to the compute type on the way."""
-    if x.is_cuda and (_fits(x, weight) or _tiles_fit(x, weight)):
+    if _taken(x, weight):
         (T, K), N, lib = x.shape, weight.shape[0], _lib.load_decoder()
         splits = lib.ed_tile_gemm_splits(T, N, K)
         run = _tile_gemm if splits > 0 else _decode_gemm

@@ -99,9 +99,3 @@ def test_casts(operands, product):
         ops.linear(x, w)
     with pytest.raises(Called):
         ops.linear(x, torch.nn.Parameter(w, requires_grad=False))
-
-
-def test_sparse_weights(operands):
-    x, w = operands
-    sparse = w.float().to_sparse()
-    assert not ops._fits(x, sparse.to(BF16)) and not ops._tiles_fit(x, sparse.to(BF16))
