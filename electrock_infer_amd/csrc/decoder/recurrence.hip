@@ -339,6 +339,11 @@ __device__ __forceinline__ u32x2_t read_column(const uint16_t* piece) {
     return w;
 }
 
+// Whether a kernel multiplies by parts.  Not the 16 waves that a delta rule's values beyond 128 need for their norm: 128 registers a lane are
+// too few for the parts, and what they spill costs more than the products (us of a call, 8192 tokens, 16 heads: 128 x 256 1086 by parts,
+// 770 as they are; 64 x 256 663 / 423); unless the state alone spills (256 x 256 2392 / 2481).
+constexpr bool chunk_parts(int threads, int ndt) { return threads <= 512 || ndt > 8; }
+
 // One workgroup per (chunk, head, group of column tiles), one wave per tile of 16 state columns; waves without a tile help
 // with the loads.  Additive rule: a workgroup may take all columns of several heads that share keys (`group`), which then are split
 // once.  OUTPUT: from the state in front of the chunk; else from zero, with the identity's columns behind the state's for the
@@ -350,15 +355,17 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     constexpr int kPart = kBlock * DP, kTile = 3 * kPart;
     static_assert(NDT % 2 == 0, "a step of the products is two tiles");
     constexpr bool kRoom = THREADS <= 512 && NDT <= 8;                 // for operands ahead of their products in registers
+    constexpr bool kParts = chunk_parts(THREADS, NDT);
     const int waves = blockDim.x / kWave;
     extern __shared__ __attribute__((aligned(16))) uint16_t operands[];
     uint16_t* Ks = operands;                               // [2][3 parts][16][DP]
     // Q by its parts as well, [2][3 parts][16][DP], where the delta rule splits the state for K anyway; for the additive rule as it is,
     // [2][16][D + 4]: splitting the state costs more than the float32 products it saves
-    constexpr int kQPitch = D + 4;
+    constexpr int kPitch = D + 4, kFloatTile = kBlock * kPitch;
     uint16_t* Qs = Ks + 2 * kTile;
-    float* Qf = reinterpret_cast<float*>(Qs);
-    float* Rs = reinterpret_cast<float*>(Qs + 2 * kTile);              // [2][THREADS / 64][16] partial sums of squares (delta rule)
+    float* Kf = reinterpret_cast<float*>(operands);        // !kParts: both as they are, [2][16][D + 4]
+    float* Qf = kParts ? reinterpret_cast<float*>(Qs) : Kf + 2 * kFloatTile;
+    float* Rs = kParts ? reinterpret_cast<float*>(Qs + 2 * kTile) : Qf + 2 * kFloatTile;      // [2][THREADS / 64][16] partial sums of squares (delta rule)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
     const int4 ch = p.chunks[blockIdx.x];
@@ -381,8 +388,9 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
 
     // Column `col` of the state, rows lq * D / 4 + dt * 4 + r: two tiles are eight rows of a lane that lie side by side, as a
     // product over the state takes them, and the pieces of a key that one tile takes lie a quarter of its row apart (so that they,
-    // and 16 rows of either operand, fall on different banks).
+    // and 16 rows of either operand, fall on different banks).  !kParts: a tile's 16 rows side by side.
     f32x4_t st[NDT];
+    auto row_of = [&](int dt) { return kParts ? lq * (D / 4) + dt * 4 : dt * 16 + lq * 4; };
     const int64_t head_state = static_cast<int64_t>(dim) * vdim;
     float* slot = p.states + (static_cast<int64_t>(p.slots[ch.x]) * p.heads + h) * head_state;
     const bool chunked = p.chunk_states != nullptr;
@@ -392,7 +400,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int d = lq * (D / 4) + dt * 4 + r;
+            const int d = row_of(dt) + r;
             st[dt][r] = identity ? (d == col ? 1.0f : 0.0f) : (!from_zero && v_ok && d < dim) ? mine[static_cast<int64_t>(d) * vdim + col] : 0.0f;
         }
     const float norm_w = OUTPUT && DELTA && v_ok ? p.norm_w[col] : 0.0f;
@@ -434,7 +442,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     };
     auto fetch = [&](int b) {
         const int64_t row0 = static_cast<int64_t>(ch.y) + b * kBlock;
-        if (b == 0 || b == n_blocks - 1) place(min(kBlock, ch.z - b * kBlock) - 1);
+        if (!kParts || b == 0 || b == n_blocks - 1) place(min(kBlock, ch.z - b * kBlock) - 1);
         const float *k0 = kg + row0 * kq_pitch, *q0 = qg + row0 * kq_pitch;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
@@ -479,7 +487,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     for (int b = 0; b < n_blocks; ++b) {
         uint16_t* kb = Ks + (b & 1) * kTile;
         uint16_t* qb = Qs + (b & 1) * kTile;
-        float* qf = Qf + (b & 1) * kBlock * kQPitch;
+        float *kf = Kf + (b & 1) * kFloatTile, *qf = Qf + (b & 1) * kFloatTile;
         const int n = min(kBlock, ch.z - b * kBlock);
         auto keep = [&](uint16_t* to, f32x4_t v, bool exists) {
             const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -491,9 +499,12 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
         for (int i = 0; i < kPieces; ++i) {
             const int e = tid + i * static_cast<int>(blockDim.x), t = e / (D / 4), d = (e - t * (D / 4)) * 4;
             if (t < kBlock) {
-                keep(kb + t * DP + d, rk[i], t < n && d < dp);
-                if (DELTA && OUTPUT) keep(qb + t * DP + d, rq[i], t < n && d < dp);
-                if (!DELTA && OUTPUT) *reinterpret_cast<f32x4_t*>(qf + t * kQPitch + d) = d < dp ? rq[i] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                const bool exists = t < n && d < dp;
+                const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (kParts) keep(kb + t * DP + d, rk[i], exists);
+                else *reinterpret_cast<f32x4_t*>(kf + t * kPitch + d) = exists ? rk[i] : zero;
+                if (kParts && DELTA && OUTPUT) keep(qb + t * DP + d, rq[i], exists);
+                else if (OUTPUT) *reinterpret_cast<f32x4_t*>(qf + t * kPitch + d) = exists ? rq[i] : zero;
             }
         }
         f32x4_t scores_b, inverse_b, decay_b, rest_b, beta_b;
@@ -517,13 +528,11 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
             take();
         }
         if (b + 1 < n_blocks) fetch(b + 1);
-        if (!has_tile) {
-            if (OUTPUT && DELTA && b > 0) finish(b - 1);
-            continue;
-        }
+        if (OUTPUT && DELTA && b > 0 && (!kParts || !has_tile)) finish(b - 1);
+        if (!has_tile) continue;
         // Operands from LDS a step ahead of the products, K's and Q's sums in turn: every product of a sum waits for the one before.
         f32x4_t u, ks = {0.0f, 0.0f, 0.0f, 0.0f}, o = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (DELTA) {
+        if (DELTA && kParts) {
             constexpr int kTwo = kRoom && OUTPUT ? 1 : 0;
             Split8 ka[1 + kTwo], qa[1 + kTwo];
             auto rows = [&](int k) {
@@ -555,16 +564,24 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
                 }
             }
         }
-        if (!DELTA && OUTPUT) {
+        if (!kParts) {
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) {
-                const f32x4_t q4 = *reinterpret_cast<const f32x4_t*>(qf + l16 * kQPitch + lq * (D / 4) + dt * 4);
+                const f32x4_t k4 = *reinterpret_cast<const f32x4_t*>(kf + l16 * kPitch + row_of(dt));
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ks = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[r], st[dt][r], ks, 0, 0, 0);
+            }
+        }
+        if ((!DELTA || !kParts) && OUTPUT) {
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                const f32x4_t q4 = *reinterpret_cast<const f32x4_t*>(qf + l16 * kPitch + row_of(dt));
 #pragma unroll
                 for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[r], st[dt][r], o, 0, 0, 0);
                 if (kRoom && dt % 2 != 0) __builtin_amdgcn_sched_barrier(0);      // (all of them at once do not fit the registers)
             }
         }
-        if (OUTPUT && DELTA && b > 0) finish(b - 1);
+        if (kParts && OUTPUT && DELTA && b > 0) finish(b - 1);
         // the keys by column, for the update: on their way while u is made
         const uint16_t* kc = kb + (lq * 4 + (l16 >> 2)) * DP + (l16 & 3) * (D / 4);
         constexpr int kRing = !kRoom ? 1 : OUTPUT || DELTA ? 2 : 4;
@@ -600,6 +617,13 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
         const bf16x8_t u32 = join(us.part[2], us.part[1]), u21 = join(us.part[1], us.part[0]), u11 = join(us.part[0], us.part[0]);
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
+            if (!kParts) {
+                st[dt] *= whole;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    st[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[(lq * 4 + r) * kPitch + dt * 16 + l16], u[r], st[dt], 0, 0, 0);
+                continue;
+            }
             if (!kRoom) columns(dt);
             const bf16x8_t k12 = join(kt[dt % kRing][0], kt[dt % kRing][1]), k13 = join(kt[dt % kRing][0], kt[dt % kRing][2]);
             if (kRoom && dt + kRing < NDT) columns(dt + kRing);
@@ -639,7 +663,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int d = lq * (D / 4) + dt * 4 + r;
+                    const int d = row_of(dt) + r;
                     if (d < dp) m[d * dp + col] = st[dt][r];
                 }
         }
@@ -649,7 +673,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int d = lq * (D / 4) + dt * 4 + r;
+            const int d = row_of(dt) + r;
             if (v_ok && d < dim) mine[static_cast<int64_t>(d) * vdim + col] = st[dt][r];
         }
     if (!OUTPUT && !DELTA && tile == 0 && lane == 0) p.chunk_trans[static_cast<int64_t>(blockIdx.x) * p.heads + h] = log_sum;
@@ -907,7 +931,9 @@ int launch_conv(const RecurProblem& p, hipStream_t s) {
 
 template <typename Elem, int NDT, bool DELTA, bool OUTPUT, int THREADS>
 int launch_chunks(const RecurProblem& p, int tiles, int waves, int group, hipStream_t s) {
-    const size_t keys = sizeof(uint16_t) * 2 * 3 * kBlock * (NDT * 16 + 8), queries = DELTA ? keys : sizeof(float) * 2 * kBlock * (NDT * 16 + 4);
+    const size_t parts = sizeof(uint16_t) * 2 * 3 * kBlock * (NDT * 16 + 8), whole = sizeof(float) * 2 * kBlock * (NDT * 16 + 4);
+    constexpr bool kParts = chunk_parts(THREADS, NDT);
+    const size_t keys = kParts ? parts : whole, queries = kParts && DELTA ? parts : whole;
     const size_t lds = keys + (OUTPUT ? queries : 0) + (DELTA && OUTPUT ? sizeof(float) * 2 * THREADS / kWave * kBlock : 0);
     const int rc = allow_lds(reinterpret_cast<const void*>(recur_chunk_kernel<Elem, NDT, DELTA, OUTPUT, THREADS>), lds);
     if (rc != 0) return rc;

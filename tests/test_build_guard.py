@@ -72,3 +72,12 @@ def test_compiler_release_is_pinned(tmp_path, monkeypatch):
     monkeypatch.setenv("ELECTROCK_ALLOW_ANY_HIPCC", "1")
     assert "9.9.1" in _build.check_compiler(str(fake))
     assert _build.VALIDATED_HIP in _build.check_compiler(_build.hipcc_path())      # the image's own compiler
+
+
+def test_a_form_of_a_kernel_may_have_limits_of_its_own():
+    limits = {"gemm_tile_kernel:ELb0ELi0ELb1E": {"max_vgprs": 256, "min_vgprs": 200, "lds": 0, "scratch": 64}}
+    assert len(_build.check_kernel_resources(report(scratch=64, spill=16), limits)) == 1
+    with pytest.raises(RuntimeError, match="scratch 68"):
+        _build.check_kernel_resources(report(scratch=68, spill=17), limits)
+    with pytest.raises(RuntimeError, match="no resource report for any gemm_tile_kernel:ELi7E"):
+        _build.check_kernel_resources(report(), {"gemm_tile_kernel:ELi7E": limits.popitem()[1]})

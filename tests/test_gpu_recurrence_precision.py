@@ -9,9 +9,10 @@ from tests.test_gpu_nunivik_ops import EPS, F32, N, Feed, rand, recurrent, slots
 pytestmark = pytest.mark.gpu
 
 
-# one and two pieces of a key per thread, heads that share a workgroup (with waves left over), columns and rows that end inside a tile
+# one and two pieces of a key per thread, heads that share a workgroup (with waves left over), columns and rows that end inside a tile;
+# heads of more than eight column tiles, whose output pass has a workgroup of its own kind (of 9, 10 and 16 waves)
 @pytest.mark.parametrize("entry", [delta(4, 2, 128, 128, 4), delta(2, 2, 256, 64, 4), delta(2, 1, 70, 40, 4), mamba(8, 1, 128, 64, 4, 2), mamba(6, 2, 40, 24, 4),
-                                   mamba(2, 1, 200, 130, 4)],
+                                   mamba(2, 1, 200, 130, 4), delta(2, 1, 128, 256, 4), delta(2, 2, 40, 130, 4), delta(1, 1, 64, 160, 4), delta(1, 1, 256, 144, 4)],
                          ids=lambda e: e["type"] + "-" + "-".join(str(v) for v in e["mixer"].values()))
 @pytest.mark.parametrize("a_log", [-12.0, 1.0])
 def test_distance_from_64_bits(entry, a_log):
