@@ -57,10 +57,11 @@ GUARDED_KERNELS = {
 
 # The same for libelectrock_decoder.so (two waves share a SIMD); behind a colon: template arguments of some of a kernel's forms, and
 # "scratch": bytes a lane that they may have.  Recurrences: passes that run with four waves per SIMD (additive rule, first pass of the
-# delta rule), and the 16 waves of the delta rule's wide heads, whose 128 registers are short (more than this was a third slower).
+# delta rule; what they spill belongs to the second pass and lies outside of the blocks' loops), and the 16 waves of the delta rule's wide
+# heads, whose 128 registers are short (more than this was a third slower).
 GUARDED_DECODER_KERNELS = {
     "tile_gemm_kernel": {"max_vgprs": 256, "min_vgprs": 24, "lds": 0},
-    **{f"recur_chunk_kernel:ELi{n}ELb{delta}ELb{output}ELi512E": {"max_vgprs": 128, "min_vgprs": 24, "lds": 0}
+    **{f"recur_chunk_kernel:ELi{n}ELb{delta}ELb{output}ELi512E": {"max_vgprs": 128, "min_vgprs": 24, "lds": 256, "scratch": 128}
        for n in (2, 4, 8) for delta, output in ((0, 0), (0, 1), (1, 0))},
     **{f"recur_chunk_kernel:ELi{n}ELb1ELb1ELi1024E": {"max_vgprs": 128, "min_vgprs": 24, "lds": 0, "scratch": scratch}
        for n, scratch in ((2, 16), (4, 96), (8, 256))},

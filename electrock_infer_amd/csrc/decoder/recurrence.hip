@@ -282,7 +282,10 @@ __global__ __launch_bounds__(256) void recur_block_kernel(RecurProblem p, int he
 // bf16 values: 8 bits each, rounded to nearest, so that the first two leave a remainder of 2^-18 and all three one of 2^-27 at most.  Of
 // the nine products the six that reach 2^-24 are added up, in float32, the smallest first.  Against float64 this is no further off than
 // float32 products (1536 tokens, decays from 1 - 6e-6 to e^-2.7 a token: 7.7e-7 / 8.0e-7 where everything is kept, 5.2e-7 / 5.3e-7 where
-// it fades); six bf16 products take 96 cycles where eight float32 ones take 256.  (An infinite operand makes NaN, not infinity.)
+// it fades); six bf16 products take 96 cycles where eight float32 ones take 256.  The parts of an infinite value, or one beyond the largest
+// bf16, are no numbers, and a key, an update or a state with such parts leaves NaN in the state until the chunk ends (a query's are asked
+// for): such a chunk is computed once more, with float32 products.  No time without one (8192 tokens: 407 / 409 and 332 / 334 us a call).
+constexpr float kMostPart = 3.3895314e38f;            // the largest bf16
 //
 // What bounds the kernel now is instructions: a block is 60-80 matrix and 130-500 vector instructions per wave (splitting the state 180,
 // scaling it 32, a share of the keys 50), and the chain from the barrier through LDS, sums, u and update.  So operands are read from LDS
@@ -347,15 +350,14 @@ constexpr bool chunk_parts(int threads, int ndt) { return threads <= 512 || ndt 
 // One workgroup per (chunk, head, group of column tiles), one wave per tile of 16 state columns; waves without a tile help
 // with the loads.  Additive rule: a workgroup may take all columns of several heads that share keys (`group`), which then are split
 // once.  OUTPUT: from the state in front of the chunk; else from zero, with the identity's columns behind the state's for the
-// delta rule.
-template <typename Elem, int NDT, bool DELTA, bool OUTPUT, int THREADS>
-__global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void recur_chunk_kernel(RecurProblem p, int group) {
+// delta rule.  True, for the whole workgroup and without a state written, where the parts did not hold a value (`kParts`).
+template <typename Elem, int NDT, bool DELTA, bool OUTPUT, int THREADS, bool kParts>
+__device__ __forceinline__ bool chunk_pass(const RecurProblem& p, int group, int tid, dim3 block) {
     typedef typename Elem::storage S;
     constexpr int D = NDT * 16, DP = D + 8, kPieces = (NDT + 7) / 8;   // four-float pieces of a block's k (q) per thread
     constexpr int kPart = kBlock * DP, kTile = 3 * kPart;
     static_assert(NDT % 2 == 0, "a step of the products is two tiles");
     constexpr bool kRoom = THREADS <= 512 && NDT <= 8;                 // for operands ahead of their products in registers
-    constexpr bool kParts = chunk_parts(THREADS, NDT);
     const int waves = blockDim.x / kWave;
     extern __shared__ __attribute__((aligned(16))) uint16_t operands[];
     uint16_t* Ks = operands;                               // [2][3 parts][16][DP]
@@ -367,11 +369,11 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     float* Qf = kParts ? reinterpret_cast<float*>(Qs) : Kf + 2 * kFloatTile;
     float* Rs = kParts ? reinterpret_cast<float*>(Qs + 2 * kTile) : Qf + 2 * kFloatTile;      // [2][THREADS / 64][16] partial sums of squares (delta rule)
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
-    const int4 ch = p.chunks[blockIdx.x];
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
+    const int4 ch = p.chunks[block.x];
     const int dim = p.dim, vdim = p.vdim, dp = (dim + 15) / 16 * 16, v_tiles = (vdim + 15) / 16;
     const bool several = !DELTA && group > 1;
-    const int h = several ? blockIdx.y * group + min(wave / v_tiles, group - 1) : blockIdx.y, tile = several ? wave % v_tiles : blockIdx.z * waves + wave;
+    const int h = several ? static_cast<int>(block.y) * group + min(wave / v_tiles, group - 1) : static_cast<int>(block.y), tile = several ? wave % v_tiles : static_cast<int>(block.z) * waves + wave;
     const int g = h / (p.heads / p.kv_heads);
     const bool identity = !OUTPUT && DELTA && tile >= v_tiles;
     const bool has_tile = (several ? wave < group * v_tiles : tile < v_tiles) || (identity && tile < v_tiles + dp / 16);
@@ -384,7 +386,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     const S* gate = OUTPUT && DELTA ? static_cast<const S*>(p.gate) + h * vdim + tile * 16 : nullptr;
     const int n_blocks = (ch.z + kBlock - 1) / kBlock;
     const int64_t rec_pitch = static_cast<int64_t>(p.heads) * recur_record(DELTA);
-    const float* rec0 = p.blocks + (static_cast<int64_t>(blockIdx.x) * (p.chunk_tokens / kBlock) * p.heads + h) * recur_record(DELTA);
+    const float* rec0 = p.blocks + (static_cast<int64_t>(block.x) * (p.chunk_tokens / kBlock) * p.heads + h) * recur_record(DELTA);
 
     // Column `col` of the state, rows lq * D / 4 + dt * 4 + r: two tiles are eight rows of a lane that lie side by side, as a
     // product over the state takes them, and the pieces of a key that one tile takes lie a quarter of its row apart (so that they,
@@ -394,7 +396,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     const int64_t head_state = static_cast<int64_t>(dim) * vdim;
     float* slot = p.states + (static_cast<int64_t>(p.slots[ch.x]) * p.heads + h) * head_state;
     const bool chunked = p.chunk_states != nullptr;
-    float* mine = chunked ? p.chunk_states + (static_cast<int64_t>(blockIdx.x) * p.heads + h) * head_state : slot;
+    float* mine = chunked ? p.chunk_states + (static_cast<int64_t>(block.x) * p.heads + h) * head_state : slot;
     const bool from_zero = !OUTPUT || (!chunked && p.starts[ch.x] == 0);
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
@@ -411,7 +413,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     // them (what does not exist is made zero where it is used).
     // (The additive rule's output pass and the delta rule's first one ask for a block's record when they start on it: one set of registers instead of two is what lets
     // a CU have four waves per SIMD.)
-    constexpr bool kLate = OUTPUT != DELTA;
+    constexpr bool kAhead = kParts || THREADS > 512, kLate = OUTPUT != DELTA || !kAhead;     // (a second pass loads a block when it starts on it)
     f32x4_t rk[kPieces], rq[kPieces], scores, inverse, decay, rest, beta;
     float block_decay, block_log;
     S v[4] = {}, gt[4] = {};                          // (as stored: a conversion here would wait for the load)
@@ -482,13 +484,14 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
     };
     if (OUTPUT && DELTA)              // (waves that do not exist add nothing)
         for (int i = tid; i < 2 * THREADS / kWave * kBlock; i += static_cast<int>(blockDim.x)) Rs[i] = 0.0f;
-    float log_sum = 0.0f;
-    fetch(0);
+    float log_sum = 0.0f, largest_q = 0.0f;
+    if (kAhead) fetch(0);
     for (int b = 0; b < n_blocks; ++b) {
         uint16_t* kb = Ks + (b & 1) * kTile;
         uint16_t* qb = Qs + (b & 1) * kTile;
         float *kf = Kf + (b & 1) * kFloatTile, *qf = Qf + (b & 1) * kFloatTile;
         const int n = min(kBlock, ch.z - b * kBlock);
+        if (!kAhead) fetch(b);
         auto keep = [&](uint16_t* to, f32x4_t v, bool exists) {
             const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
             const Split4 s = split4(exists ? v : zero);
@@ -503,8 +506,11 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
                 const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
                 if (kParts) keep(kb + t * DP + d, rk[i], exists);
                 else *reinterpret_cast<f32x4_t*>(kf + t * kPitch + d) = exists ? rk[i] : zero;
-                if (kParts && DELTA && OUTPUT) keep(qb + t * DP + d, rq[i], exists);
-                else if (OUTPUT) *reinterpret_cast<f32x4_t*>(qf + t * kPitch + d) = exists ? rq[i] : zero;
+                if (kParts && DELTA && OUTPUT) {
+                    keep(qb + t * DP + d, rq[i], exists);
+                    largest_q = fmaxf(fmaxf(fmaxf(largest_q, fabsf(rq[i][0])), fmaxf(fabsf(rq[i][1]), fabsf(rq[i][2]))), fabsf(rq[i][3]));
+                }
+                if (OUTPUT && !(kParts && DELTA)) *reinterpret_cast<f32x4_t*>(qf + t * kPitch + d) = exists ? rq[i] : zero;
             }
         }
         f32x4_t scores_b, inverse_b, decay_b, rest_b, beta_b;
@@ -527,7 +533,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
             records(b);
             take();
         }
-        if (b + 1 < n_blocks) fetch(b + 1);
+        if (kAhead && b + 1 < n_blocks) fetch(b + 1);
         if (OUTPUT && DELTA && b > 0 && (!kParts || !has_tile)) finish(b - 1);
         if (!has_tile) continue;
         // Operands from LDS a step ahead of the products, K's and Q's sums in turn: every product of a sum waits for the one before.
@@ -655,9 +661,17 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
         __syncthreads();
         finish(n_blocks - 1);
     }
-    if (OUTPUT && chunked) return;
+    if (kParts) {
+        float sum = 0.0f;             // (NaN if a value is infinite or none)
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum = fmaf(st[dt][r], 0.0f, sum);
+        if (__syncthreads_or(sum != sum || largest_q > kMostPart)) return true;
+    }
+    if (OUTPUT && chunked) return false;
     if (identity) {
-        float* m = p.chunk_trans + (static_cast<int64_t>(blockIdx.x) * p.heads + h) * dp * dp;
+        float* m = p.chunk_trans + (static_cast<int64_t>(block.x) * p.heads + h) * dp * dp;
         if (has_tile) {
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
@@ -667,7 +681,7 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
                     if (d < dp) m[d * dp + col] = st[dt][r];
                 }
         }
-        return;
+        return false;
     }
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
@@ -676,7 +690,25 @@ __global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void
             const int d = row_of(dt) + r;
             if (v_ok && d < dim) mine[static_cast<int64_t>(d) * vdim + col] = st[dt][r];
         }
-    if (!OUTPUT && !DELTA && tile == 0 && lane == 0) p.chunk_trans[static_cast<int64_t>(blockIdx.x) * p.heads + h] = log_sum;
+    if (!OUTPUT && !DELTA && tile == 0 && lane == 0) p.chunk_trans[static_cast<int64_t>(block.x) * p.heads + h] = log_sum;
+    return false;
+}
+
+template <typename Elem, int NDT, bool DELTA, bool OUTPUT, int THREADS>
+__global__ __launch_bounds__(THREADS, (DELTA && OUTPUT) || NDT > 8 ? 2 : 4) void recur_chunk_kernel(RecurProblem p, int group) {
+    if constexpr (chunk_parts(THREADS, NDT)) {
+        if (!chunk_pass<Elem, NDT, DELTA, OUTPUT, THREADS, true>(p, group, threadIdx.x, blockIdx)) return;
+        // Again, as float32.  (Everything is read anew: what the passes shared would be kept in registers during the first.)
+        auto args = __builtin_amdgcn_kernarg_segment_ptr();
+        int tid = threadIdx.x;
+        dim3 block = blockIdx;
+        asm volatile("" : "+s"(args), "+v"(tid), "+s"(block.x), "+s"(block.y), "+s"(block.z));
+        RecurProblem again;
+        __builtin_memcpy(&again, (const void*)args, sizeof(again));
+        chunk_pass<Elem, NDT, DELTA, OUTPUT, THREADS, false>(again, group, tid, block);
+    } else {
+        chunk_pass<Elem, NDT, DELTA, OUTPUT, THREADS, false>(p, group, threadIdx.x, blockIdx);
+    }
 }
 
 // ---- prompts: contribution of every chunk -> state in front of it; the state behind the last chunk goes to the slot ----
