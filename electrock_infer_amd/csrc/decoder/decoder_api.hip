@@ -221,9 +221,7 @@ int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int s
 }
 
 int ed_tile_gemm_splits(int64_t T, int N, int K) {
-    if (!tile_gemm_pays(T, N, K, 0, true)) return 0;
-    const int splits = tile_gemm_splits(T, N, K);
-    return T <= 64 && splits == 1 ? 0 : splits;      // (a decode batch that is not split: as its whole results)
+    return tile_gemm_pays(T, N, K, 0, true) ? tile_gemm_splits(T, N, K) : 0;
 }
 
 int ed_tile_gemm_pays(int64_t T, int N, int K, int act) { return act >= 0 && act <= 2 && tile_gemm_pays(T, N, K, act, false) ? 1 : 0; }

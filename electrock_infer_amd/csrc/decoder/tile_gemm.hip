@@ -311,7 +311,10 @@ bool tile_gemm_pays(int64_t T, int N, int K, int act, bool parts) {
                    size <= (int64_t{1} << 25) ? 320 : size <= (int64_t{1} << 26) ? 224 : 96);
 }
 
-int tile_gemm_splits(int64_t T, int N, int K) { return plan(T, N, K, 0, true, 1, 8).splits; }
+// (33 to 64 tokens and rows that are about a CU's worth of tiles: two ranges, where the estimate sees no difference.  us with the norm that
+// adds them up, 64 tokens, one / two: 6144 x 1024 13.5 / 12.8, 8192 x 1024 14.8 / 14.6, 8192 x 2048 18.4 / 17.4; 33 tokens 12.8 / 11.6,
+// 14.0 / 13.1, 17.0 / 15.6; 10240 x 1024, 64 tokens 13.9 / 16.5)
+int tile_gemm_splits(int64_t T, int N, int K) { return plan(T, N, K, 0, true, T > 32 && T <= 64 && N <= 8192 ? 2 : 1, 8).splits; }
 
 int launch_tile_gemm(const TileGemm& g, hipStream_t s) {
     const int form = plan(g.T, g.N, g.K, g.act, g.f32, g.splits, g.splits).form;

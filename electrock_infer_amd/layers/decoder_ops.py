@@ -147,7 +147,7 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor, exact: bool = False) -> 
         splits = splits or lib.ed_decode_gemm_splits(T, N, K)
         if splits > 1:
             return run(x, weight, torch.empty(splits, T, N, dtype=torch.float32, device=x.device), splits, N, 0)
-        if splits == 1 and T > 64:
+        if splits == 1 and T > 64:                    # (a decode batch's whole results: whichever kernel is the fastest for those)
             return _tile_gemm(x, weight, torch.empty(T, N, dtype=torch.float32 if exact else x.dtype, device=x.device), 1, N, 0)
     return linear_f32(x, weight) if exact else linear(x, weight)
 

@@ -66,7 +66,8 @@ int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int s
 
 /* The same product and activations for any number of rows, x_stride and w_stride elements apart (multiples of 8; x, w, out from a
  * 16-byte boundary); float32 results without an activation.  ed_tile_gemm_pays: 1 if that is faster than the library's product and
- * the kernel of its activation; ed_tile_gemm_splits: ranges of K where the results may stay partial sums, 0 if another product is faster. */
+ * the kernel of its activation; ed_tile_gemm_splits: ranges of K where the results may stay partial sums, 1 if whole results are faster
+ * than any number of ranges (of a decode batch by the product that is fastest for those), 0 if another product is. */
 int ed_tile_gemm_splits(int64_t T, int N, int K);
 int ed_tile_gemm_pays(int64_t T, int N, int K, int act);
 int ed_tile_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out, int out_dtype, int splits, int64_t T, int N,

@@ -49,3 +49,26 @@ def test_host_tensors_and_gradients_are_the_librarys():
     x, w = torch.randn(100, 512).to(torch.bfloat16), torch.randn(1024, 512).to(torch.bfloat16)
     assert not ops._tiles_fit(x, w) and torch.equal(ops.linear(x, w), torch.nn.functional.linear(x, w))
     assert ops._plain(x, w) and not ops._plain(x.requires_grad_(), w)
+
+
+def test_partial_sums_are_the_tiled_kernels_or_whole(monkeypatch):
+    # us as two ranges of the weight-streaming kernel / of the tiled one, with the norm behind them, 64 tokens: 6144 x 1024 16.6 / 12.8,
+    # 8192 x 1024 18.5 / 14.6, 8192 x 2048 20.7 / 17.4
+    lib, calls = _lib.load_decoder(), []
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: True), raising=False)
+    monkeypatch.setattr(ops, "_tile_gemm", lambda x, w, out, splits, cols, act: calls.append(("tile", splits)) or out)
+    monkeypatch.setattr(ops, "_decode_gemm", lambda x, w, out, splits, cols, act: calls.append(("stream", splits)) or out)
+    for T, N, K, want in ((33, 6144, 1024, ("tile", 2)), (64, 6144, 1024, ("tile", 2)), (33, 8192, 1024, ("tile", 2)), (64, 8192, 1024, ("tile", 2)),
+                          (33, 8192, 2048, ("tile", 2)), (64, 8192, 2048, ("tile", 2)), (64, 5632, 1024, ("tile", 2)), (64, 12288, 2048, ("tile", 1)),
+                          (24, 8192, 2048, ("tile", 1)), (24, 6144, 1024, ("stream", 1)), (8, 2048, 2048, ("stream", lib.ed_decode_gemm_splits(8, 2048, 2048)))):
+        x, w = torch.zeros(T, K, dtype=torch.bfloat16), torch.zeros(N, K, dtype=torch.bfloat16)
+        for exact in (False, True):
+            out = ops.linear_parts(x, w, exact)
+            assert calls.pop() == want and not calls, (T, N, K)
+            assert out.shape[-2:] == (T, N) and out.dtype == (torch.float32 if exact or out.dim() == 3 else torch.bfloat16)
+        # 0 says that another product is the faster one, not that this one stays whole
+        if lib.ed_tile_gemm_splits(T, N, K) == 1:
+            assert lib.ed_decode_gemm_splits(T, N, K) == 1
+    # wherever the rule takes partial sums, the other kernel is not asked
+    for T, N, K in itertools.product((17, 33, 64), range(512, 16384, 512), (1024, 1088, 2048, 6144)):
+        assert lib.ed_tile_gemm_splits(T, N, K) >= 1, (T, N, K)
