@@ -291,6 +291,23 @@ bool decode_pays(int64_t T, int64_t rows, int K, int act, bool parts) {
     if (act == 2) return (rows >= 10240 && K >= 1024) || (rows >= 8192 && T > 8 && K > 1024) || (rows >= 6144 && T > 32);
     return rows > 8192 || (rows >= 6144 && (T > 32 || (K > 1024 && (T > 4 || rows >= 8192))));
 }
+// Whole results of more tokens than a short prompt's, for `rows` weight rows (x and weights as the kernels before leave them; this /
+// library's time over 12 widths of 72 to 1536 rows, 1030 to 16384 tokens):
+//   * K up to 512: 0.5 to 1.0 up to 8192 tokens (T = 16384 1.05 to 1.36, 1536 rows and 3072 tokens 1.10 to 1.19); where the rows are the
+//     many, up to 1536 x 2048 0.77 to 0.98 (1280 x 4096 1.13, x 8192 1.38);
+//   * K = 1024: 0.7 to 0.9 for a million results or up to 2048 tokens (512 rows, 4096 tokens 1.29; 1024 rows 1.19);
+//   * K = 1536, 2048: 0.6 to 0.85 for 128 to 192 rows and 3072 or 4096 tokens, else the library's tiles are as fast (256 to 512 rows, 4096
+//     tokens 1.10 to 1.47), and beyond they are faster (K = 4096, 512 rows, 4096 tokens 1.61);
+//   * with an activation, whose kernel is saved, 0.4 to 0.95 (384 to 640 rows of K = 2048, 3072 and more tokens 1.0 to 1.25).
+bool prompt_pays(int64_t T, int64_t rows, int K, int act) {
+    const int64_t results = T * rows;
+    if (act != 0) return K <= 512 ? T <= 16384 : K <= 1024 ? T <= 8192 : K <= 2048 && T <= 8192 && (results <= (1 << 20) || rows > 640);
+    if (rows > T) return (K <= 512 && results <= 3 << 20) || (K <= 1024 && results <= 2 << 20);
+    if (K <= 512) return T <= 8192 && (rows < 1536 || T <= 2048);
+    if (K <= 1024) return (T <= 2048 && rows < 1536) || (T <= 8192 && results <= 1 << 20);
+    return K <= 2048 && rows > 96 && rows <= 192 && T >= 3072 && T <= 4096;
+}
+
 }  // namespace
 
 // Where this is the faster way (and the host's 15 us a call come on top): up to as many rows as the library needs for tiles of
@@ -298,14 +315,27 @@ bool decode_pays(int64_t T, int64_t rows, int K, int act, bool parts) {
 // 14.2 / 16.2; 8192 x 2048 500 rows 23.0 / 25.3, 700 31.6 / 28.5; 6144 x 4096 300 rows 28.5 / 29.7, 420 33.6 / 31.8; 12288 x 4096 200 rows
 // 37.0 / 40.1, 300 51.3 / 50.3.  An activation saves the kernel behind the library's product (12288 x 4096, 512 rows 58.1 / 51.7 + 6.5); partial sums
 // fill the chip where rows and weights are few (4096 x 8192, 512 rows 42.8 / 52.6, 700 60.4 / 54.8; 2048 x 6144, 1024 rows 36.4 / 40.8).
+// Over 1024 to 16384 weight rows, K of 512 to 12288 and 65 to 1024 tokens 0.84 of the library's time on the average, 0.71 with an activation,
+// 0.87 for partial sums with the norm behind them; single shapes, where the library's tiles happen to fit, up to 1.2 (3072 x 2048, 384
+// tokens 1.20; partial sums 1536 x 4096, 896 tokens 1.25).
+//   * Beyond 256 tokens no more results than its tiles take in a few rounds (K = 512, 16384 rows, 640 tokens 1.46, 896 1.39; K = 1024, 8192 rows,
+//     640 tokens 1.24, 12288 rows, 300 tokens 1.19; with an activation K = 1024, 16384 rows, 640 tokens 1.30), and no square of 3072 and more
+//     (4096 x 4096, 65 to 100 tokens 1.2, 300 to 512 1.06 to 1.26).
+//   * Rows that are no multiple of four are stored value by value: 2048 tokens, K = 512 511 rows 0.78, 1001 0.94, 1301 1.10; 300 tokens, 4098
+//     x 2048 1.18, partial sums of 2050 x 2048 1.36.
+//   * No partial sums for more tokens than the estimate was fitted to, or for fewer rows: the end of a layer with a token input takes whole
+//     results in one launch (128 rows of K = 1024, 4096 tokens, two ranges and four launches 26.7, library and one launch 19.0).
 bool tile_gemm_pays(int64_t T, int N, int K, int act, bool parts) {
     if (!tile_gemm_supported(T, N, K)) return false;
     const int64_t rows = act == 2 ? 2 * static_cast<int64_t>(N) : N;
     if (T <= 64) return decode_pays(T, rows, K, act, parts);
     const int64_t few = T < rows ? T : rows, many = T < rows ? rows : T, size = many * K;
     if (few <= 64 || many < 1024) return false;
+    if (N % 4 != 0 && (parts ? T > 128 : T * N > (int64_t{1} << (act == 0 ? 30 : 32)) / K)) return false;
+    if (parts && (T > 1024 || N < 1024)) return false;
     if (parts) return K >= 512 && (few <= 512 || (few <= 1024 && many <= 2048 && size <= (int64_t{1} << 24)));
-    if (K > many) return false;
+    if (K > many || (K == many && K > 2048) || (T > 1024 && !prompt_pays(T, rows, K, act))) return false;
+    if (few > 256 && T <= 1024 && T * rows > (act != 0 ? int64_t{1} << 23 : int64_t{7} << 19)) return false;
     if (act != 0) return few <= (size <= (int64_t{1} << 24) ? 1024 : size <= (int64_t{1} << 26) ? 512 : 96);
     return few <= (size <= (int64_t{1} << 21) ? 1536 : size <= (int64_t{1} << 23) ? 1024 : size <= (int64_t{1} << 24) ? 512 :
                    size <= (int64_t{1} << 25) ? 320 : size <= (int64_t{1} << 26) ? 224 : 96);

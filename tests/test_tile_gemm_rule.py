@@ -72,3 +72,26 @@ def test_partial_sums_are_the_tiled_kernels_or_whole(monkeypatch):
     # wherever the rule takes partial sums, the other kernel is not asked
     for T, N, K in itertools.product((17, 33, 64), range(512, 16384, 512), (1024, 1088, 2048, 6144)):
         assert lib.ed_tile_gemm_splits(T, N, K) >= 1, (T, N, K)
+
+
+def test_where_the_rule_ends():
+    pays = _lib.load_decoder().ed_tile_gemm_pays
+    # sections and widths of few rows: to so many tokens, by K; with an activation further
+    for rows, K, to in ((128, 512, 8192), (512, 512, 8192), (1024, 512, 8192), (1536, 512, 2048), (128, 1024, 8192), (256, 1024, 4096), (512, 1024, 2048),
+                        (1024, 1024, 2048), (72, 2048, 0), (512, 1536, 0), (1024, 2048, 0), (512, 4096, 0)):
+        assert [pays(T, rows, K, 0) for T in (1536, 2048, 4096, 8192, 8193, 16384)] == [int(T <= to) for T in (1536, 2048, 4096, 8192, 8193, 16384)], (rows, K)
+    assert [pays(T, 192, 2048, 0) for T in (2048, 3072, 4096, 4097)] == [0, 1, 1, 0]
+    for rows, K, to in ((512, 512, 16384), (1024, 1024, 8192), (512, 2048, 2048), (1024, 2048, 8192), (512, 4096, 0)):
+        assert [pays(T, rows, K, 1) for T in (2048, 8192, 16384, 16385)] == [int(T <= to) for T in (2048, 8192, 16384, 16385)], (rows, K)
+        assert [pays(T, rows // 2, K, 2) for T in (2048, 8192, 16384, 16385)] == [pays(T, rows, K, 1) for T in (2048, 8192, 16384, 16385)]
+    # more tokens than rows of a short prompt, on wide weights
+    assert [pays(1344, N, 512, 0) for N in (2048, 3072)] == [pays(1152, N, 256, 0) for N in (2048, 4096)] == [1, 0]
+    assert [pays(T, 8192, 1024, 0) for T in (256, 448, 640)] == [1, 1, 0] and [pays(T, 16384, 1024, 1) for T in (512, 640)] == [1, 0]
+    assert [pays(100, N, K, 0) for N, K in ((2048, 2048), (4096, 4096), (8192, 4096), (4096, 2048))] == [1, 0, 1, 1]
+    # results that are stored one by one
+    assert [pays(2048, N, 512, 0) for N in (1001, 1301, 1300)] == [pays(100, 4098, 2048, 0), pays(300, 4098, 2048, 0), 1] == [1, 0, 1]
+    # partial sums: within the tokens and rows that the estimate was fitted to
+    splits = _lib.load_decoder().ed_tile_gemm_splits
+    for T, N, K in itertools.product((1024, 1025, 2048, 16384), (72, 128, 512, 1020), (512, 2048, 8192)):
+        assert splits(T, N, K) == 0, (T, N, K)
+    assert splits(1025, 2048, 2048) == splits(300, 2050, 2048) == 0 < splits(1024, 2048, 2048) and splits(100, 2050, 2048) > 0
