@@ -1,4 +1,5 @@
-"""The weight-streaming product of decode batches at the edges of its tiles and of the rule that picks them."""
+"""The weight-streaming product of decode batches at the edges of its tiles and of the rule that picks them: the kernel itself into memory
+that holds NaN, and the layers' functions, which take the tiled kernel or the library where those are faster."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -26,7 +27,41 @@ def off(got, want):
 F32_TOL, BF16_TOL = 1e-5, 2.0 ** -8 + 1e-5
 
 
-# tokens: around every tile edge; rows: ones, twos and fours of 16 per workgroup, remainders; k: one step, a range that waves share unevenly
+def product(x, w, cols, splits=1, act=0, dtype=BF16):
+    """The kernel itself, with a row behind the result that has to stay."""
+    T, K = x.shape
+    full = torch.full((splits * T + 1, cols), float("nan"), dtype=dtype, device="cuda")
+    code = _lib.load_decoder().ed_decode_gemm(x.data_ptr(), w.data_ptr(), full.data_ptr(), _lib.dtype_code(dtype), splits, T, cols, K, act,
+                                              _lib.current_stream(x.device))
+    assert code == 0 and bool(full[-1].isnan().all())
+    return full[:-1].view(splits, T, cols)
+
+
+# Every form: tokens in ones to fours of 16; rows in ones (to 4096), twos (to 8192 or, up to 32 tokens, 9216), fours of eight waves (to 16384, from 33
+# tokens) and of four waves, at their edges and with remainders; k: one step, fewer steps than waves, a range that waves share unevenly
+@pytest.mark.parametrize("T", [1, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(1, 64), (50, 192), (4096, 576), (4102, 128), (8192, 192), (8198, 64), (9216, 64), (9222, 128), (16384, 64), (16390, 192), (20000, 1088)])
+def test_every_form_of_the_kernel(T, N, K):
+    announce(f"decode gemm forms {T} {N} {K}")
+    x, w, want = operands(T, N, K)
+    assert off(product(x, w, N)[0], want) < BF16_TOL
+    assert off(product(x, w, N, dtype=torch.float32)[0], want) < F32_TOL
+    assert off(product(x, w, N, act=1)[0], F.relu(want) ** 2) < BF16_TOL
+    if N % 2 == 0:
+        half = N // 2
+        assert off(product(x, w, half, act=2)[0], F.silu(want[:, :half]) * want[:, half:]) < BF16_TOL
+
+
+# (rows in 32s and, from 33 tokens and 4096 rows on, in 64s where as many ranges fill the chip)
+@pytest.mark.parametrize("T", [1, 17, 33, 64])
+@pytest.mark.parametrize("N,K,splits", [(40, 8192, 8), (2048, 6144, 4), (4096, 1024, 2), (4130, 2048, 4), (4160, 4096, 3), (512, 1088, 17)])
+def test_every_form_of_partial_sums(T, N, K, splits):
+    announce(f"decode gemm forms of parts {T} {N} {K} {splits}")
+    x, w, want = operands(T, N, K)
+    assert off(product(x, w, N, splits, dtype=torch.float32).sum(0), want) < F32_TOL
+
+
+# tokens: around every tile edge; rows: few, a remainder, as many as the rule takes to either kernel; k: one step, a range that waves share unevenly
 @pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 48, 49, 63, 64])
 @pytest.mark.parametrize("N,K", [(1, 64), (50, 192), (4096, 128), (4100, 576), (8200, 64), (16400, 128)])
 def test_products(T, N, K):
