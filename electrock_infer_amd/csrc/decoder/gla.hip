@@ -11,7 +11,9 @@
 // workgroup is one (chunk, head), one wave a v tile.  Bound: instructions and the chain through a block (its matrix units are a third
 // busy), so a block loaded ahead has two barriers: its operands lie in one of two places, and the norm of its outputs, which needs all waves' sums
 // of squares, is finished in the next one (us for 8 x 1024 tokens, 16 heads of 64 x 128, before and now: first pass 43 and 37, output
-// pass 102 and 90; loads without branches are half of it).  Everything that reaches the state is float32: the operands are
+// pass 102 and 90; loads without branches are half of it).  The second place costs LDS (128 x 128: 73 KB a workgroup instead of 45), which
+// pays at every size: a call of 8 x 1024 tokens and 32 heads, 128 x 128 855 and 719, 96 x 128 819 and 681, 100 x 120 792 and 656, 32 x 64
+// 238 and 223.  Everything that reaches the state is float32: the operands are
 // products of the bf16 projections with float32 decays, and no exponent is positive except in the block's own 16 x 16
 // scores, where exp(-bl_s) is used as a factor only while the whole block decays by less than 2^-kFactorLimit.  (The
 // logarithms are kept to base 2.)

@@ -279,10 +279,10 @@ __global__ __launch_bounds__(256) void recur_block_kernel(RecurProblem p, int he
 
 // ---- prompts: a chunk's blocks, one after the other ----
 // Products with the state (but the additive rule's read-out) run on the bf16 matrix units, every float32 operand as the sum of three
-// bf16 values: 8 bits each, rounded to nearest, so that the first two leave a remainder of 2^-18 and all three one of 2^-27 at most.  Of
-// the nine products the six that reach 2^-24 are added up, in float32, the smallest first.  Against float64 this is no further off than
-// float32 products (1536 tokens, decays from 1 - 6e-6 to e^-2.7 a token: 7.7e-7 / 8.0e-7 where everything is kept, 5.2e-7 / 5.3e-7 where
-// it fades); six bf16 products take 96 cycles where eight float32 ones take 256.  The parts of an infinite value, or one beyond the largest
+// bf16 values: 8 bits each, rounded to nearest, together all 24 (the second is 2^-8 of the first at most, the third 2^-17).  Of the nine
+// products the six down to 2^-17 of the first are added up, in float32, the smallest first; the others are 2^-25 of it at most.  Against
+// float64 this is no further off than float32 products (1536 tokens, 4 heads of 128 x 128, this / those: 8.3e-7 / 8.5e-7 where everything is
+// kept, 7.06e-7 / 7.06e-7 with decays of e^-2.7 a token; over five mixers and four decays at most 1.001 of theirs); six bf16 products take 96 cycles where eight float32 ones take 256.  The parts of an infinite value, or one beyond the largest
 // bf16, are no numbers, and a key, an update or a state with such parts leaves NaN in the state until the chunk ends (a query's are asked
 // for): such a chunk is computed once more, with float32 products.  No time without one (8192 tokens: 407 / 409 and 332 / 334 us a call).
 constexpr float kMostPart = 3.3895314e38f;            // the largest bf16

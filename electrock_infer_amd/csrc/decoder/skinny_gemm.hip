@@ -223,6 +223,8 @@ bool decode_gemm_supported(int64_t T, int N, int K) { return T > 0 && T <= 64 &&
 //     21.0 / 14.1; gated, 2048 rows x 12288, T = 40 34.4 / 23.3), or one tile to a CU still takes 16384 steps;
 //   * rows of 64 to a workgroup leave CUs without one (9216 to 15360; 12288 x 4096, T = 24 28.5 / 26.5, T = 8 26.4 / 30.4);
 //   * there are more than 48 tokens, whose rows every workgroup reads: unless the weights are small or an activation comes along.
+// (Layers ask for the tiled kernel first: ungated products of more than 8192 rows, and of 6144 from 33 tokens on, come here through
+// ed_decode_gemm and ed_skinny_gemm only.)
 bool decode_gemm_pays(int64_t T, int rows, int K, int act, bool f32) {
     if (!decode_gemm_supported(T, rows, K)) return false;
     if (rows <= 2048) {

@@ -11,7 +11,7 @@
 // costs the host 3 us instead of 20.
 //
 // Decode batches.  Bound: the weights' stream.  One tile of tokens, weights past the caches' order of use (non-temporal), and the
-// ring keeps 40-80 KB per workgroup in flight without a register, while the kernel of skinny_gemm.hip asks for a step's rows, waits and
+// ring keeps 54-72 KB per workgroup (120 in tiles of 64 x 128) in flight without a register, while the kernel of skinny_gemm.hip asks for a step's rows, waits and
 // multiplies.  us, this / that one, weights from memory: 12288 x 4096, 23 tokens 20.1 / 25.5, one 18.9 / 22.8; 4096 x 12288 parts, 64 tokens
 // 21.0 / 26.3, one 17.4 / 20.2; 2048 x 6144 parts, 64 tokens 9.4 / 12.7; gated 2 x 4096 x 2048, 64 tokens 10.9 / 14.5; 32000 x 4096
 // float32, 64 tokens 43.0 / 53.0 (6.1 TB/s).  That one shares K out over a workgroup's waves and stays ahead where the rows are few and the
