@@ -3,8 +3,9 @@
 // A workgroup makes BM token rows x BN weight rows, a wave 16 x 16 pieces of it.  Both operands go from memory straight to LDS,
 // 128 bytes of a row per step, in a ring of STAGES stages of which all but the one that is multiplied are in flight.
 //
-// Short prompts.  Bound: what a CU takes in.  Rows that lie apart arrive at about 70 bytes per ns and CU whatever the tile, the waves
-// and the depth of the ring (64 x 64: 0.23 us a step, 64 x 128 0.33, 128 x 128 0.48, 128 x 256 0.78; 1 KB pieces would reach 105),
+// Short prompts.  Bound: what a CU takes in.  Rows that L2 holds arrive at up to 125 bytes per ns and CU, whatever the width of the pieces,
+// rows from beyond at 61 with all CUs, and the products and LDS reads of a step beside the copies cost another quarter (a step of 128 x
+// 128 x 64, us: copies alone 0.26, products alone 0.23, all with operands in L2 0.36, weights from memory 0.45-0.52),
 // so a tile is as large as still leaves every CU one, and K is split where the results may stay partial sums.  us, this / the
 // library's product (and the kernel of its activation), weights from memory: 300 tokens, 6144 x 2048 squared ReLU 16.7 / 17.7 + 4.2,
 // 2048 x 6144 parts 18.1 / 26.9, 2048 x 2048 parts 8.5 / 11.5, 4096 x 12288 parts 45.9 / 66.1, 2048 x 512 5.1 / 7.0; and a call
@@ -17,11 +18,13 @@
 // float32, 64 tokens 43.0 / 53.0 (6.1 TB/s).  That one shares K out over a workgroup's waves and stays ahead where the rows are few and the
 // results whole (3072 x 2048, one token 7.7 / 5.7).
 //
-// The sum of a result runs over K from a place that depends on its tile of columns (tiles side by side ask for different
-// parts of their rows at a time).
+// The sum of a result runs over K from a place that depends on its tile (tiles side by side ask for different parts of their rows at
+// a time).
 #include "decoder.h"
 #include "mma.h"
 #include "../lds_copy.h"
+
+#include <type_traits>
 
 namespace em {
 namespace {
@@ -62,12 +65,13 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
     const int wm = wave % WM, wn = wave / WM;
-    // an XCD takes neighbouring tiles, those of one column first: its L2 reads a weight row once
-    const int tiles = m_tiles * n_tiles, per_xcd = (tiles + kXcds - 1) / kXcds;
-    const int local = blockIdx.x / kXcds, tile = blockIdx.x % kXcds * per_xcd + local;
-    if (local >= per_xcd || tile >= tiles) return;
-    const int nt = tile / m_tiles, m0 = (tile - nt * m_tiles) * BM, n0 = nt * kOutCols;
-    const int splits = gridDim.y, split = blockIdx.y, steps = K / kStepK;
+    // an XCD takes neighbouring tiles of one range of K, those of one column first: its L2 reads a weight row once, and the token rows
+    // of few ranges
+    const int splits = gridDim.y, tiles = m_tiles * n_tiles, all = tiles * splits, per_xcd = (all + kXcds - 1) / kXcds;
+    const int id = blockIdx.y * gridDim.x + blockIdx.x, local = id / kXcds, item = id % kXcds * per_xcd + local;
+    if (local >= per_xcd || item >= all) return;
+    const int split = item / tiles, tile = item - split * tiles;
+    const int nt = tile / m_tiles, mt = tile - nt * m_tiles, m0 = mt * BM, n0 = nt * kOutCols, steps = K / kStepK;
     const int s0 = static_cast<int>(static_cast<int64_t>(steps) * split / splits);
     const int nk = static_cast<int>(static_cast<int64_t>(steps) * (split + 1) / splits) - s0;
 
@@ -90,7 +94,10 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
         src[i] += static_cast<int64_t>(s0) * kStepK + piece;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
-    const int rot = (nt * 5) % nk;       // tiles side by side start at different places of their rows
+    // Tiles side by side start at different places of their rows, and those that share weight rows a little behind each other: the first
+    // brings a row into L2 and the others find it there (steps per column / row tile, us: 300 x 2048 x 6144 parts 5 / 0 18.0, 1 / 2 17.2, 1000 x
+    // 2048 x 6144 parts 32.9, 30.3; 5 / 4 loses the rows again: 300 x 4096 x 12288 parts 59.6 instead of 38.5).  Gated: 5 / 0, halves lie far apart.
+    const int rot = (m_tiles == 1 || ACT == 2 ? nt * 5 : nt + mt * 2) % nk;
     auto place = [&](int step) {         // elements into the range of K
         const int k = step + rot;
         return (k >= nk ? k - nk : k) * kStepK;
@@ -114,64 +121,63 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
         w_at[h] = G::kXBytes + wn * NF * 2048 + row;
     }
     M::frag fx[2][MF], fw[2][NF];
-    auto read = [&](int slot, int h) {
+    constexpr int kReads = NF + MF, kProducts = NF * MF;
+    auto read_one = [&](int slot, int h, int r) {
         const uint8_t* s = smem + slot * G::kStageBytes;
-#pragma unroll
-        for (int n = 0; n < NF; ++n) fw[h][n] = *reinterpret_cast<const M::frag*>(s + w_at[h] + n * 2048);
-#pragma unroll
-        for (int m = 0; m < MF; ++m) fx[h][m] = *reinterpret_cast<const M::frag*>(s + x_at[h] + m * 2048);
+        if (r < NF) fw[h][r] = *reinterpret_cast<const M::frag*>(s + w_at[h] + r * 2048);
+        else fx[h][r - NF] = *reinterpret_cast<const M::frag*>(s + x_at[h] + (r - NF) * 2048);
     };
-    auto multiply = [&](int h) {
+    // The products of half a stage.  Between them, in this order whatever the compiler would like: the reads of the half behind it and
+    // (COPIES) the copies of the stage `at` into slot `to`.  Back to back either would hold the wave's products up.
+    auto half = [&](auto copies, int h, int from, int at, int to) {
 #pragma unroll
-        for (int n = 0; n < NF; ++n)
+        for (int j = 0; j < kProducts; ++j) {
+            const int n = j / MF, m = n % 2 == 0 ? j % MF : MF - 1 - j % MF;      // (neighbours share an operand)
 #pragma unroll
-            for (int m = 0; m < MF; ++m) acc[n][m] = M::mac(fw[h][n], fx[h][m], acc[n][m]);
+            for (int i = (j * kReads + kProducts - 1) / kProducts; i < ((j + 1) * kReads + kProducts - 1) / kProducts; ++i) read_one(from, 1 - h, i);
+            acc[n][m] = M::mac(fw[h][n], fx[h][m], acc[n][m]);
+            if constexpr (decltype(copies)::value) {
+#pragma unroll
+                for (int i = j * G::kCopies / kProducts; i < (j + 1) * G::kCopies / kProducts; ++i) copy(i, at, to);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     for (int s = 0; s < STAGES && s < nk; ++s)
 #pragma unroll
         for (int i = 0; i < G::kCopies; ++i) copy(i, place(s), s);
     wait_stages<G::kCopies, STAGES - 1>(nk - 1);
     block_barrier();
-    read(0, 0);
+#pragma unroll
+    for (int i = 0; i < kReads; ++i) read_one(0, 0, i);
     int slot = 0;
     auto advance = [&]() {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // this wave has read its own of the stage
         block_barrier();
     };
+    constexpr std::true_type kWithCopies{};
+    constexpr std::false_type kWithout{};
     int k = 0;
     for (; k + STAGES < nk; ++k) {
-        read(slot, 1);
-        multiply(0);
+        half(kWithout, 0, slot, 0, 0);
         wait_dma<(STAGES - 2) * G::kCopies>();                     // the next stage has landed
         advance();
-        // the copies into the slot that is free now, one by one between products: back to back they would hold the wave up
-        const int next = slot + 1 == STAGES ? 0 : slot + 1, at = place(k + STAGES);
-        read(next, 0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < NF * MF; ++j) {
-            acc[j / MF][j % MF] = M::mac(fw[1][j / MF], fx[1][j % MF], acc[j / MF][j % MF]);
-            constexpr int kProducts = NF * MF;
-            if ((j + 1) * G::kCopies / kProducts > j * G::kCopies / kProducts) {
-#pragma unroll
-                for (int i = j * G::kCopies / kProducts; i < (j + 1) * G::kCopies / kProducts; ++i) copy(i, at, slot);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
+        const int next = slot + 1 == STAGES ? 0 : slot + 1;
+        half(kWithCopies, 1, next, place(k + STAGES), slot);       // (into the slot that is free now)
         slot = next;
     }
     for (; k + 1 < nk; ++k) {
-        read(slot, 1);
-        multiply(0);
+        half(kWithout, 0, slot, 0, 0);
         wait_stages<G::kCopies, STAGES - 2>(nk - 2 - k);
         advance();
         slot = slot + 1 == STAGES ? 0 : slot + 1;
-        read(slot, 0);
-        multiply(1);
+        half(kWithout, 1, slot, 0, 0);
     }
-    read(slot, 1);
-    multiply(0);
-    multiply(1);
+    half(kWithout, 0, slot, 0, 0);
+#pragma unroll
+    for (int n = 0; n < NF; ++n)
+#pragma unroll
+        for (int m = 0; m < MF; ++m) acc[n][m] = M::mac(fw[1][n], fx[1][m], acc[n][m]);
 
     // element i of a fragment: token l16, column lq * 4 + i
 #pragma unroll
