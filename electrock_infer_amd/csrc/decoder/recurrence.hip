@@ -78,16 +78,29 @@ __device__ __forceinline__ void load_channels(const typename Elem::storage* src,
 }
 
 // ---- prompts: convolutions, unit vectors, decays ----
-// A wave takes 16 tokens of kConvPiece channels: four per lane, of as many q or k heads as fit (a head has a power of two of
-// lanes, `head_lanes`) or of v; the last waves' share is decays and betas, one per lane.  K >= taps: rows that a lane keeps.  VEC: all
-// counts and offsets are multiples of four.
-template <typename Elem, int K, bool VEC>
+// every value's sum over `lanes` neighbouring lanes (a power of two), in all of them
+template <int N>
+__device__ __forceinline__ void add_heads(float (&v)[N], int lanes) {
+    if (lanes >= 16) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = row_sum(v[i]);
+    }
+    for (int off = lanes >= 16 ? 16 : 1; off < lanes; off *= 2) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] += __shfl_xor(v[i], off);
+    }
+}
+// A wave takes TOKENS tokens of kConvPiece channels: four per lane, of as many q or k heads as fit (a head has a power of two of
+// lanes, `head_lanes`) or of v; the last waves' share is decays and betas, one per lane.  K >= taps: rows that a lane keeps; TOKENS >= K - 1,
+// so that only a portion's first piece reads the ring.  VEC: all counts and offsets are multiples of four.
+template <typename Elem, int K, bool VEC, int TOKENS>
 __global__ __launch_bounds__(256) void recur_conv_kernel(RecurProblem p, int head_lanes) {
+    static_assert(TOKENS >= K - 1 && kBlock % TOKENS == 0, "the ring's readers");
     typedef typename Elem::storage S;
     const int4 ch = p.chunks[blockIdx.x];
-    const int first = blockIdx.y * kBlock;
+    const int first = blockIdx.y * TOKENS;
     if (first >= ch.z) return;
-    const int n = min(kBlock, ch.z - first), seq = ch.x;
+    const int n = min(TOKENS, ch.z - first), seq = ch.x;
     const int64_t row0 = static_cast<int64_t>(ch.y) + first;
     const int q_begin = p.q_begin[seq], n_seq = p.q_begin[seq + 1] - q_begin;
     const int at0 = static_cast<int>(row0) - q_begin;          // in this step's portion of the sequence
@@ -111,9 +124,9 @@ __global__ __launch_bounds__(256) void recur_conv_kernel(RecurProblem p, int hea
     const int channel0 = (is_v ? 2 * p.kv_heads * p.dim : is_q ? 0 : p.kv_heads * p.dim) + begin;
     S* ring = static_cast<S*>(p.ring) + static_cast<int64_t>(p.slots[seq]) * p.taps * channels + channel0;
 
-    float cur[kBlock][4];
+    float cur[TOKENS][4];
 #pragma unroll
-    for (int t = 0; t < kBlock; ++t) load_channels<Elem, VEC>(src + (row0 + min(t, n - 1)) * p.stride, c, count, cur[t]);
+    for (int t = 0; t < TOKENS; ++t) load_channels<Elem, VEC>(src + (row0 + min(t, n - 1)) * p.stride, c, count, cur[t]);
     float w[K][4], bias[4];                                     // w[i]: of the row K - 1 - i tokens back
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -140,46 +153,52 @@ __global__ __launch_bounds__(256) void recur_conv_kernel(RecurProblem p, int hea
             else if (pos0 >= back) load_channels<Elem, VEC>(ring + static_cast<int64_t>((pos0 - back) % p.taps) * channels, c, count, hist[i]);
         }
     }
-    const int dp = (p.dim + 15) / 16 * 16;
+    // (results take the projections' registers, so that the sums of all tokens' vectors are added up side by side)
+    float ss[TOKENS];
 #pragma unroll
-    for (int t = 0; t < kBlock; ++t) {
-        float y[4], ss = 0.0f;
+    for (int t = 0; t < TOKENS; ++t) {
+        ss[t] = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            y[j] = bias[j];
+            float y = bias[j];
 #pragma unroll
             for (int i = 0; i < K - 1; ++i) {
-                y[j] = fmaf(w[i][j], hist[i][j], y[j]);
+                y = fmaf(w[i][j], hist[i][j], y);
                 hist[i][j] = i + 1 < K - 1 ? hist[i + 1][j] : cur[t][j];
             }
-            y[j] = silu_fast(fmaf(w[K - 1][j], cur[t][j], y[j]));
-            ss = fmaf(y[j], y[j], ss);
+            cur[t][j] = silu_fast(fmaf(w[K - 1][j], cur[t][j], y));
+            ss[t] = fmaf(cur[t][j], cur[t][j], ss[t]);
         }
-        const int64_t row = row0 + t;
-        if (is_v) {
-            S* dst = static_cast<S*>(p.v_f) + row * v_count + begin;
+    }
+    if (is_v) {
+        S* dst = static_cast<S*>(p.v_f) + row0 * v_count + begin;
+#pragma unroll
+        for (int t = 0; t < TOKENS; ++t, dst += v_count) {
             if (VEC) {
                 if (c < count && t < n) {
                     S s4[4];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) s4[j] = Elem::store(y[j]);
+                    for (int j = 0; j < 4; ++j) s4[j] = Elem::store(cur[t][j]);
                     __builtin_memcpy(__builtin_assume_aligned(dst + c, sizeof(s4)), s4, sizeof(s4));
                 }
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    if (c + j < count && t < n) dst[c + j] = Elem::store(y[j]);
+                    if (c + j < count && t < n) dst[c + j] = Elem::store(cur[t][j]);
             }
-        } else {
-            float scale = is_q ? p.q_scale : 1.0f;
-            if (p.unit_eps > 0.0f) {
-                for (int off = head_lanes / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
-                scale *= __builtin_amdgcn_rsqf(ss + p.unit_eps);
-            }
-            // (channels beyond dim are zero: their weights are)
-            float* dst = (is_q ? p.q_f : p.k_f) + (row * p.kv_heads + g) * dp;
-            if (c < dp && count > 0 && t < n) *reinterpret_cast<f32x4_t*>(dst + c) = f32x4_t{y[0] * scale, y[1] * scale, y[2] * scale, y[3] * scale};
         }
+    } else {
+        const int dp = (p.dim + 15) / 16 * 16;
+        float scale[TOKENS];
+        if (p.unit_eps > 0.0f) add_heads(ss, head_lanes);
+#pragma unroll
+        for (int t = 0; t < TOKENS; ++t) scale[t] = (is_q ? p.q_scale : 1.0f) * (p.unit_eps > 0.0f ? __builtin_amdgcn_rsqf(ss[t] + p.unit_eps) : 1.0f);
+        // (channels beyond dim are zero: their weights are)
+        float* dst = (is_q ? p.q_f : p.k_f) + (row0 * p.kv_heads + g) * dp;
+#pragma unroll
+        for (int t = 0; t < TOKENS; ++t, dst += p.kv_heads * dp)
+            if (c < dp && count > 0 && t < n)
+                *reinterpret_cast<f32x4_t*>(dst + c) = f32x4_t{cur[t][0] * scale[t], cur[t][1] * scale[t], cur[t][2] * scale[t], cur[t][3] * scale[t]};
     }
     if (at0 != 0) return;
     // (the lane that reads the ring's old rows of these channels is the one that replaces them)
@@ -742,10 +761,16 @@ __global__ __launch_bounds__(256) void recur_scan_kernel(RecurProblem p) {
 }
 
 // Delta rule: by a matrix.  One workgroup per (head, 16 state columns, sequence), one wave per 16 rows.
+// A chain of chunks, bound by how fast one CU takes a chunk's matrix in: a wave's 16 rows lie whole in memory and are loaded so, 1 KB an
+// instruction, and turned into operands through LDS that is the wave's own (loaded as operands, 16 pieces of 64 bytes an instruction, 16 chunks
+// of 16 heads of 128 x 128 took 44.7 us instead of 31.4, five chunks of five sequences 53.0 instead of 38.3; the products alone are 0.9 us a
+// chunk.  Matrices of 256 rows have no room there and are loaded as operands).
 template <int NDT>
 __global__ __launch_bounds__(NDT * kWave) void recur_matrix_scan_kernel(RecurProblem p) {
-    constexpr int kPitch = NDT * 16 + 4;
+    constexpr bool kStaged = NDT <= 8;
+    constexpr int kPitch = NDT * 16 + 4, kPieces = NDT * 4, kSwap = kPieces < 16 ? kPieces - 1 : 15;       // 16-byte pieces of a row
     __shared__ __attribute__((aligned(16))) float state[2][16 * kPitch];      // column by column
+    __shared__ __attribute__((aligned(16))) f32x4_t rows[kStaged ? NDT : 1][kStaged ? 16 * kPieces : 1];    // piece c of row r at c ^ (r & kSwap)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lq = lane >> 4;
     const int col = blockIdx.y * 16 + l16, h = blockIdx.x, s = blockIdx.z;   // (a head's workgroups share an L2)
     const int dim = p.dim, vdim = p.vdim, dp = (dim + 15) / 16 * 16;
@@ -756,11 +781,18 @@ __global__ __launch_bounds__(NDT * kWave) void recur_matrix_scan_kernel(RecurPro
     float* cs = p.chunk_states + static_cast<int64_t>(h) * n;
     const int row = wave * 16 + lq * 4, k_tiles = dp / 16;
     const bool has_rows = wave * 16 < dp, zero = p.starts[s] == 0;
-    const float* mr = p.chunk_trans + h * m_size + static_cast<int64_t>(has_rows ? wave * 16 + l16 : 0) * dp + lq * 4;
+    const float* mr = p.chunk_trans + h * m_size + static_cast<int64_t>(has_rows ? wave * 16 : 0) * dp;
     // a chunk's matrix and contribution, in flight two chunks ahead (one, where the registers do not hold three matrices)
-    constexpr int kAhead = NDT <= 8 ? 2 : 1;
+    constexpr int kAhead = kStaged ? 2 : 1;
     bool ok[4];
     f32x4_t cur, add[kAhead], m4[kAhead][NDT];
+    int at[NDT], put[NDT];              // of load k: elements into the wave's rows, and where it goes in LDS
+#pragma unroll
+    for (int k = 0; k < NDT; ++k) {
+        const int kk = min(k, k_tiles - 1), i = kk * kWave + lane, r = i / (dp / 4), c = i - r * (dp / 4);
+        at[k] = kStaged ? i * 4 : l16 * dp + lq * 4 + kk * 16;
+        put[k] = r * kPieces + (c ^ (r & kSwap));
+    }
     // (addresses are held inside instead of loads being skipped: waits can count straight-line loads)
     int64_t from[4];
     auto fetch = [&](int c, f32x4_t& to_add, f32x4_t (&to)[NDT]) {
@@ -768,15 +800,15 @@ __global__ __launch_bounds__(NDT * kWave) void recur_matrix_scan_kernel(RecurPro
 #pragma unroll
         for (int r = 0; r < 4; ++r) to_add[r] = cs[c * pitch + from[r]];
 #pragma unroll
-        for (int k = 0; k < NDT; ++k) to[k] = *reinterpret_cast<const f32x4_t*>(mr + c * m_pitch + min(k, k_tiles - 1) * 16);
+        for (int k = 0; k < NDT; ++k) to[k] = *reinterpret_cast<const f32x4_t*>(mr + c * m_pitch + at[k]);
     };
     auto advance = [&](int c, f32x4_t& my_add, f32x4_t (&mine)[NDT]) {
         float* buf = state[(c - c0) & 1];
         *reinterpret_cast<f32x4_t*>(buf + l16 * kPitch + row) = cur;
-        f32x4_t sum[2] = {my_add, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}}, now[NDT];
-        if (kAhead == 2) {
+        f32x4_t sum[2] = {my_add, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}};
+        if constexpr (kStaged) {
 #pragma unroll
-            for (int k = 0; k < NDT; ++k) now[k] = mine[k];
+            for (int k = 0; k < NDT; ++k) rows[wave][put[k]] = mine[k];
             fetch(c + 2, my_add, mine);
         }
 #pragma unroll
@@ -787,11 +819,11 @@ __global__ __launch_bounds__(NDT * kWave) void recur_matrix_scan_kernel(RecurPro
         for (int k = 0; k < NDT; ++k) {
             // (rows beyond dim are zero here, whatever stands in the matrix)
             const f32x4_t s4 = *reinterpret_cast<const f32x4_t*>(buf + l16 * kPitch + k * 16 + lq * 4);
+            const f32x4_t m = kStaged ? rows[wave][l16 * kPieces + ((min(k, k_tiles - 1) * 4 + lq) ^ (l16 & kSwap))] : mine[k];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                sum[r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kAhead == 2 ? now[k][r] : mine[k][r], s4[r], sum[r & 1], 0, 0, 0);
+            for (int r = 0; r < 4; ++r) sum[r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], s4[r], sum[r & 1], 0, 0, 0);
         }
-        if (kAhead == 1) fetch(c + 1, my_add, mine);
+        if constexpr (!kStaged) fetch(c + 1, my_add, mine);
         cur = sum[0] + sum[1];
 #pragma unroll
         for (int r = 0; r < 4; ++r) cur[r] = ok[r] ? cur[r] : 0.0f;
@@ -951,13 +983,19 @@ template <typename Elem>
 int launch_conv(const RecurProblem& p, hipStream_t s) {
     int head_lanes = 1;
     while (head_lanes * 4 < round_up(p.dim, 16)) head_lanes *= 2;
-    const int units = static_cast<int>(2 * ceil_div(p.kv_heads, kWave / head_lanes) + ceil_div(p.heads * p.vdim, kConvPiece) + ceil_div(kBlock * p.heads, kWave));
-    const dim3 grid(static_cast<unsigned>(p.n_chunks), static_cast<unsigned>(p.chunk_tokens / kBlock), static_cast<unsigned>(ceil_div(units, 4)));
+    auto units = [&](int tokens) { return 2 * ceil_div(p.kv_heads, kWave / head_lanes) + ceil_div(p.heads * p.vdim, kConvPiece) + ceil_div(tokens * p.heads, kWave); };
+    auto grid = [&](int tokens) {
+        return dim3(static_cast<unsigned>(p.n_chunks), static_cast<unsigned>(p.chunk_tokens / tokens), static_cast<unsigned>(ceil_div(units(tokens), 4)));
+    };
     auto aligned = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % (4 * sizeof(typename Elem::storage)) == 0; };
     const bool vec = p.dim % 4 == 0 && p.vdim % 4 == 0 && p.stride % 4 == 0 && aligned(p.q) && aligned(p.k) && aligned(p.v);
-    if (p.taps > 4) launch((recur_conv_kernel<Elem, kMaxTaps, false>), grid, dim3(256), 0, s, p, head_lanes);
-    else if (vec) launch((recur_conv_kernel<Elem, 4, true>), grid, dim3(256), 0, s, p, head_lanes);
-    else launch((recur_conv_kernel<Elem, 4, false>), grid, dim3(256), 0, s, p, head_lanes);
+    // Where the waves of 16 tokens are few, four of them: the way of one token's channels is what a short prompt waits for, and the rows read
+    // twice lie in L2 (us, 16 / 4 tokens a wave, heads of 128: 320 tokens 10.0 / 6.3, 1024 10.4 / 9.6, 3200 19.3 / 18.6, 8192 35.9 / 38.4).
+    const bool few = int64_t{p.n_chunks} * (p.chunk_tokens / kBlock) * units(kBlock) <= 8192;
+    if (p.taps > 4) launch((recur_conv_kernel<Elem, kMaxTaps, false, kBlock>), grid(kBlock), dim3(256), 0, s, p, head_lanes);
+    else if (vec && few) launch((recur_conv_kernel<Elem, 4, true, 4>), grid(4), dim3(256), 0, s, p, head_lanes);
+    else if (vec) launch((recur_conv_kernel<Elem, 4, true, kBlock>), grid(kBlock), dim3(256), 0, s, p, head_lanes);
+    else launch((recur_conv_kernel<Elem, 4, false, kBlock>), grid(kBlock), dim3(256), 0, s, p, head_lanes);
     return launch_status();
 }
 
