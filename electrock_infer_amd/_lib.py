@@ -52,7 +52,7 @@ DECODER_SYMBOLS = (
     "ed_recur_record", "ed_recur_prefill", "ed_recur_step",
     "ed_attn_row_elems", "ed_attn_splits", "ed_attn_prepare", "ed_attn_paged", "ed_attn_prompt_supported", "ed_attn_prompt",
     "ed_latent_row_elems", "ed_latent_splits", "ed_latent_waves", "ed_latent_prepare", "ed_latent_paged", "ed_head_gemm", "ed_latent_gather",
-    "ed_latent_prompt_supported", "ed_latent_prompt",
+    "ed_latent_prompt_supported", "ed_latent_prompt", "ed_latent_prompt_behind",
 )
 
 
@@ -236,6 +236,7 @@ def load_decoder() -> ctypes.CDLL:
         "ed_head_gemm": [vp, i64, i64, vp, vp, i64, i64, i64, i32, i32, i32, i32, vp],
         "ed_latent_prompt_supported": [i32, i32, i32],
         "ed_latent_prompt": [ctypes.POINTER(LatentPromptArgs), vp],
+        "ed_latent_prompt_behind": [ctypes.POINTER(LatentPromptArgs), i32, vp],
         "ed_latent_gather": [vp, vp, i32, i32, vp, vp, i32, i32, i32, vp, i32, vp],
     }
     for name, argtypes in signatures.items():

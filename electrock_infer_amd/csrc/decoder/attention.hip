@@ -370,8 +370,7 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
                 s[n][r] = key <= pos && key >= low ? v : -INFINITY;
                 mx = fmaxf(mx, s[n][r]);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = column_max(mx);
         const float mn = fmaxf(m, mx), base = mn == -INFINITY ? 0.0f : mn;
         const float alpha = Precise<Elem>::exp(m - base);
         m = mn;
@@ -396,8 +395,7 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = column_sum(l);
     if (lq == 0) {
         wave_m[wave][l16] = m;
         wave_l[wave][l16] = l;
@@ -662,8 +660,7 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
                 for (int n = 0; n < 4; ++n)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[n][j][r]);
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                mx = column_max(mx);
                 const float mn = fmaxf(m[j], mx);
                 base = mn == -INFINITY ? 0.0f : mn;
                 alpha[j] = exp2_fast(m[j] - base);
@@ -698,8 +695,7 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        l[j] += __shfl_xor(l[j], 16);
-        l[j] += __shfl_xor(l[j], 32);
+        l[j] = column_sum(l[j]);
         const float inv = 1.0f / l[j];
         const int t = t0 + wave * kRowsPerWave + j * 16 + l16;
         if (t >= nq) continue;

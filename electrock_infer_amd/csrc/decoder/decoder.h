@@ -18,6 +18,23 @@ __device__ __forceinline__ float add_rotated(float v) {
 }
 __device__ __forceinline__ float row_sum(float v) { return add_rotated<1>(add_rotated<2>(add_rotated<4>(add_rotated<8>(v)))); }
 
+// the largest value and the sum over the four lanes that share lane % 16, in all of them (rows of lanes change places inside the vector unit)
+__device__ __forceinline__ f32x2_t swap_rows(float v, bool halves) {
+    const uint32_t b = __float_as_uint(v);
+    const auto r = halves ? __builtin_amdgcn_permlane32_swap(b, b, false, false) : __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    return f32x2_t{__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ float column_max(float v) {
+    const f32x2_t a = swap_rows(v, false);
+    const f32x2_t b = swap_rows(fmaxf(a[0], a[1]), true);
+    return fmaxf(b[0], b[1]);
+}
+__device__ __forceinline__ float column_sum(float v) {
+    const f32x2_t a = swap_rows(v, false);
+    const f32x2_t b = swap_rows(a[0] + a[1], true);
+    return b[0] + b[1];
+}
+
 // Lets a kernel take `bytes` of dynamic LDS (one CU has 160 KB); 0, or the runtime's error.
 constexpr size_t kLdsPerCu = 160 * 1024;
 inline int allow_lds(const void* kernel, size_t bytes) {
@@ -212,6 +229,6 @@ struct LatentPromptProblem {
     float scale;
 };
 bool latent_prompt_supported(int dim, int rot, int vdim);
-int launch_latent_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s);
+int launch_latent_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, int max_context, hipStream_t s);
 
 }  // namespace em

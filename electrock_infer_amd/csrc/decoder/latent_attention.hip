@@ -530,8 +530,7 @@ __global__ __launch_bounds__(256, 1) void latent_wave_kernel(LatentProblem p, in
             s[r] = tile * kWaveKeys + lq * 4 + r <= pos ? s[r] * p.scale : -INFINITY;
             mx = fmaxf(mx, s[r]);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = column_max(mx);
         // m need not be the maximum: while no row's scores exceed it by more than kSlack the weights stay below e^kSlack and
         // the accumulators as they are (their way through the vector unit costs more than the tile's products)
         if (__any(mx > m + kSlack)) {
@@ -561,8 +560,7 @@ __global__ __launch_bounds__(256, 1) void latent_wave_kernel(LatentProblem p, in
         row = next_row;
         next_row = row_of(tile + 8);
     }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = column_sum(l);
     if (lq == 0) {
         wave_m[wave][l16] = m;
         wave_l[wave][l16] = l;
