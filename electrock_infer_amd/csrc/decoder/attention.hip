@@ -478,13 +478,12 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
 // to 64, whose few tiles do not pay for the second form of the scores, are 1 to 4 % slower (1 x 173 8.5 -> 8.7).
 constexpr float kTanhRange = 0.6f;
 constexpr int kTileKeys = 64;
-constexpr int kRowsPerWave = 32;
-constexpr int kRows = 4 * kRowsPerWave;
 
-// GROUPS: workgroups that a CU is to hold
-template <int DKT, int DVT, int GROUPS>
+// QT: 16-query tiles of a wave; GROUPS: workgroups that a CU is to hold
+template <int DKT, int DVT, int QT, int GROUPS>
 __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p) {
     typedef Mma<BF16Elem> M;
+    constexpr int kRowsPerWave = 16 * QT, kRows = 4 * kRowsPerWave;
     constexpr int LPK = DKT * 32 + 8, LPV = DVT * 16 + 8;
     constexpr bool kPoly = DKT <= 4;       // registers enough for a second form of the scores
     constexpr int kFetchK = kTileKeys * DKT * 4 / 256, kFetchV = kTileKeys * DVT * 2 / 256;
@@ -503,9 +502,9 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
     const int tile0 = max(0, start + t0 - window + 1) / kTileKeys, tile1 = last_pos / kTileKeys + 1;
     const int first_pos = start + t0 + wave * kRowsPerWave;          // of this wave's first query
 
-    typename M::frag fq[2][DKT];
+    typename M::frag fq[QT][DKT];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < QT; ++j) {
         const int t = min(t0 + wave * kRowsPerWave + j * 16 + l16, nq - 1);
         const uint16_t* q = static_cast<const uint16_t*>(p.q_out) + ((row0 + static_cast<int64_t>(t)) * p.heads + h) * dp;
 #pragma unroll
@@ -546,15 +545,22 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
 #pragma unroll
         for (int i = 0; i < kFetchV; ++i) rv[i] = M::load(values + cv + at_v[i]);
     };
-    f32x4_t o[DVT][2];
+    f32x4_t o[DVT][QT];
 #pragma unroll
-    for (int d = 0; d < DVT; ++d) o[d][0] = o[d][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int d = 0; d < DVT; ++d)
+#pragma unroll
+        for (int j = 0; j < QT; ++j) o[d][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const bool capped = p.softcap > 0.0f, fixed = capped && p.softcap <= kFixedCap;
     const float c2 = p.scale * kLog2e, cap2 = p.softcap * kLog2e, in_cap = capped ? 2.0f * kLog2e * p.scale / p.softcap : 0.0f;
     const float to_cap = capped ? p.scale / p.softcap : 0.0f;
     const float tanh0 = cap2 * 0.99999994f, tanh1 = cap2 * -0.33332309f, tanh2 = cap2 * 0.13310173f, tanh3 = cap2 * -0.05210148f, tanh4 = cap2 * 0.015475428f;
     // running maxima in units of log2 (not kept where the cap stands for them); l: this lane's share
-    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
+    float m[QT], l[QT];
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+        m[j] = -INFINITY;
+        l[j] = 0.0f;
+    }
 
     keep_rows(tile0, page_of(tile0));
     keep_rows(tile0 + 1, page_of(tile0 + 1));
@@ -585,16 +591,18 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
         // no key of this tile for this wave's queries
         if (k0 > first_pos + kRowsPerWave - 1 || k0 + kTileKeys - 1 < first_pos - window + 1) continue;
 
-        f32x4_t s[4][2];
+        f32x4_t s[4][QT];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) s[n][0] = s[n][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int j = 0; j < QT; ++j) s[n][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k = 0; k < DKT; ++k)
 #pragma unroll
             for (int n = 0; n < 4; ++n) {
                 const typename M::frag fk = M::load(Ks + (n * 16 + l16) * LPK + k * 32 + lq * 8);
-                s[n][0] = M::mac(fk, fq[0][k], s[n][0]);
-                s[n][1] = M::mac(fk, fq[1][k], s[n][1]);
+#pragma unroll
+                for (int j = 0; j < QT; ++j) s[n][j] = M::mac(fk, fq[j][k], s[n][j]);
             }
         // scores in units of log2; with a fixed maximum their distance to it
         if (kPoly && fixed) {
@@ -602,14 +610,14 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
 #pragma unroll
             for (int n = 0; n < 4; ++n)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < QT; ++j)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) top = fmaxf(top, fabsf(s[n][j][r]));
             if (__all(top * fabsf(to_cap) <= kTanhRange)) {
 #pragma unroll
                 for (int n = 0; n < 4; ++n)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
+                    for (int j = 0; j < QT; ++j) {
                         const f32x4_t x = s[n][j] * to_cap, u = x * x;
                         f32x4_t t = fma4(fma4(f32x4_t(tanh4), u, f32x4_t(tanh3)), u, f32x4_t(tanh2));
                         t = fma4(fma4(t, u, f32x4_t(tanh1)), u, f32x4_t(tanh0));
@@ -619,7 +627,7 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
 #pragma unroll
                 for (int n = 0; n < 4; ++n)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
+                    for (int j = 0; j < QT; ++j)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) s[n][j][r] = -2.0f * cap2 * __builtin_amdgcn_rcpf(exp2_fast(s[n][j][r] * in_cap) + 1.0f);
             }
@@ -627,33 +635,34 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
 #pragma unroll
             for (int n = 0; n < 4; ++n)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < QT; ++j)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
                         s[n][j][r] = fmaf(-2.0f * cap2, __builtin_amdgcn_rcpf(exp2_fast(s[n][j][r] * in_cap) + 1.0f), cap2);
         } else {
 #pragma unroll
-            for (int n = 0; n < 4; ++n) {
-                s[n][0] *= c2;
-                s[n][1] *= c2;
-            }
+            for (int n = 0; n < 4; ++n)
+#pragma unroll
+                for (int j = 0; j < QT; ++j) s[n][j] *= c2;
         }
         if (k0 + kTileKeys - 1 > first_pos || k0 < first_pos + kRowsPerWave - window) {
 #pragma unroll
             for (int n = 0; n < 4; ++n)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < QT; ++j)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int gap = first_pos + j * 16 + l16 - (k0 + n * 16 + lq * 4 + r);
                         if (gap < 0 || gap >= window) s[n][j][r] = -INFINITY;
                     }
         }
-        typename M::frag fp[2][2];   // [32-key step][query tile]
-        float alpha[2] = {1.0f, 1.0f};
+        typename M::frag fp[2][QT];   // [32-key step][query tile]
+        float alpha[QT];
+        bool same = true;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < QT; ++j) {
             float base = kPoly ? 0.0f : cap2;
+            alpha[j] = 1.0f;
             if (!fixed) {
                 float mx = -INFINITY;
 #pragma unroll
@@ -676,25 +685,25 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
                     fp[n >> 1][j][(n & 1) * 4 + r] = static_cast<__bf16>(e);
                 }
             l[j] = l[j] * alpha[j] + sum;
+            same = same && alpha[j] == 1.0f;
         }
-        if (!fixed && !__all(alpha[0] == 1.0f && alpha[1] == 1.0f)) {
+        if (!fixed && !__all(same)) {
 #pragma unroll
-            for (int d = 0; d < DVT; ++d) {
-                o[d][0] *= alpha[0];
-                o[d][1] *= alpha[1];
-            }
+            for (int d = 0; d < DVT; ++d)
+#pragma unroll
+                for (int j = 0; j < QT; ++j) o[d][j] *= alpha[j];
         }
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
             for (int d = 0; d < DVT; ++d) {
                 const typename M::frag fv = load_columns<BF16Elem>(Vs, LPV, k * 32 + lq * 4, k * 32 + 16 + lq * 4, d * 16, l16);
-                o[d][0] = M::mac(fv, fp[k][0], o[d][0]);
-                o[d][1] = M::mac(fv, fp[k][1], o[d][1]);
+#pragma unroll
+                for (int j = 0; j < QT; ++j) o[d][j] = M::mac(fv, fp[k][j], o[d][j]);
             }
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < QT; ++j) {
         l[j] = column_sum(l[j]);
         const float inv = 1.0f / l[j];
         const int t = t0 + wave * kRowsPerWave + j * 16 + l16;
@@ -756,20 +765,33 @@ int keys_paged(const AttnProblem& p, int n_seqs, int max_q, int splits, float* p
 // 47.5 / 38.6; 8 x 221, 512, 13.2 / 13.8; 16 x 59, 128, 5.3 / 5.7).
 constexpr int64_t kTwoPerCu = 512;
 
+template <int DKT, int DVT, int QT, int GROUPS>
+int launch_queries(const AttnProblem& p, int n_seqs, int max_q, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(p.heads), static_cast<unsigned>(ceil_div(max_q, 64 * QT)), static_cast<unsigned>(n_seqs));
+    launch((attn_prompt_kernel<DKT, DVT, QT, GROUPS>), grid, dim3(256), 0, s, p);
+    return launch_status();
+}
+
+// 64 queries to a workgroup where 128 leave CUs without work: half the products, exponentials and sums to a tile, whose chain a wave
+// waits for (us, 128 / 64 queries, 16 heads of 128, cap 30, workgroups of 64: 80, 300 tokens behind 500 31.3 / 24.1; 16, 64 behind 1000 38.3 /
+// 29.2; 256, one prompt of 1000 37.7 / 29.1; 512, 2048 70.3 / 57.0, 8 x 256 behind 1000 53.5 / 49.7, 16 x 128 9.8 / 9.7; heads of 256 / 128, whose
+// 128 queries spill: 256, 66.3 / 34.3; beyond, 640, 10 x 256 behind 1000 65.8 / 72.0; 768, 24 x 128 14.3 / 16.0).  Portions from the start of long
+// prompts, whose first queries see few keys and leave their CUs early, gain beyond that (768, 3 x 1000 51.0 / 40.8, 2 x 1536 58.4 / 50.8, 752,
+// 3000 105 / 83; 1024, 4096 143 / 142, 4 x 1000 51.2 / 55.3, 4096 with a window of 1024 59.5 / 73.5).
+bool few_queries(const AttnProblem& p, int n_seqs, int max_q) {
+    const int64_t groups = ceil_div(max_q, 64) * p.heads * n_seqs, context = static_cast<int64_t>(p.table_width) * p.block_size;
+    return groups <= 512 || (groups <= 800 && max_q >= 960 && context <= max_q + max_q / 4 && (p.window <= 0 || p.window >= max_q));
+}
+
 template <int DKT>
 int launch_prompt(const AttnProblem& p, int n_seqs, int max_q, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(p.heads), static_cast<unsigned>(ceil_div(max_q, kRows)), static_cast<unsigned>(n_seqs));
-    if (p.vdim > 64) {
-        launch((attn_prompt_kernel<DKT, 8, 2>), grid, dim3(256), 0, s, p);
-        return launch_status();
-    }
+    // (heads of up to 64 under a cap keep 32 queries to a wave: which form of tanh a wave's scores take shows in their last bits)
+    const bool few = few_queries(p, n_seqs, max_q) && (DKT > 2 || p.softcap <= 0.0f || p.softcap > kFixedCap);
+    if (p.vdim > 64) return few ? launch_queries<DKT, 8, 1, 2>(p, n_seqs, max_q, s) : launch_queries<DKT, 8, 2, 2>(p, n_seqs, max_q, s);
+    if (few) return launch_queries<DKT, 4, 1, 2>(p, n_seqs, max_q, s);
     if constexpr (DKT == 2)
-        if (static_cast<int64_t>(grid.x) * grid.y * grid.z > kTwoPerCu) {
-            launch((attn_prompt_kernel<DKT, 4, 3>), grid, dim3(256), 0, s, p);
-            return launch_status();
-        }
-    launch((attn_prompt_kernel<DKT, 4, 2>), grid, dim3(256), 0, s, p);
-    return launch_status();
+        if (ceil_div(max_q, 128) * p.heads * n_seqs > kTwoPerCu) return launch_queries<DKT, 4, 2, 3>(p, n_seqs, max_q, s);
+    return launch_queries<DKT, 4, 2, 2>(p, n_seqs, max_q, s);
 }
 
 }  // namespace
