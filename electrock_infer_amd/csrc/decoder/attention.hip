@@ -107,8 +107,9 @@ __global__ __launch_bounds__(256) void attn_prepare_kernel(AttnProblem p) {
 }
 
 // The same for the rows of a prompt, bf16: a wave per token, L lanes with eight elements each to a head, everything a group of heads
-// needs requested before the first of them is normed.  Bound: the rows' bytes (8192 tokens, 16 + 4 heads of 128, 100 MB: 56 -> 35 us;
-// a workgroup per token took a head per wave, four bytes per lane and a load's way at a time).
+// needs requested before the first of them is normed, and the first group before the turns are computed.  Bound: the rows' bytes (8192
+// tokens, 16 + 4 heads of 128, 100 MB: 56 -> 35 us; a workgroup per token took a head per wave, four bytes per lane and a load's way at
+// a time); of few tokens a wave's way, whose groups of heads then go to waves of their own (gridDim.y).
 template <int L>
 __global__ __launch_bounds__(256) void attn_prepare_rows_kernel(AttnProblem p, int64_t T) {
     constexpr int kHeads = kWave / L, kAhead = 4;
@@ -119,8 +120,24 @@ __global__ __launch_bounds__(256) void attn_prepare_rows_kernel(AttnProblem p, i
     const int half = p.rot / 2, all = p.heads + p.kv_heads, vp = attn_pitch(p.vdim), row = attn_row_elems(p.kv_heads, L * 8, p.vdim);
     const uint16_t *q = static_cast<const uint16_t*>(p.q) + t * p.stride + c, *k = static_cast<const uint16_t*>(p.k) + t * p.stride + c;
     uint16_t* q_out = static_cast<uint16_t*>(p.q_out) + t * p.heads * (L * 8) + c;
-    uint16_t* cached = static_cast<uint16_t*>(p.cache) + static_cast<int64_t>(p.cache_rows[t]) * row;
-    const float pos = static_cast<float>(p.positions[t]);
+    const int32_t cache_row = p.cache_rows[t];
+    const float pos = static_cast<float>(p.positions[t]), lambda = p.mix != nullptr ? *p.mix : 0.0f;
+    u32x4_t rows[kAhead];
+    auto request = [&](int u0) {
+#pragma unroll
+        for (int n = 0; n < kAhead; ++n) {
+            const int u = min(u0 + n * kHeads, all - 1);
+            rows[n] = *reinterpret_cast<const u32x4_t*>(u < p.heads ? q + u * (L * 8) : k + (u - p.heads) * (L * 8));
+        }
+    };
+    const int first = sub + static_cast<int>(blockIdx.y) * kHeads * kAhead, step = static_cast<int>(gridDim.y) * kHeads * kAhead;
+    request(first);
+    float wq[8], wk[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        wq[i] = p.q_norm != nullptr ? p.q_norm[c + i] : 1.0f;
+        wk[i] = p.k_norm != nullptr ? p.k_norm[c + i] : 1.0f;
+    }
     for (int i = lane; i < half; i += kWave) sincosf(pos * p.inv_freq[i], &turns[wave][1][i], &turns[wave][0][i]);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const bool turned = c < p.rot;
@@ -129,19 +146,9 @@ __global__ __launch_bounds__(256) void attn_prepare_rows_kernel(AttnProblem p, i
         cosine = *reinterpret_cast<const f32x4_t*>(&turns[wave][0][j * 4]);
         sine = *reinterpret_cast<const f32x4_t*>(&turns[wave][1][j * 4]);
     }
-    float wq[8], wk[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        wq[i] = p.q_norm != nullptr ? p.q_norm[c + i] : 1.0f;
-        wk[i] = p.k_norm != nullptr ? p.k_norm[c + i] : 1.0f;
-    }
-    for (int u0 = sub; u0 < all + sub; u0 += kHeads * kAhead) {
-        u32x4_t rows[kAhead];
-#pragma unroll
-        for (int n = 0; n < kAhead; ++n) {
-            const int u = min(u0 + n * kHeads, all - 1);
-            rows[n] = *reinterpret_cast<const u32x4_t*>(u < p.heads ? q + u * (L * 8) : k + (u - p.heads) * (L * 8));
-        }
+    uint16_t* cached = static_cast<uint16_t*>(p.cache) + static_cast<int64_t>(cache_row) * row;
+    for (int u0 = first; u0 < all + sub; u0 += step) {
+        if (u0 != first) request(u0);
 #pragma unroll
         for (int n = 0; n < kAhead; ++n) {
             const int u = u0 + n * kHeads;
@@ -154,8 +161,13 @@ __global__ __launch_bounds__(256) void attn_prepare_rows_kernel(AttnProblem p, i
                 ss = fmaf(x[2 * i], x[2 * i], fmaf(x[2 * i + 1], x[2 * i + 1], ss));
             }
             if ((is_q ? p.q_norm : p.k_norm) != nullptr) {
+                if (L == 32) ss += __shfl_xor(ss, 16);
+                if (L >= 16) {
+                    ss = row_sum(ss);
+                } else {
 #pragma unroll
-                for (int off = L / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+                    for (int off = L / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+                }
                 const float rstd = 1.0f / sqrtf(ss / static_cast<float>(L * 8) + p.eps);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) x[i] *= rstd * (is_q ? wq[i] : wk[i]);
@@ -169,7 +181,7 @@ __global__ __launch_bounds__(256) void attn_prepare_rows_kernel(AttnProblem p, i
             if (u < all) *reinterpret_cast<u32x4_t*>(is_q ? q_out + u * (L * 8) : cached + (u - p.heads) * (L * 8) + c) = out;
         }
     }
-    const float lambda = p.mix != nullptr ? *p.mix : 0.0f;
+    if (blockIdx.y != gridDim.y - 1) return;
     for (int i = lane * 8; i < p.kv_heads * vp; i += kWave * 8) {              // (vdim is a multiple of eight: heads side by side)
         u32x4_t v = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(p.v) + t * p.stride + i);
         if (p.mix != nullptr) {
@@ -833,7 +845,9 @@ int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int
 
 int launch_attn_prepare(const AttnProblem& p, int64_t T, hipStream_t s) {
     if (prepare_rows(p, T)) {
-        const dim3 rows(static_cast<unsigned>(ceil_div(T, 4)));
+        const int64_t at_once = 4 * kWave * 8 / p.dim, parts = ceil_div(p.heads + p.kv_heads, at_once);
+        // (us, a wave per token / per group of heads: 300 tokens of 16 + 4 heads 9.4 / 7.3, 810 of 32 + 8 13.0 / 13.5, 2640 of 16 + 4 16.6 / 20.0)
+        const dim3 rows(static_cast<unsigned>(ceil_div(T, 4)), T <= 512 ? static_cast<unsigned>(parts) : 1u);
         if (p.dim == 64) launch(attn_prepare_rows_kernel<8>, rows, dim3(256), 0, s, p, T);
         else if (p.dim == 128) launch(attn_prepare_rows_kernel<16>, rows, dim3(256), 0, s, p, T);
         else launch(attn_prepare_rows_kernel<32>, rows, dim3(256), 0, s, p, T);
