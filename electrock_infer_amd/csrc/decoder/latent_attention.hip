@@ -565,39 +565,46 @@ __global__ __launch_bounds__(256, 1) void latent_wave_kernel(LatentProblem p, in
         wave_m[wave][l16] = m;
         wave_l[wave][l16] = l;
     }
+    float sk = 0.0f;                         // (requested in front of the barriers)
+    if (tid < 16 && r0 + tid < rows) sk = p.sink[(r0 + tid) % p.heads];
     __syncthreads();
     float* Os = reinterpret_cast<float*>(lds_raw);                   // [4][16][kSums]
 #pragma unroll
     for (int d = 0; d < NT; ++d) *reinterpret_cast<f32x4_t*>(Os + (wave * 16 + l16) * L::kSums + d * 16 + lq * 4) = o[d];
+    // a row's waves against each other: their weights, and with one range the sink and the division
+    if (tid < 16 && r0 + tid < rows) {
+        float top = splits == 1 ? sk : -INFINITY, sum = 0.0f, weight[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) top = fmaxf(top, wave_m[w][tid]);
+        const float base = top == -INFINITY ? 0.0f : top;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            weight[w] = expf(wave_m[w][tid] - base);
+            sum = fmaf(wave_l[w][tid], weight[w], sum);
+        }
+        const float inv = splits == 1 ? 1.0f / (sum + expf(sk - base)) : 1.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) wave_l[w][tid] = weight[w] * inv;
+        if (splits > 1) {
+            const int64_t at = static_cast<int64_t>(q0) * p.heads + r0 + tid;
+            part_ml[(at * splits + split) * 2] = top;
+            part_ml[(at * splits + split) * 2 + 1] = sum;
+        }
+    }
     __syncthreads();
     for (int i = tid; i < 16 * (pitch_c / 4); i += 256) {
         const int rr = i / (pitch_c / 4), c = (i - rr * (pitch_c / 4)) * 4;
         if (r0 + rr >= rows) continue;
         const int64_t at = static_cast<int64_t>(q0) * p.heads + r0 + rr;
-        const float sk = p.sink[(r0 + rr) % p.heads];
-        float top = splits == 1 ? sk : -INFINITY;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) top = fmaxf(top, wave_m[w][rr]);
-        const float base = top == -INFINITY ? 0.0f : top;
-        float sum = 0.0f;
         f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const float weight = expf(wave_m[w][rr] - base);
-            sum = fmaf(wave_l[w][rr], weight, sum);
-            v += *reinterpret_cast<const f32x4_t*>(Os + (w * 16 + rr) * L::kSums + c) * weight;
-        }
+        for (int w = 0; w < 4; ++w) v += *reinterpret_cast<const f32x4_t*>(Os + (w * 16 + rr) * L::kSums + c) * wave_l[w][rr];
         if (splits == 1) {
-            const float inv = 1.0f / (sum + expf(sk - base));
             uint16_t* out = static_cast<uint16_t*>(p.out) + at * pitch_c + c;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) out[j] = f32_to_bf16_bits(c + j < p.rank ? v[j] * inv : 0.0f);
+            for (int j = 0; j < 4; ++j) out[j] = f32_to_bf16_bits(c + j < p.rank ? v[j] : 0.0f);
         } else {
             *reinterpret_cast<f32x4_t*>(part_o + (at * splits + split) * pitch_c + c) = v;
-            if (c == 0) {
-                part_ml[(at * splits + split) * 2] = top;
-                part_ml[(at * splits + split) * 2 + 1] = sum;
-            }
         }
     }
 }
