@@ -96,6 +96,19 @@ struct TokenSideProblem {
 };
 int launch_token_gate(const void* x, const void* gate, const int32_t* tokens, const void* table, int64_t table_stride,
                       int column0, void* g, int64_t T, int W, int dim, int dtype, hipStream_t s);
+struct TokenInputProblem {
+    const uint16_t *x, *gate, *proj;      // [T, W], [dim, W], [W, dim]
+    const int32_t* tokens;
+    const uint16_t* table;
+    int64_t table_stride;
+    int column0;
+    float* parts;                         // [n_parts, T, dim]
+    uint16_t* out;                        // [T, W]
+    int64_t T;
+    int W, dim, n_parts;
+};
+int token_input_parts(int64_t T, int W, int dim);
+int launch_token_input(const TokenInputProblem& p, hipStream_t s);
 bool token_side_supported(int W, int dim);
 inline bool token_side_packable(int W, int dim) { return W % 128 == 0 && dim % 32 == 0; }
 bool token_side_pack_pays(int64_t T, int W, int dim);

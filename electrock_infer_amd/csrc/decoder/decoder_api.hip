@@ -258,6 +258,25 @@ int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const 
     return launch_token_gate(x, gate, tokens, table, table_stride, column0, g, T, W, dim, dtype, as_stream(stream));
 }
 
+int ed_token_input_parts(int64_t T, int W, int dim) { return T > kMaxRows ? 0 : token_input_parts(T, W, dim); }
+
+int ed_token_input(const void* x, const void* gate, const void* proj, const int32_t* tokens, const void* table, int64_t table_stride,
+                   int column0, float* parts, int n_parts, void* out, int64_t T, int W, int dim, void* stream) {
+    if (T < 0 || T > kMaxRows || column0 < 0 || column0 + static_cast<int64_t>(dim) > table_stride) return EM_ERR_BAD_SHAPE;
+    if (T == 0) return 0;
+    if (token_input_parts(T, W, dim) == 0) return EM_ERR_UNSUPPORTED;
+    if (n_parts < 1 || n_parts > W / 32 || n_parts > 65535) return EM_ERR_BAD_SHAPE;
+    if (!x || !gate || !proj || !tokens || !table || !parts || !out) return EM_ERR_NULL_POINTER;
+    if (!aligned16(x) || !aligned16(gate) || !aligned16(proj) || !aligned16(parts) || !aligned16(out) || column0 % 4 != 0 || table_stride % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(table) % 8 != 0)
+        return EM_ERR_ALIGNMENT;
+    TokenInputProblem p;
+    p.x = static_cast<const uint16_t*>(x); p.gate = static_cast<const uint16_t*>(gate); p.proj = static_cast<const uint16_t*>(proj);
+    p.tokens = tokens; p.table = static_cast<const uint16_t*>(table); p.table_stride = table_stride; p.column0 = column0;
+    p.parts = parts; p.out = static_cast<uint16_t*>(out); p.T = T; p.W = W; p.dim = dim; p.n_parts = n_parts;
+    return launch_token_input(p, as_stream(stream));
+}
+
 int ed_token_side_supported(int W, int dim) { return token_side_supported(W, dim) ? 1 : 0; }
 
 namespace {

@@ -12,6 +12,8 @@
 // bytes of the rows and, in between, the address unit that serves the weights' fragments.  Packed weights lie in operand order,
 // a wave's load is 1 KB that lies whole instead of 16 half-used lines, and what this saves in registers keeps the rows, which
 // were read twice before (8192 rows, with the packing: W = 1024 46.9 -> 32.7 us, 2048 84.2 -> 67.8, 4096 215 -> 145).
+#include <algorithm>
+
 #include "decoder.h"
 #include "mma.h"
 
@@ -83,6 +85,128 @@ __global__ __launch_bounds__(kThreads) void token_gate_kernel(const typename Ele
             for (int w = 0; w < kWaves; ++w) z += part[w][tid];
             const float e = Elem::load(table[static_cast<int64_t>(tokens[t0 + r]) * table_stride + column0 + d]);
             g[(t0 + r) * dim + d] = Elem::store(gelu_tanh(z) * e);
+        }
+    }
+}
+
+// The same and the projection behind it, p = proj g, in two launches of which neither waits for one CU's share of the weights: the gate product's
+// k is shared out over workgroups, which leave partial sums, and every workgroup of the projection adds up those of its tokens, a
+// few KB, in front of the gelu.  (As token_gate_kernel takes it, 23 tokens of 4096 columns are eight workgroups that bring in 256 KB each,
+// and more tokens are read once per 16 rows of the gate.)  MT: 16-token tiles of a workgroup; ND: 16-row tiles of the gate.
+template <int ND>
+__global__ __launch_bounds__(256) void token_parts_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gate, float* __restrict__ parts,
+                                                          int64_t T, int W) {
+    typedef Mma<BF16Elem> M;
+    constexpr int kAhead = ND <= 4 ? 4 : 2, kWavesHere = 4, kCols = ND * 16;
+    __shared__ __attribute__((aligned(16))) float sums[kWavesHere][16][kCols + 4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 16;
+    const int steps = W / 32, first = static_cast<int>(static_cast<int64_t>(steps) * blockIdx.y / gridDim.y),
+              end = static_cast<int>(static_cast<int64_t>(steps) * (blockIdx.y + 1) / gridDim.y);
+    const uint16_t *xr = x + min(t0 + l16, T - 1) * W + lq * 8, *wr[ND];
+#pragma unroll
+    for (int n = 0; n < ND; ++n) wr[n] = gate + static_cast<int64_t>(n * 16 + l16) * W + lq * 8;
+    f32x4_t acc[ND];
+#pragma unroll
+    for (int n = 0; n < ND; ++n) acc[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = first + wave; s < end; s += kWavesHere * kAhead) {
+        M::frag fx[kAhead], fw[kAhead][ND];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int k = min(s + u * kWavesHere, end - 1) * 32;
+            fx[u] = M::load(xr + k);
+#pragma unroll
+            for (int n = 0; n < ND; ++n) fw[u][n] = M::load(wr[n] + k);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (s + u * kWavesHere >= end) break;
+#pragma unroll
+            for (int n = 0; n < ND; ++n) acc[n] = M::mac(fw[u][n], fx[u], acc[n]);
+        }
+    }
+    // element i of a fragment: token l16, gate row lq * 4 + i
+#pragma unroll
+    for (int n = 0; n < ND; ++n) *reinterpret_cast<f32x4_t*>(&sums[wave][l16][n * 16 + lq * 4]) = acc[n];
+    __syncthreads();
+    float* out = parts + (static_cast<int64_t>(blockIdx.y) * T + t0) * kCols;
+    for (int i = tid; i < 16 * (kCols / 4); i += 256) {
+        const int t = i / (kCols / 4), c = (i - t * (kCols / 4)) * 4;
+        if (t0 + t >= T) break;
+        f32x4_t v = *reinterpret_cast<const f32x4_t*>(&sums[0][t][c]);
+#pragma unroll
+        for (int w = 1; w < kWavesHere; ++w) v += *reinterpret_cast<const f32x4_t*>(&sums[w][t][c]);
+        *reinterpret_cast<f32x4_t*>(out + t * kCols + c) = v;
+    }
+}
+
+// MT: 16-token tiles of a workgroup; ND: 32-element steps of g; NT: 16-column tiles of a wave
+template <int MT, int ND, int NT>
+__global__ __launch_bounds__(256) void token_proj_kernel(const float* __restrict__ parts, int n_parts, const int32_t* __restrict__ tokens,
+                                                         const uint16_t* __restrict__ table, int64_t table_stride, int column0,
+                                                         const uint16_t* __restrict__ proj, uint16_t* __restrict__ out, int64_t T, int W) {
+    typedef Mma<BF16Elem> M;
+    constexpr int kCols = ND * 32, LPG = kCols + 8, kPieces = MT * 16 * (kCols / 4) / 256, kMost = 8;
+    __shared__ __attribute__((aligned(16))) uint16_t Gs[MT * 16 * LPG];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * (16 * MT);
+    M::frag fw[NT][ND];
+    auto fetch = [&](int n0) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int k = 0; k < ND; ++k) fw[n][k] = M::load(proj + static_cast<int64_t>(min(n0 + n * 16 + l16, W - 1)) * kCols + k * 32 + lq * 8);
+    };
+    const int first = (static_cast<int>(blockIdx.y) * 4 + wave) * (NT * 16), step = static_cast<int>(gridDim.y) * (NT * 64);
+    fetch(first);
+    static_assert(MT * 16 * (kCols / 4) % 256 == 0 || MT * 16 * (kCols / 4) == 128, "pieces of four to a thread");
+    constexpr bool kHalf = kPieces == 0;                 // (16 tokens of 32 columns: every other wave)
+#pragma unroll
+    for (int i = 0; i < (kHalf ? 1 : kPieces); ++i) {
+        const int e = tid + i * 256, t = e / (kCols / 4), c = (e - t * (kCols / 4)) * 4;
+        if (kHalf && tid >= 128) break;
+        const int64_t row = min(t0 + t, T - 1);
+        const float* from = parts + row * kCols + c;
+        u32x2_t side;
+        __builtin_memcpy(&side, __builtin_assume_aligned(table + static_cast<int64_t>(tokens[row]) * table_stride + column0 + c, 8), 8);
+        f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int p0 = 0; p0 < n_parts; p0 += kMost) {
+            f32x4_t v[kMost];
+#pragma unroll
+            for (int j = 0; j < kMost; ++j) v[j] = *reinterpret_cast<const f32x4_t*>(from + static_cast<int64_t>(min(p0 + j, n_parts - 1)) * T * kCols);
+#pragma unroll
+            for (int j = 0; j < kMost; ++j)
+                if (p0 + j < n_parts) z += v[j];
+        }
+        const u32x2_t g = {pack_bf16(gelu_tanh(z[0]) * bf16_lo(side[0]), gelu_tanh(z[1]) * bf16_hi(side[0])),
+                           pack_bf16(gelu_tanh(z[2]) * bf16_lo(side[1]), gelu_tanh(z[3]) * bf16_hi(side[1]))};
+        *reinterpret_cast<u32x2_t*>(Gs + t * LPG + c) = g;
+    }
+    __syncthreads();
+    M::frag fg[MT][ND];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int k = 0; k < ND; ++k) fg[m][k] = M::load(Gs + (m * 16 + l16) * LPG + k * 32 + lq * 8);
+    for (int n0 = first; n0 < W; n0 += step) {
+        f32x4_t acc[NT][MT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                acc[n][m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k = 0; k < ND; ++k) acc[n][m] = M::mac(fw[n][k], fg[m][k], acc[n][m]);
+            }
+        if (n0 + step < W) fetch(n0 + step);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int64_t t = t0 + m * 16 + l16;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const int c = n0 + n * 16 + lq * 4;
+                if (t < T && c < W) *reinterpret_cast<u32x2_t*>(out + t * W + c) = u32x2_t{pack_bf16(acc[n][m][0], acc[n][m][1]), pack_bf16(acc[n][m][2], acc[n][m][3])};
+            }
         }
     }
 }
@@ -401,6 +525,55 @@ int launch_token_gate(const void* x, const void* gate, const int32_t* tokens, co
         launch((token_gate_kernel<F32Elem>), grid, dim3(kThreads), 0, s, static_cast<const float*>(x),
                static_cast<const float*>(gate), tokens, static_cast<const float*>(table), table_stride, column0,
                static_cast<float*>(g), T, W, dim);
+    return launch_status();
+}
+
+// How many ranges of W the gate product is shared out over: a workgroup for every CU (of 16 tokens, or the tiled product's of 64), 256
+// columns at least, and as few sums to add up as still pay; 0: the gate and the projection one by one (what this does not take, and where
+// it is not faster).  us, one by one / this, gates of 64: W = 4096, one token 9.5 / 6.8, 23 12.2 / 8.4, 64 13.2 / 8.6, 300 13.9 / 11.4, 1000 16.6 /
+// 15.0, 2244 33.5 / 24.6, 6000 66.5 / 41.7; 2048, one 6.8 / 6.2, 23 8.4 / 7.0, 300 9.7 / 9.2, 700 10.7 / 11.8, 1000 11.0 / 11.7, 1500 15.9 / 15.0, 3500 25.7 / 22.6.
+constexpr int64_t kFewTokens = 64, kSomeTokens = 512;
+int token_input_parts(int64_t T, int W, int dim) {
+    if (T <= 0 || W <= 0 || W % 64 != 0 || (dim != 32 && dim != 64 && dim != 128) || (T > kFewTokens && !tile_gemm_supported(T, dim, W))) return 0;
+    if (T > kSomeTokens && T < 1280 && W <= 2048) return 0;
+    const int64_t groups = T > kFewTokens ? ceil_div(T, 64) * ceil_div(dim, 64) : ceil_div(T, 16), most = std::max(W / 256, 1);
+    return static_cast<int>(std::min<int64_t>({most, std::max<int64_t>(1, 256 / groups), T > kSomeTokens ? 4 : T > kFewTokens ? 8 : 16}));
+}
+
+int launch_token_input(const TokenInputProblem& p, hipStream_t s) {
+    if (p.T > kFewTokens) {
+        TileGemm g{};
+        g.x = p.x; g.x_stride = p.W; g.w = p.gate; g.w_stride = p.W; g.out = p.parts; g.f32 = true;
+        g.splits = p.n_parts; g.T = static_cast<int>(p.T); g.N = p.dim; g.K = p.W;
+        const int rc = launch_tile_gemm(g, s);
+        if (rc != 0) return rc;
+    }
+#define EM_PARTS(ND) launch((token_parts_kernel<ND>), dim3(static_cast<unsigned>(ceil_div(p.T, 16)), static_cast<unsigned>(p.n_parts)), dim3(256), 0, s, p.x, p.gate, p.parts, p.T, p.W)
+    // how many workgroups share a row's columns: two to a CU, as every one adds up its tokens' sums anew
+    auto columns = [&](int mt, int nt) {
+        const int64_t groups = ceil_div(p.T, 16 * mt), all = ceil_div(p.W, 64 * nt);
+        return static_cast<unsigned>(std::min<int64_t>(all, std::max<int64_t>(1, ceil_div(512, groups))));
+    };
+#define EM_PROJ(MT, ND, NT)                                                                                                              \
+    launch((token_proj_kernel<MT, ND, NT>), dim3(static_cast<unsigned>(ceil_div(p.T, 16 * MT)), columns(MT, NT)), dim3(256), 0, s, \
+           p.parts, p.n_parts, p.tokens, p.table, p.table_stride, p.column0, p.proj, p.out, p.T, p.W)
+#define EM_BOTH(ND)                                         \
+    do {                                                    \
+        if (p.T <= kFewTokens) {                            \
+            EM_PARTS(2 * ND);                               \
+            EM_PROJ(1, ND, 1);                              \
+        } else if (p.T <= kSomeTokens) {                    \
+            EM_PROJ(1, ND, 4);                              \
+        } else {                                            \
+            EM_PROJ(2, ND, 4);                              \
+        }                                                   \
+    } while (0)
+    if (p.dim == 32) EM_BOTH(1);
+    else if (p.dim == 64) EM_BOTH(2);
+    else EM_BOTH(4);
+#undef EM_BOTH
+#undef EM_PROJ
+#undef EM_PARTS
     return launch_status();
 }
 

@@ -221,6 +221,23 @@ def token_gate(x: torch.Tensor, gate: torch.Tensor, tokens: torch.Tensor, table:
     return g
 
 
+def token_input(x: torch.Tensor, gate: torch.Tensor, proj: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor, column0: int) -> torch.Tensor:
+    """(gelu_tanh(x @ gate^T) * table[tokens, column0 : column0 + dim]) @ proj^T: two launches that share the gate's weights out over the
+    chip, or ``token_gate`` and ``linear`` where those take the call or are the faster way."""
+    (T, W), dim, lib = x.shape, gate.shape[0], _lib.load_decoder()
+    if x.is_cuda and _plain(x, gate) and _dense(x, gate) and type(proj) in _PLAIN_TYPES and proj.dtype is _BF16 and proj.shape == (W, dim) and \
+            proj.is_contiguous() and proj.device == x.device and not (proj.requires_grad and torch.is_grad_enabled()) and table.dtype is _BF16 and \
+            table.stride(1) == 1 and (table.stride(0) | column0) % 4 == 0 and proj.data_ptr() % 16 == 0 and table.data_ptr() % 8 == 0:
+        parts = lib.ed_token_input_parts(T, W, dim)
+        if parts > 0:
+            sums, out = torch.empty(parts, T, dim, dtype=torch.float32, device=x.device), torch.empty_like(x)
+            code = lib.ed_token_input(x.data_ptr(), gate.data_ptr(), proj.data_ptr(), tokens.data_ptr(), table.data_ptr(), table.stride(0), column0,
+                                      sums.data_ptr(), parts, out.data_ptr(), T, W, dim, _lib.current_stream(x.device))
+            _lib.check_decoder(code, "token_input")
+            return out
+    return linear(token_gate(x, gate, tokens, table, column0), proj)
+
+
 def pad_k(w: torch.Tensor) -> torch.Tensor:
     """[heads, N, K] with K zero-padded to a multiple of 32: the operand form of ``head_gemm``."""
     return F.pad(w, (0, -w.shape[-1] % 32)).contiguous()

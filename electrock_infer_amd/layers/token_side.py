@@ -4,7 +4,7 @@ import torch
 from torch import nn
 
 from .. import _lib
-from .decoder_ops import ADD_NORMED, linear, residual_norm, token_gate
+from .decoder_ops import ADD_NORMED, residual_norm, token_input
 
 
 class TokenSideInput(nn.Module):
@@ -29,7 +29,7 @@ class TokenSideInput(nn.Module):
 
     def forward(self, x: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
         """x [T, width] (the stream in the compute type) -> what is to be normed with ``norm`` and added."""
-        return linear(token_gate(x, self.gate, tokens, table, self.column0), self.proj)
+        return token_input(x, self.gate, self.proj, tokens, table, self.column0)
 
     def close_layer(self, x: torch.Tensor, y: torch.Tensor, post_w: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor,
                     eps: float, out: torch.Tensor, next_w) -> None:

@@ -77,6 +77,16 @@ int ed_tile_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_strid
 int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const void* table, int64_t table_stride,
                   int column0, void* g, int64_t T, int W, int dim, int dtype, void* stream);
 
+/*
+ * proj (gelu_tanh(gate x) * table[tokens, column0 : column0 + dim]) in bf16, x [T, W], gate [dim, W], proj [W, dim], out [T, W]: the token
+ * gate and the projection behind it.  parts: room for [n_parts, T, dim] float32 partial sums of the gate product;
+ * ed_token_input_parts: how many to ask for, 0: sizes that it does not take (W % 64, dim of 32, 64 and 128) or that are faster one by one.
+ * column0 and table_stride are multiples of four.
+ */
+int ed_token_input_parts(int64_t T, int W, int dim);
+int ed_token_input(const void* x, const void* gate, const void* proj, const int32_t* tokens, const void* table, int64_t table_stride,
+                   int column0, float* parts, int n_parts, void* out, int64_t T, int W, int dim, void* stream);
+
 /* The end of a layer with a per-layer token input in one launch (bf16; W a multiple of 4, see
  * ed_token_side_supported):
  *   x += y / rms(y) * post_w;  g = gelu_tanh(gate x) * table[tokens[t]][column0 ...];  p = proj g;
