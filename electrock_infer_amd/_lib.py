@@ -258,9 +258,13 @@ def check_decoder(code: int, what: str) -> None:
 
 
 _dtype_codes = {}
+_raw_stream = None      # torch's (torch is imported where it is first needed)
 
 
 def dtype_code(dtype) -> int:
+    code = _dtype_codes.get(dtype)
+    if code is not None:
+        return code
     if not _dtype_codes:
         import torch
         _dtype_codes.update({torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16})
@@ -271,11 +275,15 @@ def dtype_code(dtype) -> int:
 
 
 def current_stream(device) -> int:
-    """The handle of torch's current stream of a device (without the Stream object that wraps it: 0.3 us instead of 3.5,
+    """The handle of torch's current stream of a device (without the Stream object that wraps it: 0.2 us instead of 3.5,
     on every launch)."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        _raw_stream = torch._C._cuda_getCurrentRawStream, torch.device
+    if type(device) is _raw_stream[1] and device.type == "cuda" and device.index is not None:
+        return _raw_stream[0](device.index)
     import torch
-    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
-        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

@@ -48,13 +48,17 @@ def _dense(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0
 
 
-def _row_stride(t: torch.Tensor) -> int:
-    return t.stride(0) if t.shape[0] > 1 else t.shape[1]       # (a single row's may be anything)
-
-
-def _rows_apart(t: torch.Tensor) -> bool:
-    """Whole rows from 16-byte boundaries."""
-    return t.stride(1) == 1 and _row_stride(t) >= t.shape[1] and _row_stride(t) % 8 == 0 and t.data_ptr() % 16 == 0
+def _pitch(t: torch.Tensor, columns: int) -> int:
+    """Elements from row to row of a matrix of whole rows from 16-byte boundaries, else 0.  (Asked twice for every product: the common
+    answer costs 0.4 us of the host's time, the general one 1.6.)"""
+    if t.is_contiguous():
+        pitch = columns
+    else:
+        stride, step = t.stride()
+        pitch = stride if t.shape[0] > 1 else columns          # (a single row's may be anything)
+        if step != 1 or pitch < columns:
+            return 0
+    return pitch if pitch % 8 == 0 and t.data_ptr() % 16 == 0 else 0
 
 
 def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -64,12 +68,15 @@ def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def _tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Operands of the tiled kernel beyond a decode batch: any rows from 16-byte boundaries."""
-    return x.is_cuda and _plain(x, weight) and x.shape[0] > 64 and _rows_apart(x) and _rows_apart(weight)
+    return x.is_cuda and _plain(x, weight) and x.shape[0] > 64 and _pitch(x, x.shape[1]) > 0 and _pitch(weight, x.shape[1]) > 0
 
 
 def _taken(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Either of the two, asked once."""
-    return x.is_cuda and _plain(x, weight) and (_dense(x, weight) if x.shape[0] <= 64 else _rows_apart(x) and _rows_apart(weight))
+    if not x.is_cuda or not _plain(x, weight):
+        return False
+    T, K = x.shape
+    return _dense(x, weight) if T <= 64 else _pitch(x, K) > 0 and _pitch(weight, K) > 0
 
 
 def _decode_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
@@ -80,9 +87,10 @@ def _decode_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, split
 
 
 def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
-    code = _lib.load_decoder().ed_tile_gemm(x.data_ptr(), _row_stride(x), weight.data_ptr(), _row_stride(weight), out.data_ptr(),
-                                            _lib.dtype_code(out.dtype), splits, x.shape[0], cols, x.shape[1], act,
-                                            _lib.current_stream(x.device))
+    T, K = x.shape
+    a, b = x.stride(0) if T > 1 else K, weight.stride(0) if cols > 1 else _pitch(weight, K)         # (checked by who calls this)
+    code = _lib.load_decoder().ed_tile_gemm(x.data_ptr(), a, weight.data_ptr(), b, out.data_ptr(), _lib.dtype_code(out.dtype), splits, T, cols,
+                                            K, act, _lib.current_stream(x.device))
     _lib.check_decoder(code, "tile_gemm")
     return out
 
@@ -143,12 +151,14 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor, exact: bool = False) -> 
     if _taken(x, weight):
         (T, K), N, lib = x.shape, weight.shape[0], _lib.load_decoder()
         splits = lib.ed_tile_gemm_splits(T, N, K)
-        run = _tile_gemm if splits > 0 else _decode_gemm
-        splits = splits or lib.ed_decode_gemm_splits(T, N, K)
         if splits > 1:
-            return run(x, weight, torch.empty(splits, T, N, dtype=torch.float32, device=x.device), splits, N, 0)
+            return _tile_gemm(x, weight, torch.empty(splits, T, N, dtype=torch.float32, device=x.device), splits, N, 0)
         if splits == 1 and T > 64:                    # (a decode batch's whole results: whichever kernel is the fastest for those)
             return _tile_gemm(x, weight, torch.empty(T, N, dtype=torch.float32 if exact else x.dtype, device=x.device), 1, N, 0)
+        if splits == 0:
+            splits = lib.ed_decode_gemm_splits(T, N, K)
+            if splits > 1:
+                return _decode_gemm(x, weight, torch.empty(splits, T, N, dtype=torch.float32, device=x.device), splits, N, 0)
     return linear_f32(x, weight) if exact else linear(x, weight)
 
 
@@ -172,12 +182,16 @@ def residual_norm(update: int, x: torch.Tensor, y: Optional[torch.Tensor], post_
     the next sublayer's input into ``out`` (rows may be strided): x / rms(x) * next_w, or x itself, in out's type.
     ``y`` [T, W] or partial sums [parts, T, W] (``linear_parts``)."""
     T, W = x.shape
-    parts = y.shape[0] if y is not None and y.dim() == 3 else 1
-    dtype = out.dtype if out is not None else (y.dtype if y is not None else x.dtype)
-    code = _lib.load_decoder().ed_residual_norm(
-        update, x.data_ptr(), _ptr(y), _lib.dtype_code(y.dtype if y is not None else dtype), parts, _ptr(post_w), _ptr(next_w),
-        _ptr(out), out.stride(0) if out is not None else 0, T, W, float(eps), _lib.dtype_code(dtype),
-        _lib.current_stream(x.device))
+    y_ptr, parts, y_type = None, 1, None
+    if y is not None:
+        y_ptr, y_type = y.data_ptr(), y.dtype
+        if y.dim() == 3:
+            parts = y.shape[0]
+    out_ptr, out_stride, dtype = None, 0, y_type if y_type is not None else x.dtype
+    if out is not None:
+        out_ptr, out_stride, dtype = out.data_ptr(), out.stride(0), out.dtype
+    code = _lib.load_decoder().ed_residual_norm(update, x.data_ptr(), y_ptr, _lib.dtype_code(y_type or dtype), parts, _ptr(post_w), _ptr(next_w),
+                                                out_ptr, out_stride, T, W, float(eps), _lib.dtype_code(dtype), _lib.current_stream(x.device))
     _lib.check_decoder(code, "residual_norm")
 
 

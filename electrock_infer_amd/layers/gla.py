@@ -50,12 +50,14 @@ class GatedLinearAttention(nn.Module):
         if batch.max_q == 1:
             _lib.check_decoder(lib.ed_gla_step(byref(a), stream), "gla_step")
         else:
-            log_decay = torch.empty(T, self.heads * self.dim, dtype=torch.float32, device=h.device)
-            a.log_decay, a.chunks, a.seq_chunks = log_decay.data_ptr(), batch.chunks.data_ptr(), batch.seq_chunks.data_ptr()
+            # float32 scratch in one piece: decays, and with several chunks to a sequence their states and decays
+            channels = self.heads * self.dim
+            chunks = batch.n_chunks if batch.n_chunks > batch.n_seqs else 0
+            scratch = torch.empty(-(-(T + chunks) * channels // 4) * 4 + chunks * channels * self.vdim, dtype=torch.float32, device=h.device)
+            a.log_decay, a.chunks, a.seq_chunks = scratch.data_ptr(), batch.chunks.data_ptr(), batch.seq_chunks.data_ptr()
             a.n_chunks, a.chunk_tokens = batch.n_chunks, batch.chunk_tokens
-            if batch.n_chunks > batch.n_seqs:
-                cs = torch.empty(batch.n_chunks, *self.state_shape(), dtype=torch.float32, device=h.device)
-                cd = torch.empty(batch.n_chunks, self.heads * self.dim, dtype=torch.float32, device=h.device)
-                a.chunk_states, a.chunk_decay = cs.data_ptr(), cd.data_ptr()
+            if chunks:
+                a.chunk_decay = a.log_decay + T * channels * 4
+                a.chunk_states = a.log_decay + -(-(T + chunks) * channels // 4) * 16
             _lib.check_decoder(lib.ed_gla_prefill(byref(a), stream), "gla_prefill")
         return linear_parts(out, self.o)

@@ -65,15 +65,17 @@ class DecayedRecurrence(nn.Module):
         if batch.max_q == 1:
             _lib.check_decoder(lib.ed_recur_step(byref(a), stream), "recur_step")
             return out
-        f32 = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)
+        # scratch in one piece, every part from a 256-byte boundary
         H, padded, chunks = self.heads, -(-self.dim // 16) * 16, batch.n_chunks
-        scratch = {"q_rows": f32(T, self.kv_heads, padded), "k_rows": f32(T, self.kv_heads, padded), "v_rows": torch.empty_like(out),
-                   "rates": f32(T, H, 2), "blocks": f32(chunks, batch.chunk_tokens // 16, H, lib.ed_recur_record(int(delta)))}
+        parts = [("q_rows", T * self.kv_heads * padded * 4), ("k_rows", T * self.kv_heads * padded * 4), ("v_rows", T * H * self.vdim * out.element_size()),
+                 ("rates", T * H * 8), ("blocks", chunks * (batch.chunk_tokens // 16) * H * lib.ed_recur_record(int(delta)) * 4)]
         if chunks > batch.n_seqs:
-            scratch["chunk_states"] = f32(chunks, *self.state_shape())
-            scratch["chunk_trans"] = f32(chunks, H, padded, padded) if delta else f32(chunks, H)
-        for name, t in scratch.items():
-            setattr(a, name, t.data_ptr())
+            parts += [("chunk_states", chunks * H * self.dim * self.vdim * 4), ("chunk_trans", chunks * H * (padded * padded if delta else 1) * 4)]
+        scratch = torch.empty(sum(-(-size // 256) * 256 for _, size in parts), dtype=torch.uint8, device=dev)
+        at = scratch.data_ptr()
+        for name, size in parts:
+            setattr(a, name, at)
+            at += -(-size // 256) * 256
         a.q_begin, a.chunks, a.seq_chunks = batch.q_begin.data_ptr(), batch.chunks.data_ptr(), batch.seq_chunks.data_ptr()
         a.n_chunks, a.chunk_tokens = chunks, batch.chunk_tokens
         _lib.check_decoder(lib.ed_recur_prefill(byref(a), stream), "recur_prefill")
