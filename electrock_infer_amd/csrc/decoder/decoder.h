@@ -62,6 +62,21 @@ bool decode_gemm_pays(int64_t T, int rows, int K, int act, bool f32);
 int skinny_splits(int T, int N, int K);
 int launch_skinny_gemm(const void* x, const void* w, void* out, bool f32, int splits, int T, int N, int K, int act, hipStream_t s);
 
+// ---- norm_gemm.hip ----
+struct NormGemm {
+    const float *x, *post_w, *next_w;    // [T, K], [K], [K] or null
+    const void* y;                       // [parts, T, K]
+    const uint16_t* w;                   // [N, K]; act 2: [2 N, K]
+    float* x_out;                        // [T, K], not x
+    uint16_t* out;                       // [T, N]
+    bool y_bf16;
+    int parts, T, N, K, act;
+    float eps;
+};
+bool norm_gemm_supported(int64_t T, int N, int K, int act);
+bool norm_gemm_pays(int T, int N, int K, int act);
+int launch_norm_gemm(const NormGemm& g, hipStream_t s);
+
 // ---- tile_gemm.hip ----
 struct TileGemm {
     const uint16_t *x, *w;       // rows x_stride and w_stride elements apart

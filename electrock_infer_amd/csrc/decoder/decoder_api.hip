@@ -220,6 +220,26 @@ int ed_decode_gemm(const void* x, const void* w, void* out, int out_dtype, int s
     return launch_skinny_gemm(x, w, out, out_dtype == EM_DTYPE_F32, splits, static_cast<int>(T), N, K, act, as_stream(stream));
 }
 
+int ed_norm_gemm_supported(int64_t T, int N, int K, int act) { return norm_gemm_supported(T, N, K, act) ? 1 : 0; }
+
+int ed_norm_gemm_pays(int64_t T, int N, int K, int act) { return norm_gemm_supported(T, N, K, act) && norm_gemm_pays(static_cast<int>(T), N, K, act) ? 1 : 0; }
+
+int ed_norm_gemm(const float* x, const void* y, int y_dtype, int y_parts, const float* post_w, const float* next_w, float* x_out, const void* w,
+                 void* out, int64_t T, int N, int K, int act, double eps, void* stream) {
+    if (!dtype_ok(y_dtype)) return EM_ERR_BAD_DTYPE;
+    if (T == 0) return 0;
+    if (!norm_gemm_supported(T, N, K, act)) return EM_ERR_UNSUPPORTED;
+    if (y_parts < 1 || y_parts > 64 || (y_parts > 1 && y_dtype != EM_DTYPE_F32)) return EM_ERR_BAD_SHAPE;
+    if (!x || !y || !post_w || !x_out || !w || !out) return EM_ERR_NULL_POINTER;
+    if (x == x_out) return EM_ERR_BAD_SHAPE;
+    if (!aligned16(x) || !aligned16(y) || !aligned16(post_w) || !aligned16(next_w) || !aligned16(x_out) || !aligned16(w)) return EM_ERR_ALIGNMENT;
+    NormGemm g;
+    g.x = x; g.post_w = post_w; g.next_w = next_w; g.y = y; g.w = static_cast<const uint16_t*>(w); g.x_out = x_out;
+    g.out = static_cast<uint16_t*>(out); g.y_bf16 = y_dtype == EM_DTYPE_BF16; g.parts = y_parts;
+    g.T = static_cast<int>(T); g.N = N; g.K = K; g.act = act; g.eps = static_cast<float>(eps);
+    return launch_norm_gemm(g, as_stream(stream));
+}
+
 int ed_tile_gemm_splits(int64_t T, int N, int K) {
     return tile_gemm_pays(T, N, K, 0, true) ? tile_gemm_splits(T, N, K) : 0;
 }

@@ -1,0 +1,278 @@
+// out = act(h w^T) for the row or two h that a residual norm leaves (bf16):
+//     x_out = x + y / rms(y) * post_w,   h = next_w ? x_out / rms(x_out) * next_w : x_out, rounded to bf16
+// One launch instead of two.  Every workgroup norms the rows anew while its weights, all of a wave's part of them at K <= 4096, are on
+// their way; the first one leaves the stream behind, in a place of its own, since the others still read x.
+//
+// Bound: the way from a launch to the first bytes, and the weights' bytes.  As in skinny_gemm.hip the waves share out k, load eight rows
+// of 128 bytes at a time and turn them through LDS of their own.  The rows' loads come first (they return in order), so that their two
+// sums over the workgroup run beside the weights' way.  A decode step of one token (width 2048, sixteen norms of which fifteen go this way)
+// 418 -> 389 us, width 4096 832 -> 785; another order of the columns in every workgroup changes nothing.
+#include <algorithm>
+
+#include "decoder.h"
+#include "mma.h"
+
+namespace em {
+namespace {
+
+constexpr int kStepK = 64;
+constexpr int kPitch = kStepK + 8;       // elements of a row in LDS
+constexpr int kWaves = 8, kThreads = kWaves * kWave;
+constexpr int kGroups = 256;             // a workgroup to a CU
+
+__device__ __forceinline__ u32x4_t load_once(const uint16_t* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+}
+__device__ __forceinline__ bf16x8_t as_frag(u32x4_t w) {
+    bf16x8_t f;
+    __builtin_memcpy(&f, &w, 16);
+    return f;
+}
+
+// LDS: the rows, a stretch of weights per wave, the waves' sums
+constexpr int rows_bytes(int rows, int K) { return rows * (K + 8) * 2; }
+constexpr int stage_bytes(int nt) { return kWaves * nt * 16 * kPitch * 2; }
+constexpr int sums_bytes(int rows, int nt) { return kWaves * rows * 16 * nt * 4; }
+
+// ROWS: rows that are normed; COLS: pieces of four columns to a thread (K <= 2048 * COLS); NT: tiles of 16 weight rows; AHEAD: steps in flight
+template <int ROWS, int COLS, int NT, int AHEAD, bool GLU>
+__global__ __launch_bounds__(kThreads) void norm_gemm_kernel(NormGemm g) {
+    typedef Mma<BF16Elem> M;
+    static_assert(!GLU || NT % 2 == 0, "tiles of both halves");
+    constexpr int kCols = 16 * NT, kOutCols = GLU ? kCols / 2 : kCols;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ float scratch[2][ROWS][kWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4, l8 = lane >> 3, c8 = (lane & 7) * 8;
+    const int K = g.K, T = g.T, N = g.N;
+    uint16_t* hs = reinterpret_cast<uint16_t*>(lds);
+    uint16_t* ws = reinterpret_cast<uint16_t*>(lds + rows_bytes(ROWS, K)) + wave * NT * 16 * kPitch;
+    float* sums = reinterpret_cast<float*>(lds + rows_bytes(ROWS, K) + stage_bytes(NT));
+
+    // ---- the rows' loads, then the weights' ----
+    constexpr int kParts = 4;            // partial sums requested at once
+    float xv[ROWS][COLS][4], v[kParts][ROWS][COLS][4], pw[COLS][4], nw[COLS][4];
+    auto load_y = [&](int part, int r, int c, float (&to)[4]) {
+        const int64_t at = (static_cast<int64_t>(part) * T + r) * K + c;
+        if (g.y_bf16) {
+            const u32x2_t b = *reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(g.y) + at);
+            to[0] = bf16_lo(b[0]); to[1] = bf16_hi(b[0]); to[2] = bf16_lo(b[1]); to[3] = bf16_hi(b[1]);
+        } else {
+            const f32x4_t f = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(g.y) + at);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) to[e] = f[e];
+        }
+    };
+    auto load_f = [](const float* p, float (&to)[4]) {
+        const f32x4_t f = *reinterpret_cast<const f32x4_t*>(p);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) to[e] = f[e];
+    };
+#pragma unroll
+    for (int i = 0; i < COLS; ++i) {
+        const int c = min((tid + i * kThreads) * 4, K - 4);
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+#pragma unroll
+            for (int p = 0; p < kParts; ++p) load_y(min(p, g.parts - 1), min(r, T - 1), c, v[p][r][i]);
+            load_f(g.x + static_cast<int64_t>(min(r, T - 1)) * K + c, xv[r][i]);
+        }
+        load_f(g.post_w + c, pw[i]);
+        if (g.next_w != nullptr) load_f(g.next_w + c, nw[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int n0 = blockIdx.x * kOutCols, steps = K / kStepK;
+    const int mine = steps / kWaves, s0 = mine * wave, s1 = s0 + mine;
+    const uint16_t* wr[NT][2];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c = n0 + (GLU ? n / 2 : n) * 16 + h * 8 + l8;      // (columns beyond N are not stored)
+            wr[n][h] = g.w + (static_cast<int64_t>(c < N ? c : N - 1) + (GLU ? (n & 1) * static_cast<int64_t>(N) : 0)) * K + c8;
+        }
+    u32x4_t fw[AHEAD][NT][2];
+    auto fetch = [&](int s) {            // (a step behind the last is the last one again)
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) fw[u][n][h] = load_once(wr[n][h] + min(s + u, s1 - 1) * kStepK);
+    };
+    fetch(s0);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the norm ----
+    auto row_total = [&](float (&sum)[ROWS], int at) {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            sum[r] = column_sum(row_sum(sum[r]));
+            if (lane == 0) scratch[at][r][wave] = sum[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            sum[r] = 0.0f;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) sum[r] += scratch[at][r][w];
+            sum[r] = 1.0f / sqrtf(sum[r] / static_cast<float>(K) + g.eps);
+        }
+    };
+    float rstd[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        rstd[r] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < COLS; ++i) {
+#pragma unroll
+            for (int p = 1; p < kParts; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[0][r][i][e] += p < g.parts ? v[p][r][i][e] : 0.0f;
+            for (int p = kParts; p < g.parts; ++p) {
+                float more[4];
+                load_y(p, min(r, T - 1), min((tid + i * kThreads) * 4, K - 4), more);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[0][r][i][e] += more[e];
+            }
+            if ((tid + i * kThreads) * 4 < K) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rstd[r] = fmaf(v[0][r][i][e], v[0][r][i][e], rstd[r]);
+            }
+        }
+    }
+    row_total(rstd, 0);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < COLS; ++i) {
+            const int c = (tid + i * kThreads) * 4;
+            if (c >= K) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                xv[r][i][e] = xv[r][i][e] + v[0][r][i][e] * rstd[r] * pw[i][e];
+                sum = fmaf(xv[r][i][e], xv[r][i][e], sum);
+            }
+            if (blockIdx.x == 0 && r < T) *reinterpret_cast<f32x4_t*>(g.x_out + static_cast<int64_t>(r) * K + c) = f32x4_t{xv[r][i][0], xv[r][i][1], xv[r][i][2], xv[r][i][3]};
+        }
+        rstd[r] = sum;
+    }
+    if (g.next_w != nullptr) row_total(rstd, 1);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int i = 0; i < COLS; ++i) {
+            const int c = (tid + i * kThreads) * 4;
+            if (c >= K) continue;
+            if (g.next_w != nullptr) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xv[r][i][e] = xv[r][i][e] * rstd[r] * nw[i][e];
+            }
+            *reinterpret_cast<u32x2_t*>(hs + r * (K + 8) + c) = u32x2_t{pack_bf16(xv[r][i][0], xv[r][i][1]), pack_bf16(xv[r][i][2], xv[r][i][3])};
+        }
+    __syncthreads();
+
+    // ---- the product ----
+    f32x4_t acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint16_t* hr = hs + (l16 % ROWS) * (K + 8) + lq * 8;          // (rows of the tile beyond ROWS repeat them and are not stored)
+    for (int s = s0; s < s1; s += AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            if (s + u >= s1) continue;
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4_t*>(ws + (n * 16 + h * 8 + l8) * kPitch + c8) = fw[u][n][h];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (the stretch is this wave's own)
+            typename M::frag ax[2], aw[NT][2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                ax[h] = as_frag(*reinterpret_cast<const u32x4_t*>(hr + (s + u) * kStepK + h * 32));
+#pragma unroll
+                for (int n = 0; n < NT; ++n) aw[n][h] = as_frag(*reinterpret_cast<const u32x4_t*>(ws + (n * 16 + l16) * kPitch + h * 32 + lq * 8));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[n] = M::mac(ax[h], aw[n][h], acc[n]);
+        }
+        if (s + AHEAD < s1) fetch(s + AHEAD);
+    }
+    if (lq == 0) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) sums[(wave * ROWS + r) * kCols + n * 16 + l16] = acc[n][r];
+    }
+    __syncthreads();
+    for (int i = tid; i < ROWS * kOutCols; i += kThreads) {
+        const int t = i / kOutCols, c = i % kOutCols;
+        if (t >= T || n0 + c >= N) continue;
+        const float* at = sums + t * kCols + (GLU ? c / 16 * 32 + c % 16 : c);
+        float a = 0.0f, b = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) {
+            a += at[k * ROWS * kCols];
+            if (GLU) b += at[k * ROWS * kCols + 16];
+        }
+        if (GLU) a = silu(a) * b;
+        else if (g.act == 1) {
+            a = fmaxf(a, 0.0f);
+            a *= a;
+        }
+        g.out[static_cast<int64_t>(t) * N + n0 + c] = f32_to_bf16_bits(a);
+    }
+}
+
+template <int ROWS, int COLS, int NT, int AHEAD, bool GLU>
+int launch_one(const NormGemm& g, hipStream_t s) {
+    const size_t bytes = rows_bytes(ROWS, g.K) + stage_bytes(NT) + sums_bytes(ROWS, NT);
+    const int rc = allow_lds(reinterpret_cast<const void*>(norm_gemm_kernel<ROWS, COLS, NT, AHEAD, GLU>), bytes);
+    if (rc != 0) return rc;
+    launch((norm_gemm_kernel<ROWS, COLS, NT, AHEAD, GLU>), dim3(static_cast<unsigned>(ceil_div(g.N, (GLU ? 8 : 16) * NT))), dim3(kThreads), bytes, s, g);
+    return launch_status();
+}
+
+// Tiles of weight rows to a workgroup: as many as leave one workgroup to a CU.
+int tiles_of(int N, int act) {
+    const int tiles = static_cast<int>(ceil_div(act == 2 ? 2 * static_cast<int64_t>(N) : N, 16)), nt = static_cast<int>(ceil_div(tiles, kGroups));
+    return act == 2 ? (nt + 1) / 2 * 2 : nt;
+}
+
+template <int ROWS, int COLS>
+int launch_rows(const NormGemm& g, hipStream_t s) {
+    constexpr int kAhead = 4;
+    const int nt = tiles_of(g.N, g.act);
+    if (g.act == 2) return nt == 2 ? launch_one<ROWS, COLS, 2, kAhead, true>(g, s) : launch_one<ROWS, COLS, 4, 4, true>(g, s);
+    if (nt == 1) return launch_one<ROWS, COLS, 1, kAhead, false>(g, s);
+    if (nt == 2) return launch_one<ROWS, COLS, 2, kAhead, false>(g, s);
+    if (nt == 3) return launch_one<ROWS, COLS, 3, kAhead, false>(g, s);
+    return launch_one<ROWS, COLS, 4, 4, false>(g, s);
+}
+
+}  // namespace
+
+bool norm_gemm_supported(int64_t T, int N, int K, int act) {
+    return T > 0 && T <= 2 && N > 0 && N <= 16 * kGroups * 4 && K >= 512 && K <= 4096 && K % 512 == 0 && act >= 0 && act <= 2 && tiles_of(N, act) <= 4;
+}
+
+// Where one launch is faster than the norm's and the product's (us in a graph, two / one; y in parts and no next_w; weights read from memory).
+// One row: K = 1024, 3072 rows 6.0 / 3.9; 2048, 3072 rows 7.5 / 5.0, 6176 9.6 / 7.6, 8832 11.1 / 10.6, gated 2 x 4096 11.1 / 8.7-10.1, 12800 13.9 /
+// 13.9; 4096, 6144 rows 15.3 / 12-13, 12288 20.5 / 18.2, 12800 22.8 / 20.5, gated 2 x 8192 28.3 / 24-33.  The second sum that next_w brings costs
+// 0.5 to 0.8.  Two rows: 3072 rows of 2048 7.6 / 5.7, 6176 9.6 / 8.2, 8832 11.0 / 11.1, gated 2 x 4096 11.8 / 9.6-10.8; 12288 of 4096 20.6 / 19.3,
+// 12800 with next_w 23.1 / 23.9, gated 2 x 8192 28.7 / 28.7-34.  Four rows: the rows' bytes and sums are what a workgroup waits for (6176 rows of
+// 2048 9.7 / 9.7, with next_w 10.0 / 12.0), so no more than two are taken.
+bool norm_gemm_pays(int T, int N, int K, int act) {
+    const int64_t rows = act == 2 ? 2 * static_cast<int64_t>(N) : N;
+    return T == 1 ? K > 2048 || rows < 12288 : rows <= (K > 2048 ? 12288 : 8192);
+}
+
+int launch_norm_gemm(const NormGemm& g, hipStream_t s) {
+    if (g.T == 1) return g.K <= 2048 ? launch_rows<1, 1>(g, s) : launch_rows<1, 2>(g, s);
+    return g.K <= 2048 ? launch_rows<2, 1>(g, s) : launch_rows<2, 2>(g, s);
+}
+
+}  // namespace em

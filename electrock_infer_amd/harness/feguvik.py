@@ -11,7 +11,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from ..layers.decoder_ops import ADD_NORMED, KEEP, REPLACE, embed_rows, linear_parts, residual_norm
+from ..layers.decoder_ops import KEEP, REPLACE, embed_rows, linear_parts, normed_rows, residual_norm, stream_behind
 from ..layers.dense_mlp import DenseMLP
 from ..layers.gla import GatedLinearAttention
 from ..layers.latent_attention import LatentAttention
@@ -165,26 +165,34 @@ class FeguvikForCausalLM(DecoderModel):
         opens_pass = lambda r: r < n_runs and self.runs[r][1] is not None and self.runs[r][0] == cfg.loop.start
 
         def open_run(r, update):
-            """``update(out, norm)`` changes the stream and writes x / rms(x) * norm, or x for None: what run ``r`` reads."""
+            """``update(out, norm, reader)`` changes the stream and leaves x / rms(x) * norm, or x for None: what run ``r`` reads."""
             norm = self.layers[self.runs[r][0]].norm1 if r < n_runs else self.final_norm
+            rows = h
             if not opens_pass(r):
-                update(h, norm)
+                rows = update(h, norm, self.layers[self.runs[r][0]].mix if r < n_runs and self.layer_hook is None else None)
             else:
-                update(both[:, :W], None)
+                update(both[:, :W], None, None)
             if self.layer_hook is not None and r > 0:
                 self.layer_hook(r - 1, x)
             if opens_pass(r):
                 residual_norm(REPLACE, x, linear_parts(both, self.loop_in, exact=True), self.loop_step[self.runs[r][1]], eps, h, norm)
+            return rows
 
-        open_run(0, lambda out, norm: residual_norm(KEEP, x, None, None, eps, out, norm))
+        def first_rows(out, norm, reader):
+            residual_norm(KEEP, x, None, None, eps, out, norm)
+            return out
+
+        rows = open_run(0, first_rows)
         for r, (i, _) in enumerate(self.runs):
             layer = self.layers[i]
-            y, post = layer.mix(h, batch, self.caches[r]), layer.post1
+            y, post = layer.mix(rows, batch, self.caches[r]), layer.post1
+            x = stream_behind(rows, x)
             if layer.mlp is not None:
-                residual_norm(ADD_NORMED, x, y, post, eps, h, layer.norm2)
-                y, post = layer.mlp(h), layer.post2
+                rows = normed_rows(x, y, post, eps, h, layer.norm2, layer.mlp)
+                y, post = layer.mlp(rows), layer.post2
+                x = stream_behind(rows, x)
             if layer.side is not None:
-                open_run(r + 1, lambda out, norm: layer.side.close_layer(x, y, post, batch.tokens, self.side_embed, eps, out, norm))
+                rows = open_run(r + 1, lambda out, norm, reader: layer.side.close_layer(x, y, post, batch.tokens, self.side_embed, eps, out, norm, reader))
             else:
-                open_run(r + 1, lambda out, norm: residual_norm(ADD_NORMED, x, y, post, eps, out, norm))
+                rows = open_run(r + 1, lambda out, norm, reader: normed_rows(x, y, post, eps, out, norm, reader))
         return h

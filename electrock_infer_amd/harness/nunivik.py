@@ -11,7 +11,7 @@ import torch
 from torch import nn
 
 from ..layers.attention import CarriedValues, SoftmaxAttention
-from ..layers.decoder_ops import ADD_NORMED, embed_rows, residual_norm
+from ..layers.decoder_ops import embed_rows, normed_rows, stream_behind
 from ..layers.dense_mlp import DenseMLP
 from ..layers.recurrent import GatedDeltaRule, StateSpaceMixer
 from .batch import RaggedBatch
@@ -127,13 +127,18 @@ class NunivikForCausalLM(DecoderModel):
         cfg, eps = self.cfg, self.cfg.norm_eps
         h = torch.empty(batch.tokens.numel(), cfg.width, dtype=self.head.dtype, device=self.head.device)
         x = embed_rows(batch.tokens, self.embed, cfg.embedding_scale, h)        # h: the stream in the compute type
-        carried = CarriedValues()
+        carried, rows = CarriedValues(), h
         for i, layer in enumerate(self.layers):
             last = self.final_norm if i + 1 == len(self.layers) else None
-            y = layer.mix(h, batch, self.caches[i], carried)
-            residual_norm(ADD_NORMED, x, y, layer.norm1, eps, h, last if layer.mlp is None else None)
+            # (who reads a layer's rows: nobody waits for a product where a hook reads the stream, or behind the last layer)
+            after = self.layers[i + 1].mix if last is None and self.layer_hook is None else None
+            y = layer.mix(rows, batch, self.caches[i], carried)
+            x = stream_behind(rows, x)
+            rows = normed_rows(x, y, layer.norm1, eps, h, last if layer.mlp is None else None, after if layer.mlp is None else layer.mlp)
             if layer.mlp is not None:
-                residual_norm(ADD_NORMED, x, layer.mlp(h), layer.norm2, eps, h, last)
+                y = layer.mlp(rows)
+                x = stream_behind(rows, x)
+                rows = normed_rows(x, y, layer.norm2, eps, h, last, after)
             if self.layer_hook is not None:
                 self.layer_hook(i, x)
         return h

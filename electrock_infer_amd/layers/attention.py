@@ -21,6 +21,7 @@ class CarriedValues:
 
 class SoftmaxAttention(nn.Module):
 
+    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
     PROMPT_TOKENS = 48           # portions from this length on go to the kernel for prompts, if it takes the sizes
 
     def __init__(self, width: int, heads: int, kv_heads: int, dim: int, vdim: int, scale: float, eps: float, dtype,

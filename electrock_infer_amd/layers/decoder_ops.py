@@ -6,6 +6,7 @@ from typing import Optional
 import torch
 import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
+from torch.nn.modules.module import _global_forward_hooks as _global_hooks, _global_forward_pre_hooks as _global_pre_hooks
 from torch.overrides import _get_current_function_mode_stack
 from torch.utils._device import DeviceContext
 
@@ -115,9 +116,66 @@ def _skinny_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
     return lib.ed_tile_gemm_splits(x.shape[0], *weight.shape) or lib.ed_decode_gemm_splits(x.shape[0], *weight.shape)
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
+class NormedRows:
+    """The rows that ``residual_norm(ADD_NORMED, x, y, post_w, eps, out, next_w)`` would leave in ``out``, for one product that norms them
+    itself (``linear``, ``linear_silu_gate``); ``stream``: x, or behind that product the float32 rows that stand for it."""
+
+    __slots__ = ("x", "y", "post_w", "next_w", "eps", "out", "spare", "stream", "shape", "dtype", "device")
+
+    def __init__(self, x, y, post_w, next_w, eps, out, spare):
+        self.x, self.y, self.post_w, self.next_w, self.eps, self.out, self.spare, self.stream = x, y, post_w, next_w, eps, out, spare, x
+        self.shape, self.dtype, self.device = out.shape, out.dtype, out.device
+
+    def settle(self) -> torch.Tensor:
+        """The rows themselves."""
+        residual_norm(ADD_NORMED, self.x, self.y, self.post_w, self.eps, self.out, self.next_w)
+        return self.out
+
+    def product(self, weight: torch.Tensor, cols: int, act: int) -> Optional[torch.Tensor]:
+        """act(rows @ weight^T) in one launch, or None."""
+        lib, out = _lib.load_decoder(), self.out
+        T, K = out.shape
+        if not (_plain(out, weight) and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and lib.ed_norm_gemm_pays(T, cols, K, act) == 1):
+            return None
+        result = torch.empty(T, cols, dtype=_BF16, device=out.device)
+        y = self.y
+        code = lib.ed_norm_gemm(self.x.data_ptr(), y.data_ptr(), _lib.dtype_code(y.dtype), y.shape[0] if y.dim() == 3 else 1, self.post_w.data_ptr(),
+                                _ptr(self.next_w), self.spare.data_ptr(), weight.data_ptr(), result.data_ptr(), T, cols, K, act, float(self.eps),
+                                _lib.current_stream(out.device))
+        _lib.check_decoder(code, "norm_gemm")
+        self.stream = self.spare
+        return result
+
+
+def _unwatched(module) -> bool:
+    return not _global_hooks and not _global_pre_hooks and not any(m._forward_hooks or m._forward_pre_hooks for m in module.modules())
+
+
+def normed_rows(x: torch.Tensor, y: torch.Tensor, post_w: torch.Tensor, eps: float, out: torch.Tensor, next_w: Optional[torch.Tensor], reader):
+    """``residual_norm(ADD_NORMED, ...)`` for rows that ``reader`` reads next: ``out``, or for a row or two ``NormedRows``, where it is a layer
+    of this package that hands them to one product and nobody watches what it is given."""
+    T, K = out.shape
+    if T <= 2 and getattr(reader, "takes_normed_rows", False) and _unwatched(reader) and x.is_cuda and x.is_contiguous() and y.is_contiguous() and out.is_contiguous() and out.dtype is _BF16 and \
+            (y.dtype is _BF16 and y.dim() == 2 or y.dtype is torch.float32) and (x.data_ptr() | y.data_ptr()) % 16 == 0 and \
+            _lib.load_decoder().ed_norm_gemm_supported(T, 1, K, 0) == 1:
+        return NormedRows(x, y, post_w, next_w, eps, out, torch.empty_like(x))
+    residual_norm(ADD_NORMED, x, y, post_w, eps, out, next_w)
+    return out
+
+
+def stream_behind(rows, x: torch.Tensor) -> torch.Tensor:
+    """The float32 stream behind the product that read ``rows``: x, or what stands for it from there on."""
+    return rows.stream if type(rows) is NormedRows else x
+
+
+def linear(x, weight: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
     """act(x @ weight^T) in x's type: a kernel of this package for decode batches and short prompts, a library product otherwise;
-    ``act``: None or 'relu_squared'."""
+    ``act``: None or 'relu_squared'.  ``x``: a matrix, or ``NormedRows``."""
+    if type(x) is NormedRows:
+        out = x.product(weight, weight.shape[0], int(act is not None))
+        if out is not None:
+            return out
+        x = x.settle()
     out = _own(x, weight, weight.shape[0], int(act is not None))
     if out is not None:
         return out
@@ -125,8 +183,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, act: Optional[str] = None) -> 
     return relu_squared_(out) if act is not None else out
 
 
-def linear_silu_gate(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """silu(x @ gate^T) * (x @ up^T) for ``weight`` = [gate; up]: one launch for a decode batch or a short prompt."""
+def linear_silu_gate(x, weight: torch.Tensor) -> torch.Tensor:
+    """silu(x @ gate^T) * (x @ up^T) for ``weight`` = [gate; up]: one launch for a decode batch or a short prompt.  ``x``: a matrix, or
+    ``NormedRows``."""
+    if type(x) is NormedRows:
+        out = x.product(weight, weight.shape[0] // 2, 2) if weight.shape[0] % 2 == 0 else None
+        if out is not None:
+            return out
+        x = x.settle()
     (T, _), ff = x.shape, weight.shape[0] // 2
     out = _own(x, weight, ff, 2) if weight.shape[0] == 2 * ff else None
     if out is not None:

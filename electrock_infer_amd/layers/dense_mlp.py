@@ -8,6 +8,7 @@ from .decoder_ops import StackedRows, linear, linear_parts, linear_silu_gate
 class DenseMLP(nn.Module):
     """``activation``: 'relu_squared', or 'silu_gate' for a gated one, whose two input matrices are stacked in ``up``."""
 
+    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
     ACTIVATIONS = ("relu_squared", "silu_gate")
 
     def __init__(self, width: int, ff: int, dtype, activation: str = "relu_squared"):

@@ -10,6 +10,8 @@ from .decoder_ops import StackedLinear, byref, linear_parts
 class GatedLinearAttention(nn.Module):
     """Projections stacked in one matrix: q, k, v, the output gate g and the first factor a1 of the decay."""
 
+    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
+
     def __init__(self, width: int, heads: int, dim: int, vdim: int, tau: float, decay_rank: int, eps: float, dtype):
         super().__init__()
         self.heads, self.dim, self.vdim, self.tau, self.rank, self.eps = heads, dim, vdim, tau, decay_rank, eps

@@ -14,6 +14,7 @@ def rotary_frequencies(dims: int, base: float, factor: float = 1.0) -> torch.Ten
 
 class LatentAttention(nn.Module):
 
+    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
     PROMPT_TOKENS = 64           # portions from this length on write their keys and values out, if the kernel takes the sizes
 
     def __init__(self, width: int, heads: int, dim: int, rot_dim: int, vdim: int, kv_rank: int, scale: float,

@@ -20,6 +20,8 @@ class DecayedRecurrence(nn.Module):
     """What both mixers share: q, k [kv_heads, dim] and v [heads, vdim] from convolutions over ``in_proj``'s sections of
     these names, decay inputs in its section ``decay``, and the recurrence itself."""
 
+    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
+
     def __init__(self, width: int, heads: int, kv_heads: int, dim: int, vdim: int, taps: int, eps: float, sections: Dict[str, int],
                  conv_bias: bool, dtype):
         super().__init__()

@@ -4,7 +4,7 @@ import torch
 from torch import nn
 
 from .. import _lib
-from .decoder_ops import ADD_NORMED, residual_norm, token_input
+from .decoder_ops import ADD_NORMED, normed_rows, residual_norm, token_input
 
 
 class TokenSideInput(nn.Module):
@@ -32,9 +32,9 @@ class TokenSideInput(nn.Module):
         return token_input(x, self.gate, self.proj, tokens, table, self.column0)
 
     def close_layer(self, x: torch.Tensor, y: torch.Tensor, post_w: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor,
-                    eps: float, out: torch.Tensor, next_w) -> None:
+                    eps: float, out: torch.Tensor, next_w, reader=None):
         """Everything from the feed-forward's result ``y`` to the next layer's input: the stream ``x`` takes the normed y,
-        then the token's input; ``out`` (rows may be strided) = x / rms(x) * next_w, or x.  One launch for a bfloat16
+        then the token's input; ``out`` (rows may be strided) = x / rms(x) * next_w, or x: returned, or ``NormedRows`` for ``reader``.  One launch for a bfloat16
         prompt of a width its kernel takes; a few rows are better spread over the chip in four."""
         T, W = x.shape
         lib, dim = _lib.load_decoder(), self.gate.shape[0]
@@ -48,7 +48,7 @@ class TokenSideInput(nn.Module):
                        table.data_ptr(), table.stride(0), self.column0, self.norm.data_ptr(), None if next_w is None else next_w.data_ptr(),
                        out.data_ptr(), out.stride(0), T, W, dim, float(eps), stream)
             _lib.check_decoder(code, "token_side")
-            return
+            return out
         rows = torch.empty(T, W, dtype=out.dtype, device=x.device)
         residual_norm(ADD_NORMED, x, y, post_w, eps, rows)
-        residual_norm(ADD_NORMED, x, self(rows, tokens, table), self.norm, eps, out, next_w)
+        return normed_rows(x, self(rows, tokens, table), self.norm, eps, out, next_w, reader)

@@ -73,6 +73,18 @@ int ed_tile_gemm_pays(int64_t T, int N, int K, int act);
 int ed_tile_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out, int out_dtype, int splits, int64_t T, int N,
                  int K, int act, void* stream);
 
+/*
+ * A residual norm and the product behind it for one or two rows (bf16 weights and results), one launch:
+ *     x_out = x + y / rms(y) * post_w,   out = act(h w^T),   h = next_w ? x_out / rms(x_out) * next_w : x_out, rounded to bf16.
+ * x, x_out float32 [T, K] (not the same memory); y [y_parts, T, K] float32 partial sums, or bf16 with y_parts 1; w and act as in
+ * ed_decode_gemm.  ed_norm_gemm_supported: 1 where it takes the sizes (K a multiple of 512 up to 4096, at most 16384 rows of w),
+ * _pays: where it is faster than the two.
+ */
+int ed_norm_gemm_supported(int64_t T, int N, int K, int act);
+int ed_norm_gemm_pays(int64_t T, int N, int K, int act);
+int ed_norm_gemm(const float* x, const void* y, int y_dtype, int y_parts, const float* post_w, const float* next_w, float* x_out, const void* w,
+                 void* out, int64_t T, int N, int K, int act, double eps, void* stream);
+
 /* g [T, dim] = gelu_tanh(x gate^T) * table[tokens[t]][column0 + c]; x [T, W], gate [dim, W]. */
 int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const void* table, int64_t table_stride,
                   int column0, void* g, int64_t T, int W, int dim, int dtype, void* stream);
