@@ -847,7 +847,10 @@ __global__ __launch_bounds__(NDT * kWave) void recur_matrix_scan_kernel(RecurPro
 }
 
 // ---- decoding: one new token per sequence ----
-// A thread holds VEC columns of up to ROWS rows of the state.
+// A thread holds VEC columns of up to ROWS rows of the state.  Bound: the states' bytes, read and written once a step, past the caches' order of
+// use (us, loads and stores in it / past it: 64 sequences of 64 heads of 128 x 64, 268 MB, 62.5 / 51.2, 8 of them 11.3 / 8.9, 128 112 / 97; the delta
+// rule, 16 heads of 128 x 128, 23 sequences 15.2 / 13.1, 64 27.3 / 26.3, 128 71 / 52; a single sequence is the same; either alone gives a third).
+// Asking for a thread's channels and taps together, beside the state or in front of it, spills (one sequence of the delta rule 9.2 / 9.8-10.3).
 template <typename Elem, bool DELTA, int VEC, int ROWS>
 __global__ __launch_bounds__(1024) void recur_step_kernel(RecurProblem p) {
     typedef typename Elem::storage S;
@@ -868,7 +871,7 @@ __global__ __launch_bounds__(1024) void recur_step_kernel(RecurProblem p) {
 #pragma unroll
     for (int u = 0; u < ROWS; ++u) {
         const int d = grp + u * groups;
-        if (grp < groups && d < dim && pos > 0) x[u] = *reinterpret_cast<const vec_t*>(st + d * vdim + c);
+        if (grp < groups && d < dim && pos > 0) x[u] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(st + d * vdim + c));
         else x[u] = static_cast<vec_t>(0.0f);
     }
     const f32x2_t rate = decay_and_beta<Elem>(p, s, h);
@@ -950,7 +953,7 @@ __global__ __launch_bounds__(1024) void recur_step_kernel(RecurProblem p) {
             if (!DELTA) x[u] *= decay;
             x[u] += u_new * (lk[d] * k_scale);
             o += x[u] * (lqv[d] * q_scale);
-            *reinterpret_cast<vec_t*>(st + d * vdim + c) = x[u];
+            __builtin_nontemporal_store(x[u], reinterpret_cast<vec_t*>(st + d * vdim + c));
         }
     }
     if (grp < groups) *reinterpret_cast<vec_t*>(lo + grp * vdim + c) = o;
