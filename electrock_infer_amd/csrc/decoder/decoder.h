@@ -233,6 +233,7 @@ bool latent_supported(int heads, int dim, int rot, int rank);
 int latent_splits(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64_t max_q, int64_t keys);
 bool latent_waves(int dtype, int rank, int rot, int heads, int64_t n_seqs, int64_t max_q, int64_t keys);
 int launch_latent_prepare(const LatentProblem& p, int64_t T, hipStream_t s);
+int launch_latent_front(const LatentProblem& p, const void* uk, int64_t T, hipStream_t s);
 int launch_latent_paged(const LatentProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml,
                         int64_t T, hipStream_t s);
 int launch_head_gemm(const void* a, int64_t a_row, int64_t a_head, const void* b, void* out, int64_t o_row,

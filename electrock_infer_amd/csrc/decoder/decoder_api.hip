@@ -454,6 +454,15 @@ int ed_latent_prepare(const ed_latent_args* a, void* stream) {
     return launch_latent_prepare(latent_problem(*a), a->T, as_stream(stream));
 }
 
+int ed_latent_front(const ed_latent_args* a, const void* uk, void* stream) {
+    const int rc = check_latent(a);
+    if (rc != 0 || a->T == 0) return rc;
+    if (!a->q || !a->down || !a->latent_w || (a->rot > 0 && !a->inv_freq) || !a->positions || !a->cache_rows || !a->cache || !a->q_latent || !uk)
+        return EM_ERR_NULL_POINTER;
+    if (!aligned16(uk)) return EM_ERR_ALIGNMENT;
+    return launch_latent_front(latent_problem(*a), uk, a->T, as_stream(stream));
+}
+
 int ed_latent_paged(const ed_latent_args* a, void* stream) {
     const int rc = check_latent(a);
     if (rc != 0 || a->T == 0) return rc;

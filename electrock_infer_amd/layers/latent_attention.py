@@ -69,9 +69,9 @@ class LatentAttention(nn.Module):
                             max_q=batch.max_q, table_width=batch.table_width, block_size=cache.shape[1], splits=1,
                             heads=self.heads, dim=self.dim, rot=self.rot, rank=self.rank, dtype=_lib.dtype_code(h.dtype),
                             scale=self.scale, eps=self.eps)
-        _lib.check_decoder(_lib.load_decoder().ed_latent_prepare(byref(a), _lib.current_stream(dev)), "latent_prepare")
         o = torch.empty(T, self.heads * self.vdim, dtype=h.dtype, device=dev)
         if self.writes_out(batch, h.dtype):
+            _lib.check_decoder(_lib.load_decoder().ed_latent_prepare(byref(a), _lib.current_stream(dev)), "latent_prepare")
             self._attend_written_out(p, batch, cache, o)
         else:
             self._attend_paged(a, p, batch, o)
@@ -91,8 +91,9 @@ class LatentAttention(nn.Module):
             part_o = torch.empty(T * H * a.splits * self.pitch, dtype=torch.float32, device=dev)
             part_ml = torch.empty(T * H * a.splits * 2, dtype=torch.float32, device=dev)
             a.part_o, a.part_ml = part_o.data_ptr(), part_ml.data_ptr()
-        head_gemm(p, p.stride(0), self.dim + self.rot, self.uk_t, self.dim, q_lat, H * self.pitch, self.pitch, T)
-        _lib.check_decoder(_lib.load_decoder().ed_latent_paged(byref(a), _lib.current_stream(dev)), "latent_paged")
+        lib, stream = _lib.load_decoder(), _lib.current_stream(dev)
+        _lib.check_decoder(lib.ed_latent_front(byref(a), self.uk_t.data_ptr(), stream), "latent_front")
+        _lib.check_decoder(lib.ed_latent_paged(byref(a), stream), "latent_paged")
         head_gemm(o_lat, H * self.pitch, self.pitch, self.uv_p, self.rank, o, H * self.vdim, self.vdim, T)
 
     def _attend_written_out(self, p: torch.Tensor, batch, cache: torch.Tensor, o: torch.Tensor) -> None:

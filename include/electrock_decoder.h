@@ -270,6 +270,9 @@ int ed_latent_splits(int dtype, int heads, int rank, int rot, int n_seqs, int ma
 int ed_latent_waves(int dtype, int heads, int rank, int rot, int n_seqs, int max_q, int max_context);
 /* Norm of the latent, rotation of the key part (both into the cache) and of q's rotated parts (in place). */
 int ed_latent_prepare(const ed_latent_args* a, void* stream);
+/* ed_latent_prepare, and q_latent [T, heads, round_up(rank, 8)] = q's other parts times uk [heads, rank, round_up(dim, 32)], zeros in the
+ * padding of dim: for a few tokens in one launch. */
+int ed_latent_front(const ed_latent_args* a, const void* uk, void* stream);
 /* out = sum_j p_j c_j per row and head, p = softmax of (q_latent . c_j + q_rot . k_rot_j) * scale over the keys
  * j <= position with exp(sink) added to the denominator; the keys of a row are shared out over `splits` (<= 256) workgroups. */
 int ed_latent_paged(const ed_latent_args* a, void* stream);
