@@ -266,21 +266,21 @@ template <typename Elem> __host__ __device__ constexpr int value_pitch(int dvt) 
 template <typename Elem> __host__ __device__ constexpr int tile_pitch(int dkt, int dvt) {     // of keys and values in one stretch
     return sizeof(typename Elem::storage) == 2 && dkt <= 4 && dkt * 2 > dvt ? value_pitch<Elem>(dkt * 2) : value_pitch<Elem>(dvt);
 }
-template <typename Elem> __host__ __device__ constexpr int paged_lds(int dkt, int dvt) {   // keys, then values of a wave's tile; later the waves' results
-    const int tiles = 4 * kKeys * tile_pitch<Elem>(dkt, dvt) * static_cast<int>(sizeof(typename Elem::storage)), results = 4 * 16 * (dvt * 16 + 4) * 4;
+template <typename Elem> __host__ __device__ constexpr int paged_lds(int dkt, int dvt, int waves) {   // keys, then values of a wave's tile; later the waves' results
+    const int tiles = waves * kKeys * tile_pitch<Elem>(dkt, dvt) * static_cast<int>(sizeof(typename Elem::storage)), results = waves * 16 * (dvt * 16 + 4) * 4;
     return tiles > results ? tiles : results;
 }
 
 // DKT: 32-element steps of dim; DVT: 16-element tiles of vdim
-template <typename Elem, int DKT, int DVT, bool ONCE>
-__global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) void attn_paged_kernel(AttnProblem p, int splits,
+template <typename Elem, int DKT, int DVT, bool ONCE, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave, WAVES == 4 && sizeof(typename Elem::storage) == 2 ? 2 : 1) void attn_paged_kernel(AttnProblem p, int splits,
                                                                                                     float* __restrict__ part_o,
                                                                                                     float* __restrict__ part_ml) {
     typedef typename Elem::storage S;
     typedef Mma<Elem> M;
     constexpr int LPT = tile_pitch<Elem>(DKT, DVT), kPieces = kKeys * DVT * 2 / kWave, kRowsAtOnce = kKeys / kPieces, LPO = DVT * 16 + 4;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-    __shared__ float wave_m[4][16], wave_l[4][16];
+    __shared__ float wave_m[WAVES][16], wave_l[WAVES][16];
     const int share = p.heads / p.kv_heads;
     const int seq = blockIdx.y / p.kv_heads, g = blockIdx.y - seq * p.kv_heads, split = blockIdx.z;
     const int q0 = p.q_begin[seq], rows = (p.q_begin[seq + 1] - q0) * share, r0 = blockIdx.x * 16;
@@ -336,12 +336,12 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
             fv[i] = load_rows<Elem, ONCE>(values + static_cast<int64_t>(max(__shfl(row, v_key + i * kRowsAtOnce), 0)) * row_elems);
         }
     };
-    int row = row_of(tile0 + wave), next_row = row_of(tile0 + wave + 4);
+    int row = row_of(tile0 + wave), next_row = row_of(tile0 + wave + WAVES);
     if (kAhead && tile0 + wave < tile1) {
         load_keys(row);
         load_values(row);
     }
-    for (int tile = tile0 + wave; tile < tile1; tile += 4) {
+    for (int tile = tile0 + wave; tile < tile1; tile += WAVES) {
         if (!kAhead) load_values(row);
         if (kAhead) {
 #pragma unroll
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
         }
         if (kAhead) load_values(next_row);
         row = next_row;
-        next_row = row_of(tile + 8);
+        next_row = row_of(tile + 2 * WAVES);
         float mx = -INFINITY;
 #pragma unroll
         for (int n = 0; n < 2; ++n)
@@ -413,19 +413,21 @@ __global__ __launch_bounds__(256, sizeof(typename Elem::storage) == 2 ? 2 : 1) v
         wave_l[wave][l16] = l;
     }
     __syncthreads();
-    float* Os = reinterpret_cast<float*>(lds_raw);                   // [4][16][LPO]
+    float* Os = reinterpret_cast<float*>(lds_raw);                   // [WAVES][16][LPO]
 #pragma unroll
     for (int d = 0; d < DVT; ++d)
         *reinterpret_cast<f32x4_t*>(Os + (wave * 16 + l16) * LPO + d * 16 + lq * 4) = o[d];
     __syncthreads();
-    for (int i = tid; i < 16 * DVT * 16; i += 256) {
+    for (int i = tid; i < 16 * DVT * 16; i += WAVES * kWave) {
         const int rr = i / (DVT * 16), c = i - rr * (DVT * 16);
         if (r0 + rr >= rows || c >= p.vdim) continue;
-        const float top = fmaxf(fmaxf(wave_m[0][rr], wave_m[1][rr]), fmaxf(wave_m[2][rr], wave_m[3][rr]));
+        float top = wave_m[0][rr];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) top = fmaxf(top, wave_m[w][rr]);
         const float base = top == -INFINITY ? 0.0f : top;
         float sum = 0.0f, v = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < WAVES; ++w) {
             const float weight = Precise<Elem>::exp(wave_m[w][rr] - base);
             sum = fmaf(wave_l[w][rr], weight, sum);
             v = fmaf(Os[(w * 16 + rr) * LPO + c], weight, v);
@@ -736,13 +738,13 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
     }
 }
 
-template <typename Elem, int DKT, int DVT, bool ONCE>
+template <typename Elem, int DKT, int DVT, bool ONCE, int WAVES>
 int launch_groups(const AttnProblem& p, int row_groups, int n_seqs, int splits, float* part_o, float* part_ml, hipStream_t s) {
-    const size_t lds = paged_lds<Elem>(DKT, DVT);
-    const int rc = allow_lds(reinterpret_cast<const void*>(attn_paged_kernel<Elem, DKT, DVT, ONCE>), lds);
+    const size_t lds = paged_lds<Elem>(DKT, DVT, WAVES);
+    const int rc = allow_lds(reinterpret_cast<const void*>(attn_paged_kernel<Elem, DKT, DVT, ONCE, WAVES>), lds);
     if (rc != 0) return rc;
     const dim3 grid(static_cast<unsigned>(row_groups), static_cast<unsigned>(n_seqs * p.kv_heads), static_cast<unsigned>(splits));
-    launch((attn_paged_kernel<Elem, DKT, DVT, ONCE>), grid, dim3(256), lds, s, p, splits, part_o, part_ml);
+    launch((attn_paged_kernel<Elem, DKT, DVT, ONCE, WAVES>), grid, dim3(WAVES * kWave), lds, s, p, splits, part_o, part_ml);
     return launch_status();
 }
 
@@ -750,8 +752,15 @@ template <typename Elem, int DKT, int DVT>
 int launch_paged(const AttnProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml, int64_t T, hipStream_t s) {
     const int row_groups = static_cast<int>(ceil_div(static_cast<int64_t>(max_q) * (p.heads / p.kv_heads), 16));
     constexpr bool kBf16 = sizeof(typename Elem::storage) == 2;
-    const int rc = kBf16 && row_groups == 1 ? launch_groups<Elem, DKT, DVT, kBf16>(p, row_groups, n_seqs, splits, part_o, part_ml, s)
-                                            : launch_groups<Elem, DKT, DVT, false>(p, row_groups, n_seqs, splits, part_o, part_ml, s);
+    // Eight waves share out a context that nothing else does, where no CU has a second workgroup to fill its waits: twice the bytes in flight
+    // and half of the steps of the longest context (us, four / eight waves, 64 sequences of 16 heads on 4: 1023 keys 31.1 / 28.8, 512 to 1535 of
+    // them 40.4 / 33.0, 4000 103 / 92, heads of 64 22.1 / 16.5; 33 sequences 26.7 / 21.1; up to 200 keys the same).
+    constexpr int kMany = kBf16 && DKT <= 4 ? 8 : 4;
+    const bool many = splits == 1 && row_groups == 1 && n_seqs * p.kv_heads <= 256 && static_cast<int64_t>(p.table_width) * p.block_size > 4 * kKeys;
+    int rc;
+    if (kBf16 && many) rc = launch_groups<Elem, DKT, DVT, kBf16, kMany>(p, row_groups, n_seqs, splits, part_o, part_ml, s);
+    else if (kBf16 && row_groups == 1) rc = launch_groups<Elem, DKT, DVT, kBf16, 4>(p, row_groups, n_seqs, splits, part_o, part_ml, s);
+    else rc = launch_groups<Elem, DKT, DVT, false, 4>(p, row_groups, n_seqs, splits, part_o, part_ml, s);
     if (rc != 0 || splits == 1) return rc;
     launch((attn_combine_kernel<Elem>), dim3(static_cast<unsigned>(T * p.heads)), dim3(kWave), 0, s, part_o, part_ml, splits, p.vdim,
            static_cast<typename Elem::storage*>(p.out));
@@ -822,8 +831,8 @@ bool attn_supported(int heads, int kv_heads, int dim, int vdim, int rot) {
 // next tile in flight hide its way with other workgroups (float32, 64 + 64: 24 x 2000 keys in threes 50.0, eights 31.8; bf16,
 // 192 + 64 in threes 40.8, eights 30.3).  A CU's second workgroup of the form that reads its rows once gains little, as the pages
 // come near memory's rate: where every CU has one without a split, that is worth a launch only behind long contexts (64 sequences
-// of 1024 keys in ones 33.5, twos 35.0; 2048 keys 58.9 / 58.5, 4096 108.5 / 102.8; and a recorded step plans for up to twice the
-// keys that it has: 1064 of 2048 36.3 / 38.9).
+// of 1024 keys in ones 33.5, twos 35.0; 2048 keys 58.9 / 58.5; and a recorded step plans for up to twice the keys that it has: 1064 of
+// 2048 36.3 / 38.9).
 int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int64_t max_q, int64_t keys) {
     const int64_t row_groups = ceil_div(max_q * (heads / kv_heads), 16), groups = row_groups * n_seqs * kv_heads, most = ceil_div(keys, 4 * kKeys);
     const bool bf16 = dtype == EM_DTYPE_BF16, ahead = bf16 && dim <= 128, once = bf16 && row_groups == 1;
@@ -841,6 +850,16 @@ int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int
         best = static_cast<int>(s);
     }
     return best;
+}
+
+// The layer's choice: a context that is not split has eight waves where it has a CU to itself, and that is the faster way from 160 workgroups
+// on, and from 112 behind short contexts (us, 16 heads on 4, ones / the best split: 64 x 4000 keys 90.3 / 94.9, 48 x 1023 24.1 / 27.3, 48 x 4000 72.2 /
+// 74.9; 32 x 500 13.6 / 14.6, 32 x 1023 20.9 / 20.8, 32 x 4000 60.0 / 54.3; 24 x 1023 20.2 / 19.6, 24 x 4000 57.7 / 45.5).
+int attn_ranges(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int64_t max_q, int64_t keys) {
+    const int64_t groups = n_seqs * kv_heads;
+    const bool many = dtype == EM_DTYPE_BF16 && dim <= 128 && max_q * (heads / kv_heads) <= 16 && groups <= 256;
+    if (many && (groups >= 160 || (groups >= 112 && keys <= 1536))) return 1;
+    return attn_splits(dtype, heads, kv_heads, dim, n_seqs, max_q, keys);
 }
 
 int launch_attn_prepare(const AttnProblem& p, int64_t T, hipStream_t s) {

@@ -201,6 +201,7 @@ __host__ __device__ constexpr int attn_row_elems(int kv_heads, int dim, int vdim
 constexpr int kAttnMaxSplits = 64;
 bool attn_supported(int heads, int kv_heads, int dim, int vdim, int rot);
 int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int64_t max_q, int64_t keys);
+int attn_ranges(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int64_t max_q, int64_t keys);
 bool attn_prompt_supported(int dim, int vdim);
 int launch_attn_prepare(const AttnProblem& p, int64_t T, hipStream_t s);
 int launch_attn_paged(const AttnProblem& p, int n_seqs, int max_q, int splits, float* part_o, float* part_ml, int64_t T, hipStream_t s);

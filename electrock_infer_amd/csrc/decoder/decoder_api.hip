@@ -397,10 +397,18 @@ int ed_recur_step(const ed_recur_args* a, void* stream) {
 
 int ed_attn_row_elems(int kv_heads, int dim, int vdim) { return attn_row_elems(kv_heads, dim, vdim); }
 
+namespace {
+bool attn_plan_ok(int dtype, int heads, int kv_heads, int dim, int vdim, int n_seqs, int max_q, int max_keys) {
+    return dtype_ok(dtype) && attn_supported(heads, kv_heads, dim, vdim, 0) && n_seqs > 0 && n_seqs <= kMaxSeqs && max_q > 0 && max_q <= kMaxRows && max_keys > 0;
+}
+}  // namespace
+
 int ed_attn_splits(int dtype, int heads, int kv_heads, int dim, int vdim, int n_seqs, int max_q, int max_keys) {
-    if (!dtype_ok(dtype) || !attn_supported(heads, kv_heads, dim, vdim, 0) || n_seqs <= 0 || n_seqs > kMaxSeqs || max_q <= 0 || max_q > kMaxRows || max_keys <= 0)
-        return 0;
-    return attn_splits(dtype, heads, kv_heads, dim, n_seqs, max_q, max_keys);
+    return attn_plan_ok(dtype, heads, kv_heads, dim, vdim, n_seqs, max_q, max_keys) ? attn_splits(dtype, heads, kv_heads, dim, n_seqs, max_q, max_keys) : 0;
+}
+
+int ed_attn_ranges(int dtype, int heads, int kv_heads, int dim, int vdim, int n_seqs, int max_q, int max_keys) {
+    return attn_plan_ok(dtype, heads, kv_heads, dim, vdim, n_seqs, max_q, max_keys) ? attn_ranges(dtype, heads, kv_heads, dim, n_seqs, max_q, max_keys) : 0;
 }
 
 int ed_attn_prepare(const ed_attn_args* a, void* stream) {

@@ -62,7 +62,7 @@ class SoftmaxAttention(nn.Module):
     def splits(self, batch) -> int:
         """Ranges that the keys are shared out over."""
         keys = min(batch.max_context, self.window + batch.max_q) if self.window else batch.max_context
-        return _lib.load_decoder().ed_attn_splits(_lib.dtype_code(self.o.dtype), self.heads, self.kv_heads, self.dim, self.vdim, batch.n_seqs,
+        return _lib.load_decoder().ed_attn_ranges(_lib.dtype_code(self.o.dtype), self.heads, self.kv_heads, self.dim, self.vdim, batch.n_seqs,
                                                   batch.max_q, keys)
 
     def forward(self, h: torch.Tensor, batch, cache: torch.Tensor, carried: Optional[CarriedValues] = None) -> torch.Tensor:

@@ -225,6 +225,9 @@ int ed_attn_row_elems(int kv_heads, int dim, int vdim);
 /* Ranges of keys that fill the chip, for n_seqs portions of at most max_q tokens that see at most max_keys keys (0: sizes that are
  * not taken). */
 int ed_attn_splits(int dtype, int heads, int kv_heads, int dim, int vdim, int n_seqs, int max_q, int max_keys);
+/* The same, but one range where ed_attn_paged then gives every workgroup a CU and eight waves: the faster choice; any number of ranges
+ * gives the same result up to the order of sums. */
+int ed_attn_ranges(int dtype, int heads, int kv_heads, int dim, int vdim, int n_seqs, int max_q, int max_keys);
 /* Norms, rotation and mixing: keys and values into the cache, queries into q_rows. */
 int ed_attn_prepare(const ed_attn_args* a, void* stream);
 /* Any portions; the keys of a row are shared out over `splits` (<= 64) workgroups. */
