@@ -33,6 +33,7 @@ class RaggedBatch:
     k_lens: torch.Tensor            # [n_seqs] context length, this step's tokens included
     k_begin: torch.Tensor           # [n_seqs + 1] first of a sequence's padded keys
     logit_rows: torch.Tensor        # rows whose logits are wanted
+    every_row: bool = False         # those are all rows, in their order
 
 
 @dataclass
@@ -165,4 +166,5 @@ def make_ragged(seqs: List[Sequence], block_size: int, chunk_tokens: int, device
     view["chunks"] = view["chunks"].view(-1, 4)
     return RaggedBatch(buffer=dev, n_seqs=n_seqs, max_q=max(counts, default=1),
                        max_context=padding.table_width * block_size if padding is not None else max(contexts),
-                       table_width=width, n_chunks=len(chunks) // 4, chunk_tokens=chunk_tokens, padded_keys=k_begin[-1], **view)
+                       table_width=width, n_chunks=len(chunks) // 4, chunk_tokens=chunk_tokens, padded_keys=k_begin[-1],
+                       every_row=rows is None and len(wanted) == q_begin[-1], **view)

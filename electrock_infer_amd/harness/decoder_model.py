@@ -84,4 +84,5 @@ class DecoderModel(nn.Module):
     # ---- forward ----
     def compute_logits(self, hidden: torch.Tensor, batch: RaggedBatch) -> torch.Tensor:
         """float32 logits of the batch's wanted rows."""
-        return linear_f32(hidden.index_select(0, batch.logit_rows), self.head)
+        rows = hidden if batch.every_row else hidden.index_select(0, batch.logit_rows)       # (2-5 us of a decode step)
+        return linear_f32(rows, self.head)

@@ -50,3 +50,15 @@ def test_padded_steps_overwrite_the_buffer():
     fresh = make_ragged(second, 16, 16, "cpu", padding=pad)
     assert torch.equal(kept.buffer, fresh.buffer)
     assert fresh.tokens.tolist()[3] == 0 and fresh.cache_rows.tolist()[3] == 90 * 16 and fresh.state_slots.tolist()[3] == 3
+
+
+def test_every_row_is_wanted_of_single_tokens_only():
+    def seq(n, start, slot):
+        s = Sequence([1] * (start + n), SamplingParams(temperature=0.0, max_tokens=4))
+        s.block_table, s.state_slot, s.num_computed_tokens, s.num_scheduled_tokens = [slot], slot, start, n
+        return s
+    one, two = seq(1, 3, 0), seq(2, 0, 1)
+    assert make_ragged([one], 16, 64, "cpu").every_row and make_ragged([one, seq(1, 0, 1)], 16, 64, "cpu").every_row
+    assert not make_ragged([one, two], 16, 64, "cpu").every_row and not make_ragged([one], 16, 64, "cpu", rows=[0]).every_row
+    padded = make_ragged([one], 16, 64, "cpu", padding=DecodePadding(4, 8, 9, 9))
+    assert padded.every_row and padded.logit_rows.tolist() == [0, 1, 2, 3]
