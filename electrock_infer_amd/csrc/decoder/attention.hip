@@ -9,8 +9,8 @@
 // transposing reads.
 //
 // paged_kernel: any portion, both types; a wave takes tiles of 32 keys for 16 (token, head) rows that share a key/value
-// head, on its own, and the workgroup's four waves add up at the end.  prompt_kernel: long portions, bf16; 128 queries of
-// a head per workgroup, 32 per wave, tiles of 64 keys shared by the four waves.
+// head, on its own, and the workgroup's four or eight waves add up at the end.  prompt_kernel: long portions, bf16; 128 or 64
+// queries of a head per workgroup, 32 or 16 per wave, tiles of 64 keys shared by four waves.
 #include "decoder.h"
 #include "mma.h"
 

@@ -1,6 +1,7 @@
 // A per-layer token input.  token_gate_kernel is the gate product with its epilogue,
 //     g[t] = gelu_tanh(gate x_t) * side[token_t],
-// spread over as many workgroups as there are 16 x 16 tiles of g: what decoding needs.  token_side_kernel is the end of a
+// spread over as many workgroups as there are 16 x 16 tiles of g; token_parts_kernel and token_proj_kernel share the gate out over the chip
+// and make the projection too (bf16, few rows).  token_side_kernel is the end of a
 // layer in one launch (bf16), for prompts, where there are rows enough to fill the chip with 16 each:
 //     x <- x + y / rms(y) * post_w                       (the feed-forward's result)
 //     g  = gelu_tanh(gate x) * side[token]
