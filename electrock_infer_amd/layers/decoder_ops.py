@@ -147,6 +147,13 @@ class NormedRows:
         return result
 
 
+def _takes_rows(module) -> bool:
+    """Whether a layer's own forward is one of those that hand their input to one product: said by the class that defines it, so that a
+    forward put in its place, by a subclass or on the object, gets a tensor."""
+    defined = next((vars(c) for c in type(module).__mro__ if "forward" in vars(c)), {})
+    return defined.get("takes_normed_rows", False) and "forward" not in vars(module)
+
+
 def _unwatched(module) -> bool:
     return not _global_hooks and not _global_pre_hooks and not any(m._forward_hooks or m._forward_pre_hooks for m in module.modules())
 
@@ -155,7 +162,7 @@ def normed_rows(x: torch.Tensor, y: torch.Tensor, post_w: torch.Tensor, eps: flo
     """``residual_norm(ADD_NORMED, ...)`` for rows that ``reader`` reads next: ``out``, or for a row or two ``NormedRows``, where it is a layer
     of this package that hands them to one product and nobody watches what it is given."""
     T, K = out.shape
-    if T <= 2 and getattr(reader, "takes_normed_rows", False) and _unwatched(reader) and x.is_cuda and x.is_contiguous() and y.is_contiguous() and out.is_contiguous() and out.dtype is _BF16 and \
+    if T <= 2 and reader is not None and _takes_rows(reader) and _takes_rows(getattr(reader, "in_proj", reader)) and _unwatched(reader) and x.is_cuda and x.is_contiguous() and y.is_contiguous() and out.is_contiguous() and out.dtype is _BF16 and \
             (y.dtype is _BF16 and y.dim() == 2 or y.dtype is torch.float32) and (x.data_ptr() | y.data_ptr()) % 16 == 0 and \
             _lib.load_decoder().ed_norm_gemm_supported(T, 1, K, 0) == 1:
         return NormedRows(x, y, post_w, next_w, eps, out, torch.empty_like(x))
@@ -360,6 +367,8 @@ class StackedRows:
 class StackedLinear(torch.nn.Module):
     """Several projections of one input as a single matrix.  A section starts at a multiple of eight rows (zeros between),
     so that vector loads of its outputs are aligned."""
+
+    takes_normed_rows = True
 
     def __init__(self, width: int, sections, dtype):
         super().__init__()

@@ -20,8 +20,6 @@ class DecayedRecurrence(nn.Module):
     """What both mixers share: q, k [kv_heads, dim] and v [heads, vdim] from convolutions over ``in_proj``'s sections of
     these names, decay inputs in its section ``decay``, and the recurrence itself."""
 
-    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
-
     def __init__(self, width: int, heads: int, kv_heads: int, dim: int, vdim: int, taps: int, eps: float, sections: Dict[str, int],
                  conv_bias: bool, dtype):
         super().__init__()
@@ -86,6 +84,8 @@ class DecayedRecurrence(nn.Module):
 
 class GatedDeltaRule(DecayedRecurrence):
 
+    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
+
     def __init__(self, width: int, heads: int, kv_heads: int, dim: int, vdim: int, taps: int, eps: float, dtype):
         super().__init__(width, heads, kv_heads, dim, vdim, taps, eps,
                          {"q": kv_heads * dim, "k": kv_heads * dim, "v": heads * vdim, "gate": heads * vdim, "decay": heads,
@@ -105,6 +105,8 @@ class GatedDeltaRule(DecayedRecurrence):
 
 class StateSpaceMixer(DecayedRecurrence):
     """Mamba-2: q, k and v are C, B and x; a skip per head; the gated output is normed in ``norm_groups`` parts."""
+
+    takes_normed_rows = True     # (its input goes to one product: decoder_ops.normed_rows)
 
     def __init__(self, width: int, heads: int, groups: int, state: int, vdim: int, taps: int, norm_groups: int, eps: float, dtype):
         inner, shared = heads * vdim, groups * state

@@ -78,3 +78,24 @@ def test_rows_reach_the_product_either_way(T, K):
             assert torch.equal(seen[0], want)
         assert (stream - kept).abs().max() <= 2.0 ** -22 * kept.abs().max()
         assert (out.float() - ops.linear(want, w).float()).abs().max() <= 2.0 ** -6 * out.float().abs().max()      # (a row's last bit may turn)
+
+
+@pytest.mark.parametrize("change", ["subclass", "object", "projection", "none"])
+def test_a_forward_of_ones_own_gets_a_tensor(change):
+    from electrock_infer_amd.layers.attention import SoftmaxAttention
+    from electrock_infer_amd.layers.dense_mlp import DenseMLP
+    x, y, w = torch.randn(1, 1024, device="cuda"), torch.randn(2, 1, 1024, device="cuda"), torch.ones(1024, device="cuda")
+
+    class Own(DenseMLP):
+        def forward(self, h):
+            return super().forward(h * 1)
+
+    if change == "projection":
+        reader = SoftmaxAttention(1024, 8, 2, 64, 64, 1.0, 1e-6, BF16)
+        reader.in_proj = torch.nn.Linear(1024, 768)
+    else:
+        reader = (Own if change == "subclass" else DenseMLP)(1024, 512, BF16)
+        if change == "object":
+            reader.forward = lambda h: h * 1
+    rows = ops.normed_rows(x, y, w, 1e-6, torch.empty(1, 1024, dtype=BF16, device="cuda"), None, reader)
+    assert (type(rows) is ops.NormedRows) == (change == "none")
