@@ -86,6 +86,7 @@ struct TileGemm {
     int splits, T, N, K, act;
 };
 constexpr int64_t kTileGemmRows = 1 << 20;
+constexpr int kMostSplits = 64;   // ranges of K, each of one step of 64 at least
 bool tile_gemm_supported(int64_t T, int N, int K);
 bool tile_gemm_pays(int64_t T, int N, int K, int act, bool parts);
 int tile_gemm_splits(int64_t T, int N, int K);
@@ -123,6 +124,7 @@ struct TokenInputProblem {
     int W, dim, n_parts;
 };
 int token_input_parts(int64_t T, int W, int dim);
+int token_input_most_parts(int64_t T, int W);
 int launch_token_input(const TokenInputProblem& p, hipStream_t s);
 bool token_side_supported(int W, int dim);
 inline bool token_side_packable(int W, int dim) { return W % 128 == 0 && dim % 32 == 0; }

@@ -251,7 +251,7 @@ int ed_tile_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_strid
     if (out_dtype != EM_DTYPE_BF16 && out_dtype != EM_DTYPE_F32) return EM_ERR_BAD_DTYPE;
     if (T == 0) return 0;
     if (!tile_gemm_supported(T, N, K)) return EM_ERR_UNSUPPORTED;
-    if (splits < 1 || splits > 64 || splits > K / 64 || act < 0 || act > 2 || (splits > 1 && (act != 0 || out_dtype != EM_DTYPE_F32)) ||
+    if (splits < 1 || splits > kMostSplits || splits > K / 64 || act < 0 || act > 2 || (splits > 1 && (act != 0 || out_dtype != EM_DTYPE_F32)) ||
         (act != 0 && out_dtype != EM_DTYPE_BF16) || x_stride < K || w_stride < K)
         return EM_ERR_BAD_SHAPE;
     if (!x || !w || !out) return EM_ERR_NULL_POINTER;
@@ -285,7 +285,7 @@ int ed_token_input(const void* x, const void* gate, const void* proj, const int3
     if (T < 0 || T > kMaxRows || column0 < 0 || column0 + static_cast<int64_t>(dim) > table_stride) return EM_ERR_BAD_SHAPE;
     if (T == 0) return 0;
     if (token_input_parts(T, W, dim) == 0) return EM_ERR_UNSUPPORTED;
-    if (n_parts < 1 || n_parts > W / 32 || n_parts > 65535) return EM_ERR_BAD_SHAPE;
+    if (n_parts < 1 || n_parts > token_input_most_parts(T, W)) return EM_ERR_BAD_SHAPE;
     if (!x || !gate || !proj || !tokens || !table || !parts || !out) return EM_ERR_NULL_POINTER;
     if (!aligned16(x) || !aligned16(gate) || !aligned16(proj) || !aligned16(parts) || !aligned16(out) || column0 % 4 != 0 || table_stride % 4 != 0 ||
         reinterpret_cast<uintptr_t>(table) % 8 != 0)

@@ -541,6 +541,9 @@ int token_input_parts(int64_t T, int W, int dim) {
     return static_cast<int>(std::min<int64_t>({most, std::max<int64_t>(1, 256 / groups), T > kSomeTokens ? 4 : T > kFewTokens ? 8 : 16}));
 }
 
+// The most ranges that the kernel of the gate product makes: none of them empty (its steps are of 32 columns, the tiled product's of 64).
+int token_input_most_parts(int64_t T, int W) { return T > kFewTokens ? std::min(W / 64, kMostSplits) : std::min(W / 32, 65535); }
+
 int launch_token_input(const TokenInputProblem& p, hipStream_t s) {
     if (p.T > kFewTokens) {
         TileGemm g{};
