@@ -18,8 +18,10 @@
 // float32, 64 tokens 43.0 / 53.0 (6.1 TB/s).  That one shares K out over a workgroup's waves and stays ahead where the rows are few and the
 // results whole (3072 x 2048, one token 7.7 / 5.7).
 //
-// The sum of a result runs over K from a place that depends on its tile (tiles side by side ask for different parts of their rows at
-// a time).
+// The sum of a result runs over K from a place that depends on its tile of columns (tiles side by side ask for different parts of their
+// rows at a time), and on nothing else: tokens that are alike have the same results wherever they stand.  Tiles that share weight rows a
+// little behind each other too, so that the first brings them into L2, would be 2 to 5 % of a few products (us, 300 x 2048 x 6144 parts 17.4 / 17.8,
+// 1000 x 3072 x 2048 20.0 / 21.0, 1000 x 12288 x 4096 111.6 / 115) and lose as much of others (300 x 2048 x 2048 parts 8.2 / 7.7).
 #include "decoder.h"
 #include "mma.h"
 #include "../lds_copy.h"
@@ -94,10 +96,7 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void tile_gemm_kernel(const uint1
         src[i] += static_cast<int64_t>(s0) * kStepK + piece;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
-    // Tiles side by side start at different places of their rows, and those that share weight rows a little behind each other: the first
-    // brings a row into L2 and the others find it there (steps per column / row tile, us: 300 x 2048 x 6144 parts 5 / 0 18.0, 1 / 2 17.2, 1000 x
-    // 2048 x 6144 parts 32.9, 30.3; 5 / 4 loses the rows again: 300 x 4096 x 12288 parts 59.6 instead of 38.5).  Gated: 5 / 0, halves lie far apart.
-    const int rot = (m_tiles == 1 || ACT == 2 ? nt * 5 : nt + mt * 2) % nk;
+    const int rot = nt * 5 % nk;
     auto place = [&](int step) {         // elements into the range of K
         const int k = step + rot;
         return (k >= nk ? k - nk : k) * kStepK;
