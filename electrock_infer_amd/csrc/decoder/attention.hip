@@ -482,7 +482,7 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
 // and its second product for the scores, with two waves on a SIMD.  So a score is kept cheap and a tile free of waits:
 //   * the cap's tanh takes two of the three slow instructions of a score (exponential, reciprocal).  Up to kTanhRange caps
 //     tanh(x) is x times a polynomial of degree four in x * x (its coefficients as written: 9.1e-8 of the value at the end of the
-//     range, in float32 with the cap in them 1.5e-7, one to two units in the last place); a wave whose 32 x 64 scores all lie there takes it, four scores in step, others take the exponential.  Caps
+//     range, in float32 with the cap in them 1.5e-7, one to two units in the last place); 16 queries whose 16 x 64 scores all lie there take it, four scores in step, others take the exponential.  Caps
 //     are chosen far above ordinary scores.
 //   * the page of a tile's keys is asked for a tile ahead of its use and in front of the loads that use the one before, and the
 //     rows are read from LDS in front of the barrier; loads have no condition of their own (keys behind the last stand for it).
@@ -530,8 +530,8 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
     const int32_t* table = p.tables + static_cast<int64_t>(seq) * p.table_width;
     const uint16_t* keys = static_cast<const uint16_t*>(p.cache) + g * dp;
     const uint16_t* values = static_cast<const uint16_t*>(p.cache) + p.kv_heads * dp + g * vp;
-    // the page of the key that thread tid < 64 looks up; keys behind the last one stand for it (their scores are masked)
-    auto key_of = [&](int tile) { return min(tile * kTileKeys + tid, last_pos); };
+    // the page of the key that thread tid < 64 looks up; keys behind the portion's last stand for it (their scores are masked)
+    auto key_of = [&](int tile) { return min(tile * kTileKeys + tid, start + nq - 1); };
     auto page_of = [&](int tile) { return tid < kTileKeys ? table[key_of(tile) / p.block_size] : 0; };
     auto keep_rows = [&](int tile, int page) {
         if (tid < kTileKeys) Kr[tile & 1][tid] = static_cast<int64_t>(page * p.block_size + key_of(tile) % p.block_size) * row_elems;
@@ -620,30 +620,34 @@ __global__ __launch_bounds__(256, GROUPS) void attn_prompt_kernel(AttnProblem p)
             }
         // scores in units of log2; with a fixed maximum their distance to it
         if (kPoly && fixed) {
-            float top = 0.0f;
+            // The form of tanh shows in a score's last bits, so 16 queries choose it for themselves: theirs do not depend on how many a wave
+            // has, and so not on the portions beside this one.
+            bool small[QT];
 #pragma unroll
-            for (int n = 0; n < 4; ++n)
-#pragma unroll
-                for (int j = 0; j < QT; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) top = fmaxf(top, fabsf(s[n][j][r]));
-            if (__all(top * fabsf(to_cap) <= kTanhRange)) {
+            for (int j = 0; j < QT; ++j) {
+                float top = 0.0f;
 #pragma unroll
                 for (int n = 0; n < 4; ++n)
 #pragma unroll
-                    for (int j = 0; j < QT; ++j) {
+                    for (int r = 0; r < 4; ++r) top = fmaxf(top, fabsf(s[n][j][r]));
+                small[j] = __all(top * fabsf(to_cap) <= kTanhRange);
+            }
+#pragma unroll
+            for (int j = 0; j < QT; ++j) {
+                if (small[j]) {
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) {
                         const f32x4_t x = s[n][j] * to_cap, u = x * x;
                         f32x4_t t = fma4(fma4(f32x4_t(tanh4), u, f32x4_t(tanh3)), u, f32x4_t(tanh2));
                         t = fma4(fma4(t, u, f32x4_t(tanh1)), u, f32x4_t(tanh0));
                         s[n][j] = fma4(x, t, f32x4_t(-cap2));
                     }
-            } else {
+                } else {
 #pragma unroll
-                for (int n = 0; n < 4; ++n)
-#pragma unroll
-                    for (int j = 0; j < QT; ++j)
+                    for (int n = 0; n < 4; ++n)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) s[n][j][r] = -2.0f * cap2 * __builtin_amdgcn_rcpf(exp2_fast(s[n][j][r] * in_cap) + 1.0f);
+                }
             }
         } else if (capped) {
 #pragma unroll
@@ -806,8 +810,7 @@ bool few_queries(const AttnProblem& p, int n_seqs, int max_q) {
 
 template <int DKT>
 int launch_prompt(const AttnProblem& p, int n_seqs, int max_q, hipStream_t s) {
-    // (heads of up to 64 under a cap keep 32 queries to a wave: which form of tanh a wave's scores take shows in their last bits)
-    const bool few = few_queries(p, n_seqs, max_q) && (DKT > 2 || p.softcap <= 0.0f || p.softcap > kFixedCap);
+    const bool few = few_queries(p, n_seqs, max_q);
     if (p.vdim > 64) return few ? launch_queries<DKT, 8, 1, 2>(p, n_seqs, max_q, s) : launch_queries<DKT, 8, 2, 2>(p, n_seqs, max_q, s);
     if (few) return launch_queries<DKT, 4, 1, 2>(p, n_seqs, max_q, s);
     if constexpr (DKT == 2)
