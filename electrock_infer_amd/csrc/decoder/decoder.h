@@ -261,6 +261,6 @@ struct LatentPromptProblem {
     float scale;
 };
 bool latent_prompt_supported(int dim, int rot, int vdim);
-int launch_latent_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, int max_context, hipStream_t s);
+int launch_latent_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s);
 
 }  // namespace em

@@ -509,9 +509,9 @@ int ed_latent_gather(const void* cache, const int32_t* tables, int table_width, 
 
 int ed_latent_prompt_supported(int dim, int rot, int vdim) { return latent_prompt_supported(dim, rot, vdim) ? 1 : 0; }
 
-int ed_latent_prompt(const ed_latent_prompt_args* a, void* stream) { return ed_latent_prompt_behind(a, 0, stream); }
+int ed_latent_prompt_behind(const ed_latent_prompt_args* a, int, void* stream) { return ed_latent_prompt(a, stream); }
 
-int ed_latent_prompt_behind(const ed_latent_prompt_args* a, int max_context, void* stream) {
+int ed_latent_prompt(const ed_latent_prompt_args* a, void* stream) {
     if (!a) return EM_ERR_NULL_POINTER;
     if (a->n_seqs < 0 || a->n_seqs > kMaxSeqs || a->max_q < 0 || a->max_q > kMaxRows || a->heads <= 0 || !(a->scale > 0.0f)) return EM_ERR_BAD_SHAPE;
     if (!latent_prompt_supported(a->dim, a->rot, a->vdim) || a->q_stride % 8 != 0 || a->k_stride % 8 != 0 ||
@@ -531,7 +531,7 @@ int ed_latent_prompt_behind(const ed_latent_prompt_args* a, int max_context, voi
     p.q_begin = a->q_begin; p.starts = a->starts; p.k_begin = a->k_begin;
     p.heads = a->heads; p.dim = a->dim; p.rot = a->rot; p.vdim = a->vdim;
     p.scale = a->scale;
-    return launch_latent_prompt(p, a->n_seqs, a->max_q, max_context, as_stream(stream));
+    return launch_latent_prompt(p, a->n_seqs, a->max_q, as_stream(stream));
 }
 
 }  // extern "C"

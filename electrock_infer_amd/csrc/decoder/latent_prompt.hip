@@ -17,31 +17,21 @@ namespace {
 constexpr int kTileKeys = 64;
 constexpr float kLog2e = 1.4426950408889634f;
 
-// LDS of four waves: a tile's keys and transposed values, and where there are several fours, their results in its place
-template <int DKT, int DVT, int QT, int GROUPS>
-constexpr int lds_bytes() {
-    constexpr int tile = 2 * (kTileKeys * (DKT * 32 + 8) + DVT * 16 * (kTileKeys + 8)), results = GROUPS == 1 ? 0 : 256 * QT * (DVT * 16 + 8);
-    return tile > results ? tile : results;
-}
-
-// DKT: 32-element steps of dim + rot; DVT: 16-element tiles of vdim; QT: 16-query tiles of a wave; GROUPS: of four waves that take the
-// tiles of the same queries in turn and add up at the end
-template <int DKT, int DVT, int QT, int GROUPS>
-__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 2 : 1) void latent_prompt_kernel(LatentPromptProblem p) {
+// DKT: 32-element steps of dim + rot; DVT: 16-element tiles of vdim; QT: 16-query tiles of a wave
+template <int DKT, int DVT, int QT>
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentPromptProblem p) {
     typedef Mma<BF16Elem> M;
     constexpr int kRowsPerWave = 16 * QT, kRows = 4 * kRowsPerWave;
     constexpr int LPK = DKT * 32 + 8, LPV = kTileKeys + 8;
     constexpr int kFetchK = kTileKeys * DKT * 4 / 256, kFetchV = DVT * 16 * (kTileKeys / 8) / 256;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / 256);
-    uint16_t* Ks = reinterpret_cast<uint16_t*>(smem + group * lds_bytes<DKT, DVT, QT, GROUPS>());
-    uint16_t* Vs = Ks + kTileKeys * LPK;
+    __shared__ __attribute__((aligned(16))) uint16_t Ks[kTileKeys * LPK];
+    __shared__ __attribute__((aligned(16))) uint16_t Vs[DVT * 16 * LPV];
     const int h = blockIdx.x, seq = blockIdx.z;
     const int row0 = p.q_begin[seq], nq = p.q_begin[seq + 1] - row0;
     const int t0 = (static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y)) * kRows;  // long rows start first
     if (t0 >= nq) return;
     const int start = p.starts[seq];
-    const int tid = threadIdx.x % 256, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
     const int D = p.dim + p.rot;
     const int64_t k0 = p.k_begin[seq];
     const int n_tiles = (start + min(t0 + kRows, nq) + kTileKeys - 1) / kTileKeys;
@@ -89,9 +79,8 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 2 : 1) void latent_prom
     }
     const float c2 = p.scale * kLog2e;
 
-    if (group < n_tiles) fetch(group);
-    for (int round = 0; round < n_tiles; round += GROUPS) {
-        const int tile = round + group;
+    fetch(0);
+    for (int tile = 0; tile < n_tiles; ++tile) {
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < kFetchK; ++i) {
@@ -109,8 +98,8 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 2 : 1) void latent_prom
             *reinterpret_cast<u32x2_t*>(Vs + d * LPV + at + 8) = w[1];
         }
         __syncthreads();
-        if (tile + GROUPS < n_tiles) fetch(tile + GROUPS);
-        if ((GROUPS > 1 && tile >= n_tiles) || tile * kTileKeys > first_pos + kRowsPerWave - 1) continue;   // no key of this tile for this wave's queries
+        if (tile + 1 < n_tiles) fetch(tile + 1);
+        if (tile * kTileKeys > first_pos + kRowsPerWave - 1) continue;   // no key of this tile for this wave's queries
 
         f32x4_t s[4][QT];
 #pragma unroll
@@ -177,36 +166,6 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 2 : 1) void latent_prom
                 for (int j = 0; j < QT; ++j) o[d][j] = M::mac(fv, fp[k][j], o[d][j]);
             }
     }
-    if constexpr (GROUPS > 1) {
-        // the other groups' outputs, maxima and sums, lane by lane, through the tiles' LDS
-        __syncthreads();
-        if (group > 0) {
-            f32x4_t* mine = reinterpret_cast<f32x4_t*>(Ks) + tid;
-#pragma unroll
-            for (int d = 0; d < DVT; ++d)
-#pragma unroll
-                for (int j = 0; j < QT; ++j) mine[(d * QT + j) * 256] = o[d][j];
-            f32x2_t* ml = reinterpret_cast<f32x2_t*>(Ks + 256 * DVT * QT * 8) + tid;
-#pragma unroll
-            for (int j = 0; j < QT; ++j) ml[j * 256] = f32x2_t{m[j], l[j]};
-        }
-        __syncthreads();
-        if (group > 0) return;
-#pragma unroll
-        for (int g = 1; g < GROUPS; ++g) {
-            const uint8_t* theirs = smem + g * lds_bytes<DKT, DVT, QT, GROUPS>();
-#pragma unroll
-            for (int j = 0; j < QT; ++j) {
-                const f32x2_t ml = reinterpret_cast<const f32x2_t*>(theirs + 256 * DVT * QT * 16)[j * 256 + tid];
-                const float mn = fmaxf(m[j], ml[0]), base = mn == -INFINITY ? 0.0f : mn;
-                const float here = __builtin_amdgcn_exp2f(m[j] - base), there = __builtin_amdgcn_exp2f(ml[0] - base);
-                m[j] = mn;
-                l[j] = l[j] * here + ml[1] * there;
-#pragma unroll
-                for (int d = 0; d < DVT; ++d) o[d][j] = o[d][j] * here + reinterpret_cast<const f32x4_t*>(theirs)[(d * QT + j) * 256 + tid] * there;
-            }
-        }
-    }
     const float sk = p.sink[h] * kLog2e;
 #pragma unroll
     for (int j = 0; j < QT; ++j) {
@@ -227,13 +186,10 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 2 : 1) void latent_prom
     }
 }
 
-template <int DKT, int DVT, int QT, int GROUPS>
+template <int DKT, int DVT, int QT>
 int launch_tiles(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s) {
-    constexpr size_t kLds = static_cast<size_t>(GROUPS) * lds_bytes<DKT, DVT, QT, GROUPS>();
-    const int rc = allow_lds(reinterpret_cast<const void*>(latent_prompt_kernel<DKT, DVT, QT, GROUPS>), kLds);
-    if (rc != 0) return rc;
     const dim3 grid(static_cast<unsigned>(p.heads), static_cast<unsigned>(ceil_div(max_q, 64 * QT)), static_cast<unsigned>(n_seqs));
-    launch((latent_prompt_kernel<DKT, DVT, QT, GROUPS>), grid, dim3(256 * GROUPS), kLds, s, p);
+    launch((latent_prompt_kernel<DKT, DVT, QT>), grid, dim3(256), 0, s, p);
     return launch_status();
 }
 
@@ -243,31 +199,27 @@ int launch_tiles(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_
 // 4 x 512 25.7 / 24.0; 384, 3072 123 / 88; 512, 4 x 1024 55.8 / 57.1, 4096 163 / 152, behind 4000 328 / 385; 1024, 8192
 // 397 / 520; a little below 512, portions that end early in their last 128 queries lose: 480, 15 x 200, heads of 128 + 32 21.5 /
 // 24.2).  Keys of up to 128 elements under values of more than 64 gain little from it, and only while the workgroups of 64 have a
-// CU each (96 + 32, values of 128: 128, 1000 behind 1000 56.6 / 51.4; 256, 2 x 1000 behind 3000 107 / 126).
-// Where workgroups of 64 are few and the longest context is known to make seven tiles, eight waves take them,
-// every other tile each four of them: half the chain, on SIMDs that held one wave (us, four waves / eight, heads of 128 + 64: 80 workgroups, 300
-// tokens behind 1000 34.2 / 29.8; 256, one prompt of 1000 28.0 / 24.7; 384, 1536 43.4 / 35.7; 512, two rounds of them, 32.0 / 32.9; seven tiles
-// 14.6 / 14.5, five 11.3 / 12.0; 96 + 32, 80 workgroups 32.8 / 26.4).  Three fours spill: 37.0.
+// CU each (96 + 32, values of 128: 128, 1000 behind 1000 56.6 / 51.4; 256, 2 x 1000 behind 3000 107 / 126).  A query's sums keep
+// their order either way.  (Eight waves, every other tile each four of them, are faster where workgroups of 64 are few, 300 tokens behind 1000
+// 35.5 / 29.2, one prompt of 1000 28.6 / 23.7, but add up in an order that would then depend on the other portions; eight that share every tile's
+// keys and value columns in the same order wait for each other twice a tile: 35.8, 28.6.)
 template <int DKT, int DVT>
 constexpr int64_t few_workgroups() { return DKT <= 4 && DVT > 4 ? 160 : 448; }
 
 template <int DKT, int DVT>
-int launch_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, int max_context, hipStream_t s) {
-    if (ceil_div(max_q, 128) * p.heads * n_seqs < few_workgroups<DKT, DVT>()) {
-        if (ceil_div(max_q, 64) * p.heads * n_seqs <= 384 && max_context > 6 * kTileKeys) return launch_tiles<DKT, DVT, 1, 2>(p, n_seqs, max_q, s);
-        return launch_tiles<DKT, DVT, 1, 1>(p, n_seqs, max_q, s);
-    }
-    return launch_tiles<DKT, DVT, 2, 1>(p, n_seqs, max_q, s);
+int launch_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s) {
+    if (ceil_div(max_q, 128) * p.heads * n_seqs < few_workgroups<DKT, DVT>()) return launch_tiles<DKT, DVT, 1>(p, n_seqs, max_q, s);
+    return launch_tiles<DKT, DVT, 2>(p, n_seqs, max_q, s);
 }
 
 template <int DVT>
-int dispatch_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, int max_context, hipStream_t s) {
+int dispatch_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s) {
     const int D = p.dim + p.rot;
-    if (D <= 64) return launch_prompt<2, DVT>(p, n_seqs, max_q, max_context, s);
-    if (D <= 96) return launch_prompt<3, DVT>(p, n_seqs, max_q, max_context, s);
-    if (D <= 128) return launch_prompt<4, DVT>(p, n_seqs, max_q, max_context, s);
-    if (D <= 192) return launch_prompt<6, DVT>(p, n_seqs, max_q, max_context, s);
-    return launch_prompt<8, DVT>(p, n_seqs, max_q, max_context, s);
+    if (D <= 64) return launch_prompt<2, DVT>(p, n_seqs, max_q, s);
+    if (D <= 96) return launch_prompt<3, DVT>(p, n_seqs, max_q, s);
+    if (D <= 128) return launch_prompt<4, DVT>(p, n_seqs, max_q, s);
+    if (D <= 192) return launch_prompt<6, DVT>(p, n_seqs, max_q, s);
+    return launch_prompt<8, DVT>(p, n_seqs, max_q, s);
 }
 
 }  // namespace
@@ -277,8 +229,8 @@ bool latent_prompt_supported(int dim, int rot, int vdim) {
     return dim > 0 && dim % 8 == 0 && rot >= 0 && rot % 8 == 0 && dim + rot <= 256 && vdim > 0 && vdim % 4 == 0 && vdim <= 128;
 }
 
-int launch_latent_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, int max_context, hipStream_t s) {
-    return p.vdim <= 64 ? dispatch_prompt<4>(p, n_seqs, max_q, max_context, s) : dispatch_prompt<8>(p, n_seqs, max_q, max_context, s);
+int launch_latent_prompt(const LatentPromptProblem& p, int n_seqs, int max_q, hipStream_t s) {
+    return p.vdim <= 64 ? dispatch_prompt<4>(p, n_seqs, max_q, s) : dispatch_prompt<8>(p, n_seqs, max_q, s);
 }
 
 }  // namespace em

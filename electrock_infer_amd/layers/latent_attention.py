@@ -111,4 +111,4 @@ class LatentAttention(nn.Module):
                                   q_begin=batch.q_begin.data_ptr(), starts=batch.starts.data_ptr(),
                                   k_begin=batch.k_begin.data_ptr(), n_seqs=batch.n_seqs, max_q=batch.max_q, heads=self.heads,
                                   dim=self.dim, rot=self.rot, vdim=self.vdim, scale=self.scale)
-        _lib.check_decoder(lib.ed_latent_prompt_behind(byref(a), batch.max_context, stream), "latent_prompt")
+        _lib.check_decoder(lib.ed_latent_prompt(byref(a), stream), "latent_prompt")

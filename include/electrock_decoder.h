@@ -312,7 +312,7 @@ typedef struct ed_latent_prompt_args {
 
 int ed_latent_prompt_supported(int dim, int rot, int vdim);
 int ed_latent_prompt(const ed_latent_prompt_args* a, void* stream);
-/* The same for contexts of up to max_context keys, this portion's included (0: not known): a hint for how the work is shared out. */
+/* The same, by callers that know the longest context, max_context keys: the results do not depend on it, nor does anything else. */
 int ed_latent_prompt_behind(const ed_latent_prompt_args* a, int max_context, void* stream);
 
 #ifdef __cplusplus
