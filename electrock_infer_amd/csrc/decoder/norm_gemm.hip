@@ -1,14 +1,12 @@
 // out = act(h w^T) for the row or two h that a residual norm leaves (bf16):
 //     x_out = x + y / rms(y) * post_w,   h = next_w ? x_out / rms(x_out) * next_w : x_out, rounded to bf16
-// One launch instead of two.  Every workgroup norms the rows anew while its weights, all of a wave's part of them at K <= 4096, are on
-// their way; the first one leaves the stream behind, in a place of its own, since the others still read x.
+// One launch instead of two.  Every workgroup norms the rows anew while its weights, all of a wave's part of them at K <= 2048 and half of it
+// at 4096, are on their way; the first one leaves the stream behind, in a place of its own, since the others still read x.
 //
 // Bound: the way from a launch to the first bytes, and the weights' bytes.  As in skinny_gemm.hip the waves share out k, load eight rows
 // of 128 bytes at a time and turn them through LDS of their own.  The rows' loads come first (they return in order), so that their two
 // sums over the workgroup run beside the weights' way.  A decode step of one token (width 2048, sixteen norms of which fifteen go this way)
-// 418 -> 389 us, width 4096 832 -> 785; another order of the columns in every workgroup changes nothing.
-#include <algorithm>
-
+// with this and without it, nothing else changed: 437 -> 401 us; another order of the columns in every workgroup changes nothing.
 #include "decoder.h"
 #include "mma.h"
 
@@ -246,11 +244,11 @@ template <int ROWS, int COLS>
 int launch_rows(const NormGemm& g, hipStream_t s) {
     constexpr int kAhead = 4;
     const int nt = tiles_of(g.N, g.act);
-    if (g.act == 2) return nt == 2 ? launch_one<ROWS, COLS, 2, kAhead, true>(g, s) : launch_one<ROWS, COLS, 4, 4, true>(g, s);
+    if (g.act == 2) return nt == 2 ? launch_one<ROWS, COLS, 2, kAhead, true>(g, s) : launch_one<ROWS, COLS, 4, kAhead, true>(g, s);
     if (nt == 1) return launch_one<ROWS, COLS, 1, kAhead, false>(g, s);
     if (nt == 2) return launch_one<ROWS, COLS, 2, kAhead, false>(g, s);
     if (nt == 3) return launch_one<ROWS, COLS, 3, kAhead, false>(g, s);
-    return launch_one<ROWS, COLS, 4, 4, false>(g, s);
+    return launch_one<ROWS, COLS, 4, kAhead, false>(g, s);
 }
 
 }  // namespace
@@ -259,15 +257,21 @@ bool norm_gemm_supported(int64_t T, int N, int K, int act) {
     return T > 0 && T <= 2 && N > 0 && N <= 16 * kGroups * 4 && K >= 512 && K <= 4096 && K % 512 == 0 && act >= 0 && act <= 2 && tiles_of(N, act) <= 4;
 }
 
-// Where one launch is faster than the norm's and the product's (us in a graph, two / one; y in parts and no next_w; weights read from memory).
-// One row: K = 1024, 3072 rows 6.0 / 3.9; 2048, 3072 rows 7.5 / 5.0, 6176 9.6 / 7.6, 8832 11.1 / 10.6, gated 2 x 4096 11.1 / 8.7-10.1, 12800 13.9 /
-// 13.9; 4096, 6144 rows 15.3 / 12-13, 12288 20.5 / 18.2, 12800 22.8 / 20.5, gated 2 x 8192 28.3 / 24-33.  The second sum that next_w brings costs
-// 0.5 to 0.8.  Two rows: 3072 rows of 2048 7.6 / 5.7, 6176 9.6 / 8.2, 8832 11.0 / 11.1, gated 2 x 4096 11.8 / 9.6-10.8; 12288 of 4096 20.6 / 19.3,
-// 12800 with next_w 23.1 / 23.9, gated 2 x 8192 28.7 / 28.7-34.  Four rows: the rows' bytes and sums are what a workgroup waits for (6176 rows of
+// Where one launch is faster than the norm's and the product's (us in a graph, two / one; y in parts and no next_w, whose second sum costs
+// the one 0.3 to 0.7 and the two 0.1 to 0.8; weights read from memory).  A wave has K / 512 steps and asks for four at a time, so K of 5 to 6 x 512
+// and more than four ask for some twice: large products of such K lose.  One row: 3072 rows of 512 5.3 / 3.9, 16384 7.9 / 8.8; 12000 of 1024
+// 9.1 / 8.3, 16384 10.4 / 11.7; 2048, 3072 rows 7.4 / 5.2, 8832 10.8 / 10.4, 12000 12.8-13.3 / 13.0-13.2, gated 2 x 4096 10.9 / 8.7-10.1, 2 x 5632
+// 12.9 / 12.8; 2560, 8192 11.8 / 10.8, 12288 14.8 / 15.2; 3072, 9216 14.0 / 14.1, 16384 20.3 / 21.4; 3584, 12288 19.1 / 16.6; 4096, 6144 14.7 /
+// 10.8-14.2, 12288 20.5 / 18.0, 16384 26.9 / 24.8.  Two rows: 8192 of 2048 10.4 / 9.7, 8832 10.9 / 11.3; 8192 of 3072 13.0 / 12.4, 9216 14.2 / 15.2;
+// 12288 of 3584 19.2 / 17.8, of 4096 20.9 / 19.1, 8192 of 4096 16.3 / 14-18.  Long gated rows, whose halves lie a power of two apart: 2 x 4096 of
+// 4096 16.2 / 12.7 and 16.4 / 13.9, but 2 x 6144 21.3 / 19.4-26.5 and 21.4 / 20.7-27.7, 2 x 8192 28.2 / 24.0-32.9, by the queue that runs it; a step of
+// one token with 2 x 8192, width 4096, 879 either way.  Four rows: the rows' bytes and sums are what a workgroup waits for (6176 rows of
 // 2048 9.7 / 9.7, with next_w 10.0 / 12.0), so no more than two are taken.
 bool norm_gemm_pays(int T, int N, int K, int act) {
     const int64_t rows = act == 2 ? 2 * static_cast<int64_t>(N) : N;
-    return T == 1 ? K > 2048 || rows < 12288 : rows <= (K > 2048 ? 12288 : 8192);
+    if (act == 2 && K > 2048) return rows <= 8192;
+    if (K >= 3584) return T == 1 || rows <= 12288;
+    return T == 1 ? rows < 12288 : rows <= 8192;
 }
 
 int launch_norm_gemm(const NormGemm& g, hipStream_t s) {
