@@ -48,7 +48,7 @@ DECODER_SYMBOLS = (
     "ed_version", "ed_embed", "ed_residual_norm", "ed_relu_squared", "ed_silu_gate", "ed_gated_norm", "ed_argmax", "ed_token_gate", "ed_skinny_gemm_splits", "ed_skinny_gemm",
     "ed_norm_gemm_supported", "ed_norm_gemm_pays", "ed_norm_gemm", "ed_decode_gemm_splits", "ed_decode_gemm_pays", "ed_decode_gemm_plain_pays", "ed_decode_gemm",
     "ed_tile_gemm_splits", "ed_tile_gemm_pays", "ed_tile_gemm",
-    "ed_token_input_parts", "ed_token_input", "ed_token_side_supported", "ed_token_side", "ed_token_side_packable", "ed_token_side_pack_pays", "ed_token_side_pack", "ed_token_side_packed", "ed_gla_prefill", "ed_gla_step",
+    "ed_token_input_parts", "ed_token_input_pays", "ed_token_input", "ed_token_side_supported", "ed_token_side", "ed_token_side_packable", "ed_token_side_pack_pays", "ed_token_side_pack", "ed_token_side_packed", "ed_gla_prefill", "ed_gla_step",
     "ed_recur_record", "ed_recur_prefill", "ed_recur_step",
     "ed_attn_row_elems", "ed_attn_splits", "ed_attn_ranges", "ed_attn_prepare", "ed_attn_paged", "ed_attn_prompt_supported", "ed_attn_prompt",
     "ed_latent_row_elems", "ed_latent_splits", "ed_latent_waves", "ed_latent_prepare", "ed_latent_front", "ed_latent_paged", "ed_head_gemm", "ed_latent_gather",
@@ -225,6 +225,7 @@ def load_decoder() -> ctypes.CDLL:
         "ed_attn_prompt": [ctypes.POINTER(AttnArgs), vp],
         "ed_token_gate": [vp, vp, vp, vp, i64, i32, vp, i64, i32, i32, i32, vp],
         "ed_token_input_parts": [i64, i32, i32],
+        "ed_token_input_pays": [i64, i32, i32],
         "ed_token_input": [vp, vp, vp, vp, vp, i64, i32, vp, i32, vp, i64, i32, i32, vp],
         "ed_token_side_supported": [i32, i32],
         "ed_token_side": [vp, vp, vp, vp, vp, vp, vp, i64, i32, vp, vp, vp, i64, i64, i32, i32, dbl, vp],

@@ -124,6 +124,7 @@ struct TokenInputProblem {
     int W, dim, n_parts;
 };
 int token_input_parts(int64_t T, int W, int dim);
+bool token_input_pays(int64_t T, int W, int dim);
 int token_input_most_parts(int64_t T, int W);
 int launch_token_input(const TokenInputProblem& p, hipStream_t s);
 bool token_side_supported(int W, int dim);

@@ -280,6 +280,8 @@ int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const 
 
 int ed_token_input_parts(int64_t T, int W, int dim) { return T > kMaxRows ? 0 : token_input_parts(T, W, dim); }
 
+int ed_token_input_pays(int64_t T, int W, int dim) { return T <= kMaxRows && token_input_pays(T, W, dim) ? 1 : 0; }
+
 int ed_token_input(const void* x, const void* gate, const void* proj, const int32_t* tokens, const void* table, int64_t table_stride,
                    int column0, float* parts, int n_parts, void* out, int64_t T, int W, int dim, void* stream) {
     if (T < 0 || T > kMaxRows || column0 < 0 || column0 + static_cast<int64_t>(dim) > table_stride) return EM_ERR_BAD_SHAPE;

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kThreads) void token_gate_kernel(const typename Ele
 // The same and the projection behind it, p = proj g, in two launches of which neither waits for one CU's share of the weights: the gate product's
 // k is shared out over workgroups, which leave partial sums, and every workgroup of the projection adds up those of its tokens, a
 // few KB, in front of the gelu.  (As token_gate_kernel takes it, 23 tokens of 4096 columns are eight workgroups that bring in 256 KB each,
-// and more tokens are read once per 16 rows of the gate.)  MT: 16-token tiles of a workgroup; ND: 16-row tiles of the gate.
+// and more tokens are read once per 16 rows of the gate.)  ND: 16-row tiles of the gate.
 template <int ND>
 __global__ __launch_bounds__(256) void token_parts_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gate, float* __restrict__ parts,
                                                           int64_t T, int W) {
@@ -530,15 +530,30 @@ int launch_token_gate(const void* x, const void* gate, const int32_t* tokens, co
 }
 
 // How many ranges of W the gate product is shared out over: a workgroup for every CU (of 16 tokens, or the tiled product's of 64), 256
-// columns at least, and as few sums to add up as still pay; 0: the gate and the projection one by one (what this does not take, and where
-// it is not faster).  us, one by one / this, gates of 64: W = 4096, one token 9.5 / 6.8, 23 12.2 / 8.4, 64 13.2 / 8.6, 300 13.9 / 11.4, 1000 16.6 /
-// 15.0, 2244 33.5 / 24.6, 6000 66.5 / 41.7; 2048, one 6.8 / 6.2, 23 8.4 / 7.0, 300 9.7 / 9.2, 700 10.7 / 11.8, 1000 11.0 / 11.7, 1500 15.9 / 15.0, 3500 25.7 / 22.6.
+// columns at least, and as few sums to add up as still pay; 0: what this does not take, and numbers of tokens that leave the tiled product few
+// workgroups (gates of 64, W = 2048, 700 tokens one by one 10.7, this 11.8; 1000 11.0 / 11.7).
 constexpr int64_t kFewTokens = 64, kSomeTokens = 512;
 int token_input_parts(int64_t T, int W, int dim) {
     if (T <= 0 || W <= 0 || W % 64 != 0 || (dim != 32 && dim != 64 && dim != 128) || (T > kFewTokens && !tile_gemm_supported(T, dim, W))) return 0;
     if (T > kSomeTokens && T < 1280 && W <= 2048) return 0;
     const int64_t groups = T > kFewTokens ? ceil_div(T, 64) * ceil_div(dim, 64) : ceil_div(T, 16), most = std::max(W / 256, 1);
     return static_cast<int>(std::min<int64_t>({most, std::max<int64_t>(1, 256 / groups), T > kSomeTokens ? 4 : T > kFewTokens ? 8 : 16}));
+}
+
+// Where this is faster than the gate and the projection one by one: from this width on, by the gate's rows and the tokens (us, one by one / this.
+// Gates of 32: 1 x 256 6.0 / 5.2, 64 x 2048 9.1 / 5.8; 300 x 512 6.7 / 7.1, x 1024 8.0 / 7.3; 1280 x 512 7.0 / 7.6, x 1024 8.5 / 7.9.  Of 64: 1 x 1024
+// 5.9 / 6.1, x 2048 6.8 / 6.1, x 4096 9.3 / 6.7, 23 x 512 5.9 / 6.3, x 1024 6.7 / 6.3, x 4096 12.2 / 8.4; 300 x 1024 7.8 / 8.3, x 2048 9.7 / 9.1, x 4096
+// 13.9 / 11.2; 1280 x 1024 10.6 / 10.7, 4000 18.2 / 16.6, 2244 x 2048 20.9 / 19.0, x 4096 33.7 / 24.6.  Of 128: 1 x 8192 14.1 / 15.1, 23 x 3072 10.9 /
+// 12.3, x 4096 12.6 / 12.4; 128 x 3072 11.6 / 11.3, x 4096 13.2 / 11.8, 300 x 4096 14.4 / 15.0, x 8192 23.1 / 21.3; 1000 x 3072 20.3 / 19.4; 1280 x 1024
+// 12.8 / 14.7, x 2048 19.6 / 18.5, 4000 41.1 / 30.6).
+bool token_input_pays(int64_t T, int W, int dim) {
+    if (token_input_parts(T, W, dim) == 0) return false;
+    constexpr int kNever = 1 << 30;
+    int least;
+    if (T <= kFewTokens) least = dim == 32 ? 256 : dim == 64 ? (T < 16 ? 2048 : 1024) : (T < 16 ? kNever : 4096);
+    else if (T <= kSomeTokens) least = dim == 32 ? 1024 : dim == 64 ? 2048 : T <= 128 ? 4096 : 8192;
+    else least = dim == 32 || (dim == 64 && T >= 4000) ? 1024 : 2048;
+    return W >= least;
 }
 
 // The most ranges that the kernel of the gate product makes: none of them empty (its steps are of 32 columns, the tiled product's of 64).

@@ -313,8 +313,8 @@ def token_input(x: torch.Tensor, gate: torch.Tensor, proj: torch.Tensor, tokens:
     if x.is_cuda and _plain(x, gate) and _dense(x, gate) and type(proj) in _PLAIN_TYPES and proj.dtype is _BF16 and proj.shape == (W, dim) and \
             proj.is_contiguous() and proj.device == x.device and not (proj.requires_grad and torch.is_grad_enabled()) and table.dtype is _BF16 and \
             table.stride(1) == 1 and (table.stride(0) | column0) % 4 == 0 and proj.data_ptr() % 16 == 0 and table.data_ptr() % 8 == 0:
-        parts = lib.ed_token_input_parts(T, W, dim)
-        if parts > 0:
+        if lib.ed_token_input_pays(T, W, dim) == 1:
+            parts = lib.ed_token_input_parts(T, W, dim)
             sums, out = torch.empty(parts, T, dim, dtype=torch.float32, device=x.device), torch.empty_like(x)
             code = lib.ed_token_input(x.data_ptr(), gate.data_ptr(), proj.data_ptr(), tokens.data_ptr(), table.data_ptr(), table.stride(0), column0,
                                       sums.data_ptr(), parts, out.data_ptr(), T, W, dim, _lib.current_stream(x.device))

@@ -92,11 +92,12 @@ int ed_token_gate(const void* x, const void* gate, const int32_t* tokens, const 
 /*
  * proj (gelu_tanh(gate x) * table[tokens, column0 : column0 + dim]) in bf16, x [T, W], gate [dim, W], proj [W, dim], out [T, W]: the token
  * gate and the projection behind it.  parts: room for [n_parts, T, dim] float32 partial sums of the gate product;
- * ed_token_input_parts: how many to ask for, 0: sizes that it does not take (W % 64, dim of 32, 64 and 128) or that are faster one by one;
- * any number up to W / 32 for at most 64 tokens, up to W / 64 and 64 for more, is taken.
+ * ed_token_input_parts: how many to ask for, 0: sizes that it does not take (W % 64, dim of 32, 64 and 128; 513 to 1279 tokens of at most
+ * 2048 columns); any number up to W / 32 for at most 64 tokens, up to W / 64 and 64 for more, is taken.  _pays: where it is faster than the two.
  * column0 and table_stride are multiples of four.
  */
 int ed_token_input_parts(int64_t T, int W, int dim);
+int ed_token_input_pays(int64_t T, int W, int dim);
 int ed_token_input(const void* x, const void* gate, const void* proj, const int32_t* tokens, const void* table, int64_t table_stride,
                    int column0, float* parts, int n_parts, void* out, int64_t T, int W, int dim, void* stream);
 
