@@ -1076,8 +1076,9 @@ int launch_step(const RecurProblem& p, hipStream_t s) {
     const int cgs = p.vdim / VEC;
     // A workgroup that has a CU to itself is shorter with twice the waves and half the rows to each; more of them get in each other's way (us, 256 /
     // 512 threads: delta rule of 16 heads of 128 x 128, one sequence 9.2 / 8.3, 8 10.3 / 9.4, 16 11.8 / 11.4, 64 26.5 / 29.6; 64 heads of 128 x 64, one
-    // 6.4 / 6.2, 4 7.2 / 6.8, 16 13.5 / 16.7; 1024 threads are slower everywhere).
-    int threads = static_cast<int64_t>(p.heads) * p.n_seqs <= 256 ? 512 : 256;
+    // 6.4 / 6.2, 4 7.2 / 6.8, 16 13.5 / 16.7; 1024 threads are slower everywhere), and so does a small state, whose sums over the waves are what it
+    // takes (8 heads of 32 x 32, delta rule 7.2 / 8.0, of 64 x 64 7.2 / 7.5, 80 x 80 7.6 / 7.5; additive 32 x 32 5.0 / 5.4, 48 x 5 8.4 / 9.1).
+    int threads = static_cast<int64_t>(p.heads) * p.n_seqs <= 256 && p.dim * p.vdim >= 6400 ? 512 : 256;
     while (threads < 1024 && (threads / cgs == 0 || ceil_div(p.dim, threads / cgs) > ROWS)) threads *= 2;
     const size_t lds = sizeof(float) * (static_cast<size_t>(threads / cgs) * p.vdim + p.vdim + 2 * p.dim);
     launch((recur_step_kernel<Elem, DELTA, VEC, ROWS>), dim3(static_cast<unsigned>(p.heads), static_cast<unsigned>(p.n_seqs)),
