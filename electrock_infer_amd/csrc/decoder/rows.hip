@@ -1,5 +1,7 @@
 // Row kernels of a decoder whose residual stream is float32: embedding, post-norm residual update fused with the next
 // layer's pre-norm, squared ReLU, gated SiLU, and the gated norm of a mixer's output.
+#include <algorithm>
+
 #include "decoder.h"
 
 namespace em {
@@ -328,7 +330,7 @@ __global__ __launch_bounds__(THREADS) void gated_norm_kernel(typename Elem::stor
 }
 
 // Place of the largest value of a row, the first one where several are equal; a NaN is larger than every number.  One
-// workgroup per row, eight vectors of it requested at once: 32000 columns take a way to memory and a pass over 32
+// workgroup per row, up to AHEAD vectors to a thread requested at once: 32000 columns take a way to memory and a pass over 32
 // values a thread: the maximum of a piece first, two values to an instruction, its first place only where it brings anything, and over the
 // wave without LDS (us: one row 7.8 -> 5.1, 64 rows 8.7 -> 5.9, 128256 columns 22.7 -> 14.1; the library 10.7 and 11.3 for 32000).
 constexpr int kArgmaxThreads = 1024;
@@ -363,24 +365,24 @@ __device__ __forceinline__ int wave_argmax(float& value, int place) {
     value = most;
     return place;
 }
-template <int VEC>
+template <int VEC, int AHEAD>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const float* __restrict__ x, int V, int32_t* __restrict__ out) {
-    constexpr int kAhead = 8, kWaves = kArgmaxThreads / kWave;
-    __shared__ float best_v[kWaves];
-    __shared__ int best_i[kWaves];
+    __shared__ float best_v[kArgmaxThreads / kWave];
+    __shared__ int best_i[kArgmaxThreads / kWave];
+    const int step = static_cast<int>(blockDim.x) * VEC, waves = static_cast<int>(blockDim.x) / kWave;
     const float* row = x + static_cast<int64_t>(blockIdx.x) * V;
     float value = -INFINITY;
     int place = V;
-    for (int c0 = threadIdx.x * VEC; c0 < V; c0 += kAhead * kArgmaxThreads * VEC) {
-        float v[kAhead][VEC], most = -INFINITY;
+    for (int c0 = threadIdx.x * VEC; c0 < V; c0 += AHEAD * step) {
+        float v[AHEAD][VEC], most = -INFINITY;
         bool nan = false;
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i) RowIo<F32Elem, VEC>::load(row + min(c0 + i * kArgmaxThreads * VEC, V - VEC), v[i]);
+        for (int i = 0; i < AHEAD; ++i) RowIo<F32Elem, VEC>::load(row + min(c0 + i * step, V - VEC), v[i]);
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i)
+        for (int i = 0; i < AHEAD; ++i)
 #pragma unroll
             for (int j = 0; j < VEC; ++j) {
-                if (c0 + i * kArgmaxThreads * VEC >= V) v[i][j] = -INFINITY;      // (V is a multiple of VEC)
+                if (c0 + i * step >= V) v[i][j] = -INFINITY;      // (V is a multiple of VEC)
                 most = fmaxf(most, v[i][j]);
                 nan = nan || v[i][j] != v[i][j];
             }
@@ -388,10 +390,10 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const float* __r
         const bool seek = value == value && (nan || most > value || place == V);
         if (!seek) continue;
 #pragma unroll
-        for (int i = kAhead - 1; i >= 0; --i)
+        for (int i = AHEAD - 1; i >= 0; --i)
 #pragma unroll
             for (int j = VEC - 1; j >= 0; --j)
-                if (nan ? v[i][j] != v[i][j] : v[i][j] == most) place = c0 + i * kArgmaxThreads * VEC + j;
+                if (nan ? v[i][j] != v[i][j] : v[i][j] == most) place = c0 + i * step + j;
         value = nan ? NAN : most;
     }
     place = wave_argmax(value, place);
@@ -401,8 +403,8 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const float* __r
     }
     __syncthreads();
     if (threadIdx.x >= kWave) return;
-    value = best_v[threadIdx.x % kWaves];
-    place = wave_argmax(value, best_i[threadIdx.x % kWaves]);
+    value = best_v[threadIdx.x % waves];
+    place = wave_argmax(value, best_i[threadIdx.x % waves]);
     if (threadIdx.x == 0) out[blockIdx.x] = place;
 }
 
@@ -531,10 +533,17 @@ int launch_silu_gate(const void* u, void* out, int64_t T, int ff, int dtype, hip
     return launch_status();
 }
 
+// No more vectors to a thread than a row has for it: a pass over places that are not there takes as long as one over others (us, eight to a thread
+// / as here: one row of 1000 3.8 / 2.3, 5000 5.3 / 3.0, 16384 5.3 / 3.8; 1000 rows of 1000 11.7 / 3.2, 4096 18.2 / 5.4, 8192 18.2 / 6.6); where rows
+// fill the chip the next workgroup hides a row's way (256 of 32000 7.1 / 6.9, of 128256 24.8 / 22.0, 1000 of 32000 27.3 / 21.7).
 int launch_argmax(const float* x, int64_t T, int V, int32_t* out, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(T)), block(kArgmaxThreads);
-    if (V % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0) launch((argmax_kernel<4>), grid, block, 0, s, x, V, out);
-    else launch((argmax_kernel<1>), grid, block, 0, s, x, V, out);
+    const bool vec = V % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    const dim3 grid(static_cast<unsigned>(T)), block(vec ? static_cast<unsigned>(std::min<int64_t>(kArgmaxThreads, round_up(V / 4, kWave))) : kArgmaxThreads);
+    if (!vec) launch((argmax_kernel<1, 8>), grid, block, 0, s, x, V, out);
+    else if (V <= 4 * kArgmaxThreads) launch((argmax_kernel<4, 1>), grid, block, 0, s, x, V, out);
+    else if (V <= 8 * kArgmaxThreads) launch((argmax_kernel<4, 2>), grid, block, 0, s, x, V, out);
+    else if (V <= 16 * kArgmaxThreads || T >= 256) launch((argmax_kernel<4, 4>), grid, block, 0, s, x, V, out);
+    else launch((argmax_kernel<4, 8>), grid, block, 0, s, x, V, out);
     return launch_status();
 }
 
