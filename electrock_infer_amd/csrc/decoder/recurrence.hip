@@ -993,8 +993,9 @@ int launch_conv(const RecurProblem& p, hipStream_t s) {
     auto aligned = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % (4 * sizeof(typename Elem::storage)) == 0; };
     const bool vec = p.dim % 4 == 0 && p.vdim % 4 == 0 && p.stride % 4 == 0 && aligned(p.q) && aligned(p.k) && aligned(p.v);
     // Where the waves of 16 tokens are few, four of them: the way of one token's channels is what a short prompt waits for, and the rows read
-    // twice lie in L2 (us, 16 / 4 tokens a wave, heads of 128: 320 tokens 10.0 / 6.3, 1024 10.4 / 9.6, 3200 19.3 / 18.6, 8192 35.9 / 38.4).
-    const bool few = int64_t{p.n_chunks} * (p.chunk_tokens / kBlock) * units(kBlock) <= 8192;
+    // twice lie in L2 (us, 16 / 4 tokens a wave, heads of 128: 320 tokens 10.0 / 6.3, 1024 10.4 / 9.6, 3200 19.3 / 18.6, 8192 35.9 / 38.4; the whole
+    // prefill of 24 heads of 64 x 64, 3505 tokens, 3066 waves of 16, 80.2 / 74.9, 7500, 6566, 114.6 / 117.8, 16 x 512, 7168, 97.7 / 101.3).
+    const bool few = int64_t{p.n_chunks} * (p.chunk_tokens / kBlock) * units(kBlock) <= 6144;
     if (p.taps > 4) launch((recur_conv_kernel<Elem, kMaxTaps, false, kBlock>), grid(kBlock), dim3(256), 0, s, p, head_lanes);
     else if (vec && few) launch((recur_conv_kernel<Elem, 4, true, 4>), grid(4), dim3(256), 0, s, p, head_lanes);
     else if (vec) launch((recur_conv_kernel<Elem, 4, true, kBlock>), grid(kBlock), dim3(256), 0, s, p, head_lanes);
