@@ -855,13 +855,20 @@ int attn_splits(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int
     return best;
 }
 
-// The layer's choice: a context that is not split has eight waves where it has a CU to itself, and that is the faster way from 160 workgroups
-// on, and from 112 behind short contexts (us, 16 heads on 4, ones / the best split: 64 x 4000 keys 90.3 / 94.9, 48 x 1023 24.1 / 27.3, 48 x 4000 72.2 /
-// 74.9; 32 x 500 13.6 / 14.6, 32 x 1023 20.9 / 20.8, 32 x 4000 60.0 / 54.3; 24 x 1023 20.2 / 19.6, 24 x 4000 57.7 / 45.5).
+// The layer's choice: a context that is not split has eight waves where it has a CU to itself.  us, one range / the split's choice, 16 heads on 4 of
+// 128, equal contexts, the same ones behind a plan for twice their keys, and one as long as the plan among others of 1000, which one range
+// walks through alone:
+//     192 workgroups  1023 keys 24.5 / 29.3;  4096 73.3 / 79.3, 41.1 / 46.1, 55.0 / 53.5;  16000 264 / 276, 139 / 148, 184 / 176
+//     (33 sequences and 15 rows of padding 1000 keys 21.2 / 25.4, 8000 113 / 118);  256  4096 91.6 / 95.9, 59.5 / 63.9
+//     176  2048 38.9 / 44.5;  4096 68.9 / 90.0, 39.1 / 52.2, 54.9 / 43.5;  8192 130 / 134, 69.4 / 74.4, 99 / 62
+//     160  2048 36.9 / 43.2, 22.9 / 28.1, 32.0 / 33.3;  4096 65.9 / 65.0, 36.9 / 39.6, 54.5 / 43.0;  16384 243 / 222, 124 / 118, 190 / 127;  heads of
+//     64  2048 24.6 / 27.9;  4096 43.8 / 36.9;  8192 82.4 / 69.5
+//     128  1536 28.1 / 29.5;  2048 34.9 / 33.1;  112  500 13.7 / 15.2, 1023 21.0 / 20.8, 1536 27.3 / 25.4, half of a plan for 1024 13.9 / 16.4
+// So: from 176 workgroups on, up to the contexts that this was measured at; from 160 and from 112 behind short ones.
 int attn_ranges(int dtype, int heads, int kv_heads, int dim, int64_t n_seqs, int64_t max_q, int64_t keys) {
     const int64_t groups = n_seqs * kv_heads;
     const bool many = dtype == EM_DTYPE_BF16 && dim <= 128 && max_q * (heads / kv_heads) <= 16 && groups <= 256;
-    if (many && (groups >= 160 || (groups >= 112 && keys <= 1536))) return 1;
+    if (many && ((groups >= 176 && keys <= 16384) || (groups >= 160 && keys <= 2048) || (groups >= 112 && keys <= 1536))) return 1;
     return attn_splits(dtype, heads, kv_heads, dim, n_seqs, max_q, keys);
 }
 
