@@ -488,8 +488,7 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
 //     rows are read from LDS in front of the barrier; loads have no condition of their own (keys behind the last stand for it).
 // One prompt of 8192 tokens, 16 heads of 128, cap 30: 427 -> 386 us, window 1024: 119.5 -> 112.6; scores beyond the range
 // 422 -> 401, no cap 386 -> 368; 8 x 1000 tokens, heads of 64: 63.4 -> 60.3; heads of 256 / 64: 249 -> 228, 256 / 128
-// 644 -> 608.  Two tiles in LDS with one barrier a tile were no faster (394 us, 114).  Capped portions of up to 500 tokens with heads of up
-// to 64, whose few tiles do not pay for the second form of the scores, are 1 to 4 % slower (1 x 173 8.5 -> 8.7).
+// 644 -> 608.  Two tiles in LDS with one barrier a tile were no faster (394 us, 114).
 constexpr float kTanhRange = 0.6f;
 constexpr int kTileKeys = 64;
 
@@ -798,11 +797,14 @@ int launch_queries(const AttnProblem& p, int n_seqs, int max_q, hipStream_t s) {
 }
 
 // 64 queries to a workgroup where 128 leave CUs without work: half the products, exponentials and sums to a tile, whose chain a wave
-// waits for (us, 128 / 64 queries, 16 heads of 128, cap 30, workgroups of 64: 80, 300 tokens behind 500 31.3 / 24.1; 16, 64 behind 1000 38.3 /
-// 29.2; 256, one prompt of 1000 37.7 / 29.1; 512, 2048 70.3 / 57.0, 8 x 256 behind 1000 53.5 / 49.7, 16 x 128 9.8 / 9.7; heads of 256 / 128, whose
-// 128 queries spill: 256, 66.3 / 34.3; beyond, 640, 10 x 256 behind 1000 65.8 / 72.0; 768, 24 x 128 14.3 / 16.0).  Portions from the start of long
-// prompts, whose first queries see few keys and leave their CUs early, gain beyond that (768, 3 x 1000 51.0 / 40.8, 2 x 1536 58.4 / 50.8, 752,
-// 3000 105 / 83; 1024, 4096 143 / 142, 4 x 1000 51.2 / 55.3, 4096 with a window of 1024 59.5 / 73.5).
+// waits for (us, 128 / 64 queries, 16 heads of 128, cap 30, workgroups of 64: 80, 300 tokens behind 500 31.0 / 23.7; 16, 64 behind 1000 38.8 /
+// 29.3; 256, one prompt of 1000 37.2 / 28.7; 512, 2048 69.7 / 56.3, 8 x 256 behind 1000 49.8 / 46.1, 16 x 128 9.9 / 9.8; heads of 64, 512, 2048 54.3 /
+// 42.3, 8 x 256 behind 1000 39.0 / 32.7; of 256 / 128, whose 128 queries spill: 256, 64.7 / 35.2).  Beyond two to a CU every workgroup pays for the
+// keys that it brings in for itself: 576, 9 x 256 behind 1000 62.9 / 68.5; 528, 3 x 700 behind 4000 192 / 215; 768, 12 x 256 18.9 / 21.2; 832, 4 x 800
+// 36.4 / 40.8.  Portions from the start of long prompts gain beyond that, as their first queries see few keys and leave their CUs early, up to 800
+// (720, 3 x 960 47.7 / 36.4; 768, 3 x 1000 50.8 / 40.9, 2 x 1536 59.1 / 49.7; 800, 3200 111.8 / 86.7, behind 800 141 / 135, behind 3200 224 / 280; with
+// a window that all but the first fill: 768, 2 x 1536 of 512 35.1 / 40.9).  The lines lie where both sides were measured and not at the crossing:
+// shorter ones that would gain too (720, 3 x 900 46.6 / 35.4; 560, 5 x 448 25.2 / 17.4) stay with 128, and 880, 3500 123 / 105.
 bool few_queries(const AttnProblem& p, int n_seqs, int max_q) {
     const int64_t groups = ceil_div(max_q, 64) * p.heads * n_seqs, context = static_cast<int64_t>(p.table_width) * p.block_size;
     return groups <= 512 || (groups <= 800 && max_q >= 960 && context <= max_q + max_q / 4 && (p.window <= 0 || p.window >= max_q));
