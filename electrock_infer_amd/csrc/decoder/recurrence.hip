@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void recur_block_kernel(RecurProblem p, int he
         }
         if (!DELTA) continue;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        // column l16 of the inverse of the unit lower triangular matrix, row by row (each quarter of the wave on its own)
+        // column l16 of the inverse of the unit lower triangular matrix, row by row (each few of the wave on its own)
         float inv[kBlock];
 #pragma unroll
         for (int t = 0; t < kBlock; ++t) {
@@ -408,7 +408,7 @@ __device__ __forceinline__ bool chunk_pass(const RecurProblem& p, int group, int
     const float* rec0 = p.blocks + (static_cast<int64_t>(block.x) * (p.chunk_tokens / kBlock) * p.heads + h) * recur_record(DELTA);
 
     // Column `col` of the state, rows lq * D / 4 + dt * 4 + r: two tiles are eight rows of a lane that lie side by side, as a
-    // product over the state takes them, and the pieces of a key that one tile takes lie a quarter of its row apart (so that they,
+    // product over the state takes them, and the pieces of a key that one tile takes lie a few of its row apart (so that they,
     // and 16 rows of either operand, fall on different banks).  !kParts: a tile's 16 rows side by side.
     f32x4_t st[NDT];
     auto row_of = [&](int dt) { return kParts ? lq * (D / 4) + dt * 4 : dt * 16 + lq * 4; };
@@ -847,20 +847,21 @@ __global__ __launch_bounds__(NDT * kWave) void recur_matrix_scan_kernel(RecurPro
 }
 
 // ---- decoding: one new token per sequence ----
-// A thread holds VEC columns of up to ROWS rows of the state.  Bound: the states' bytes, read and written once a step, past the caches' order of
+// A thread holds VEC columns of up to ROWS rows of the state, and sums of every SHARESth of them (2: in the order of twice the threads, so
+// that a sequence's sums are the same whatever the launch).  Bound: the states' bytes, read and written once a step, past the caches' order of
 // use (us, loads and stores in it / past it: 64 sequences of 64 heads of 128 x 64, 268 MB, 62.5 / 51.2, 8 of them 11.3 / 8.9, 128 112 / 97; the delta
 // rule, 16 heads of 128 x 128, 23 sequences 15.2 / 13.1, 64 27.3 / 26.3, 128 71 / 52; a single sequence is the same; either alone gives a third).
 // Asking for a thread's channels and taps together, beside the state or in front of it, spills (one sequence of the delta rule 9.2 / 9.8-10.3).
-template <typename Elem, bool DELTA, int VEC, int ROWS>
-__global__ __launch_bounds__(1024) void recur_step_kernel(RecurProblem p) {
+template <typename Elem, bool DELTA, int VEC, int ROWS, int SHARES>
+__global__ __launch_bounds__(1024) void recur_step_kernel(RecurProblem p, int groups) {
     typedef typename Elem::storage S;
     typedef float vec_t __attribute__((ext_vector_type(VEC)));
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ float red[2][16];
     const int dim = p.dim, vdim = p.vdim, threads = blockDim.x, waves = threads / kWave;
-    const int cgs = vdim / VEC, groups = threads / cgs;
-    float* lo = lds;                           // [groups][vdim]
-    float* lv = lo + groups * vdim;            // [vdim]
+    const int cgs = vdim / VEC, sums = groups * SHARES;     // groups <= threads / cgs
+    float* lo = lds;                           // [sums][vdim]
+    float* lv = lo + sums * vdim;              // [vdim]
     float* lqv = lv + vdim;                    // [dim] q
     float* lk = lqv + dim;                     // [dim] k
     const int tid = threadIdx.x, h = blockIdx.x, s = blockIdx.y, share = p.heads / p.kv_heads, g = h / share;
@@ -928,40 +929,50 @@ __global__ __launch_bounds__(1024) void recur_step_kernel(RecurProblem p) {
         for (int j = 0; j < VEC; ++j) u_new[j] = lv[c + j];
     }
     if (DELTA) {
-        vec_t sk = static_cast<vec_t>(0.0f);
+        vec_t sk[SHARES];
+#pragma unroll
+        for (int i = 0; i < SHARES; ++i) sk[i] = static_cast<vec_t>(0.0f);
 #pragma unroll
         for (int u = 0; u < ROWS; ++u) {
             const int d = grp + u * groups;
             if (grp < groups && d < dim) {
                 x[u] *= decay;
-                sk += x[u] * (lk[d] * k_scale);
+                sk[u % SHARES] += x[u] * (lk[d] * k_scale);
             }
         }
-        if (grp < groups) *reinterpret_cast<vec_t*>(lo + grp * vdim + c) = sk;
+        if (grp < groups) {
+#pragma unroll
+            for (int i = 0; i < SHARES; ++i) *reinterpret_cast<vec_t*>(lo + (grp + i * groups) * vdim + c) = sk[i];
+        }
         __syncthreads();
         if (grp < groups) {
-            for (int w = 0; w < groups; ++w) u_new -= *reinterpret_cast<const vec_t*>(lo + w * vdim + c);
+            for (int w = 0; w < sums; ++w) u_new -= *reinterpret_cast<const vec_t*>(lo + w * vdim + c);
         }
         __syncthreads();
     }
     u_new *= beta;
-    vec_t o = static_cast<vec_t>(0.0f);
+    vec_t o[SHARES];
+#pragma unroll
+    for (int i = 0; i < SHARES; ++i) o[i] = static_cast<vec_t>(0.0f);
 #pragma unroll
     for (int u = 0; u < ROWS; ++u) {
         const int d = grp + u * groups;
         if (grp < groups && d < dim) {
             if (!DELTA) x[u] *= decay;
             x[u] += u_new * (lk[d] * k_scale);
-            o += x[u] * (lqv[d] * q_scale);
+            o[u % SHARES] += x[u] * (lqv[d] * q_scale);
             __builtin_nontemporal_store(x[u], reinterpret_cast<vec_t*>(st + d * vdim + c));
         }
     }
-    if (grp < groups) *reinterpret_cast<vec_t*>(lo + grp * vdim + c) = o;
+    if (grp < groups) {
+#pragma unroll
+        for (int i = 0; i < SHARES; ++i) *reinterpret_cast<vec_t*>(lo + (grp + i * groups) * vdim + c) = o[i];
+    }
     __syncthreads();
     float sum = 0.0f;
     for (int v = tid; v < vdim; v += threads) {
         float y = p.skip != nullptr ? p.skip[h] * lv[v] : 0.0f;
-        for (int w = 0; w < groups; ++w) y += lo[w * vdim + v];
+        for (int w = 0; w < sums; ++w) y += lo[w * vdim + v];
         lo[v] = y;                              // (column v is this thread's alone)
         sum = fmaf(y, y, sum);
     }
@@ -1079,11 +1090,18 @@ int launch_step(const RecurProblem& p, hipStream_t s) {
     // 512 threads: delta rule of 16 heads of 128 x 128, one sequence 9.2 / 8.3, 8 10.3 / 9.4, 16 11.8 / 11.4, 64 26.5 / 29.6; 64 heads of 128 x 64, one
     // 6.4 / 6.2, 4 7.2 / 6.8, 16 13.5 / 16.7; 1024 threads are slower everywhere), and so does a small state, whose sums over the waves are what it
     // takes (8 heads of 32 x 32, delta rule 7.2 / 8.0, of 64 x 64 7.2 / 7.5, 80 x 80 7.6 / 7.5; additive 32 x 32 5.0 / 5.4, 48 x 5 8.4 / 9.1).
-    int threads = static_cast<int64_t>(p.heads) * p.n_seqs <= 256 && p.dim * p.vdim >= 6400 ? 512 : 256;
-    while (threads < 1024 && (threads / cgs == 0 || ceil_div(p.dim, threads / cgs) > ROWS)) threads *= 2;
-    const size_t lds = sizeof(float) * (static_cast<size_t>(threads / cgs) * p.vdim + p.vdim + 2 * p.dim);
-    launch((recur_step_kernel<Elem, DELTA, VEC, ROWS>), dim3(static_cast<unsigned>(p.heads), static_cast<unsigned>(p.n_seqs)),
-           dim3(static_cast<unsigned>(threads)), lds, s, p);
+    // Sums are taken in one order either way, so a sequence's state does not depend on how many others decode beside it: two sums to a thread cost
+    // nothing but for the delta rule with values of 64 (64 heads, 16 sequences 16.3 / 16.9, 64 61.2 / 60.6).
+    const int few = 256 / cgs;                               // groups of rows that 256 threads make
+    const bool enough = few > 0 && ceil_div(p.dim, few) <= ROWS, large = p.dim * p.vdim >= 6400;
+    const bool twice = enough && large && static_cast<int64_t>(p.heads) * p.n_seqs <= 256;
+    int threads = enough && !twice ? 256 : 512;
+    while (!enough && threads < 1024 && (threads / cgs == 0 || ceil_div(p.dim, threads / cgs) > ROWS)) threads *= 2;
+    const int groups = !enough ? threads / cgs : twice ? 2 * few : few, shares = enough && large && !twice ? 2 : 1;
+    const size_t lds = sizeof(float) * (static_cast<size_t>(groups) * shares * p.vdim + p.vdim + 2 * p.dim);
+    const dim3 grid(static_cast<unsigned>(p.heads), static_cast<unsigned>(p.n_seqs)), block(static_cast<unsigned>(threads));
+    if (shares == 2) launch((recur_step_kernel<Elem, DELTA, VEC, ROWS, 2>), grid, block, lds, s, p, groups);
+    else launch((recur_step_kernel<Elem, DELTA, VEC, ROWS, 1>), grid, block, lds, s, p, groups);
     return launch_status();
 }
 

@@ -1,4 +1,4 @@
-"""A decoding step of a recurrence with a small state: the same bits for a sequence alone and beside others, as its workgroups are the same."""
+"""A decoding step of a recurrence: the same bits for a sequence alone and beside others, though few heads have wider workgroups."""
 from ctypes import byref
 
 import pytest
@@ -11,8 +11,11 @@ BF16 = torch.bfloat16
 
 
 @pytest.mark.parametrize("delta", [False, True])
-@pytest.mark.parametrize("H,G,dim,vdim,n", [(129, 3, 20, 12, 2), (130, 2, 48, 5, 2), (64, 8, 64, 64, 5), (8, 8, 32, 32, 40)])
-def test_small_states(delta, H, G, dim, vdim, n):
+# small states, whose workgroups are the same; large ones in every form: rows that twice the threads do not share evenly, columns one by one, a
+# state that takes twice the threads in any case
+@pytest.mark.parametrize("H,G,dim,vdim,n", [(129, 3, 20, 12, 2), (130, 2, 48, 5, 2), (64, 8, 64, 64, 5), (8, 8, 32, 32, 40), (40, 8, 128, 128, 7), (64, 1, 128, 64, 5),
+                                            (100, 4, 100, 72, 3), (100, 4, 96, 75, 3), (100, 4, 256, 64, 3), (90, 3, 80, 80, 3)])
+def test_alone_and_beside_others(delta, H, G, dim, vdim, n):
     g = torch.Generator(device="cuda").manual_seed(H + dim + delta)
     rand = lambda *s: torch.randn(*s, device="cuda", generator=g) * 0.5
     ch = 2 * G * dim + H * vdim
