@@ -67,17 +67,17 @@ def _fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return _plain(x, weight) and x.shape[0] <= 64 and _dense(x, weight)
 
 
-def _tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Operands of the tiled kernel beyond a decode batch: any rows from 16-byte boundaries."""
-    return x.is_cuda and _plain(x, weight) and x.shape[0] > 64 and _pitch(x, x.shape[1]) > 0 and _pitch(weight, x.shape[1]) > 0
-
-
 def _taken(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Either of the two, asked once."""
+    """Operands of either kernel, asked once: those of a decode batch, and beyond one any rows from 16-byte boundaries."""
     if not x.is_cuda or not _plain(x, weight):
         return False
     T, K = x.shape
     return _dense(x, weight) if T <= 64 else _pitch(x, K) > 0 and _pitch(weight, K) > 0
+
+
+def _tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Operands of the tiled kernel beyond a decode batch."""
+    return _taken(x, weight) and x.shape[0] > 64
 
 
 def _decode_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, splits: int, cols: int, act: int) -> torch.Tensor:
@@ -162,7 +162,8 @@ def normed_rows(x: torch.Tensor, y: torch.Tensor, post_w: torch.Tensor, eps: flo
     """``residual_norm(ADD_NORMED, ...)`` for rows that ``reader`` reads next: ``out``, or for a row or two ``NormedRows``, where it is a layer
     of this package that hands them to one product and nobody watches what it is given."""
     T, K = out.shape
-    if T <= 2 and reader is not None and _takes_rows(reader) and _takes_rows(getattr(reader, "in_proj", reader)) and _unwatched(reader) and x.is_cuda and x.is_contiguous() and y.is_contiguous() and out.is_contiguous() and out.dtype is _BF16 and \
+    if T <= 2 and reader is not None and _takes_rows(reader) and _takes_rows(getattr(reader, "in_proj", reader)) and _unwatched(reader) and \
+            x.is_cuda and x.is_contiguous() and y.is_contiguous() and out.is_contiguous() and out.dtype is _BF16 and \
             (y.dtype is _BF16 and y.dim() == 2 or y.dtype is torch.float32) and (x.data_ptr() | y.data_ptr()) % 16 == 0 and \
             _lib.load_decoder().ed_norm_gemm_supported(T, 1, K, 0) == 1:
         return NormedRows(x, y, post_w, next_w, eps, out, torch.empty_like(x))
